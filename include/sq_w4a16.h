@@ -54,6 +54,9 @@ extern "C" {
                                   * distance ahead of the arithmetic, activations staged in LDS first; K beyond 4096
                                   * is split through the workspace */
 
+#define SQ_ALGO_RING 7           /* any M: 32 .. 128-row tiles, eight waves in two alternating groups, K split inside
+                                  * the workgroup (and over workgroups through the workspace) */
+
 /* Library version (major*10000 + minor*100 + patch). */
 int sq_version(void);
 

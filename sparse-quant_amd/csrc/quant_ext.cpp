@@ -120,7 +120,7 @@ std::pair<at::Tensor, at::Tensor> l1_view_of_l2(const at::Tensor& W, const at::T
     return {w1, zs1};
 }
 
-// Workspace of the split-K kernels (5..1024 tokens): one zero-initialised buffer per
+// Workspace of the kernels that split K over workgroups (3..1024 tokens): one zero-initialised buffer per
 // (device, stream), grown on demand and kept for the life of the process.  Calls on one
 // stream are ordered, which is what sharing a workspace requires.  Under HIP graph capture
 // the buffer must already exist (run the call once on the capturing stream beforehand).
@@ -210,7 +210,8 @@ at::Tensor gemm_impl(const at::Tensor& I, const at::Tensor& W, const at::Tensor&
     void* ws_ptr = nullptr;
     size_t ws_bytes = 0;
     at::Tensor ws;
-    if (M > 2 && M <= 1024 && ((algo & 0xFF) == SQ_ALGO_AUTO || (algo & 0xFF) == SQ_ALGO_SKINNY_WS || (algo & 0xFF) == SQ_ALGO_STREAM)) {
+    if (M > 2 && M <= 1024 && ((algo & 0xFF) == SQ_ALGO_AUTO || (algo & 0xFF) == SQ_ALGO_SKINNY_WS || (algo & 0xFF) == SQ_ALGO_STREAM ||
+        (algo & 0xFF) == SQ_ALGO_RING)) {
         ws = workspace_for(I, stream, sq_w4a16_workspace_bytes((int)M, N, (int)K));
         ws_ptr = ws.data_ptr();
         ws_bytes = (size_t)ws.numel();

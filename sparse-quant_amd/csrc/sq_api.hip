@@ -92,21 +92,17 @@ int tuned_lookup(int M, int N, int K, int g, bool has_ws) {
 enum : unsigned {
     P_LARGE = 1u << 0,      // N * K >= 2^25 elements (fc1 / fc2 class)
     P_WS = 1u << 1,         // a workspace for the decode kernels' K split is at hand
-    P_GEMM_WS = 1u << 2,    // a workspace for the tiled GEMM's K split is at hand
-    P_G128 = 1u << 3,       // group size 128
-    P_G128_64 = 1u << 4,    // group size 128 or 64
-    P_K128 = 1u << 5,       // K a multiple of 128
-    P_K256 = 1u << 6,       // K a multiple of 256
-    P_K_LE_4096 = 1u << 7,
-    P_K_LE_8192 = 1u << 8,
-    P_K_LE_32768 = 1u << 9,
-    P_WIDE = 1u << 10,      // the two-tile streaming kernel applies and its workgroups come in one round or fill their rounds
-    P_SMALL = 1u << 11,     // N * K <= 2^22 elements and K <= 2048
-    P_N_GE_8192 = 1u << 12, // 32 or more 256-column tiles: a K split of up to 8 gives every CU a workgroup of the tiled GEMM
-    P_K_LE_1536 = 1u << 13,
-    P_CHUNK_FILL = 1u << 14,  // the least K split of the streaming kernel fills 3/4 or more of a workgroup's 32 chunks
+    P_G128_64 = 1u << 2,    // group size 128 or 64
+    P_K128 = 1u << 3,       // K a multiple of 128
+    P_K_LE_4096 = 1u << 4,
+    P_K_LE_8192 = 1u << 5,
+    P_K_LE_32768 = 1u << 6,
+    P_SMALL = 1u << 7,        // N * K <= 2^22 elements and K <= 1536
+    P_OVER_16M = 1u << 8,     // N * K > 2^24 elements
+    P_CHUNK_FILL = 1u << 9,   // the least K split of the streaming kernel fills 3/4 or more of a workgroup's 32 chunks
+    P_RING = 1u << 10,        // the ring kernel can address the operands
+    P_SHORT_ROUNDS = 1u << 11,  // many rounds of 128 x 256 tiles over a short K (see builtin_choice)
 };
-constexpr int ALGO_TWO_BLOCKS = 100;  // internal: the split-K decode kernel on two blocks of up to 32 tokens
 struct ChoiceRule {
     int m_lo, m_hi;
     unsigned need, forbid;
@@ -114,6 +110,11 @@ struct ChoiceRule {
     const char* measured;
 };
 const ChoiceRule kChoiceRules[] = {
+    // 5..16 tokens where a K range of the streaming kernel would leave its chunk slots part empty, and at group size 32
+    {5, 16, P_LARGE | P_G128_64 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
+     "8 / 16 tokens: 15360x5120 13.9 vs 16.0 / 19.0 (streaming kernel), 13696x5120 13.4 vs 15.7 / 19.3"},
+    {5, 16, P_OVER_16M | P_RING, P_G128_64, SQ_ALGO_RING,
+     "16 tokens, group size 32: 5120x5120 10.3 vs 19.2, 12288x4096 12.2 vs 15.4, 4096x11008 13.0 vs 15.4; 4096x4096 8.6 vs 8.4"},
     // the streaming decode kernel, 5..16 tokens (3..4 on large weights); K beyond 4096 is split through the workspace
     {5, 16, P_G128_64 | P_K128 | P_K_LE_4096, 0, SQ_ALGO_STREAM,
      "8 tokens: fc1 10.0 vs 13.3 (split-K kernel), q/k/v in one launch 8.6 vs 12.1, 4096x4096 4.9 vs 6.5 (GEMV)"},
@@ -122,57 +123,30 @@ const ChoiceRule kChoiceRules[] = {
     {3, 4, P_LARGE | P_G128_64 | P_K128 | P_WS | P_K_LE_32768 | P_CHUNK_FILL, 0, SQ_ALGO_STREAM,
      "4 tokens: fc2 11.9 vs 13.6 (GEMV); 13824x5120, whose K ranges fill 20 of a workgroup's 32 chunks: 14.6 vs 13.9 (GEMV)"},
     // small weights at 17..32 tokens: the 16-column kernel (one launch, no exchange between workgroups)
-    {17, 32, P_SMALL, 0, SQ_ALGO_SKINNY,
-     "32 tokens: 2048x2048 7.4 vs 8.6 (split-K kernel), 1024x1024 4.9 vs 6.9, 3072x768 4.8 vs 6.6"},
-    // its two-tile variant, 17..32 tokens
-    {17, 32, P_G128 | P_WIDE, 0, SQ_ALGO_STREAM,
-     "32 tokens: fc1 16.5 vs 17.2 (split-K kernel), q/k/v-sized 14.3 vs 15.5, fc2 18.1 vs 19.0"},
-    // large weights whose grid leaves the two-tile kernel's last round part empty or whose K leaves chunk slots of
-    // its workgroups unused: the tiled GEMM's 32-row tiles with K split through the workspace
-    {17, 32, P_LARGE | P_K256 | P_GEMM_WS | P_G128, 0, SQ_ALGO_GEMM,
-     "32 tokens: 13824x5120 20.2 vs 27.7 (two-tile kernel: 1.7 rounds of workgroups at 20 of 32 chunk slots), "
-     "28672x8192 47.2 vs 56.7, 8192x28672 45.6 vs 55.6, 5120x13824 23.3 vs 26.9, 22016x4096 24.3 vs 25.9"},
-    // the same at group size 64 and 32 (no two-tile kernel) on weights with enough columns of tiles; long K on few
-    // rows stays with the split-K kernel below (group size 64, 4096x16384: 19.6 vs 25.2 for the tiled GEMM)
-    {17, 32, P_LARGE | P_K256 | P_GEMM_WS | P_N_GE_8192, 0, SQ_ALGO_GEMM,
-     "32 tokens, group size 64: fc1 18.4, 12288x4096 16.0, 13824x5120 20.7, 28672x8192 53.6: no other kernel faster"},
-    // small weights with a short K at 33..64 tokens: still the 16-column kernel (from K = 2048 on the GEMM wins)
-    {33, 64, P_SMALL | P_K_LE_1536, 0, SQ_ALGO_SKINNY,
-     "48 tokens: 3072x768 5.6 vs 8.6 (tiled GEMM), 4096x1024 6.3 vs 8.6, 1024x1024 5.9 vs 8.1, 1536x1536 7.8 vs 9.9; "
-     "64 tokens: 6.8 vs 8.6, 7.3 vs 8.7, 6.9 vs 8.1, 9.2 vs 10.0; 2048x2048 at 64 tokens 12.0 vs 10.7"},
-    // the tiled GEMM with every operand through LDS and K split through the workspace, beyond 32 tokens
-    {33, 1 << 30, P_K256 | P_GEMM_WS, 0, SQ_ALGO_GEMM,
-     "48 tokens: 4096x4096 14.5 vs 17.2 (two blocks of the split-K kernel), fc1 24.7 vs 28.2, fc2 27.0 vs 32.3; "
-     "64 tokens: 14.5 vs 20.5 (16-column kernel)"},
-    // the split-K decode kernel: where the streaming kernels do not apply (group size 32, K no multiple of 128,
-    // grids that leave the two-tile kernel under half the chip such as 4096x4096 at 17..32 tokens)
-    {5, 32, P_WS | P_LARGE, 0, SQ_ALGO_SKINNY_WS, "16 tokens: fc1 12.5, fc2 14.7 vs 16-column kernel 19.6 / 21.7"},
-    {17, 32, P_WS, 0, SQ_ALGO_SKINNY_WS, "32 tokens: 4096x4096 9.8 vs 10.2 (two-tile kernel at 64 rows x 2048 columns)"},
-    {5, 32, P_WS, P_K_LE_8192, SQ_ALGO_SKINNY_WS, "long K: one workgroup per 16 rows cannot stage the activations in one round"},
-    {33, 48, P_WS | P_LARGE, 0, ALGO_TWO_BLOCKS, "33..48 tokens without the GEMM's workspace: fc1 30 vs 31 (tiled GEMM), fc2 35 vs 37"},
-    {33, 48, P_WS, P_K_LE_8192, ALGO_TWO_BLOCKS, "as above, long K"},
+    {17, 32, P_SMALL, 0, SQ_ALGO_SKINNY, "24 tokens: 3072x1024 4.9 vs 5.2 (ring kernel); 2048x2048 at 32 tokens 7.4 vs 6.8"},
+    // everything else from 17 tokens up
+    {17, 1 << 30, P_RING, P_SHORT_ROUNDS, SQ_ALGO_RING,
+     "see sq_gemm_ring.hip: 1.25x at 24..32 tokens, 1.4x at 40..160, 1.2x at 256..700, 1.1x at 1024..2048 (geometric means over 18 weights)"},
+    // group size 32 and long K at 5..16 tokens: the split-K decode kernel
+    {5, 16, P_WS | P_LARGE, 0, SQ_ALGO_SKINNY_WS, "16 tokens: fc1 12.5, fc2 14.7 vs 16-column kernel 19.6 / 21.7"},
+    {5, 16, P_WS, P_K_LE_8192, SQ_ALGO_SKINNY_WS, "long K: one workgroup per 16 rows cannot stage the activations in one round"},
     // the decode GEMV: up to 4 tokens, up to 8 while its staged activations fit one round
     {1, 4, 0, 0, SQ_ALGO_GEMV_FIXUP, "1 token: the four-launch layer step 27.3 per step; 4096x4096 at 4 tokens 4.4"},
     {5, 8, P_K_LE_8192, 0, SQ_ALGO_GEMV_FIXUP, "8 tokens at group size 32 (no streaming kernel): 6.5 vs 8.1 (16-column kernel)"},
-    // the 16-column kernel: no workspace, or small weights at 33..64 tokens
-    {5, 32, 0, 0, SQ_ALGO_SKINNY, "no workspace: the only kernel of this range that needs none"},
-    {33, 64, P_K_LE_8192, P_LARGE, SQ_ALGO_SKINNY, "4096x4096 at 64 tokens without the GEMM's workspace: 21 vs 46 (unsplit GEMM)"},
-    {33, 64, 0, P_GEMM_WS | P_K_LE_8192, SQ_ALGO_SKINNY, "4096x16384 at 64 tokens without a workspace: 70 vs 170 (unsplit GEMM)"},
+    // the 16-column kernel: no workspace
+    {5, 16, 0, 0, SQ_ALGO_SKINNY, "no workspace: the only kernel of this range that needs none"},
     {1, 1 << 30, 0, 0, SQ_ALGO_GEMM, "everything else: the tiled GEMM (plan_gemm picks tile height, staging and split)"},
 };
 
-int builtin_choice(int M, int N, int K, int g, bool ws_ok, bool gemm_ws) {
+int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
     unsigned p = 0;
-    if ((long)N * (long)K >= (1L << 25)) p |= P_LARGE;
+    const long nk = (long)N * (long)K;
+    if (nk >= (1L << 25)) p |= P_LARGE;
+    if (nk > (1L << 24)) p |= P_OVER_16M;
     if (ws_ok) p |= P_WS;
-    if (gemm_ws) p |= P_GEMM_WS;
-    if (g == 128) p |= P_G128;
     if (g == 128 || g == 64) p |= P_G128_64;
     if (K % 128 == 0) p |= P_K128;
-    if (K % 256 == 0) p |= P_K256;
-    if ((long)N * (long)K <= (1L << 22) && K <= 2048) p |= P_SMALL;
-    if (N >= 8192) p |= P_N_GE_8192;
-    if (K <= 1536) p |= P_K_LE_1536;
+    if (nk <= (1L << 22) && K <= 1536) p |= P_SMALL;
     {
         const int chunks = K / 128, ks0 = (chunks + 31) / 32;
         if (ks0 > 0 && chunks * 4 >= ks0 * 32 * 3) p |= P_CHUNK_FILL;
@@ -180,15 +154,14 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok, bool gemm_ws) {
     if (K <= 4096) p |= P_K_LE_4096;
     if (K <= 8192) p |= P_K_LE_8192;
     if (K <= 32768) p |= P_K_LE_32768;
-    if (M > 16 && M <= 32 && g == 128) {
-        // One workgroup per CU: W workgroups take ceil(W / 256) rounds of about the same length whatever part of
-        // their 32 chunk slots the K range fills.
-        long wgs = 0;
-        int slots = 0;
-        if (sq::skinny3_wide_shape(N, K, ws_ok, &wgs, &slots)) {
-            const long rounds = (wgs + 255) / 256;
-            if (wgs <= 256 || wgs * slots * 100 >= rounds * 256 * 32 * 95) p |= P_WIDE;
-        }
+    if (sq::gemm_ring_applies(M, N, K)) p |= P_RING;
+    if (M > 1024 && K <= 4096 && K % 256 == 0 && g >= 64) {
+        // One workgroup per CU pays its first loads and its stores in full every round, two per CU hide them behind each
+        // other: 6144x1536 at 4096 tokens (768 tiles) 82 us against the ring kernel's 95, 8192x2048 135 against 149,
+        // 16384x4096 (2048 tiles) 504 against 538, 12288x4096 (1536) 386 against 399; with fewer rounds or a longer K
+        // the ring kernel is ahead (11008x4096, 1376 tiles: 369 against 378; 4096x4096 at 2048 tokens, 256: 68 against 75).
+        const long tiles = (long)((N + 255) / 256) * ((M + 127) / 128);
+        if (tiles >= (K <= 2048 ? 384 : 1500)) p |= P_SHORT_ROUNDS;
     }
     for (const ChoiceRule& r : kChoiceRules)
         if (M >= r.m_lo && M <= r.m_hi && (p & r.need) == r.need && (p & r.forbid) == 0) return r.kernel;
@@ -222,22 +195,7 @@ int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, 
         const bool ws_ok = workspace && aligned16(workspace) &&
                            workspace_bytes >= sq::skinny2_workspace_bytes(M > 32 ? 32 : M, N, K) &&
                            (N + 63) / 64 <= 16384;
-        const bool gemm_ws = workspace && aligned16(workspace) && M > 16 &&
-                             workspace_bytes >= sq::gemm_workspace_bytes(M, N, K);
-        kernel = builtin_choice(M, N, K, group_size, ws_ok, gemm_ws);
-        if (kernel == ALGO_TWO_BLOCKS) {
-            for (int m0 = 0; m0 < M; m0 += 32) {
-                const int mb = M - m0 < 32 ? M - m0 : 32;
-                sq::Epilogue e = epi;
-                if (e.residual) e.residual += (long)m0 * N;
-                if (e.mul) e.mul += (long)m0 * N;
-                const hipError_t err = sq::launch_skinny2_tuned(
-                    static_cast<const sq::half_t*>(x) + (long)m0 * K, w, zs, static_cast<sq::half_t*>(y) + (long)m0 * N,
-                    workspace, mb, N, K, group_size, 0, e, st);
-                if (err != hipSuccess) return SQ_ERR_LAUNCH;
-            }
-            return SQ_OK;
-        }
+        kernel = builtin_choice(M, N, K, group_size, ws_ok);
     }
     switch (kernel) {
         case SQ_ALGO_GEMV:
@@ -256,10 +214,14 @@ int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, 
             return launch_code(sq::launch_skinny2_tuned(x, w, zs, y, workspace, M, N, K, group_size, tune, epi, st));
         case SQ_ALGO_STREAM: {
             if (M > 16 && M <= 32 && group_size == 128) {
+                // The two-tile streaming kernel lives on in the grouped launch of the sequence entry point; for one
+                // linear the ring kernel has taken its place (32 tokens: fc1 15.6 -> 13.4 us, 4096x11008 16.5 -> 12.9) on the
+                // shapes this id takes.
                 const bool ws_fits = workspace && aligned16(workspace) &&
                                      workspace_bytes >= sq::skinny2_workspace_bytes(M, N, K);
-                const hipError_t e = sq::launch_skinny3_wide(x, w, zs, y, ws_fits ? workspace : nullptr, M, N, K, epi, st);
-                return e == hipErrorInvalidValue ? SQ_ERR_WORKSPACE : launch_code(e);
+                if (!sq::skinny3_wide_applies(N, K, ws_fits) || !sq::gemm_ring_applies(M, N, K)) return SQ_ERR_WORKSPACE;
+                return launch_code(sq::launch_gemm_ring(x, w, zs, y, aligned16(workspace) ? workspace : nullptr,
+                                                        workspace_bytes, M, N, K, group_size, 0, epi, st));
             }
             if (M > 16 || (group_size != 128 && group_size != 64)) return SQ_ERR_BAD_ALGO;
             const bool ws_fits = workspace && aligned16(workspace) &&
@@ -271,6 +233,11 @@ int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, 
         case SQ_ALGO_GEMM:
             return launch_code(sq::launch_gemm_tuned(x, w, zs, y, aligned16(workspace) ? workspace : nullptr,
                                                      workspace_bytes, M, N, K, group_size, tune, epi, st));
+        case SQ_ALGO_RING: {
+            const hipError_t e = sq::launch_gemm_ring(x, w, zs, y, aligned16(workspace) ? workspace : nullptr, workspace_bytes,
+                                                      M, N, K, group_size, tune, epi, st);
+            return e == hipErrorInvalidValue ? SQ_ERR_WORKSPACE : launch_code(e);
+        }
         default:
             return SQ_ERR_BAD_ALGO;
     }
@@ -309,7 +276,8 @@ size_t sq_w4a16_workspace_bytes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const size_t a = sq::skinny2_workspace_bytes(M > 32 ? 32 : M, N, K);
     const size_t b = M > 16 ? sq::gemm_workspace_bytes(M, N, K) : 0;
-    return a > b ? a : b;
+    const size_t c = M > 4 ? sq::gemm_ring_workspace_bytes(M, N, K) : 0;
+    return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
 int sq_w4a16_gemm_ws(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int group_size,
@@ -335,8 +303,7 @@ static int autotune_candidates(int M, int K, int g, bool has_ws, int* out, int c
             for (int ks = 1; ks <= 8; ks *= 2)
                 if (ks == 1 ? K <= 4096 : (has_ws && K / ks >= 1024 && K / ks <= 4096)) add(SQ_ALGO_STREAM, rows[r] | (ks << 4));
     }
-    if (M > 16 && M <= 32 && g == 128) add(SQ_ALGO_STREAM, 0);
-    if (M > 2 && M <= 32 && has_ws)
+        if (M > 2 && M <= 32 && has_ws)
         for (int ks = 1; ks <= 8; ks *= 2) add(SQ_ALGO_SKINNY_WS, ks);
     if (M > 2 && M <= 64) add(SQ_ALGO_SKINNY, 0);
     if (M > 16) {
@@ -348,6 +315,11 @@ static int autotune_candidates(int M, int K, int g, bool has_ws, int* out, int c
         if (M > 64)
             for (int v = 8; v <= 10; v++) add(SQ_ALGO_GEMM, v);
     }
+    if (M > 4)
+        for (int shape = 1; shape <= 8; shape++)
+            for (int rest = 0; rest <= (has_ws ? 1 : 0); rest++)
+                for (int ks = rest ? 2 : 1; ks <= (has_ws ? 8 : 1); ks += ks < 4 ? 1 : 2)
+                    add(SQ_ALGO_RING, shape | (rest ? 0x10 : 0) | (ks << 8));
     return n;
 }
 
@@ -405,8 +377,8 @@ int sq_w4a16_autotune(const void* x, const void* w, const void* zs, void* y, int
     int best = 0;
     float t_best = t_auto;
     if (status == SQ_OK) {
-        int words[96];
-        const int n = autotune_candidates(M, K, group_size, has_ws, words, 96);
+        int words[192];
+        const int n = autotune_candidates(M, K, group_size, has_ws, words, 192);
         for (int i = 0; i < n; i++) {
             float t = 0.f;
             const int rc = time_word(words[i], &t);
@@ -473,13 +445,9 @@ int sq_w4a16_gemm_static_ws(const void* x, const void* w, const void* zs, void* 
     if (layout != SQ_LAYOUT_L1) return SQ_ERR_BAD_LAYOUT;
     // What the kernels of this token count would take from a workspace: nothing up to 2 tokens (the GEMV has
     // no workspace form), the split-K decode kernels' counters and partial tiles up to 32, the tiled GEMM's K
-    // split beyond and where the automatic choice takes it at 17..32.  A shape that wants more than the static
+    // split beyond (the ring kernel plans within whatever it is given).  A shape that wants more than the static
     // buffer is refused rather than served by a slower workspace-free kernel behind the caller's back.
-    size_t need = M <= 2 ? 0 : (M <= 32 ? sq::skinny2_workspace_bytes(M, N, K) : sq::gemm_workspace_bytes(M, N, K));
-    if (M > 16 && M <= 32 && builtin_choice(M, N, K, group_size, true, true) == SQ_ALGO_GEMM) {
-        const size_t b = sq::gemm_workspace_bytes(M, N, K);
-        if (b > need) need = b;
-    }
+    const size_t need = M <= 2 ? 0 : (M <= 32 ? sq::skinny2_workspace_bytes(M, N, K) : sq::gemm_workspace_bytes(M, N, K));
     if (need > (size_t)SQ_STATIC_WS_BYTES) return SQ_ERR_STATIC_WS;
     if (M == 0) return SQ_OK;
     if (!x || !w || !zs || !y) return SQ_ERR_NULL_POINTER;

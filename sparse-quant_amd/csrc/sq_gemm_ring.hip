@@ -1,0 +1,705 @@
+// GEMM for 17 tokens up (any group size, any K) with layout L1: the product between a weight stream and a matrix-core
+// contraction, and the contraction itself until many rounds of short K favour the two-workgroups-per-CU kernel of
+// sq_gemm.hip.
+//
+// What bounds it.  At 32..600 tokens neither HBM nor the matrix cores are full; what a CU can issue is: about five
+// vector instructions fit beside a v_mfma_f32_32x32x16_f16 (32 cycles), each further one costs five cycles or more,
+// and dequantising eight weights takes thirteen.  A workgroup with one wave per SIMD (the kernel this one replaces)
+// leaves the matrix pipe idle through every barrier, LDS trip and load issue.  Hence:
+//   * eight waves, two per SIMD, in two groups that alternate: while waves 0..3 issue the matrix instructions of a
+//     phase from registers, waves 4..7 read their operands from LDS, dequantise and request the next loads, then the
+//     groups swap at a barrier.  (Measured on a loop of the same instruction mix: both groups in step 1790 cycles per
+//     64 k of a 64-row tile, alternating 1520, matrix instructions alone 1040.)  Part of the dequantisation sits
+//     between the matrix instructions of the phase before it is needed.
+//   * K is split over the waves of the workgroup (WK groups of 64 consecutive k each per stage of KS = 64 WK), so that
+//     a weight row is read in 64..256-byte pieces, a stage holds 40..50 KB, and narrow weights fill the chip without
+//     partial tiles in memory.  The groups' sums meet in LDS at the end.
+//   * every operand goes global -> LDS by direct loads, ST - 1 stages ahead (three or four stages of a ring); rows past
+//     M are never requested (their lanes are masked, their LDS rows are zero), so padding costs no memory traffic.
+//   * where the tiles leave CUs idle, the tiles of the last, part-filled round split K over workgroups through the
+//     caller's workspace.
+// Measured (us per launch, cold weights, group size 128; before: sq_gemm.hip's 32..128-row tiles or the decode kernels):
+//   32 tokens   4096x4096 9.9 -> 8.6, 12288x4096 14.3 -> 12.3, 4096x11008 16.5 -> 12.9, 5120x13696 27.0 -> 16.6
+//   100 tokens  4096x4096 15.9 -> 11.0, 15360x5120 37.3 -> 28.8, 5120x13696 54.0 -> 30.2
+//   333 tokens  4096x4096 27.0 -> 20.2, 12288x4096 65.1 -> 47.5, 5120x13696 90.3 -> 65.0
+//   1024 tokens 4096x4096 46.0 -> 41, 5120x13696 202 -> 152; 2048 tokens 4096x16384 269 -> 243 (1.13 PFLOP/s)
+// Tried and dropped: all waves in one group with software-pipelined operands (8..15 % slower), stages of 32 k per wave
+// with twice the bytes in flight (10 % slower: a barrier per 8 matrix instructions), the group sums handed over in
+// registers' order instead of row-major slices (1..4 % slower below 256 tokens).
+//
+// Operand mapping as in sq_gemm.hip: D = X W^T with activations as A (lane = row) and weights as B (lane = column);
+// lane (ln, lc) of a wave holds k = 32 lc + 8 t .. + 7 of its 64 for slice t, one packed word of the weight row per
+// slice; W_hat = fp16((q - z) * s) bit for bit.
+// (replaces w4a16_gemm_wmma_kernel, reference: quantization/muxi/backend/w4a16_gemm.cuh:466-600, and the role of
+// turbomind::GemmS4F16, quantization/nvidia/kernel/gemm_s4_f16/gemm_template.h:358-450)
+#include "sq_common.h"
+#include "sq_kernels.h"
+
+#include <type_traits>
+
+namespace sq {
+
+constexpr size_t RING_COUNTER_BYTES = 65536;  // start of the workspace: one uint32 per tile that splits K
+
+struct RingPlan {
+    int shape, nfull, ksplit;  // tiles below nfull are computed by one workgroup, the others by ksplit each
+};
+
+namespace {
+
+__device__ __forceinline__ int swz8(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+
+// LDS layout of a stage: activations as WK tiles [BM rows][128 bytes], weights [BN rows][32 WK bytes], zeros/scales
+// [BN columns][pairs].  The 16-byte chunks of a row are permuted (by the lane that requests them: a direct load puts
+// lane l at 16 l) so that the 128-bit operand reads, lane = row, of eight and of sixteen consecutive rows fall on
+// different banks: swz8 for rows of eight chunks, wswz for weight rows of 2 WK.
+template <int WK>
+__device__ __forceinline__ int wswz(int row) {
+    if constexpr (WK == 8) return row & 15;
+    if constexpr (WK == 4) return swz8(row);
+    if constexpr (WK == 2) return ((row >> 1) & 3) ^ ((row >> 3) & 1);
+    return ((row >> 2) & 1) ^ ((row >> 3) & 1);
+}
+
+// The largest divisor of l that is at most cap and a multiple of unit.
+constexpr int ring_trip(int l, int cap, int unit) {
+    int u = cap < l ? cap : l;
+    while (l % u != 0 || u % unit != 0) u--;
+    return u;
+}
+
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST>
+struct RingShape {
+    static constexpr int NW = WM * WN * WK, NT = 64 * NW;
+    static constexpr int BM = 32 * MI * WM, BN = 32 * NI * WN, KS = 64 * WK;
+    static constexpr int XB = WK * BM * 128, WB = BN * WK * 32;
+    static constexpr int P = (KS >> GS) ? (KS >> GS) : 1;  // zeros/scales pairs per column and stage
+    static constexpr int ZB = BN * P * 4;
+    static constexpr int SB = XB + WB + ZB;
+    static constexpr int XI = XB / 1024 / NW, WI = WB / 1024 / NW;
+    static constexpr int ZL = BN * P / NW < 64 ? BN * P / NW : 64, ZI = BN * P / NW / ZL;  // lanes and instructions of a wave
+    static constexpr int PER = XI + WI + ZI;
+    static constexpr int LDS = ST * SB;
+    static constexpr int TAIL = NW * 32 * 32 * NI * 4;  // one 32-row slice of every wave's sums
+    static_assert(XI * NW * 1024 == XB && WI * NW * 1024 == WB && ZI * ZL * NW == BN * P && NW == 8, "loads divide over the waves");
+    static_assert(LDS <= 163840 && TAIL <= LDS, "fits");
+};
+
+template <int EV>
+__device__ __forceinline__ void finish_cols(float (&v)[EV], half_t* __restrict__ Y, int m, int n, int N, const Epilogue& epi) {
+    typedef _Float16 hv_t __attribute__((ext_vector_type(EV)));
+    const long idx = (long)m * N + n;
+    auto load = [&](const half_t* p, float (&o)[EV]) {
+        if ((reinterpret_cast<uintptr_t>(p) & (2 * EV - 1)) == 0) {
+            const hv_t h = *(const hv_t*)p;
+#pragma unroll
+            for (int e = 0; e < EV; e++) o[e] = (float)h[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < EV; e++) o[e] = (float)p[e];
+        }
+    };
+    float t[EV];
+    if (epi.bias) {
+        load(epi.bias + n, t);
+#pragma unroll
+        for (int e = 0; e < EV; e++) v[e] += t[e];
+    }
+    if (epi.act == 1) {
+#pragma unroll
+        for (int e = 0; e < EV; e++) v[e] = fmaxf(v[e], 0.f);
+    } else if (epi.act == 2) {
+#pragma unroll
+        for (int e = 0; e < EV; e++) v[e] = v[e] * __builtin_amdgcn_rcpf(1.f + __expf(-v[e]));
+    }
+    if (epi.mul) {
+        load(epi.mul + idx, t);
+#pragma unroll
+        for (int e = 0; e < EV; e++) v[e] *= t[e];
+    }
+    if (epi.residual) {
+        load(epi.residual + idx, t);
+#pragma unroll
+        for (int e = 0; e < EV; e++) v[e] += t[e];
+    }
+    hv_t h;
+#pragma unroll
+    for (int e = 0; e < EV; e++) h[e] = (half_t)v[e];
+    *(hv_t*)(Y + idx) = h;
+}
+
+// Direct loads by part of a wave's lanes (mask): the instruction is issued whatever the mask, so that the counted waits
+// hold for every wave.  The wave runs with all lanes active around it.
+__device__ __forceinline__ void load_to_lds_x4_masked(const void* base, uint32_t lane_byte, uint32_t lds_byte, uint64_t mask) {
+    asm volatile("s_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(lane_byte), "s"(base),
+                 "{m0}"(lds_byte), "s"(mask)
+                 : "memory");
+}
+
+__device__ __forceinline__ void load_to_lds_x1_masked(const void* base, uint32_t lane_byte, uint32_t lds_byte, uint64_t mask) {
+    asm volatile("s_mov_b64 exec, %3\n\tglobal_load_lds_dword %0, %1\n\ts_mov_b64 exec, -1" ::"v"(lane_byte), "s"(base),
+                 "{m0}"(lds_byte), "s"(mask)
+                 : "memory");
+}
+
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST>
+__global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(
+    const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS, const half_t* __restrict__ X, half_t* __restrict__ Y,
+    int M, int N, int K, int mtiles, int tiles, int nfull, int ksplit, Epilogue epi, float* part, unsigned* counters) {
+    using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
+    constexpr int BM = S::BM, BN = S::BN, KS = S::KS, SB = S::SB, XI = S::XI, WI = S::WI, ZI = S::ZI, ZL = S::ZL, PER = S::PER, P = S::P;
+    constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = S::XB + S::WB;
+    constexpr int H = MI > 3 || MI * NI > 4 ? 2 : 4, PH = 4 / H;  // 16-wide k slices per phase, phases per stage
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[S::LDS];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+
+    const NibbleMasks nm = nibble_masks();
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ln = lane & 31;
+    const int lc = lane >> 5;
+    const int kg = wave / (WM * WN);
+    const int wm = (wave / WN) % WM;
+    const int wn = wave % WN;
+
+    // Which tile, and which part of K.
+    int tile, z = 0, ks = 1, tr = 0;
+    const int rest = tiles - nfull;
+    const int id = blockIdx.x;
+    if (ksplit == 1) {
+        const int per = (tiles + 7) >> 3;
+        tile = (id & 7) * per + (id >> 3);
+        if (tile >= tiles || (id >> 3) >= per) return;
+    } else if (id < nfull) {
+        tile = (id & 7) * (nfull >> 3) + (id >> 3);
+    } else {
+        const int rid = id - nfull;
+        const int per = (rest * ksplit + 7) >> 3;
+        const int u = (rid & 7) * per + (rid >> 3);
+        if (u >= rest * ksplit || (rid >> 3) >= per) return;
+        z = u / rest;
+        tr = u - z * rest;
+        tile = nfull + tr;
+        ks = ksplit;
+    }
+    const int nt = tile / mtiles;
+    const int m0 = (tile - nt * mtiles) * BM;
+    const int n0 = nt * BN;
+    const int groups = K >> GS;
+    const int nst = (K + KS - 1) / KS;
+    const int spz = (nst + ks - 1) / ks;
+    const int it0 = z * spz;
+    const int it1 = imin(it0 + spz, nst);
+
+    // Byte offsets of this wave's loads; the part along K is a wave-uniform base.
+    uint32_t xlane[XI], wlane[WI], zlane[ZI];
+    uint64_t xmask[XI];  // lanes whose row exists; the others' LDS rows stay zero
+    constexpr uint64_t zmask = ZL == 64 ? ~0ull : (1ull << (ZL & 63)) - 1;
+#pragma unroll
+    for (int j = 0; j < XI; j++) {
+        const int ii = wave * XI + j;
+        const int R = (ii % (BM / 8)) * 8 + (lane >> 3);
+        xlane[j] = (uint32_t)((long)imin(m0 + R, M - 1) * K * 2) + (64 * (ii / (BM / 8)) + ((lane & 7) ^ swz8(R)) * 8) * 2;
+        xmask[j] = __builtin_amdgcn_ballot_w64(m0 + R < M);
+        if (m0 + R >= M) {
+            const u32x4_t zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int c = 0; c < ST; c++) *(u32x4_t*)(lds + X_OFF + c * SB + (wave * XI + j) * 1024 + lane * 16) = zero;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < WI; j++) {
+        const int R = (wave * WI + j) * (32 / WK) + lane / (2 * WK);
+        wlane[j] = (uint32_t)((long)imin(n0 + R, N - 1) * (K >> 1)) + (((lane % (2 * WK)) ^ wswz<WK>(R)) * 16);
+    }
+#pragma unroll
+    for (int j = 0; j < ZI; j++) {
+        const int d = (wave * ZI + j) * ZL + (lane & (ZL - 1));
+        zlane[j] = (uint32_t)((long)imin(n0 + d / P, N - 1) * groups * 4) + (d % P) * 4;
+    }
+    // All loads of stage it into slot c.  EDGE: the last stage of a K that ends inside it; what is missing re-reads the
+    // end of the row (and meets a scale of 0).
+    auto issue = [&](int it, int c, auto EDGE_) {
+        constexpr bool EDGE = decltype(EDGE_)::value;
+        const int k0 = it * KS, left = K - k0;
+        const uint8_t* xb = (const uint8_t*)X + (long)k0 * 2;
+        const uint8_t* wb = W + (k0 >> 1);
+        const uint8_t* zb = (const uint8_t*)ZS + (k0 >> GS) * 4;
+        const uint32_t l0 = lds0 + c * SB;
+#pragma unroll
+        for (int j = 0; j < ZI; j++) {
+            uint32_t o = zlane[j];
+            if constexpr (EDGE) {
+                const int p = ((wave * ZI + j) * ZL + (lane & (ZL - 1))) % P;
+                o = o - p * 4 + imin(p, groups - 1 - (k0 >> GS)) * 4;
+            }
+            load_to_lds_x1_masked(zb, o, l0 + Z_OFF + (wave * ZI + j) * ZL * 4, zmask);
+        }
+#pragma unroll
+        for (int j = 0; j < WI; j++) {
+            uint32_t o = wlane[j];
+            if constexpr (EDGE) {
+                const int R = (wave * WI + j) * (32 / WK) + lane / (2 * WK);
+                const int p = ((lane % (2 * WK)) ^ wswz<WK>(R)) * 16;
+                o = o - p + imin(p, (left - 32) >> 1);
+            }
+            load_to_lds_x4(wb, o, l0 + W_OFF + (wave * WI + j) * 1024);
+        }
+#pragma unroll
+        for (int j = 0; j < XI; j++) {
+            uint32_t o = xlane[j];
+            if constexpr (EDGE) {
+                const int ii = wave * XI + j;
+                const int R = (ii % (BM / 8)) * 8 + (lane >> 3);
+                const int p = (64 * (ii / (BM / 8)) + ((lane & 7) ^ swz8(R)) * 8) * 2;
+                o = o - p + imin(p, (left - 8) * 2);
+            }
+            load_to_lds_x4_masked(xb, o, l0 + X_OFF + (wave * XI + j) * 1024, xmask[j]);
+        }
+    };
+    auto issue_any = [&](int it, int c) {
+        if (it * KS + KS <= K)
+            issue(it, c, std::false_type{});
+        else
+            issue(it, c, std::true_type{});
+    };
+
+    const int xrow = X_OFF + kg * (BM * 128) + (wm * 32 * MI + ln) * 128;
+    int xoff[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) xoff[t] = xrow + (((4 * lc + t) ^ swz8(ln)) * 16);
+    const int wcol = wn * 32 * NI + ln;
+    const int woff = W_OFF + wcol * (32 * WK) + (((2 * kg + lc) ^ wswz<WK>(ln)) * 16);
+    const int zoff = Z_OFF + (wcol * P + ((64 * kg + (GS == 5 ? 32 * lc : 0)) >> GS)) * 4;
+
+    float16_t acc[MI][NI];
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[mi][ni][v] = 0.f;
+
+    half8_t a[H][MI], b[H][NI];
+    half2_t zs[NI];
+    uint32_t q[NI][H];
+    auto dequantise = [&](int t) {
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++)
+            b[t][ni] = dequant8(q[ni][t], (half2_t){zs[ni].x, zs[ni].x}, (half2_t){zs[ni].y, zs[ni].y}, nm);
+    };
+    // Phase h of stage it (slot c): the wave's operands into registers, weights dequantised.
+    auto fetch = [&](int it, int c, auto h_) {
+        constexpr int h = decltype(h_)::value;
+        const uint8_t* l = lds + c * SB;
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            zs[ni] = *(const half2_t*)(l + zoff + ni * (32 * P * 4));
+            if constexpr (H == 4) {
+                const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (32 * 32 * WK));
+#pragma unroll
+                for (int t = 0; t < 4; t++) q[ni][t] = v[t];
+            } else {
+                const u32x2_t v = *(const u32x2_t*)(l + woff + 8 * h + ni * (32 * 32 * WK));
+                q[ni][0] = v.x;
+                q[ni][1] = v.y;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < H; t++)
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) a[t][mi] = *(const half8_t*)(l + xoff[h * H + t] + mi * 4096);
+    };
+    // Weights past the end of K get the scale 0 (only the last stage can hold any).
+    auto clip = [&](int it) {
+        if (it * KS + 64 * kg + (GS == 5 ? 32 * lc : 0) >= K) {
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) zs[ni].y = (half_t)0.f;
+        }
+    };
+    // the first half of the phase's weights, finished in front of the barrier that follows
+    auto dequantise_first = [&]() {
+#pragma unroll
+        for (int t = 0; t < H / 2; t++) {
+            dequantise(t);
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) {
+                u32x4_t v = bit_cast<u32x4_t>(b[t][ni]);
+                asm volatile("" : "+v"(v));
+                b[t][ni] = bit_cast<half8_t>(v);
+            }
+        }
+    };
+    // Matrix instructions of the phase; those of its first half hide the dequantisation of the second.
+    auto compute = [&]() {
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+            for (int t = H / 2; t < H; t++) asm volatile("" : "+v"(q[ni][t]));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = H / 2; t < H; t++) dequantise(t);
+#pragma unroll
+        for (int t = 0; t < H; t++)
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t][mi], b[t][ni], acc[mi][ni], 0, 0, 0);
+        constexpr int MF = H / 2 * MI * NI, VA = (14 * NI * (H / 2) + MF - 1) / MF;
+#pragma unroll
+        for (int i = 0; i < MF; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, VA, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, MF, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (it0 < it1) {
+#pragma unroll
+        for (int s = 0; s < ST - 1; s++)
+            if (it0 + s < it1) issue_any(it0 + s, s);
+        if (it0 + ST - 1 <= it1)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        using H0 = std::integral_constant<int, 0>;
+        using H1 = std::integral_constant<int, PH - 1>;
+        // Stage it + 1 has landed: all but the loads of the younger stages are done.
+        auto landed_full = []() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory"); };
+        auto landed_all = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+        auto turn = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+        int c = 0, cp = ST - 1, it = it0;
+        auto next = [&]() {
+            cp = c;
+            c = c == ST - 1 ? 0 : c + 1;
+        };
+        const int full = it1 - (ST - 1);  // stages below it still have a stage to request
+        // Both branches pass the same barriers, two per phase: waves 0..3 fetch phase p + 1 while waves 4..7 compute
+        // phase p.  A stage's first fetch also requests stage it + ST - 1 into the slot of stage it - 1, which both
+        // groups have read by then.
+        if (wave < 4) {
+            if (it < full) {
+                fetch(it, 0, H0{});
+                issue_any(it + ST - 1, ST - 1);
+                dequantise_first();
+            } else {
+                fetch(it, 0, H0{});
+                clip(it);
+                dequantise_first();
+            }
+            turn();
+            for (; it + 1 < full; it++) {
+                compute();
+                if constexpr (PH == 2) {
+                    turn();
+                    fetch(it, c, H1{});
+                    dequantise_first();
+                    turn();
+                    compute();
+                }
+                landed_full();
+                next();
+                fetch(it + 1, c, H0{});
+                issue_any(it + ST, cp);
+                dequantise_first();
+                turn();
+            }
+            for (; it < it1; it++) {
+                compute();
+                if constexpr (PH == 2) {
+                    turn();
+                    fetch(it, c, H1{});
+                    clip(it);
+                    dequantise_first();
+                    turn();
+                    compute();
+                }
+                landed_all();
+                next();
+                if (it + 1 < it1) {
+                    fetch(it + 1, c, H0{});
+                    clip(it + 1);
+                    dequantise_first();
+                }
+                turn();
+            }
+        } else {
+            turn();
+            for (; it < full; it++) {
+                fetch(it, c, H0{});
+                issue_any(it + ST - 1, cp);
+                dequantise_first();
+                if constexpr (PH == 2) {
+                    turn();
+                    compute();
+                    turn();
+                    fetch(it, c, H1{});
+                    dequantise_first();
+                }
+                landed_full();
+                compute();
+                next();
+                turn();
+            }
+            for (; it < it1; it++) {
+                fetch(it, c, H0{});
+                clip(it);
+                dequantise_first();
+                if constexpr (PH == 2) {
+                    turn();
+                    compute();
+                    turn();
+                    fetch(it, c, H1{});
+                    clip(it);
+                    dequantise_first();
+                }
+                landed_all();
+                compute();
+                next();
+                turn();
+            }
+        }
+    }
+
+    // The K groups' sums meet in LDS, one 32-row slice of every row group at a time, and leave row-major, EV consecutive
+    // columns per thread.
+    constexpr int PT = 16 * NI / WK;     // sums per thread and slice
+    constexpr int EV = PT < 8 ? PT : 8;
+    constexpr int G = PT / EV;
+    constexpr int CPR = BN / EV;         // column chunks per row
+    constexpr int L = MI * PT / 4;       // float4 per thread
+    float* red = reinterpret_cast<float*>(lds);
+    const long tsz = (long)BM * BN;
+    float* mine = part + ((long)z * rest + tr) * tsz + tid * 4;
+    auto finish = [&](int mi, int g, float (&v)[EV]) {
+        const int ch = tid + g * S::NT;
+        const int r = ch / CPR, cc = ch % CPR;
+        const int m = m0 + (r >> 5) * (32 * MI) + 32 * mi + (r & 31);
+        const int n = n0 + cc * EV;
+        if (m < M && n < N) finish_cols<EV>(v, Y, m, n, N, epi);
+    };
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++) {
+        __syncthreads();
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                red[((kg * WM + wm) * 32 + 8 * (v >> 2) + 4 * lc + (v & 3)) * BN + wcol + 32 * ni] = acc[mi][ni][v];
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            const int ch = tid + g * S::NT;
+            const int r = ch / CPR, cc = ch % CPR;  // r: row of the WM * 32 of this slice
+            float v[EV];
+#pragma unroll
+            for (int e = 0; e < EV; e++) v[e] = red[r * BN + cc * EV + e];
+#pragma unroll
+            for (int q = 1; q < WK; q++)
+#pragma unroll
+                for (int e = 0; e < EV; e++) v[e] += red[(q * WM * 32 + r) * BN + cc * EV + e];
+            if (ks == 1) {
+                finish(mi, g, v);
+            } else {
+#pragma unroll
+                for (int h = 0; h < EV / 4; h++)
+                    store_coherent_x4(mine + ((mi * G + g) * (EV / 4) + h) * (S::NT * 4),
+                                      (float4_t){v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]});
+            }
+        }
+    }
+    if (ks > 1) {
+        // Partial tiles meet in the workspace: device-coherent stores, one counter per tile.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        unsigned* last_flag = reinterpret_cast<unsigned*>(lds);
+        if (tid == 0) {
+            const unsigned old = __hip_atomic_fetch_add(&counters[tr], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *last_flag = (old == (unsigned)(ks - 1)) ? 1u : 0u;
+        }
+        __syncthreads();
+        if (!*last_flag) return;
+        // The last of the tile's workgroups adds the partial sums in the order of the K ranges (bit-reproducible whoever
+        // comes last); up to 32 loads per thread are in flight, nothing else hides their latency.
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(part, 0, 0x7FFFFFFF, 0x00027000);
+        auto reduce = [&](auto NZ_) {
+            constexpr int NZ = decltype(NZ_)::value;          // ranges, rounded up
+            constexpr int U = ring_trip(L, 32 / NZ, EV / 4);  // float4 per thread and trip
+            static_assert(L % U == 0 && U % (EV / 4) == 0, "whole trips");
+#pragma unroll 1
+            for (int l0 = 0; l0 < L; l0 += U) {
+                u32x4_t pv[U][NZ];
+                const uint32_t base = (uint32_t)(((long)tr * tsz + (long)l0 * (S::NT * 4) + tid * 4) * 4);
+                const uint32_t zstep = (uint32_t)((long)rest * tsz * 4);
+#pragma unroll
+                for (int q = 0; q < NZ; q++)
+#pragma unroll
+                    for (int i = 0; i < U; i++)
+                        pv[i][q] = __builtin_amdgcn_raw_buffer_load_b128(rs, base + i * (S::NT * 16), q < ks ? q * zstep : 0, 16);
+#pragma unroll
+                for (int i0 = 0; i0 < U; i0 += EV / 4) {
+                    float v[EV];
+#pragma unroll
+                    for (int i = i0; i < i0 + EV / 4; i++) {
+                        float4_t sum = bit_cast<float4_t>(pv[i][0]);
+#pragma unroll
+                        for (int q = 1; q < NZ; q++)
+                            if (q < ks) sum += bit_cast<float4_t>(pv[i][q]);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[4 * (i - i0) + e] = sum[e];
+                    }
+                    const int chunk = (l0 + i0) / (EV / 4);
+                    finish(chunk / G, chunk % G, v);
+                }
+            }
+        };
+        if (ks <= 2)
+            reduce(std::integral_constant<int, 2>{});
+        else if (ks <= 4)
+            reduce(std::integral_constant<int, 4>{});
+        else
+            reduce(std::integral_constant<int, 8>{});
+        if (tid == 0) __hip_atomic_store(&counters[tr], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+}  // namespace
+
+// The shapes that are built: {MI, NI, WM, WN, WK, stages}, i.e. a (32 MI WM) x (32 NI WN) tile and 64 WK columns of K
+// per stage.  LDS holds three or four stages.
+#define SQ_RING_SHAPES(X_)                                                                                             \
+    X_(1, 1, 2, 1, 1, 8, 3) X_(2, 1, 2, 1, 2, 4, 4) X_(3, 2, 2, 1, 2, 4, 3) X_(4, 3, 1, 1, 4, 2, 4) X_(5, 2, 2, 1, 4, 2, 4) \
+        X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3) X_(8, 4, 2, 1, 4, 2, 3)
+
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST>
+static hipError_t launch_shape(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int nfull,
+                               int ksplit, Epilogue epi, void* ws, hipStream_t st) {
+    using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
+    const int mt = (M + S::BM - 1) / S::BM;
+    const int tiles = mt * ((N + S::BN - 1) / S::BN);
+    if (ksplit == 1) nfull = tiles;
+    const int grid = ksplit == 1 ? (tiles + 7) / 8 * 8 : nfull + ((tiles - nfull) * ksplit + 7) / 8 * 8;
+    hipLaunchKernelGGL((gemm_ring_kernel<MI, NI, WM, WN, WK, GS, ST>), dim3(grid), dim3(S::NT), 0, st, (const uint8_t*)w,
+                       (const half2_t*)zs, (const half_t*)x, (half_t*)y, M, N, K, mt, tiles, nfull, ksplit, epi,
+                       ws ? (float*)((char*)ws + RING_COUNTER_BYTES) : nullptr, (unsigned*)ws);
+    return hipGetLastError();
+}
+
+// What a shape costs, in us: a workgroup takes `step0 + step1 * a` per stage of K and `fixed` besides (first loads, sums,
+// stores), a = the share of the 256 CUs that its round keeps busy (memory and clock are shared); a K split adds the
+// exchange of the partial tiles, `ex0 + ex1 * parts + exmb` per MB of them.  One workgroup fills a CU.  Least-squares
+// fits to 9000 timings of 18 weights (3072 x 1024 .. 28672 x 8192) x 23 token counts (12 .. 4096) x all shapes and
+// splits: rms error 5..7 %, the choice within 0.5 % of the best in the geometric mean, 11 % at worst.
+struct RingTile {
+    int bm, bn, ks;
+    float fixed, step0, step1, ex0, ex1, exmb;
+};
+static const RingTile kRingTiles[] = {
+    {32, 64, 512, 1.723f, 0.829f, 0.160f, 0.301f, 0.226f, 0.861f},
+    {32, 128, 256, 1.498f, 0.754f, 0.096f, 0.448f, 0.304f, 0.649f},
+    {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f},
+    {96, 128, 128, 2.993f, 0.625f, 0.206f, 0.534f, 0.521f, 0.308f},
+    {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f},
+    {96, 256, 128, 4.305f, 1.017f, 0.410f, 0.106f, 1.298f, 0.243f},
+    {128, 128, 128, 3.276f, 0.802f, 0.268f, 0.000f, 0.967f, 0.278f},
+    {128, 256, 128, 4.931f, 1.142f, 0.611f, 0.100f, 1.663f, 0.230f},
+};
+constexpr int RING_SHAPES = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
+#define X_(id, MI, NI, WM, WN, WK, ST)                                                                              \
+    static_assert(id >= 1 && id <= RING_SHAPES, "a row of kRingTiles per shape");
+SQ_RING_SHAPES(X_)
+#undef X_
+
+bool gemm_ring_applies(int M, int N, int K) {
+    // operands are addressed with 32-bit byte offsets per lane
+    return (long)M * K * 2 < (1L << 32) && (long)N * (K / 2) < (1L << 32) && (long)M * N < (1L << 36);
+}
+
+static size_t ring_bytes(const RingPlan& p, int M, int N) {
+    if (p.ksplit <= 1) return 0;
+    const RingTile& t = kRingTiles[p.shape - 1];
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    return RING_COUNTER_BYTES + (size_t)(tiles - p.nfull) * p.ksplit * t.bm * t.bn * sizeof(float);
+}
+
+// The cheapest shape and K split whose partial tiles fit `ws_bytes`.  Where the tiles come in full rounds of 256 and a
+// rest, only the rest splits K.
+static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes) {
+    RingPlan best{1, 0, 1};
+    float best_us = 3.4e38f;
+    const int rows32 = (M + 31) / 32 * 32;
+    for (int s = 0; s < RING_SHAPES; s++) {
+        const RingTile& t = kRingTiles[s];
+        const int mt = (M + t.bm - 1) / t.bm;
+        if (t.bm > 64 && mt * t.bm * 2 > rows32 * 3) continue;  // a third of the matrix work would be padding
+        const long tiles = (long)mt * ((N + t.bn - 1) / t.bn);
+        const int stages = (K + t.ks - 1) / t.ks;
+        const int full = (int)(tiles >> 8), rest = (int)(tiles & 255);
+        const float one = stages * (t.step0 + t.step1) + t.fixed;
+        const float base = 2.f + full * one;
+        auto consider = [&](float us, int nfull, int ks) {
+            if (us >= best_us) return;
+            const RingPlan p{s + 1, nfull, ks};
+            if (ks > 1 && ring_bytes(p, M, N) > ws_bytes) return;
+            best_us = us;
+            best = p;
+        };
+        consider(base + (rest ? stages * (t.step0 + t.step1 * rest * (1.f / 256)) + t.fixed : 0.f), 0, 1);
+        if (ws_bytes == 0 || rest == 0) continue;
+        static const int splits[5] = {2, 3, 4, 6, 8};
+        for (int ks : splits) {
+            const long w = (long)rest * ks;
+            if (ks > stages || w > 300) break;
+            const int st = (stages + ks - 1) / ks;
+            const float ex = t.ex0 + t.ex1 * ks + t.exmb * (4e-6f * w * t.bm * t.bn);
+            const int r = (int)(w >> 8), last = (int)(w & 255);
+            consider(base + r * (st * (t.step0 + t.step1) + t.fixed) +
+                         (last ? st * (t.step0 + t.step1 * last * (1.f / 256)) + t.fixed : 0.f) + ex,
+                     full * 256, ks);
+        }
+    }
+    return best;
+}
+
+size_t gemm_ring_workspace_bytes(int M, int N, int K) {
+    return gemm_ring_applies(M, N, K) ? ring_bytes(plan_ring(M, N, K, (size_t)64 << 20), M, N) : 0;
+}
+
+// tune = 0 for the cost model's choice, else shape id | 0x10: only the tiles of the last, part-filled round of 256
+// workgroups split K | K split << 8.  hipErrorInvalidValue: not applicable (or the workspace is missing or too small).
+hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,
+                            int K, int g, int tune, Epilogue epi, hipStream_t st) {
+    if (!gemm_ring_applies(M, N, K)) return hipErrorInvalidValue;
+    RingPlan p{tune & 0xF, 0, (tune >> 8) & 0xFF};
+    if (p.shape == 0) {
+        p = plan_ring(M, N, K, ws ? ws_bytes : 0);
+    } else {
+        if (p.shape > RING_SHAPES || p.ksplit > 8) return hipErrorInvalidValue;
+        const RingTile& t = kRingTiles[p.shape - 1];
+        const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        if (tiles > (1L << 24)) return hipErrorInvalidValue;
+        if (p.ksplit < 1) p.ksplit = 1;
+        if (tune & 0x10) p.nfull = (int)(tiles / 256 * 256);
+        if (p.ksplit > 1) {
+            const size_t need = ring_bytes(p, M, N);
+            if (tiles == p.nfull || tiles - p.nfull > (long)(RING_COUNTER_BYTES / 4) || p.ksplit > (K + t.ks - 1) / t.ks ||
+                need - RING_COUNTER_BYTES >= 0x7FFFFFFFu || !ws || ws_bytes < need)
+                return hipErrorInvalidValue;
+        }
+    }
+    switch (p.shape) {
+#define X_(id, MI, NI, WM, WN, WK, ST)                                                                                    \
+    case id:                                                                                                              \
+        if (g == 128)                                                                                                     \
+            return launch_shape<MI, NI, WM, WN, WK, 7, ST>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st);         \
+        if (g == 64) return launch_shape<MI, NI, WM, WN, WK, 6, ST>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st); \
+        return launch_shape<MI, NI, WM, WN, WK, 5, ST>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st);
+        SQ_RING_SHAPES(X_)
+#undef X_
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace sq

@@ -76,17 +76,22 @@ hipError_t launch_skinny2_tuned(const void* x, const void* w, const void* zs, vo
 hipError_t launch_skinny3_tuned(const void* x, const void* w, const void* zs, void* y, void* ws, int M, int N, int K,
                                 int g, int tune, Epilogue epi, const LnPre* ln, hipStream_t st);
 hipError_t launch_skinny3_group(const SeqProblem* probs, int count, int M, void* ws, size_t ws_bytes, hipStream_t st);
-// The same kernel family for 17..32 tokens (two token tiles, activations staged in two halves); group size 128 only.
-hipError_t launch_skinny3_wide(const void* x, const void* w, const void* zs, void* y, void* ws, int M, int N, int K,
-                               Epilogue epi, hipStream_t st);
+// The same kernel family for 17..32 tokens (two token tiles), group size 128: whether it takes a weight, and the launch
+// of several linears of equal K.
 bool skinny3_wide_applies(int N, int K, bool have_ws);
-bool skinny3_wide_shape(int N, int K, bool have_ws, long* workgroups, int* slots_in_use);
 hipError_t launch_skinny3_wide_group(const SeqProblem* probs, int count, int M, void* ws, size_t ws_bytes,
                                      hipStream_t st);
 // sq_gemm.hip: any M.  tune = 32-row tiles per workgroup (1,2,4) | ksplit << 8; ws may be null.
 size_t gemm_workspace_bytes(int M, int N, int K);
 hipError_t launch_gemm_tuned(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M,
                              int N, int K, int g, int tune, Epilogue epi, hipStream_t st);
+
+// sq_gemm_ring.hip: any M, the choice from 17 tokens up.  tune = 0: the cost model's plan within ws_bytes (ws may be
+// null: K is not split over workgroups).
+bool gemm_ring_applies(int M, int N, int K);
+size_t gemm_ring_workspace_bytes(int M, int N, int K);
+hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,
+                            int K, int g, int tune, Epilogue epi, hipStream_t st);
 
 // sq_gemm2.hip: software-pipelined 128 x 256 tile variant for M > 64.
 hipError_t launch_gemm_pipe(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int g,

@@ -714,14 +714,6 @@ __device__ __forceinline__ void skinny3_wide_body(const uint8_t* __restrict__ W,
     if (tid == 0) __hip_atomic_store(&counters[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int RT, int CH>
-__global__ __launch_bounds__(SK3_NT) void skinny3_wide_kernel(const uint8_t* __restrict__ W, const uint32_t* __restrict__ ZS,
-                                                              const half_t* __restrict__ X, half_t* __restrict__ Y,
-                                                              float* part, unsigned* counters, int M, int N, int K,
-                                                              int ksplit, Epilogue epi) {
-    skinny3_wide_body<RT, CH>(W, ZS, X, Y, part, counters, M, N, K, ksplit, epi, blockIdx.x, blockIdx.x, gridDim.x);
-}
-
 template <int MROWS, int RT, int CH, bool LN, int GPC>
 __global__ __launch_bounds__(SK3_NT) void skinny3_kernel(const uint8_t* __restrict__ W, const uint32_t* __restrict__ ZS,
                                                          const half_t* __restrict__ X, half_t* __restrict__ Y,
@@ -981,31 +973,6 @@ static bool wide_fits(long blocks64, int K, bool have_ws, int* ksplit) {
 bool skinny3_wide_applies(int N, int K, bool have_ws) {
     int ks;
     return wide_fits((N + 63) / 64, K, have_ws, &ks);
-}
-
-// The same with the grid it would run: workgroups, and how many of a workgroup's 32 chunk slots its K range fills.
-bool skinny3_wide_shape(int N, int K, bool have_ws, long* workgroups, int* slots_in_use) {
-    int ks;
-    const long blocks64 = (N + 63) / 64;
-    if (!wide_fits(blocks64, K, have_ws, &ks)) return false;
-    *workgroups = blocks64 * ks;
-    *slots_in_use = (K / 128 + ks - 1) / ks;
-    return true;
-}
-
-// ws = the caller's workspace or null (then K is never split); it must hold skinny2_workspace_bytes(M, N, K).
-hipError_t launch_skinny3_wide(const void* x, const void* w, const void* zs, void* y, void* ws, int M, int N, int K,
-                               Epilogue epi, hipStream_t st) {
-    int ksplit;
-    if (M < 1 || M > 32 || !wide_fits((N + 63) / 64, K, ws != nullptr, &ksplit)) return hipErrorInvalidValue;
-    static bool allowed[64];
-    constexpr int lds = Sk3WideLds<4, 4>::BYTES;
-    const hipError_t e = allow_lds(skinny3_wide_kernel<4, 4>, lds, allowed);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((skinny3_wide_kernel<4, 4>), dim3((N + 63) / 64, ksplit), dim3(SK3_NT), lds, st, (const uint8_t*)w,
-                       (const uint32_t*)zs, (const half_t*)x, (half_t*)y,
-                       ws ? (float*)((char*)ws + SK3_COUNTER_BYTES) : nullptr, (unsigned*)ws, M, N, K, ksplit, epi);
-    return hipGetLastError();
 }
 
 hipError_t launch_skinny3_wide_group(const SeqProblem* probs, int count, int M, void* ws, size_t ws_bytes,

@@ -1,0 +1,62 @@
+"""The ring kernel (17 tokens up): every tile shape, K split and group size on ragged M, N and K against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import w4a16_oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def capi(built_lib):
+    from sqamd import capi as c
+    c.lib()
+    return c
+
+
+def to_dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+# (M, N, K, g): one row; a row past a tile; K shorter than a stage, ending inside one, inside 64 columns (group size 32);
+# N inside the first tile, one chunk past a tile; tiles beyond one round of 256 (the last case)
+CASES = [(1, 64, 128, 128), (33, 136, 640, 128), (97, 264, 1408, 128), (128, 256, 2048, 64), (100, 520, 960, 64),
+         (65, 72, 416, 32), (40, 392, 1056, 32), (300, 5128, 384, 128)]
+
+
+@pytest.mark.parametrize("m,n,k,g", CASES)
+@pytest.mark.parametrize("shape", range(1, 9))
+def test_ring_parity(capi, shape, m, n, k, g):
+    d = orc.synth_linear(n, k, g, seed=7 * n + k)
+    w_hat = orc.dequant_l1(d["w_l1"], d["zs_l1"], g)
+    x = orc.synth_x(m, k, seed=m)
+    rng = np.random.default_rng(m + n)
+    bias = rng.normal(0, 1, n).astype(np.float16)
+    res = rng.normal(0, 1, (m, n)).astype(np.float16)
+    x64, w64 = x.astype(np.float64), w_hat.astype(np.float64)
+    ref = np.maximum(x64 @ w64.T + bias.astype(np.float64), 0) + res.astype(np.float64)
+    # one rounding to fp16 and K fp32 additions, each of relative error 2^-24 of the magnitudes that meet
+    bound = 2.0 ** -11 * np.abs(ref) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(bias) + np.abs(res)) + 2.0 ** -24
+    w, zs, xd, bd, rd = to_dev(d["w_l1"]), to_dev(d["zs_l1"]), to_dev(x), to_dev(bias), to_dev(res)
+    ws = torch.zeros(65536 + (96 << 20), dtype=torch.uint8, device=DEV)
+    ran = 0
+    for rest in (0, 0x10):
+        for ks in (1, 2, 3, 8):
+            tune = shape | rest | (ks << 8)
+            y = torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV)
+            args = dict(bias=bd, residual=rd, act=capi.SQ_ACT_RELU, algo=capi.SQ_ALGO_RING | (tune << 8), ws=ws)
+            try:
+                capi.gemm_fused(xd, w, zs, n, k, g, out=y, **args)
+            except capi.SqError:
+                assert ks > 1  # fewer stages than parts, or no rest to split
+                continue
+            ran += 1
+            got = y.cpu().numpy().astype(np.float64)
+            assert np.all(np.abs(got - ref) <= bound), (hex(tune), np.max(np.abs(got - ref) / bound))
+            assert torch.equal(y, capi.gemm_fused(xd, w, zs, n, k, g, **args)), hex(tune)
+            assert capi.workspace_is_clean(ws)
+    assert ran >= 1
+    y = capi.gemm_fused(xd, w, zs, n, k, g, bias=bd, residual=rd, act=capi.SQ_ACT_RELU, algo=capi.SQ_ALGO_RING, ws=ws)
+    assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - ref) <= bound)
