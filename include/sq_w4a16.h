@@ -281,6 +281,15 @@ int sq_w4a16_gemv_sequence_tune(unsigned spin_limit, int loads_in_flight);
 int sq_w4a16_dequant(const void* w, const void* zs, void* out, int N, int K,
                      int group_size, int layout, void* stream);
 
+/* fp16 weight [N, K] -> packed codes and zeros_scales of either layout in one launch, bit for bit what the host packers
+ * (sqamd/quant_funcs.py) give with torch operations on a device tensor: round to nearest per group of group_size along
+ * K, asymmetric.  n_bit 4 or 2 (layout L1: uint8 [N, K*n_bit/8]; layout L2: always the 4-bit words int32 [K, N/8]).
+ * group_size 32, 64 or 128, K % group_size == 0; layout L2 also K % 32 == 0 and N % 32 == 0.  fake (layout L2 only, may
+ * be null): the fake-quantised weight fp16 [N, K].
+ * (reference: test/muxi/utils/quant_funcs.py:75-114, test/nvidia/utils/quant_dequant_nvidia.py:5-32) */
+int sq_w4a16_quantise(const void* w, void* q, void* zs, void* fake, int N, int K, int group_size,
+                      int n_bit, int layout, void* stream);
+
 /* zeros, scales fp16 [N, K/g] (zeros without the +64) -> zs fp16 [K/g, 2N]
  * = pairs (zero + 64, scale).  Replaces transpose_merge_zeros_scales
  * (reference: quantization/nvidia/kernel/gemm_s4_f16/format.cu:206-239). */

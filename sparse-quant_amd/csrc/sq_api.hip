@@ -688,6 +688,20 @@ int sq_w4a16_dequant(const void* w, const void* zs, void* out, int N, int K, int
     return launch_code(sq::launch_dequant_l2(w, zs, out, N, K, group_size, st));
 }
 
+int sq_w4a16_quantise(const void* w, void* q, void* zs, void* fake, int N, int K, int group_size, int n_bit, int layout,
+                      void* stream) {
+    if (layout != SQ_LAYOUT_L1 && layout != SQ_LAYOUT_L2) return SQ_ERR_BAD_LAYOUT;
+    if (group_size != 32 && group_size != 64 && group_size != 128) return SQ_ERR_BAD_GROUP;
+    if (N <= 0 || K <= 0 || K % group_size != 0 || (n_bit != 2 && n_bit != 4)) return SQ_ERR_BAD_SHAPE;
+    if (layout == SQ_LAYOUT_L2 ? (N % 32 != 0 || K > (1 << 22)) : fake != nullptr) return SQ_ERR_BAD_SHAPE;
+    if ((long)N * (long)K > (1L << 40)) return SQ_ERR_BAD_SHAPE;
+    if (!w || !q || !zs) return SQ_ERR_NULL_POINTER;
+    if (!aligned16(w) || !aligned16(q) || !aligned16(zs) || !aligned16(fake)) return SQ_ERR_MISALIGNED;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (layout == SQ_LAYOUT_L1) return launch_code(sq::launch_quantise_l1(w, q, zs, N, K, group_size, n_bit, st));
+    return launch_code(sq::launch_quantise_l2(w, q, zs, fake, N, K, group_size, n_bit, st));
+}
+
 int sq_transpose_merge_zeros_scales(const void* zeros, const void* scales, void* zs, int in_features,
                                     int out_features, int group_size, void* stream) {
     if (in_features <= 0 || out_features <= 0) return SQ_ERR_BAD_SHAPE;

@@ -13,6 +13,10 @@ namespace sq {
 hipError_t launch_dequant_l1(const void* w, const void* zs, void* out, int N, int K, int g, hipStream_t st);
 hipError_t launch_dequant_l2(const void* w, const void* zs, void* out, int N, int K, int g, hipStream_t st);
 
+// sq_quantize.hip: fp16 [N, K] -> packed codes and zeros_scales, one launch.  g in {32, 64, 128}, bits 2 or 4.
+hipError_t launch_quantise_l1(const void* w, void* q, void* zs, int N, int K, int g, int bits, hipStream_t st);
+hipError_t launch_quantise_l2(const void* w, void* q, void* zs, void* fake, int N, int K, int g, int bits, hipStream_t st);
+
 // sq_repack.hip
 hipError_t launch_transpose_merge_zeros_scales(const void* zeros, const void* scales, void* zs, int K, int N,
                                                int g, hipStream_t st);

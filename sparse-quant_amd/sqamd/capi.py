@@ -38,6 +38,7 @@ SIGNATURES = {
     "sq_workspace_reset": (_i, [_vp, ctypes.c_size_t, _vp]),
     "sq_workspace_check": (_i, [_vp, ctypes.c_size_t, _vp]),
     "sq_w4a16_dequant": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
+    "sq_w4a16_quantise": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "sq_transpose_merge_zeros_scales": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "sq_convert_ours_to_awq": (_i, [_vp, _vp, _i, _i, _vp]),
     "sq_convert_awq_to_lmdeploy": (_i, [_vp, _vp, _i, _i, _vp]),
@@ -336,6 +337,22 @@ def dequant(w, zs, n, k, group_size, layout=SQ_LAYOUT_L1, stream=None):
     _check(lib().sq_w4a16_dequant(_ptr(w), _ptr(zs), _ptr(out), n, k, group_size, layout, _stream(stream)),
            "sq_w4a16_dequant")
     return out
+
+
+def quantise(w, group_size, n_bit=4, layout=SQ_LAYOUT_L1, want_fake=False, stream=None):
+    """w fp16 [N, K] -> (packed codes, zeros_scales, fake-quantised weight or None); layout L2: 4-bit words."""
+    n, k = w.shape
+    if layout == SQ_LAYOUT_L1:
+        q = torch.empty((n, k * n_bit // 8), dtype=torch.uint8, device=w.device)
+        zs = torch.empty((n, 2 * (k // group_size)), dtype=torch.float16, device=w.device)
+    else:
+        q = torch.empty((k, n // 8), dtype=torch.int32, device=w.device)
+        zs = torch.empty((k // group_size, 2 * n), dtype=torch.float16, device=w.device)
+    fake = torch.empty((n, k), dtype=torch.float16, device=w.device) if want_fake else None
+    with torch.cuda.device(w.device):
+        _check(lib().sq_w4a16_quantise(_ptr(w), _ptr(q), _ptr(zs), _ptr(fake), n, k, group_size, n_bit, layout,
+                                       _stream(stream)), "sq_w4a16_quantise")
+    return q, zs, fake
 
 
 def transpose_merge_zeros_scales(zeros, scales, in_features, out_features, group_size, stream=None):

@@ -89,16 +89,15 @@ class WALinear(nn.Module):
     def from_float(module, w_config, a_config=None, quantize_output=False, layout="l1"):
         assert isinstance(module, nn.Linear)
         n_bit, g = w_config["n_bit"], w_config["group_size"]
+        # every buffer is replaced below: on the meta device the constructor's zeros cost no fills
         new = WALinear(module.in_features, module.out_features, w_config, a_config, w_bit=n_bit, group_size=g,
-                       bias=module.bias is not None, quantize_output=quantize_output, dev=module.weight.device,
-                       layout=layout)
+                       bias=module.bias is not None, quantize_output=quantize_output, dev="meta", layout=layout)
         if layout == "l1":
             new.weight, new.zeros_scales = quant_funcs.quant_muxi(module.weight.data, module.in_features,
                                                                   module.out_features, n_bit=n_bit, group_size=g)
         else:
-            new.weight, new.zeros_scales, _ = quant_funcs.quant_lmdeploy(module.weight.data, module.in_features,
-                                                                         module.out_features, group_size=g,
-                                                                         n_bit=n_bit)
+            new.weight, new.zeros_scales, _ = quant_funcs._lmdeploy(module.weight.data, module.in_features,
+                                                                    module.out_features, g, n_bit, want_fake=False)
         if module.bias is not None:
             new.bias = module.bias.data.half().unsqueeze(0)
         return new

@@ -2,7 +2,7 @@
 
 Mirror of the reference's Python packers (same names, same arguments, same
 tensors out), written with vectorised torch ops so they run on the device the
-weight lives on:
+weight lives on (an fp16 weight on the GPU takes one kernel instead, same bits):
 
     quant_muxi      test/muxi/utils/quant_funcs.py:75-83   (layout L1, uint8 [N, K*b/8])
     quant_lmdeploy  test/nvidia/utils/quant_dequant_nvidia.py:5-32 (layout L2, int32 [K, N/8])
@@ -17,6 +17,9 @@ weight are bit-identical to the reference's; pass `compute_dtype=torch.float32` 
 quantise an fp16 weight in fp32 instead.
 """
 import torch
+from torch.autograd import forward_ad
+
+from . import capi
 
 
 def quantize_tensor(w, n_bit, q_group_size):
@@ -69,6 +72,25 @@ def _as(weight, compute_dtype):
     return weight if compute_dtype is None else weight.to(compute_dtype)
 
 
+def _one_launch(weight, n_bit, group_size, layout):
+    """Whether the packing kernel takes this weight: a plain fp16 [N, K] device tensor, dense and 16-byte aligned, with a
+    group size the kernel is built for, and nothing that has to see the torch operations (autograd, function transforms,
+    tracing).  Everything else is packed by the torch operations below, which also raise what a bad call raises."""
+    if type(weight) not in (torch.Tensor, torch.nn.Parameter) or weight.dtype != torch.float16 or weight.dim() != 2:
+        return False
+    if not weight.is_cuda or weight.numel() == 0 or not weight.is_contiguous():
+        return False
+    if (weight.requires_grad and torch.is_grad_enabled()) or forward_ad._current_level >= 0:
+        return False
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or \
+            torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    n, k = weight.shape
+    if n_bit not in (2, 4) or group_size not in (32, 64, 128) or k % group_size != 0 or weight.data_ptr() % 16 != 0:
+        return False
+    return layout == capi.SQ_LAYOUT_L1 or (n % 32 == 0 and k <= 1 << 22)
+
+
 def quant_muxi(weight, input_features, output_features, n_bit=4, group_size=64, compute_dtype=None):
     """fp16 weight [N, K] -> (qweight uint8 [N, K*n_bit/8], zeros_scales fp16 [N, 2K/g]) in layout L1.
 
@@ -76,6 +98,8 @@ def quant_muxi(weight, input_features, output_features, n_bit=4, group_size=64, 
     scales are the same as those of the un-permuted weight.
     """
     assert weight.shape == (output_features, input_features)
+    if compute_dtype in (None, torch.float16) and _one_launch(weight, n_bit, group_size, capi.SQ_LAYOUT_L1):
+        return capi.quantise(weight, group_size, n_bit)[:2]
     q, scales, zeros = quantize_tensor(_as(weight, compute_dtype), n_bit, group_size)
     q = interleave_k(q)
     if n_bit == 4:
@@ -110,10 +134,18 @@ def quant_lmdeploy(weight, input_features, output_features, group_size=128, n_bi
     four levels and passes the words through convert_4bit_to_2bit as the reference does (:29-30),
     which returns int32 [K, N/16].
     """
+    return _lmdeploy(weight, input_features, output_features, group_size, n_bit, compute_dtype)
+
+
+def _lmdeploy(weight, input_features, output_features, group_size, n_bit, compute_dtype=None, want_fake=True):
     import quant
 
     if n_bit not in (2, 4):
         raise ValueError("n_bit must be 2 or 4")
+    if compute_dtype in (None, torch.float16) and weight.shape == (output_features, input_features) and \
+            _one_launch(weight, n_bit, group_size, capi.SQ_LAYOUT_L2):
+        qweight, zeros_scales, w_fp16 = capi.quantise(weight, group_size, n_bit, capi.SQ_LAYOUT_L2, want_fake)
+        return (convert_4bit_to_2bit(qweight) if n_bit == 2 else qweight), zeros_scales, w_fp16
     w = _as(weight, compute_dtype)
     q, scales, zeros = quantize_tensor(w, n_bit, group_size)
     g = group_size
