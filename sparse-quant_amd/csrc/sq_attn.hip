@@ -7,301 +7,345 @@
 // sparse_attention_prefill_fwd_p, sparse-attention/muxi/playground/kernels/csrc/include/
 // block_sparse_attention_lut.cuh:30-236)
 //
-// Mapping.  A workgroup (4 waves) owns one 64-row query block of one (batch, head);
-// wave w owns queries 16w .. 16w+15.  Both products are computed transposed with
-// v_mfma_f32_16x16x32_f16 so that a lane always owns ONE query (column l%16):
-//   S^T = K Q^T : A = K tile (row = key, from LDS), B = Q^T (registers, pre-scaled by
-//                 sm_scale*log2(e) and rounded to fp16 like the reference);
-//                 D: lane (query l%16) holds keys 16t + 4*(l/16) + v of key tile t.
-//   softmax     : over a lane's 16 values and the 4 lanes {l, l^16, l^32, l^48}; the
-//                 reference maximum of a query lives in its lanes and moves lazily (only when
-//                 a score exceeds it by more than 2^8), the row sum stays split over the four
-//                 lanes until the end: in the common case nothing is exchanged or rescaled.
-//   O^T = V^T P^T: B = P^T is exactly what the lane already holds: for the k-step
-//                 covering keys 32s .. 32s+31 lane group g supplies keys 32s+4g+{0..3}
-//                 and 32s+16+4g+{0..3}; A = V^T rows read from an LDS copy of the V
-//                 tile that was transposed while staging (two 64-bit reads);
-//                 D: lane (query l%16) holds head-dim rows 16*dt + 4*(l/16) + v.
-// K and V tiles are staged once per block for the four waves (global -> registers one
-// visited block ahead -> LDS); V is transposed on the way in (each thread packs two
-// adjacent keys into 32-bit LDS writes).
+// Mapping.  A workgroup of two waves owns one 64-row query block of one (batch, head) and goes through the visited
+// blocks in steps of 32 keys; a wave owns 32 queries.  Both products are computed transposed with
+// v_mfma_f32_32x32x16_f16 so that a lane always owns ONE query (column l % 32):
+//   S^T = K Q^T : A = K tile (row = key, 128-bit LDS reads), B = Q^T (registers, as given);
+//                 D: lane holds keys 8 (v / 4) + 4 (l / 32) + v % 4 of the 32.  The scores are scaled in fp32.
+//   softmax     : over a lane's 16 values and the lane pair {l, l ^ 32}; the reference maximum of a query moves
+//                 lazily (only when a score exceeds it by more than 2^8), the row sum stays split over the lane
+//                 pair until the end: in the common case nothing is exchanged or rescaled.
+//   O^T = V^T P^T: B = P^T is what the lane already holds, keys in that order; A = V^T by transposing 64-bit LDS
+//                 reads (ds_read_b64_tr_b16: four keys of one column per lane) of the V tile as it lies in memory.
+// K and V tiles go global -> LDS by direct loads, one step ahead, and are never touched by vector instructions on
+// the way; the 16-byte chunks of a row are permuted by the lane that requests them so that the operand reads of
+// neighbouring rows fall on different banks.  The visited blocks of a row come from the table 64 entries at a time,
+// in one load: which of them are padding is a ballot, so no step waits for the table.
+//
+// What bounds it.  Per step of D = 128 a wave needs 512 cycles of its matrix pipe and about 600 of vector issue (16
+// exponentials at a quarter of the rate among them); the operand reads take 512 LDS cycles per 64 x 64 block (32
+// queries per wave: each K and V value is read twice; with 16 per wave it is four times, and 1024 cycles were the
+// bound).  Four workgroups of 32 KB share a CU, two waves per SIMD, each at its own point of the step, so that one's
+// softmax and first loads run beside another's products; four waves on one 64-key step (64 KB, the key halves of a
+// query merged at the end) were 20 % slower, for the time a workgroup takes to start and end is not hidden there.
+// Measured (us; before: 16 queries per wave, K through registers, V transposed by vector instructions):
+//   32 heads x 4096 x 128, causal, 26 % of the blocks   115 -> 86 (matrix pipes busy 0.39 of the cycles)
+//   8 x 32 heads x 512 x 128, causal, 26 %               35 -> 35 (134 MB to move: 22 at the rate of a copy)
+//   8 x 16 heads x 512 x 64, 25 %                        10.1 -> 9.4
 #include "sq_common.h"
 #include "sq_kernels.h"
 
+#include <type_traits>
+
 namespace sq {
 
-#ifndef SQ_ATTN_KPAD
-#define SQ_ATTN_KPAD 16
-#endif
-#ifndef SQ_ATTN_VPAD
-#define SQ_ATTN_VPAD 12
-#endif
+namespace {
 
-// QT = 16-query tiles per wave: the workgroup has 4 / QT waves, and every K / V operand read
-// from LDS feeds QT matrix instructions.  QT = 2 was measured (3 % slower at D = 64, 30 %
-// slower at D = 128, where it needs more than 256 registers); QT = 1 is what is launched.
-template <int D, int QT>
-__global__ __launch_bounds__(256 / QT) void lut_attn_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ Kp,
-                                                            const half_t* __restrict__ V, half_t* __restrict__ O,
-                                                            const void* __restrict__ lut, int lut_is_64, int H, int S,
-                                                            int nblk_q, int nnz, int nvisit, float qk_scale,
-                                                            int causal, int total_wg) {
-    constexpr int NT = 256 / QT;                 // threads per workgroup
-    constexpr int KP = D + SQ_ATTN_KPAD;         // halves per row of the K tile in LDS
-    constexpr int VP = 64 + SQ_ATTN_VPAD;        // halves per row of the transposed V tile in LDS
-    constexpr int DK = D / 32;                   // k-steps of S^T
-    constexpr int DT = D / 16;                   // row tiles of O^T
-    constexpr int KPASS = (64 * D / 8) / NT;     // 16-byte words of the K tile per thread
-    constexpr int VPASS = (32 * D / 8) / NT;     // key pairs x 8 head-dim values of the V tile per thread
-    __shared__ __attribute__((aligned(16))) half_t ks[64 * KP];
-    __shared__ __attribute__((aligned(16))) half_t vt[D * VP];
+struct LutAttnArgs {
+    const half_t* q;
+    const half_t* k;
+    const half_t* v;
+    half_t* o;
+    const void* lut;
+    int lut_is_64, H, S, nblk, nnz, nvisit;
+    float qk_scale;  // sm_scale * log2(e)
+    int causal, total_wg;
+};
+
+// Chunk permutations inside a tile row of D halves (D / 8 chunks of 16 bytes).
+// K is read 128 bits wide by 32 lanes = rows at one chunk: 16 consecutive rows (256 bytes of LDS banks) must differ.
+template <int D>
+__device__ __forceinline__ int k_swz(int row) {
+    return D == 128 ? (row & 15) : ((row & 7) ^ ((row >> 3) & 1));
+}
+// V is read 64 bytes of a row by 8 lanes, four consecutive rows by a transposing read: the rows' 64-byte pieces must differ.
+template <int D>
+__device__ __forceinline__ int v_swz(int row) {
+    return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1);
+}
+
+typedef short short4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ short4_t lds_read_tr(const uint8_t* p) {
+    typedef __attribute__((address_space(3))) short4_t* lp;
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p));
+}
+
+template <int D>
+__global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
+    constexpr int ROW = D * 2;              // bytes of a tile row
+    constexpr int TILE = 32 * ROW;          // K or V of one step: 32 keys
+    constexpr int SB = 2 * TILE;            // a stage: K tile, V tile
+    constexpr int NK = D / 16;              // matrix steps of S^T
+    constexpr int DT = D / 32;              // 32-row tiles of O^T
+    constexpr int NL = TILE / 1024 / 2;     // direct loads per wave, operand and stage
+    constexpr int RPL = 1024 / ROW;         // tile rows per load
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * SB];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int lq = lane & 15;
-    const int g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ln = lane & 31;
+    const int lc = lane >> 5;
     // Workgroups are handed to the eight XCDs round-robin by their linear id, and every XCD has its own L2.
     // The id is therefore re-read as (XCD, slot): XCD x works through the x-th eighth of the (head, query block)
     // list, so that all query blocks of a head, which visit the same K and V rows, share one L2
-    // instead of pulling those rows into all eight.
-    const int per_xcd = (total_wg + 7) >> 3;
+    // instead of pulling those rows into all eight.  Causal: the long rows first.
+    const int per_xcd = (a.total_wg + 7) >> 3;
     const int work = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (work >= total_wg) return;
-    const int qb = work % nblk_q;
-    const int zh = work / nblk_q;
-    const int h = zh % H;
+    if (work >= a.total_wg) return;
+    const int zh = work / a.nblk;
+    const int qr = work - zh * a.nblk;
+    const int qb = a.causal ? a.nblk - 1 - qr : qr;
+    const int h = zh % a.H;
+    const int S = a.S;
     const long base = (long)zh * S * D;
-    int m[QT];  // this lane's queries
-#pragma unroll
-    for (int qt = 0; qt < QT; qt++) m[qt] = qb * 64 + 16 * (QT * wave + qt) + lq;
+    const int m = qb * 64 + 32 * wave + ln;  // this lane's query
 
-    // Q^T operands: q * (sm_scale * log2 e), rounded to fp16.
-    half8_t qf[QT][DK];
+    half8_t qf[NK];
+    {
+        const half_t* qp = a.q + base + (long)imin(m, S - 1) * D + 8 * lc;
 #pragma unroll
-    for (int qt = 0; qt < QT; qt++)
-#pragma unroll
-        for (int s = 0; s < DK; s++) {
-            const half8_t raw = *(const half8_t*)(Q + base + (long)imin(m[qt], S - 1) * D + 32 * s + 8 * g);
-#pragma unroll
-            for (int e = 0; e < 8; e++) qf[qt][s][e] = (half_t)((float)raw[e] * qk_scale);
-        }
-
-    float m_i[QT], l_i[QT];
-    float4_t acc[QT][DT];
-#pragma unroll
-    for (int qt = 0; qt < QT; qt++) {
-        m_i[qt] = -INFINITY;
-        l_i[qt] = 0.f;
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) acc[qt][dt] = (float4_t){0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < NK; s++) qf[s] = *(const half8_t*)(qp + 16 * s);
     }
 
-    const long lut_row = ((long)h * nblk_q + qb) * nnz;
-    // Tiles travel global -> registers -> LDS; the registers of the next visited block are
-    // requested before the current block is consumed, so their latency hides behind it.
-    u32x4_t kreg[KPASS];
-    half8_t v0reg[VPASS], v1reg[VPASS];
-    auto fetch = [&](int n0) {
-        // K tile: 64 keys x D halves, 16 bytes per thread per pass.
-#pragma unroll
-        for (int p = 0; p < KPASS; p++) {
-            const int idx = tid + NT * p;
-            const int key = idx / (D / 8);
-            const int c8 = idx % (D / 8);
-            kreg[p] = *(const u32x4_t*)(Kp + base + (long)imin(n0 + key, S - 1) * D + 8 * c8);
+    // The visited blocks, 64 table entries at a time: lane j holds entry j, `todo` has a bit for each that is visited.
+    const long lut_row = ((long)h * a.nblk + qb) * a.nnz;
+    int entry = 0, jbase = 0, last = -1;
+    uint64_t todo = 0;
+    auto next_block = [&]() {  // its first key, or -1
+        while (todo == 0) {
+            if (jbase >= a.nvisit) return -1;
+            const int j = jbase + lane;
+            int blk = -1;
+            if (j < a.nvisit) blk = a.lut_is_64 ? (int)((const long long*)a.lut)[lut_row + j] : ((const int*)a.lut)[lut_row + j];
+            const int up = __shfl_up(blk, 1);
+            const int prev = lane == 0 ? last : up;
+            todo = __builtin_amdgcn_ballot_w64(blk != prev && blk >= 0 && (long)blk * 64 < S);
+            entry = blk;
+            last = __builtin_amdgcn_readlane(blk, 63);
+            jbase += 64;
         }
-        // V tile: a thread takes keys 2kp, 2kp+1 and 8 head-dim values.
+        const int j = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        return __builtin_amdgcn_readlane(entry, j) * 64;
+    };
+    int n0 = next_block();
+
+    // Byte offsets of this wave's loads inside a step; load j covers tile rows RPL * (NL * wave + j) .. + RPL - 1.
+    const int lrow = lane / (D / 8);
+    const int lchunk = lane % (D / 8);
+    auto lane_offset = [&](int j, int row_max, bool is_v) {
+        const int row = RPL * (NL * wave + j) + lrow;
+        const int c = lchunk ^ (is_v ? v_swz<D>(row) : k_swz<D>(row));
+        return (uint32_t)(imin(row, row_max) * ROW + c * 16);
+    };
+    uint32_t koff[NL], voff[NL];
 #pragma unroll
-        for (int p = 0; p < VPASS; p++) {
-            const int idx = tid + NT * p;
-            const int kp = idx & 31;
-            const int c8 = idx >> 5;
-            v0reg[p] = *(const half8_t*)(V + base + (long)imin(n0 + 2 * kp, S - 1) * D + 8 * c8);
-            v1reg[p] = *(const half8_t*)(V + base + (long)imin(n0 + 2 * kp + 1, S - 1) * D + 8 * c8);
+    for (int j = 0; j < NL; j++) {
+        koff[j] = lane_offset(j, 31, false);
+        voff[j] = lane_offset(j, 31, true);
+    }
+    auto issue = [&](int n, int slot) {
+        const uint8_t* kb = (const uint8_t*)(a.k + base + (long)n * D);
+        const uint8_t* vb = (const uint8_t*)(a.v + base + (long)n * D);
+        const uint32_t l0 = lds0 + slot * SB + wave * (NL * 1024);
+        if (n + 32 <= S) {
+#pragma unroll
+            for (int j = 0; j < NL; j++) load_to_lds_x4(kb, koff[j], l0 + j * 1024);
+#pragma unroll
+            for (int j = 0; j < NL; j++) load_to_lds_x4(vb, voff[j], l0 + TILE + j * 1024);
+        } else {  // rows past the end re-read the last one (their scores are masked)
+#pragma unroll
+            for (int j = 0; j < NL; j++) load_to_lds_x4(kb, lane_offset(j, S - 1 - n, false), l0 + j * 1024);
+#pragma unroll
+            for (int j = 0; j < NL; j++) load_to_lds_x4(vb, lane_offset(j, S - 1 - n, true), l0 + TILE + j * 1024);
         }
     };
-    auto stash = [&]() {
+    if (n0 >= 0) issue(n0, 0);
+
+    // LDS byte offsets of the operand reads.
+    int kread[NK], vread[DT];
 #pragma unroll
-        for (int p = 0; p < KPASS; p++) {
-            const int idx = tid + NT * p;
-            const int key = idx / (D / 8);
-            const int c8 = idx % (D / 8);
-            *(u32x4_t*)(&ks[key * KP + 8 * c8]) = kreg[p];
-        }
-        // V transposed: 8 packed pairs vt[d][2kp .. 2kp+1] per pass.
+    for (int s = 0; s < NK; s++) kread[s] = ln * ROW + (((2 * s + lc) ^ k_swz<D>(ln)) * 16);
+    {
+        const int key = 4 * lc + ((lane & 15) >> 2);  // + 16 s + 8 i, which leave v_swz unchanged
 #pragma unroll
-        for (int p = 0; p < VPASS; p++) {
-            const int idx = tid + NT * p;
-            const int kp = idx & 31;
-            const int c8 = idx >> 5;
+        for (int dt = 0; dt < DT; dt++)
+            vread[dt] = TILE + key * ROW + (((4 * dt + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ v_swz<D>(key)) * 16) +
+                        8 * (lane & 1);
+    }
+
+    // Reference maximum of the query (0 while unset), the score above it at which it moves (any score while unset), and
+    // this lane's share of the row sum.
+    constexpr float LAZY = 8.f;
+    float ref = 0.f, limit = -INFINITY, l_i = 0.f;
+    float16_t acc[DT];
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const half2_t pr = {v0reg[p][e], v1reg[p][e]};
-                *(half2_t*)(&vt[(8 * c8 + e) * VP + 2 * kp]) = pr;
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[dt][v] = 0.f;
+
+    // Step n from slot SLOT; `next` (or -1) is requested into the other one.
+    auto visit = [&](int n, auto slot_, int next) {
+        constexpr int SLOT = decltype(slot_)::value;
+        const uint8_t* l = lds + SLOT * SB;
+        float16_t st;
+#pragma unroll
+        for (int v = 0; v < 16; v++) st[v] = 0.f;
+        // All K operands are requested at once, and all V operands ahead of the softmax: a wave has one other wave on its
+        // SIMD to hide LDS latency behind, which is not enough for a read per product.
+        half8_t kf[NK];
+#pragma unroll
+        for (int s = 0; s < NK; s++) kf[s] = *(const half8_t*)(l + kread[s]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (next >= 0) issue(next, 1 - SLOT);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < NK; s++) st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s], qf[s], st, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        short4_t vf[2][DT][2];
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) vf[s][dt][i] = lds_read_tr(l + vread[dt] + (16 * s + 8 * i) * ROW);
+        __builtin_amdgcn_sched_barrier(0);
+        // scores relative to the reference maximum, in units of log2
+#pragma unroll
+        for (int v = 0; v < 16; v++) st[v] = __builtin_fmaf(st[v], a.qk_scale, -ref);
+        // Masks (only where the step touches the end of the sequence or the causal diagonal; the test is uniform).
+        if (n + 32 > S || (a.causal && n + 31 > qb * 64 + 32 * wave)) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int key = n + 8 * (v >> 2) + 4 * lc + (v & 3);
+                const bool keep = (key < S) && (!a.causal || key <= m);
+                st[v] = keep ? st[v] : -INFINITY;
             }
         }
-    };
-    // Next visited block (first key index) or -1; a LUT entry equal to its predecessor is
-    // padding.  Uniform over the workgroup.
-    int jn = 0, last = -1;
-    auto advance = [&]() {
-        while (jn < nvisit) {
-            const int blk = lut_is_64 ? (int)((const long long*)lut)[lut_row + jn] : ((const int*)lut)[lut_row + jn];
-            jn++;
-            const bool skip = (blk == last) || blk < 0 || (long)blk * 64 >= S;
-            last = blk;
-            if (!skip) return blk * 64;
+        // The reference maximum of a query moves only when a score exceeds it by more than 2^LAZY (or when it is still
+        // unset): until then p = exp2(score) stays below 2^LAZY, well inside fp16, the final O = acc / l does not depend
+        // on the reference, and neither the accumulators nor the scores need rescaling.  The test is made per lane and
+        // voted over the wave; the maximum over a query's two lanes is formed only when it is needed.
+        float mx = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 16; v++) mx = fmaxf(mx, st[v]);
+        if (__builtin_amdgcn_ballot_w64(mx > limit) != 0) {
+            const float mq = fmaxf(mx, __shfl_xor(mx, 32));
+            const bool upd = mq > limit;
+            const float delta = upd ? mq : 0.f;
+            // a query without a reference so far has l = 0 and acc = 0: nothing to rescale
+            const float alpha = (upd && limit == LAZY) ? __builtin_amdgcn_exp2f(-delta) : 1.f;
+            ref += delta;
+            limit = upd ? LAZY : limit;
+            l_i *= alpha;
+#pragma unroll
+            for (int v = 0; v < 16; v++) st[v] -= delta;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[dt][v] *= alpha;
         }
-        return -1;
+        // p = exp2(score) (bare v_exp_f32: exp2(-inf) = 0 for masked entries), rounded to fp16 for the second product
+        // like the reference; the lane's share of the row sum is taken from the rounded pairs with one dot instruction
+        // per pair and stays in the lane until the end.
+        half8_t pk[2];
+        float rs = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) {
+            const half2_t pp = {(half_t)__builtin_amdgcn_exp2f(st[v]), (half_t)__builtin_amdgcn_exp2f(st[v + 1])};
+            rs = __builtin_amdgcn_fdot2(pp, (half2_t){(half_t)1.f, (half_t)1.f}, rs, false);
+            pk[v >> 3][v & 7] = pp.x;
+            pk[v >> 3][(v & 7) + 1] = pp.y;
+        }
+        l_i += rs;
+        // O^T += V^T P^T
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+                const u32x2_t lo2 = bit_cast<u32x2_t>(vf[s][dt][0]), hi2 = bit_cast<u32x2_t>(vf[s][dt][1]);
+                const u32x4_t vt = {lo2.x, lo2.y, hi2.x, hi2.y};
+                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bit_cast<half8_t>(vt), pk[s], acc[dt], 0, 0, 0);
+            }
     };
 
-    int n0 = advance();
-    if (n0 >= 0) fetch(n0);
+    // One barrier per step: behind it this step's tiles have landed for both waves and nobody reads the other slot any
+    // more, which the next step's loads may then fill.
+    auto landed = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    // The query operands are waited for here, together with the first tiles: left to the loop, the compiler's wait for
+    // them would sit at the first product and drain the direct loads, which it cannot count, on every iteration.
+#pragma unroll
+    for (int s = 0; s < NK; s++) {
+        u32x4_t t = bit_cast<u32x4_t>(qf[s]);
+        asm volatile("" : "+v"(t));
+        qf[s] = bit_cast<half8_t>(t);
+    }
     while (n0 >= 0) {
-        __syncthreads();  // the previous tiles are no longer read
-        stash();
-        __syncthreads();
-        const int n1 = advance();
-        if (n1 >= 0) fetch(n1);
-
-        // S^T = K Q^T for the four 16-key tiles; a K operand serves all QT query tiles.  The accumulators
-        // start at -m_ref of the lane's query, so the matrix core delivers the scores already shifted by
-        // the reference maximum and the softmax needs no subtraction.
-        float4_t st[QT][4];
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-#pragma unroll
-            for (int qt = 0; qt < QT; qt++) {
-                const float c = (m_i[qt] == -INFINITY) ? 0.f : -m_i[qt];
-                st[qt][t] = (float4_t){c, c, c, c};
-            }
-#pragma unroll
-            for (int s = 0; s < DK; s++) {
-                const half8_t a = *(const half8_t*)(&ks[(16 * t + lq) * KP + 32 * s + 8 * g]);
-#pragma unroll
-                for (int qt = 0; qt < QT; qt++)
-                    st[qt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qf[qt][s], st[qt][t], 0, 0, 0);
-            }
-        }
-        // Masks (only where the block touches the end of the sequence or the causal diagonal;
-        // the test is uniform over the workgroup).
-        const bool need_mask = (n0 + 64 > S) || (causal && n0 + 63 > qb * 64);
-        half8_t pk[QT][2];
-#pragma unroll
-        for (int qt = 0; qt < QT; qt++) {
-            if (need_mask) {
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int n = n0 + 16 * t + 4 * g + v;
-                        const bool keep = (n < S) && (!causal || n <= m[qt]);
-                        st[qt][t][v] = keep ? st[qt][t][v] : -INFINITY;
-                    }
-            }
-            // Largest shifted score of this lane.  The reference maximum m_ref of a query moves only when a
-            // score exceeds it by more than 2^LAZY (or when it is still unset): until then p = exp2(s - m_ref)
-            // stays below 2^LAZY, well inside fp16, the final O = acc / l does not depend on the reference,
-            // and neither the accumulators nor the scores need rescaling.  The test is made per lane and
-            // voted over the wave; the maximum over a query's four lanes is formed only when it is needed.
-            constexpr float LAZY = 8.f;
-            float mx = -INFINITY;
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) mx = fmaxf(mx, st[qt][t][v]);
-            const bool unset = (m_i[qt] == -INFINITY);
-            if (__builtin_amdgcn_ballot_w64(mx > LAZY || (unset && mx > -INFINITY)) != 0) {
-                float mq = fmaxf(mx, __shfl_xor(mx, 16));
-                mq = fmaxf(mq, __shfl_xor(mq, 32));
-                const bool upd = mq > LAZY || (unset && mq > -INFINITY);
-                const float delta = upd ? mq : 0.f;
-                // a query without a reference so far has l = 0 and acc = 0: nothing to rescale
-                const float alpha = (upd && !unset) ? __builtin_amdgcn_exp2f(-delta) : 1.f;
-                m_i[qt] = upd ? (unset ? delta : m_i[qt] + delta) : m_i[qt];
-                l_i[qt] *= alpha;
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) st[qt][t][v] -= delta;
-#pragma unroll
-                for (int dt = 0; dt < DT; dt++) acc[qt][dt] *= alpha;
-            }
-            // p = exp2(shifted score) (bare v_exp_f32: exp2(-inf) = 0 for masked entries), rounded to fp16
-            // for the second product like the reference; the lane's share of the row sum is taken from the
-            // rounded pairs with one dot instruction per pair and stays in the lane until the end.
-            float rs = 0.f;
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int v = 0; v < 4; v += 2) {
-                    const half2_t pp = {(half_t)__builtin_amdgcn_exp2f(st[qt][t][v]),
-                                        (half_t)__builtin_amdgcn_exp2f(st[qt][t][v + 1])};
-                    rs = __builtin_amdgcn_fdot2(pp, (half2_t){(half_t)1.f, (half_t)1.f}, rs, false);
-                    pk[qt][t >> 1][4 * (t & 1) + v] = pp.x;
-                    pk[qt][t >> 1][4 * (t & 1) + v + 1] = pp.y;
-                }
-            l_i[qt] += rs;
-        }
-
-        // O^T += V^T P^T; a V operand serves all QT query tiles.
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) {
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-                const half_t* vp = &vt[(16 * dt + lq) * VP + 32 * s + 4 * g];
-                const u32x2_t lo = *(const u32x2_t*)(vp);
-                const u32x2_t hi = *(const u32x2_t*)(vp + 16);
-                const u32x4_t a = {lo.x, lo.y, hi.x, hi.y};
-#pragma unroll
-                for (int qt = 0; qt < QT; qt++)
-                    acc[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bit_cast<half8_t>(a), pk[qt][s], acc[qt][dt],
-                                                                         0, 0, 0);
-            }
-        }
+        const int n1 = next_block();
+        const bool whole = n0 + 32 < S;  // the block has a second half
+        landed();
+        visit(n0, std::integral_constant<int, 0>{}, whole ? n0 + 32 : -1);
+        landed();
+        if (whole)
+            visit(n0 + 32, std::integral_constant<int, 1>{}, n1);
+        else if (n1 >= 0)
+            issue(n1, 0);
         n0 = n1;
     }
 
-    // O[m][16*dt + 4g + v] = acc / l.
+    // The row sum of a query is split over its two lanes.  A query row without any visible key has l = 0 and acc = 0:
+    // 0 * inf = NaN, which is also what the reference's running sums produce for such a row.
+    const float inv = 1.f / (l_i + __shfl_xor(l_i, 32));
+    // The wave's 32 x D outputs leave through its part of LDS (16-byte chunks permuted like K's) as whole rows: a lane
+    // holds four columns at a time, and 8-byte stores would cost the L2 eight times the write requests.
+    __syncthreads();
+    uint8_t* out = lds + wave * TILE;
 #pragma unroll
-    for (int qt = 0; qt < QT; qt++) {
-        // the row sum of a query is spread over its four lanes
-        float l = l_i[qt] + __shfl_xor(l_i[qt], 16);
-        l += __shfl_xor(l, 32);
-        if (m[qt] < S) {
-            // A query row without any visible key has l = 0 and acc = 0: 0 * inf = NaN, which is
-            // also what the reference's running sums produce for such a row.
-            const float inv = 1.f / l;
+    for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-            for (int dt = 0; dt < DT; dt++) {
-                half4_t o;
+        for (int i = 0; i < 4; i++) {
+            half4_t o;
 #pragma unroll
-                for (int v = 0; v < 4; v++) o[v] = (half_t)(acc[qt][dt][v] * inv);
-                *(half4_t*)(O + base + (long)m[qt] * D + 16 * dt + 4 * g) = o;
-            }
+            for (int j = 0; j < 4; j++) o[j] = (half_t)(acc[dt][4 * i + j] * inv);
+            *(half4_t*)(out + ln * ROW + (((4 * dt + i) ^ k_swz<D>(ln)) * 16) + 8 * lc) = o;
         }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < TILE / 1024; j++) {
+        const int row = RPL * j + lrow;
+        const u32x4_t t = *(const u32x4_t*)(out + row * ROW + ((lchunk ^ k_swz<D>(row)) * 16));
+        const int mr = qb * 64 + 32 * wave + row;
+        if (mr < S) *(u32x4_t*)(a.o + base + (long)mr * D + 8 * lchunk) = t;
     }
 }
+
+}  // namespace
 
 hipError_t launch_lut_attention(const void* q, const void* k, const void* v, void* o, const void* lut,
                                 int lut_elem_bytes, int Z, int H, int S, int D, int nnz, float sm_scale, int causal,
                                 hipStream_t st) {
-    const int nblk = (S + 63) / 64;
-    const int total_wg = nblk * Z * H;
-    const dim3 grid(((total_wg + 7) / 8) * 8);
-    const float qk_scale = sm_scale * 1.44269504f;
-    const int use_nnz = nnz < nblk ? nnz : nblk;  // the reference clamps NNZ to ceil(S / 64) as well
-    // (the LUT row pitch stays nnz even when fewer entries are visited)
-#define SQ_ATTN_LAUNCH(D_, QT_)                                                                                   \
-    hipLaunchKernelGGL((lut_attn_kernel<D_, QT_>), grid, dim3(256 / QT_), 0, st, (const half_t*)q, (const half_t*)k, \
-                       (const half_t*)v, (half_t*)o, lut, lut_elem_bytes == 8, H, S, nblk, nnz, use_nnz, qk_scale,   \
-                       causal, total_wg)
+    LutAttnArgs a;
+    a.q = (const half_t*)q;
+    a.k = (const half_t*)k;
+    a.v = (const half_t*)v;
+    a.o = (half_t*)o;
+    a.lut = lut;
+    a.lut_is_64 = lut_elem_bytes == 8;
+    a.H = H;
+    a.S = S;
+    a.nblk = (S + 63) / 64;
+    a.nnz = nnz;
+    a.nvisit = nnz < a.nblk ? nnz : a.nblk;  // the reference clamps NNZ to ceil(S / 64) as well (the row pitch stays nnz)
+    a.qk_scale = sm_scale * 1.44269504f;
+    a.causal = causal;
+    a.total_wg = a.nblk * Z * H;
+    const dim3 grid(((a.total_wg + 7) / 8) * 8);
     if (D == 64)
-        SQ_ATTN_LAUNCH(64, 1);
+        hipLaunchKernelGGL((lut_attn_kernel<64>), grid, dim3(128), 0, st, a);
     else
-        SQ_ATTN_LAUNCH(128, 1);
-#undef SQ_ATTN_LAUNCH
+        hipLaunchKernelGGL((lut_attn_kernel<128>), grid, dim3(128), 0, st, a);
     return hipGetLastError();
 }
 

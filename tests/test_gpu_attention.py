@@ -143,3 +143,40 @@ def test_query_rows_without_a_visible_key_are_nan(capi):
     ok = np.isfinite(ref)
     assert np.array_equal(ok, np.isfinite(out))
     assert np.max(np.abs(out[ok] - ref[ok])) <= TOL * np.max(np.abs(ref[ok]))
+
+
+def _assert_close_fp16(capi, q, k, v, lut, scale, causal):
+    ref = att.attention_ref(q, k, v, lut, scale, causal)
+    out = capi.lut_attention(torch.from_numpy(q).cuda(), torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda(),
+                             torch.from_numpy(lut).cuda(), scale, causal)
+    torch.cuda.synchronize()
+    out = out.float().cpu().numpy().astype(np.float64)
+    # Every probability is rounded to fp16 once (relative 2^-11) in the product and in the row sum alike, and the output
+    # once; scores, sums and exponentials are fp32.  A weighted mean of v moves by at most 2 * 2^-11 * max|v|, the
+    # rounding of the output adds 2^-11 * |out|.
+    assert np.all(np.isfinite(out))
+    assert np.max(np.abs(out - ref)) <= 3 * 2.0 ** -11 * np.max(np.abs(v.astype(np.float64)))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("s", [1, 31, 32, 33, 63, 65, 95, 97, 161])
+def test_attention_at_the_edges_of_a_step(capi, s, causal, d):
+    """Sequences that end inside, at and just behind a step of 32 keys; query rows likewise."""
+    rng = np.random.default_rng(s + d)
+    q, k, v = (rng.normal(size=(2, 3, s, d)).astype(np.float16) for _ in range(3))
+    lut = att.layout_to_lut(att.synth_layout(3, (s + 63) // 64, 0.7, causal, seed=s))
+    _assert_close_fp16(capi, q, k, v, lut, d ** -0.5, causal)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_table_rows_of_more_than_64_entries(capi, dtype):
+    """The table is read 64 entries at a time: padding is recognised across that border (entry 64 repeats entry 63 in
+    every even row), and a growing score makes the running maximum move late in the row."""
+    rng = np.random.default_rng(7)
+    s, d = 66 * 64 - 5, 64
+    q, k, v = (rng.normal(size=(1, 1, s, d)).astype(np.float16) for _ in range(3))
+    k *= np.linspace(0.1, 3.0, s)[None, None, :, None].astype(np.float16)
+    row = np.arange(66)
+    rows = [np.concatenate([row[:64], row[63:65]]) if i % 2 == 0 else row for i in range(66)]
+    _assert_close_fp16(capi, q, k, v, np.stack(rows)[None].astype(dtype), d ** -0.5, False)
