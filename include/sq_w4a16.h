@@ -346,6 +346,15 @@ int sq_lut_attention_fwd(const void* q, const void* k, const void* v, void* out,
                          int lut_elem_bytes, int Z, int H, int S, int D, int nnz, float sm_scale, int causal,
                          void* stream);
 
+/* The same on tensors as a model's fused projection leaves them.  strides: element strides over batch, head and row
+ * of q, of k and v (one triple for both), of out, and of the caches (12 values; 9 are read without caches), all
+ * multiples of 8, the row stride of k and v below 2^24; the D elements of a row are adjacent.  k_cache, v_cache: both
+ * NULL, or where row j of (z, h) of k and v is also stored (they must not overlap the inputs).  lut NULL: every key
+ * block is visited (causal: those up to the diagonal), nnz and lut_elem_bytes are not used. */
+int sq_lut_attention_strided(const void* q, const void* k, const void* v, void* out, void* k_cache, void* v_cache,
+                             const void* lut, int lut_elem_bytes, int Z, int H, int S, int D, int nnz,
+                             const long* strides, float sm_scale, int causal, void* stream);
+
 /* Dense decode attention, one query token per sequence (q_len == 1 < kv_len):
  *   out[b,h,:] = sum_j P[j] v[b,h,j,:],  P = softmax_j(q[b,h,:] . k[b,h,j,:] * sm_scale + mask[b,j])
  * over the first L rows of an fp16 key/value cache, softmax and accumulation in fp32 (one

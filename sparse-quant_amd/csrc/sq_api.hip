@@ -762,8 +762,35 @@ int sq_lut_attention_fwd(const void* q, const void* k, const void* v, void* out,
     if (lut_elem_bytes != 4 && lut_elem_bytes != 8) return SQ_ERR_BAD_LAYOUT;
     if (!q || !k || !v || !out || !lut) return SQ_ERR_NULL_POINTER;
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) return SQ_ERR_MISALIGNED;
-    return launch_code(sq::launch_lut_attention(q, k, v, out, lut, lut_elem_bytes, Z, H, S, D, nnz, sm_scale, causal,
-                                                static_cast<hipStream_t>(stream)));
+    const long hs = (long)S * D, zs = hs * H;
+    const sq::LutAttnStrides st = {{zs, hs, D}, {zs, hs, D}, {zs, hs, D}, {0, 0, 0}};
+    return launch_code(sq::launch_lut_attention(q, k, v, out, nullptr, nullptr, lut, lut_elem_bytes, Z, H, S, D, nnz, st,
+                                                sm_scale, causal, static_cast<hipStream_t>(stream)));
+}
+
+int sq_lut_attention_strided(const void* q, const void* k, const void* v, void* out, void* k_cache, void* v_cache,
+                             const void* lut, int lut_elem_bytes, int Z, int H, int S, int D, int nnz, const long* strides,
+                             float sm_scale, int causal, void* stream) {
+    if (Z <= 0 || H <= 0 || S <= 0 || (D != 64 && D != 128) || (lut && nnz <= 0)) return SQ_ERR_BAD_SHAPE;
+    if ((long)Z * H > 65535) return SQ_ERR_BAD_SHAPE;
+    if (lut && lut_elem_bytes != 4 && lut_elem_bytes != 8) return SQ_ERR_BAD_LAYOUT;
+    if (!q || !k || !v || !out || !strides || !k_cache != !v_cache) return SQ_ERR_NULL_POINTER;
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) return SQ_ERR_MISALIGNED;
+    if (k_cache && (!aligned16(k_cache) || !aligned16(v_cache))) return SQ_ERR_MISALIGNED;
+    sq::LutAttnStrides st;
+    for (int i = 0; i < 3; i++) {
+        st.q[i] = strides[i];
+        st.kv[i] = strides[3 + i];
+        st.o[i] = strides[6 + i];
+        st.c[i] = k_cache ? strides[9 + i] : 0;
+    }
+    for (int i = 0; i < (k_cache ? 12 : 9); i++) {
+        if (strides[i] < 0) return SQ_ERR_BAD_SHAPE;
+        if (strides[i] % 8 != 0) return SQ_ERR_MISALIGNED;
+    }
+    if (st.kv[2] >= (1L << 24)) return SQ_ERR_BAD_SHAPE;  // 32-bit byte offsets inside a step of 32 rows
+    return launch_code(sq::launch_lut_attention(q, k, v, out, k_cache, v_cache, lut, lut_elem_bytes, Z, H, S, D, nnz, st,
+                                                sm_scale, causal, static_cast<hipStream_t>(stream)));
 }
 
 int sq_decode_attention(const void* q, const void* k_new, const void* v_new, void* k_cache, void* v_cache,

@@ -32,6 +32,10 @@
 //   32 heads x 4096 x 128, causal, 26 % of the blocks   115 -> 86 (matrix pipes busy 0.39 of the cycles)
 //   8 x 32 heads x 512 x 128, causal, 26 %               35 -> 35 (134 MB to move: 22 at the rate of a copy)
 //   8 x 16 heads x 512 x 64, 25 %                        10.1 -> 9.4
+// A model's prompt reads q, k and v where the fused projection left them and stores the cache rows and a [batch, row,
+// hidden] output: the element-wise copies around the kernel cost three times its own time (8 prompts of 512 tokens, 32
+// heads of 128, per layer: six copies of 21 us and 35 -> 52 in all; without a table, against torch's attention and its
+// copies, 157 -> 59).
 #include "sq_common.h"
 #include "sq_kernels.h"
 
@@ -46,9 +50,13 @@ struct LutAttnArgs {
     const half_t* k;
     const half_t* v;
     half_t* o;
-    const void* lut;
+    half_t* kc;       // caches that receive the K and V rows, or null
+    half_t* vc;
+    const void* lut;  // null: every block (causal: up to the diagonal)
+    LutAttnStrides st;
     int lut_is_64, H, S, nblk, nnz, nvisit;
     float qk_scale;  // sm_scale * log2(e)
+    float lazy;      // log2 of how far a score may exceed the reference maximum
     int causal, total_wg;
 };
 
@@ -99,26 +107,33 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
     const int qb = a.causal ? a.nblk - 1 - qr : qr;
     const int h = zh % a.H;
     const int S = a.S;
-    const long base = (long)zh * S * D;
+    const int z = zh / a.H;
+    const half_t* kz = a.k + z * a.st.kv[0] + h * a.st.kv[1];
+    const half_t* vz = a.v + z * a.st.kv[0] + h * a.st.kv[1];
+    const int kv_row = (int)a.st.kv[2] * 2;  // bytes
     const int m = qb * 64 + 32 * wave + ln;  // this lane's query
 
     half8_t qf[NK];
     {
-        const half_t* qp = a.q + base + (long)imin(m, S - 1) * D + 8 * lc;
+        const half_t* qp = a.q + z * a.st.q[0] + h * a.st.q[1] + imin(m, S - 1) * a.st.q[2] + 8 * lc;
 #pragma unroll
         for (int s = 0; s < NK; s++) qf[s] = *(const half8_t*)(qp + 16 * s);
     }
 
     // The visited blocks, 64 table entries at a time: lane j holds entry j, `todo` has a bit for each that is visited.
     const long lut_row = ((long)h * a.nblk + qb) * a.nnz;
+    const int nvisit = a.lut ? a.nvisit : (a.causal ? qb + 1 : a.nblk);
     int entry = 0, jbase = 0, last = -1;
     uint64_t todo = 0;
     auto next_block = [&]() {  // its first key, or -1
         while (todo == 0) {
-            if (jbase >= a.nvisit) return -1;
+            if (jbase >= nvisit) return -1;
             const int j = jbase + lane;
             int blk = -1;
-            if (j < a.nvisit) blk = a.lut_is_64 ? (int)((const long long*)a.lut)[lut_row + j] : ((const int*)a.lut)[lut_row + j];
+            if (j < nvisit) {
+                blk = j;
+                if (a.lut) blk = a.lut_is_64 ? (int)((const long long*)a.lut)[lut_row + j] : ((const int*)a.lut)[lut_row + j];
+            }
             const int up = __shfl_up(blk, 1);
             const int prev = lane == 0 ? last : up;
             todo = __builtin_amdgcn_ballot_w64(blk != prev && blk >= 0 && (long)blk * 64 < S);
@@ -138,7 +153,7 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
     auto lane_offset = [&](int j, int row_max, bool is_v) {
         const int row = RPL * (NL * wave + j) + lrow;
         const int c = lchunk ^ (is_v ? v_swz<D>(row) : k_swz<D>(row));
-        return (uint32_t)(imin(row, row_max) * ROW + c * 16);
+        return (uint32_t)(imin(row, row_max) * kv_row + c * 16);
     };
     uint32_t koff[NL], voff[NL];
 #pragma unroll
@@ -147,8 +162,8 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
         voff[j] = lane_offset(j, 31, true);
     }
     auto issue = [&](int n, int slot) {
-        const uint8_t* kb = (const uint8_t*)(a.k + base + (long)n * D);
-        const uint8_t* vb = (const uint8_t*)(a.v + base + (long)n * D);
+        const uint8_t* kb = (const uint8_t*)(kz + n * a.st.kv[2]);
+        const uint8_t* vb = (const uint8_t*)(vz + n * a.st.kv[2]);
         const uint32_t l0 = lds0 + slot * SB + wave * (NL * 1024);
         if (n + 32 <= S) {
 #pragma unroll
@@ -178,7 +193,7 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
 
     // Reference maximum of the query (0 while unset), the score above it at which it moves (any score while unset), and
     // this lane's share of the row sum.
-    constexpr float LAZY = 8.f;
+    const float lazy = a.lazy;
     float ref = 0.f, limit = -INFINITY, l_i = 0.f;
     float16_t acc[DT];
 #pragma unroll
@@ -224,8 +239,8 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
                 st[v] = keep ? st[v] : -INFINITY;
             }
         }
-        // The reference maximum of a query moves only when a score exceeds it by more than 2^LAZY (or when it is still
-        // unset): until then p = exp2(score) stays below 2^LAZY, well inside fp16, the final O = acc / l does not depend
+        // The reference maximum of a query moves only when a score exceeds it by more than 2^lazy (or when it is still
+        // unset): until then p = exp2(score) stays below 2^lazy, well inside fp16, the final O = acc / l does not depend
         // on the reference, and neither the accumulators nor the scores need rescaling.  The test is made per lane and
         // voted over the wave; the maximum over a query's two lanes is formed only when it is needed.
         float mx = -INFINITY;
@@ -236,9 +251,9 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
             const bool upd = mq > limit;
             const float delta = upd ? mq : 0.f;
             // a query without a reference so far has l = 0 and acc = 0: nothing to rescale
-            const float alpha = (upd && limit == LAZY) ? __builtin_amdgcn_exp2f(-delta) : 1.f;
+            const float alpha = (upd && limit != -INFINITY) ? __builtin_amdgcn_exp2f(-delta) : 1.f;
             ref += delta;
-            limit = upd ? LAZY : limit;
+            limit = upd ? lazy : limit;
             l_i *= alpha;
 #pragma unroll
             for (int v = 0; v < 16; v++) st[v] -= delta;
@@ -317,21 +332,37 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
         const int row = RPL * j + lrow;
         const u32x4_t t = *(const u32x4_t*)(out + row * ROW + ((lchunk ^ k_swz<D>(row)) * 16));
         const int mr = qb * 64 + 32 * wave + row;
-        if (mr < S) *(u32x4_t*)(a.o + base + (long)mr * D + 8 * lchunk) = t;
+        if (mr < S) *(u32x4_t*)(a.o + z * a.st.o[0] + h * a.st.o[1] + mr * a.st.o[2] + 8 * lchunk) = t;
+    }
+    // The workgroup's own 64 rows of K and V go to the caches (their lines are in this XCD's L2).
+    if (a.kc) {
+        half_t* kcz = a.kc + z * a.st.c[0] + h * a.st.c[1];
+        half_t* vcz = a.vc + z * a.st.c[0] + h * a.st.c[1];
+#pragma unroll
+        for (int j = 0; j < TILE / 1024; j++) {
+            const int mr = qb * 64 + 32 * wave + RPL * j + lrow;
+            if (mr < S) {
+                *(u32x4_t*)(kcz + mr * a.st.c[2] + 8 * lchunk) = *(const u32x4_t*)(kz + mr * a.st.kv[2] + 8 * lchunk);
+                *(u32x4_t*)(vcz + mr * a.st.c[2] + 8 * lchunk) = *(const u32x4_t*)(vz + mr * a.st.kv[2] + 8 * lchunk);
+            }
+        }
     }
 }
 
 }  // namespace
 
-hipError_t launch_lut_attention(const void* q, const void* k, const void* v, void* o, const void* lut,
-                                int lut_elem_bytes, int Z, int H, int S, int D, int nnz, float sm_scale, int causal,
-                                hipStream_t st) {
+hipError_t launch_lut_attention(const void* q, const void* k, const void* v, void* o, void* k_cache, void* v_cache,
+                                const void* lut, int lut_elem_bytes, int Z, int H, int S, int D, int nnz,
+                                const LutAttnStrides& strides, float sm_scale, int causal, hipStream_t st) {
     LutAttnArgs a;
     a.q = (const half_t*)q;
     a.k = (const half_t*)k;
     a.v = (const half_t*)v;
     a.o = (half_t*)o;
+    a.kc = (half_t*)k_cache;
+    a.vc = (half_t*)v_cache;
     a.lut = lut;
+    a.st = strides;
     a.lut_is_64 = lut_elem_bytes == 8;
     a.H = H;
     a.S = S;
@@ -339,6 +370,10 @@ hipError_t launch_lut_attention(const void* q, const void* k, const void* v, voi
     a.nnz = nnz;
     a.nvisit = nnz < a.nblk ? nnz : a.nblk;  // the reference clamps NNZ to ceil(S / 64) as well (the row pitch stays nnz)
     a.qk_scale = sm_scale * 1.44269504f;
+    // Without a table the reference is the running maximum itself, whose probability 1 is exact in fp16: the error of a
+    // dense softmax with it (2.43e-4 of the result at 512 keys, 2.51e-4 with the lazy one) at the price of more rescaling
+    // (8 x 32 heads x 512 x 128: 51 -> 59 us).
+    a.lazy = lut ? 8.f : 0.f;
     a.causal = causal;
     a.total_wg = a.nblk * Z * H;
     const dim3 grid(((a.total_wg + 7) / 8) * 8);

@@ -102,9 +102,14 @@ hipError_t launch_gemm_pipe(const void* x, const void* w, const void* zs, void* 
                             int variant, Epilogue epi, hipStream_t st);
 
 // sq_attn.hip: LUT block-sparse attention, prefill.  D in {64, 128}; lut int32 or int64 [H, ceil(S/64), nnz].
-hipError_t launch_lut_attention(const void* q, const void* k, const void* v, void* o, const void* lut,
-                                int lut_elem_bytes, int Z, int H, int S, int D, int nnz, float sm_scale, int causal,
-                                hipStream_t st);
+// Element strides over batch, head and row (multiples of 8) of q, of k and v, of the output and of the caches that
+// receive the k and v rows (k_cache null: none).  lut null: every block.
+struct LutAttnStrides {
+    long q[3], kv[3], o[3], c[3];
+};
+hipError_t launch_lut_attention(const void* q, const void* k, const void* v, void* o, void* k_cache, void* v_cache,
+                                const void* lut, int lut_elem_bytes, int Z, int H, int S, int D, int nnz,
+                                const LutAttnStrides& strides, float sm_scale, int causal, hipStream_t st);
 
 // sq_decode_attn.hip: dense decode attention over an fp16 KV cache (one query row per sequence),
 // optionally appending the new key/value row.  Strides in elements.

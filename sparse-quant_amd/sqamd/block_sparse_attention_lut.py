@@ -23,8 +23,10 @@ def sparse_attention_prefill(q, k, v, sm_scale, lut, LT=True, BLOCK_M=64, BLOCK_
         raise TypeError("lut must be int32 or int64")
     if not q.is_cuda:
         raise RuntimeError("sparse_attention_prefill needs device tensors; there is no host path")
-    return capi.lut_attention(q.contiguous(), k.contiguous(), v.contiguous(), lut.contiguous().to(q.device),
-                              sm_scale, LT)
+    lut = lut.contiguous().to(q.device)
+    if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()) and capi.lut_attention_strided_ok(q, k, v):
+        return capi.lut_attention_strided(q, k, v, lut, sm_scale, LT)  # views of a fused projection: no copies
+    return capi.lut_attention(q.contiguous(), k.contiguous(), v.contiguous(), lut, sm_scale, LT)
 
 
 def sparse_attention(q, k, v, sm_scale, lut, LT=True, BLOCK_M=64, BLOCK_N=64, attention_mask=None,

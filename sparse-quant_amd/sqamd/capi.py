@@ -54,6 +54,7 @@ SIGNATURES = {
     "sq_w4a16_gemm_ln_fused": (_i, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i,
                                     _vp, ctypes.c_size_t, _vp]),
     "sq_lut_attention_fwd": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, ctypes.c_float, _i, _vp]),
+    "sq_lut_attention_strided": (_i, [_vp] * 7 + [_i] * 6 + [_vp, ctypes.c_float, _i, _vp]),
     "sq_embed_rows": (_i, [_vp, _vp, _vp, _vp, ctypes.c_longlong, _vp, _i, _i, ctypes.c_longlong, ctypes.c_longlong, _vp]),
     "sq_f16_gemv_parts": (_i, [_i]),
     "sq_f16_gemv": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
@@ -417,6 +418,45 @@ def lut_attention(q, k, v, lut, sm_scale, causal, stream=None):
     _check(lib().sq_lut_attention_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lut), lut.element_size(), z, h, s, d,
                                       lut.shape[-1], float(sm_scale), int(bool(causal)), _stream(stream)),
            "sq_lut_attention_fwd")
+    return out
+
+
+def _rows_readable(*tensors):
+    """Whether the attention kernel can address these [Z,H,S,D] tensors as they lie: 16-byte rows, chunks and strides."""
+    return all(t.stride(3) == 1 and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0
+               and t.stride(2) % 8 == 0 for t in tensors)
+
+
+def lut_attention_strided_ok(q, k, v, k_cache=None, v_cache=None):
+    """Whether lut_attention_strided takes these tensors."""
+    caches = () if k_cache is None else (k_cache, v_cache)
+    return (all(t.dtype == torch.float16 and t.is_cuda for t in (q, k, v) + caches) and q.shape[3] in (64, 128)
+            and q.shape == k.shape == v.shape and k.stride() == v.stride() and k.stride(2) < 1 << 24
+            and _rows_readable(q, k, v, *caches)
+            and (k_cache is None or (k_cache.stride() == v_cache.stride() and k_cache.shape == v_cache.shape
+                                     and k_cache.shape[:2] == k.shape[:2] and k_cache.shape[3] == k.shape[3]
+                                     and k_cache.shape[2] >= k.shape[2])))
+
+
+def lut_attention_strided(q, k, v, lut, sm_scale, causal, k_cache=None, v_cache=None, rows_first=False, stream=None):
+    """sq_lut_attention_strided on [Z,H,S,D] views that lut_attention_strided_ok accepts.  lut int32/int64 contiguous
+    or None (every block).  k_cache, v_cache [Z,H,Lmax,D]: rows 0..S-1 receive k and v.  Returns a contiguous
+    [Z,H,S,D], or with rows_first a contiguous [Z,S,H,D]."""
+    z, h, s, d = q.shape
+    if not lut_attention_strided_ok(q, k, v, k_cache, v_cache):
+        raise ValueError("lut_attention_strided: unsupported dtype, shape or strides")
+    if rows_first:
+        out = torch.empty((z, s, h, d), dtype=q.dtype, device=q.device)
+        o_st = (s * h * d, d, h * d)
+    else:
+        out = torch.empty((z, h, s, d), dtype=q.dtype, device=q.device)
+        o_st = (h * s * d, s * d, d)
+    c_st = (0, 0, 0) if k_cache is None else k_cache.stride()[:3]
+    strides = (ctypes.c_long * 12)(*q.stride()[:3], *k.stride()[:3], *o_st, *c_st)
+    _check(lib().sq_lut_attention_strided(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(k_cache), _ptr(v_cache), _ptr(lut),
+                                          0 if lut is None else lut.element_size(), z, h, s, d,
+                                          0 if lut is None else lut.shape[-1], strides, float(sm_scale),
+                                          int(bool(causal)), _stream(stream)), "sq_lut_attention_strided")
     return out
 
 

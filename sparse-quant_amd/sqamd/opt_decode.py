@@ -11,8 +11,9 @@ too): the decode step appends to the preallocated fp16 KV cache and attends in o
 (sq_decode_attention) that reads the position from the device, so the step is a fixed
 kernel sequence that can be captured in a HIP graph.  Prefill attention is dense causal by
 default; a layer that has been given a look-up table (`DecoderLayer.lut`, per head) runs its
-prefill through sparse_attention(q, k, v, scaling, lut, LT=True) as the reference's OPT
-attention does (test/nvidia/module/opt/modeling_opt_ours.py:435-438).
+prefill over the table's blocks (sparse_attention(q, k, v, scaling, lut, LT=True) in the reference's OPT
+attention, test/nvidia/module/opt/modeling_opt_ours.py:435-438).  Either way a prompt's attention is one kernel
+that also fills the cache (sq_lut_attention_strided).
 """
 import math
 import time
@@ -81,11 +82,22 @@ class DecoderLayer(nn.Module):
             q = self.q_proj(flat).view(b, t, self.heads, self.hd).transpose(1, 2)
             k = self.k_proj(flat).view(b, t, self.heads, self.hd).transpose(1, 2)
             v = self.v_proj(flat).view(b, t, self.heads, self.hd).transpose(1, 2)
-        if isinstance(pos0, int):
+        scale = 1.0 / math.sqrt(self.hd)
+        if isinstance(pos0, int) and pos0 == 0 and t > 1 and capi.lut_attention_strided_ok(q, k, v, kc, vc) \
+                and (self.lut is None or self.lut.dtype in (torch.int32, torch.int64)):
+            # a whole prompt: one kernel reads q, k and v where the projection left them, fills the cache and writes
+            # [b, t, hidden] (without a table: every block up to the diagonal)
+            lut = None if self.lut is None else self.lut.contiguous().to(q.device)
+            a = capi.lut_attention_strided(q, k, v, lut, scale, True, kc, vc, rows_first=True)
+            if self.capture is not None:
+                self.capture.update(q=q.detach().clone(), k=k.detach().clone(), v=v.detach().clone(),
+                                    a=a.transpose(1, 2).detach().clone())
+            a = a.view(1, b * t, hdim)
+        elif isinstance(pos0, int):
             kc[:, :, pos0:pos0 + t] = k
             vc[:, :, pos0:pos0 + t] = v
             if self.lut is not None and pos0 == 0 and t > 1:
-                a = sparse_attention(q, k, v, 1.0 / math.sqrt(self.hd), self.lut, LT=True)
+                a = sparse_attention(q, k, v, scale, self.lut, LT=True)
             else:
                 a = nn.functional.scaled_dot_product_attention(q, kc[:, :, :pos0 + t], vc[:, :, :pos0 + t],
                                                                is_causal=(t > 1))
@@ -95,7 +107,7 @@ class DecoderLayer(nn.Module):
         else:
             # graph-captured decode step: the position lives in a device tensor; one kernel appends the
             # new key/value rows to the cache and attends over rows 0 .. pos0, output already [b, 1, hidden]
-            a = capi.decode_attention(q, kc, vc, pos0, 1.0 / math.sqrt(self.hd), k_new=k, v_new=v).view(1, b * t, hdim)
+            a = capi.decode_attention(q, kc, vc, pos0, scale, k_new=k, v_new=v).view(1, b * t, hdim)
         # bias, ReLU and the two residual adds ride in the kernels' stores
         x = self.out_proj(a, residual=x.reshape(1, b * t, hdim)).view(b, t, hdim)
         if self.fuse_ln:
@@ -160,6 +172,8 @@ class OPTDecoder(nn.Module):
         for layer, (kc, vc) in zip(self.layers, cache):
             x = layer(x, kc, vc, pos0)
         x = _layernorm(self.final_ln, x[:, -1:])
+        if b <= 8 and self.hidden % 512 == 0 and 512 <= self.hidden <= 8192:  # what sq_f16_gemv takes
+            return capi.f16_gemv(x, self.lm_head).view(b, 1, -1)
         return torch.matmul(x, self.lm_head.t())  # [B, 1, vocab]
 
     @torch.no_grad()
@@ -296,11 +310,10 @@ def run_e2e(batch=8, prompt=512, new_tokens=128, layers=32, use_graph=True, seed
                  "launch" + ("; embeddings, fp16 lm_head + argmax, token feedback as three launches inside the step"
                              if fused_ends else ""),
         "prefill_ms": round(prefill_s * 1e3, 2),
-        "prefill_attention": "dense causal (torch SDPA)",
+        "prefill_attention": "dense causal (sq_lut_attention_strided without a table)",
         "prefill_lut_ms": None if prefill_lut_s is None else round(prefill_lut_s * 1e3, 2),
         "prefill_lut_attention": None if prefill_lut_s is None else
-        "sparse_attention(q, k, v, scaling, lut, LT=True) in every layer: causal per-head tables, block density %.2f, "
-        "D = 128 (sq_lut_attention_fwd)" % lut_density,
+        "causal per-head tables in every layer, block density %.2f, D = 128 (sq_lut_attention_strided)" % lut_density,
         "prefill_tok_per_s": round(batch * prompt / prefill_s, 1),
         "decode_ms_per_step": round(decode_s * 1e3 / steps, 4),
         "decode_tok_per_s": round(batch * steps / decode_s, 1),

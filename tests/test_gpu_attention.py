@@ -180,3 +180,65 @@ def test_table_rows_of_more_than_64_entries(capi, dtype):
     row = np.arange(66)
     rows = [np.concatenate([row[:64], row[63:65]]) if i % 2 == 0 else row for i in range(66)]
     _assert_close_fp16(capi, q, k, v, np.stack(rows)[None].astype(dtype), d ** -0.5, False)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("s", [2, 33, 64, 130, 200])
+def test_strided_attention_fills_the_cache(capi, s, d):
+    """Views of a fused projection [Z, S, 3, H, D]: the outputs of the contiguous path bit for bit in either output
+    order, cache rows 0..S-1 hold k and v, the rows behind them are untouched."""
+    z, h = 2, 3
+    gen = torch.Generator(device="cuda").manual_seed(s + d)
+    qkv = torch.randn((z, s, 3, h, d), device="cuda", generator=gen).half()
+    q, k, v = (qkv[:, :, j].transpose(1, 2) for j in range(3))
+    lut = torch.from_numpy(att.layout_to_lut(att.synth_layout(h, (s + 63) // 64, 0.6, True, seed=s))).cuda()
+    ref = capi.lut_attention(q.contiguous(), k.contiguous(), v.contiguous(), lut, 0.1, True)
+    kc, vc = (torch.full((z, h, s + 5, d), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+    assert capi.lut_attention_strided_ok(q, k, v, kc, vc)
+    out = capi.lut_attention_strided(q, k, v, lut, 0.1, True, kc, vc, rows_first=True)
+    assert torch.equal(out.transpose(1, 2), ref)
+    assert torch.equal(kc[:, :, :s], k) and torch.equal(vc[:, :, :s], v)
+    assert bool((kc[:, :, s:] == 7).all()) and bool((vc[:, :, s:] == 7).all())
+    assert torch.equal(capi.lut_attention_strided(q, k, v, lut, 0.1, True), ref)
+    from sqamd.block_sparse_attention_lut import sparse_attention
+    assert torch.equal(sparse_attention(q, k, v, 0.1, lut, True), ref)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("s", [2, 65, 70 * 64 + 3])
+def test_attention_without_a_table_visits_every_block(capi, s, causal):
+    gen = torch.Generator(device="cuda").manual_seed(s)
+    q, k, v = (torch.randn((1, 2, s, 64), device="cuda", generator=gen).half() for _ in range(3))
+    nb = (s + 63) // 64
+    rows = torch.arange(nb, device="cuda")
+    full = rows.expand(2, nb, nb)
+    if causal:  # padded with the diagonal block
+        full = torch.minimum(full, rows.view(1, nb, 1))
+    out = capi.lut_attention_strided(q, k, v, None, 0.125, causal)
+    ref = capi.lut_attention(q, k, v, full.contiguous(), 0.125, causal)
+    # the two differ in the reference maximum of the softmax: each is within 3 * 2^-11 * max|v| of the exact result
+    assert torch.max((out.float() - ref.float()).abs()) <= 6 * 2.0 ** -11 * v.float().abs().max()
+
+
+def test_strided_attention_refuses_what_it_cannot_address(capi):
+    import ctypes
+    L, p = capi.lib(), ctypes.c_void_p(4096)
+    st = lambda *v: (ctypes.c_long * 12)(*v)
+    good = [4096, 64, 192] * 2 + [4096, 64, 64] * 2
+    call = lambda strides, q=p, kc=None, vc=None, d=64, lut=None: L.sq_lut_attention_strided(
+        q, p, p, p, kc, vc, lut, 8, 1, 1, 64, d, 1, strides, 1.0, 0, None)
+    assert call(None) == capi.SQ_ERR_NULL_POINTER
+    assert call(st(*good), d=96) == capi.SQ_ERR_BAD_SHAPE
+    assert call(st(*good), kc=p) == capi.SQ_ERR_NULL_POINTER
+    assert call(st(*good), q=ctypes.c_void_p(4104)) == capi.SQ_ERR_MISALIGNED
+    for i in range(9):
+        assert call(st(*(good[:i] + [good[i] + 4] + good[i + 1:]))) == capi.SQ_ERR_MISALIGNED
+    assert call(st(*(good[:5] + [1 << 24] + good[6:]))) == capi.SQ_ERR_BAD_SHAPE
+    assert call(st(*(good[:2] + [-8] + good[3:]))) == capi.SQ_ERR_BAD_SHAPE
+    x = torch.zeros((1, 1, 64, 72), dtype=torch.float16, device="cuda")
+    q = x[..., :64]
+    assert capi.lut_attention_strided_ok(q, q, q)
+    assert not capi.lut_attention_strided_ok(x[..., 4:68], q, q)                  # rows not 16-byte aligned
+    assert not capi.lut_attention_strided_ok(q, q, q.contiguous())                # k and v laid out differently
+    assert not capi.lut_attention_strided_ok(q, q, q, q[:, :, :8], q[:, :, :8])   # a cache shorter than the prompt
+    assert not capi.lut_attention_strided_ok(q.float(), q, q)
