@@ -150,7 +150,7 @@ struct LnArgs {
 at::Tensor gemm_impl(const at::Tensor& I, const at::Tensor& W, const at::Tensor& ZS, int N, int group_size, int algo,
                      const c10::optional<at::Tensor>& bias = c10::nullopt,
                      const c10::optional<at::Tensor>& residual = c10::nullopt, int act = SQ_ACT_NONE,
-                     const LnArgs* ln = nullptr) {
+                     const LnArgs* ln = nullptr, bool any_rank = false) {
     SQ_CHECK_DEVICE(I);
     SQ_CHECK_DEVICE(W);
     SQ_CHECK_DEVICE(ZS);
@@ -159,12 +159,12 @@ at::Tensor gemm_impl(const at::Tensor& I, const at::Tensor& W, const at::Tensor&
     SQ_CHECK_CONTIGUOUS(ZS);
     SQ_CHECK_DTYPE(I, at::kHalf);
     SQ_CHECK_DTYPE(ZS, at::kHalf);
-    SQ_CHECK_DIMS(I, 3);
+    if (!any_rank) SQ_CHECK_DIMS(I, 3);
     SQ_CHECK_DIMS(W, 2);
     SQ_CHECK_DIMS(ZS, 2);
     const int layout = layout_of(W);
-    const int64_t M = I.size(0) * I.size(1);
-    const int64_t K = I.size(2);
+    const int64_t K = I.size(-1);
+    const int64_t M = any_rank ? I.numel() / std::max<int64_t>(K, 1) : I.size(0) * I.size(1);
     if (group_size <= 0 || K % group_size != 0) throw std::invalid_argument("embbed dim must be a multiple of group_size!");
     if (layout == SQ_LAYOUT_L1) {
         if (W.size(0) != N) throw std::invalid_argument("output dim mismatch!");
@@ -181,7 +181,9 @@ at::Tensor gemm_impl(const at::Tensor& I, const at::Tensor& W, const at::Tensor&
     TORCH_CHECK(M < (1LL << 31) && K < (1LL << 31), "problem too large");
 
     c10::DeviceGuard guard(I.device());
-    at::Tensor O = torch::empty({I.size(0), I.size(1), N}, I.options());
+    c10::SmallVector<int64_t, 5> out_sizes(I.sizes().begin(), I.sizes().end());
+    out_sizes.back() = N;
+    at::Tensor O = at::empty(out_sizes, I.options());
     const void* w_ptr = W.data_ptr();
     const void* zs_ptr = ZS.data_ptr();
     std::pair<at::Tensor, at::Tensor> keep;
@@ -361,6 +363,100 @@ at::Tensor gemm_awq_ln_fused_ut(at::Tensor I, c10::optional<at::Tensor> ln_weigh
     return gemm_impl(I, W, W_zeros_scales, N, group_size, SQ_ALGO_AUTO, bias, residual, act_code(act), &ln);
 }
 
+// WALinear.forward in one call: x of any rank (the rows are its leading dimensions), a residual of as many elements as
+// the output, the LayerNorm parameters as in gemm_awq_ln_fused_ut where with_ln is set.  The module's own reshapes,
+// its no_grad scope and the view back cost as much host time as a decode linear takes on the device (4096 x 4096, one
+// token, back to back: 9.9 us a call with them, 6.8 so; the four linears of a decoder layer of 4096 x 16384 39.6 -> 30.6).
+at::Tensor walinear_forward(const at::Tensor& x, const at::Tensor& W, const at::Tensor& W_zeros_scales,
+                            const c10::optional<at::Tensor>& bias, const c10::optional<at::Tensor>& residual,
+                            const std::string& act, const int N, const int group_size, const bool with_ln,
+                            const c10::optional<at::Tensor>& ln_weight, const c10::optional<at::Tensor>& ln_bias,
+                            double ln_eps) {
+    at::NoGradGuard no_grad;
+    const LnArgs ln{ln_weight, ln_bias, ln_eps};
+    c10::optional<at::Tensor> res;
+    if (residual.has_value() && residual->defined()) {
+        const int64_t K = x.size(-1);
+        const int64_t rows = x.numel() / std::max<int64_t>(K, 1);
+        TORCH_CHECK(residual->numel() == rows * N, "residual of ", residual->numel(), " elements for an output of ", rows,
+                    " x ", N);
+        res = residual->is_contiguous() ? *residual : residual->contiguous();
+    }
+    return gemm_impl(x.is_contiguous() ? x : x.contiguous(), W, W_zeros_scales, N, group_size, SQ_ALGO_AUTO, bias, res,
+                     act_code(act), with_ln ? &ln : nullptr, true);
+}
+
+// The two branches of sparse_attention on tensors that need no conversion (12.4 and 19.2 us of host time a call from
+// Python, 7.1 and 6.3 here: 8 x 16 heads x 512 x 64 at 25 % took 11.1 us and takes 8.7); anything else returns nothing
+// and takes the
+// general path in Python, which copies or refuses it.
+bool half_rows(const at::Tensor& t, const at::Tensor& like) {
+    return t.is_cuda() && t.device() == like.device() && t.scalar_type() == at::kHalf && t.dim() == 4 &&
+           t.stride(3) == 1 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
+}
+
+c10::optional<at::Tensor> lut_attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& lut,
+                                        double sm_scale, bool causal) {
+    if (!q.is_cuda() || !half_rows(q, q) || !half_rows(k, q) || !half_rows(v, q)) return c10::nullopt;
+    if (q.sizes() != k.sizes() || q.sizes() != v.sizes() || k.strides() != v.strides()) return c10::nullopt;
+    if (lut.device() != q.device() || !lut.is_contiguous() || lut.dim() < 1 || q.numel() == 0 || lut.numel() == 0)
+        return c10::nullopt;
+    if (lut.scalar_type() != at::kInt && lut.scalar_type() != at::kLong) return c10::nullopt;
+    const int64_t Z = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
+    const int64_t nnz = lut.size(-1);
+    if (S >= (1LL << 31) || nnz >= (1LL << 31) || Z * H > 65535) return c10::nullopt;
+    at::NoGradGuard no_grad;
+    c10::DeviceGuard guard(q.device());
+    at::Tensor out = at::empty({Z, H, S, D}, q.options());
+    const long strides[9] = {q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), H * S * D, S * D, D};
+    const int rc = sq_lut_attention_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), nullptr, nullptr,
+                                            lut.data_ptr(), (int)lut.element_size(), (int)Z, (int)H, (int)S, (int)D, (int)nnz,
+                                            strides, (float)sm_scale, causal, current_stream(q));
+    if (rc != SQ_OK) return c10::nullopt;
+    return out;
+}
+
+// Partial states and counters of the decode attention that shares a head's rows between workgroups (fewer than 256
+// heads): one zero-initialised buffer per (device, stream), of the size any such call can need (2 MB), so that it
+// never moves under a captured graph.
+at::Tensor attention_workspace_for(const at::Tensor& like, void* stream) {
+    static std::mutex mutex;
+    static std::map<std::pair<int, void*>, at::Tensor> buffers;
+    std::lock_guard<std::mutex> lock(mutex);
+    at::Tensor& ws = buffers[std::make_pair((int)like.device().index(), stream)];
+    if (!ws.defined())
+        ws = torch::zeros({(int64_t)sq_decode_attention_workspace_bytes(1, 255, 128)}, like.options().dtype(at::kByte));
+    return ws;
+}
+
+c10::optional<at::Tensor> decode_attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                           const c10::optional<at::Tensor>& mask, double sm_scale) {
+    if (!q.is_cuda() || !half_rows(q, q) || !half_rows(k, q) || !half_rows(v, q) || q.numel() == 0) return c10::nullopt;
+    const int64_t B = q.size(0), H = q.size(1), D = q.size(3), L = k.size(2);
+    if (q.size(2) != 1 || k.sizes() != v.sizes() || k.strides() != v.strides() || k.stride(2) != D || k.size(0) != B ||
+        k.size(1) != H || k.size(3) != D || L >= (1LL << 31) || B * H > (1LL << 24))
+        return c10::nullopt;
+    const void* mask_ptr = nullptr;
+    if (mask.has_value() && mask->defined()) {
+        if (mask->device() != q.device() || mask->scalar_type() != at::kHalf || !mask->is_contiguous() || mask->dim() != 4 ||
+            mask->size(0) != B || mask->size(1) != 1 || mask->size(2) != 1 || mask->size(3) != L)
+            return c10::nullopt;
+        mask_ptr = mask->data_ptr();
+    }
+    at::NoGradGuard no_grad;
+    c10::DeviceGuard guard(q.device());
+    at::Tensor out = at::empty({B, H, 1, D}, q.options());
+    void* stream = current_stream(q);
+    at::Tensor ws;
+    if (B * H < 256) ws = attention_workspace_for(q, stream);
+    const int rc = sq_decode_attention(q.data_ptr(), nullptr, nullptr, k.data_ptr(), v.data_ptr(), mask_ptr, out.data_ptr(),
+                                       (int)B, (int)H, (int)D, (int)L, q.stride(0), q.stride(1), 0, 0, k.stride(0), k.stride(1),
+                                       mask_ptr ? L : 0, (int)L, nullptr, (float)sm_scale, ws.defined() ? ws.data_ptr() : nullptr,
+                                       ws.defined() ? (size_t)ws.numel() : 0, stream);
+    if (rc != SQ_OK) return c10::nullopt;
+    return out;
+}
+
 // Same with an explicit kernel id (SQ_ALGO_* | tuning word << 8); for tests and benchmarks.
 at::Tensor gemm_awq_algo(at::Tensor I, at::Tensor W, at::Tensor W_zeros_scales, const int N, const int group_size,
                          const int algo) {
@@ -515,6 +611,9 @@ PYBIND11_MODULE(quant, m) {
           py::arg("ln_bias") = py::none(), py::arg("ln_eps") = 1e-5, py::arg("W"), py::arg("W_zeros_scales"),
           py::arg("bias") = py::none(), py::arg("residual") = py::none(), py::arg("act") = "none", py::arg("N"),
           py::arg("group_size"));
+    m.def("walinear_forward", &walinear_forward);
+    m.def("lut_attention", &lut_attention);
+    m.def("decode_attention", &decode_attention);
     m.def("gemm_awq_silu_dot_ut", &gemm_awq_silu_dot_ut, py::arg("I"), py::arg("W1") = py::none(),
           py::arg("W2") = py::none(), py::arg("ZS1") = py::none(), py::arg("ZS2") = py::none(),
           py::arg("W13") = py::none(), py::arg("ZS13") = py::none(), py::arg("M"), py::arg("N"), py::arg("K"),

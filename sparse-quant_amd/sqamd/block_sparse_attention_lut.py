@@ -10,6 +10,7 @@ here in one kernel behind sq_decode_attention.
 """
 import torch
 
+import quant
 from . import capi
 
 
@@ -23,9 +24,11 @@ def sparse_attention_prefill(q, k, v, sm_scale, lut, LT=True, BLOCK_M=64, BLOCK_
         raise TypeError("lut must be int32 or int64")
     if not q.is_cuda:
         raise RuntimeError("sparse_attention_prefill needs device tensors; there is no host path")
+    out = quant.lut_attention(q, k, v, lut, sm_scale, LT)
+    if out is not None:
+        return out
+    # something has to be copied or moved first, or is refused
     lut = lut.contiguous().to(q.device)
-    if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()) and capi.lut_attention_strided_ok(q, k, v):
-        return capi.lut_attention_strided(q, k, v, lut, sm_scale, LT)  # views of a fused projection: no copies
     return capi.lut_attention(q.contiguous(), k.contiguous(), v.contiguous(), lut, sm_scale, LT)
 
 
@@ -42,10 +45,13 @@ def sparse_attention(q, k, v, sm_scale, lut, LT=True, BLOCK_M=64, BLOCK_N=64, at
             raise ValueError("decode attention is inference only (the reference applies dropout with training=False)")
         if not q.is_cuda:
             raise RuntimeError("sparse_attention needs device tensors; there is no host path")
-        if k.stride(-1) != 1 or k.stride(2) != k.size(3) or v.stride() != k.stride():
-            k, v = k.contiguous(), v.contiguous()
         if attention_mask is not None:
             attention_mask = attention_mask.to(torch.float16).contiguous()
+        out = quant.decode_attention(q, k, v, attention_mask, sm_scale)
+        if out is not None:
+            return out
+        if k.stride(-1) != 1 or k.stride(2) != k.size(3) or v.stride() != k.stride():
+            k, v = k.contiguous(), v.contiguous()
         out = capi.decode_attention(q.contiguous(), k, v, kv_len, sm_scale, mask=attention_mask)
         return out.view(bsz, num_heads, 1, -1)
     return sparse_attention_prefill(q, k, v, sm_scale, lut, LT, BLOCK_M, BLOCK_N)

@@ -48,14 +48,18 @@ class WALinear(nn.Module):
         else:
             self.register_buffer("bias", None)
 
-    @torch.no_grad()
     def forward(self, x, residual=None, act="none", pre_ln=None):
         """y = act(x W_hat^T + bias) + residual.  With the defaults this is the reference's
         forward (gemm_awq_ut, then + bias); bias, activation and residual all ride in the
         kernel's store instead of separate element-wise launches.  pre_ln: an nn.LayerNorm (or
         any object with weight, bias, eps) applied to x first, inside the same kernel where the
         shape allows (up to 8 tokens, group size 128, 2048 < K <= 4096)."""
-        weight = self.weight
+        buffers = self._buffers  # (a look-up through the module costs four times as much, three times a call)
+        weight = buffers.get("weight")
+        zeros_scales = buffers.get("zeros_scales")
+        if weight is None or zeros_scales is None:
+            weight, zeros_scales = self.weight, self.zeros_scales
+        bias = buffers["bias"] if "bias" in buffers else self.bias
         if self.w_bit == 2:
             # uint8 [N, K/4] or int32 [K, N/16] -> the 4-bit words of the same layout, as the
             # reference's forward does on every call (test/muxi/module/qlinear/qlinear.py:61-62,
@@ -70,20 +74,13 @@ class WALinear(nn.Module):
                     self._expanded = quant.convert_2bit_to_4bit(weight)
                     self._expanded_key = key
                 weight = self._expanded
-        lead = x.shape[:-1]
-        x3 = x.reshape(1, -1, x.shape[-1]) if x.dim() != 3 else x
-        res3 = None
-        if residual is not None:
-            res3 = residual.reshape(x3.shape[0], x3.shape[1], self.out_features).contiguous()
-        if pre_ln is not None:
-            if self.layout != "l1":
-                raise NotImplementedError("pre_ln is supported in layout 'l1' only")
-            y = quant.gemm_awq_ln_fused_ut(x3.contiguous(), pre_ln.weight, pre_ln.bias, pre_ln.eps, weight,
-                                           self.zeros_scales, self.bias, res3, act, self.out_features, self.group_size)
-        else:
-            y = quant.gemm_awq_fused_ut(x3.contiguous(), weight, self.zeros_scales, self.bias, res3, act,
-                                        self.out_features, self.group_size)
-        return y.reshape(*lead, self.out_features)
+        if pre_ln is None:
+            return quant.walinear_forward(x, weight, zeros_scales, bias, residual, act, self.out_features,
+                                          self.group_size, False, None, None, 0.0)
+        if self.layout != "l1":
+            raise NotImplementedError("pre_ln is supported in layout 'l1' only")
+        return quant.walinear_forward(x, weight, zeros_scales, bias, residual, act, self.out_features, self.group_size,
+                                      True, pre_ln.weight, pre_ln.bias, pre_ln.eps)
 
     @staticmethod
     def from_float(module, w_config, a_config=None, quantize_output=False, layout="l1"):
