@@ -388,8 +388,7 @@ at::Tensor walinear_forward(const at::Tensor& x, const at::Tensor& W, const at::
 
 // The two branches of sparse_attention on tensors that need no conversion (12.4 and 19.2 us of host time a call from
 // Python, 7.1 and 6.3 here: 8 x 16 heads x 512 x 64 at 25 % took 11.1 us and takes 8.7); anything else returns nothing
-// and takes the
-// general path in Python, which copies or refuses it.
+// and takes the general path in Python, which copies or refuses it.
 bool half_rows(const at::Tensor& t, const at::Tensor& like) {
     return t.is_cuda() && t.device() == like.device() && t.scalar_type() == at::kHalf && t.dim() == 4 &&
            t.stride(3) == 1 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;

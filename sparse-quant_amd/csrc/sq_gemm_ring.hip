@@ -23,6 +23,10 @@
 //   100 tokens  4096x4096 15.9 -> 11.0, 15360x5120 37.3 -> 28.8, 5120x13696 54.0 -> 30.2
 //   333 tokens  4096x4096 27.0 -> 20.2, 12288x4096 65.1 -> 47.5, 5120x13696 90.3 -> 65.0
 //   1024 tokens 4096x4096 46.0 -> 41, 5120x13696 202 -> 152; 2048 tokens 4096x16384 269 -> 243 (1.13 PFLOP/s)
+// Tiles of 256 x 256 (two rows of waves that share the weight columns, no K groups to add up at the end, a quarter less
+// to load per product) where they fill the chip: 12288x4096 at 1024 tokens 118 -> 105, 16384x4096 at 2048 tokens
+// 269 -> 259, at 4096 tokens 537 -> 512, 15360x5120 at 4096 tokens 647 -> 610 (1.06 PFLOP/s on a box where the smaller
+// tiles reach 1.00).
 // Tried and dropped: all waves in one group with software-pipelined operands (8..15 % slower), stages of 32 k per wave
 // with twice the bytes in flight (10 % slower: a barrier per 8 matrix instructions), the group sums handed over in
 // registers' order instead of row-major slices (1..4 % slower below 256 tokens).
@@ -571,7 +575,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 // per stage.  LDS holds three or four stages.
 #define SQ_RING_SHAPES(X_)                                                                                             \
     X_(1, 1, 2, 1, 1, 8, 3) X_(2, 1, 2, 1, 2, 4, 4) X_(3, 2, 2, 1, 2, 4, 3) X_(4, 3, 1, 1, 4, 2, 4) X_(5, 2, 2, 1, 4, 2, 4) \
-        X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3) X_(8, 4, 2, 1, 4, 2, 3)
+        X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3) X_(8, 4, 2, 1, 4, 2, 3) X_(9, 4, 2, 2, 4, 1, 3)
 
 template <int MI, int NI, int WM, int WN, int WK, int GS, int ST>
 static hipError_t launch_shape(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int nfull,
@@ -605,6 +609,7 @@ static const RingTile kRingTiles[] = {
     {96, 256, 128, 4.305f, 1.017f, 0.410f, 0.106f, 1.298f, 0.243f},
     {128, 128, 128, 3.276f, 0.802f, 0.268f, 0.000f, 0.967f, 0.278f},
     {128, 256, 128, 4.931f, 1.142f, 0.611f, 0.100f, 1.663f, 0.230f},
+    {256, 256, 64, 5.673f, 0.778f, 0.907f, 0.f, 0.f, 0.f},  // never split, see plan_ring
 };
 constexpr int RING_SHAPES = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
 #define X_(id, MI, NI, WM, WN, WK, ST)                                                                              \
@@ -647,7 +652,8 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes) {
             best = p;
         };
         consider(base + (rest ? stages * (t.step0 + t.step1 * rest * (1.f / 256)) + t.fixed : 0.f), 0, 1);
-        if (ws_bytes == 0 || rest == 0) continue;
+        // (256 x 256 tiles split over K were behind smaller tiles wherever they were timed: partial tiles of 256 KB)
+        if (ws_bytes == 0 || rest == 0 || t.bm == 256) continue;
         static const int splits[5] = {2, 3, 4, 6, 8};
         for (int ks : splits) {
             const long w = (long)rest * ks;

@@ -60,3 +60,9 @@ def test_ring_parity(capi, shape, m, n, k, g):
     assert ran >= 1
     y = capi.gemm_fused(xd, w, zs, n, k, g, bias=bd, residual=rd, act=capi.SQ_ACT_RELU, algo=capi.SQ_ALGO_RING, ws=ws)
     assert np.all(np.abs(y.cpu().numpy().astype(np.float64) - ref) <= bound)
+
+
+@pytest.mark.parametrize("m,n,k,g", CASES + [(257, 264, 320, 64), (520, 136, 1056, 32)])
+def test_ring_parity_of_256_row_tiles(capi, m, n, k, g):
+    """Two rows of waves over the same weight columns: the second row of tiles full, ragged and absent."""
+    test_ring_parity(capi, 9, m, n, k, g)
