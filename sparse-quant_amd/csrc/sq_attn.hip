@@ -26,12 +26,16 @@
 // exponentials at a quarter of the rate among them); the operand reads take 512 LDS cycles per 64 x 64 block (32
 // queries per wave: each K and V value is read twice; with 16 per wave it is four times, and 1024 cycles were the
 // bound).  Four workgroups of 32 KB share a CU, two waves per SIMD, each at its own point of the step, so that one's
-// softmax and first loads run beside another's products; four waves on one 64-key step (64 KB, the key halves of a
-// query merged at the end) were 20 % slower, for the time a workgroup takes to start and end is not hidden there.
+// softmax and first loads run beside another's products.  Where there are too few workgroups for that, four waves take
+// steps of 64 keys and split them (SPLIT_WGS below).
 // Measured (us; before: 16 queries per wave, K through registers, V transposed by vector instructions):
-//   32 heads x 4096 x 128, causal, 26 % of the blocks   115 -> 86 (matrix pipes busy 0.39 of the cycles)
-//   8 x 32 heads x 512 x 128, causal, 26 %               35 -> 35 (134 MB to move: 22 at the rate of a copy)
-//   8 x 16 heads x 512 x 64, 25 %                        10.1 -> 9.4
+//   32 heads x 4096 x 128, causal, 26 % of the blocks   125 -> 87 (matrix pipes busy 0.39 of the cycles)
+//   8 x 16 heads x 4096 x 64, 25 %                       225 -> 188
+//   8 x 32 heads x 512 x 128, causal, 26 %               38.5 -> 35 (134 MB to move: 22 at the rate of a copy)
+//   8 x 16 heads x 512 x 64, 25 %                        10.2 -> 9.0
+//   16 heads x 1674 x 128, causal, 42 %                  26.4 -> 18.6;   12 heads x 128 x 64  4.2 -> 4.2
+// Of a small call's time 0.5 us was the fetch of the kernel's arguments in front of the first request: those that the
+// request of the table needs are scalars now, which arrive with the wave.
 // A model's prompt reads q, k and v where the fused projection left them and stores the cache rows and a [batch, row,
 // hidden] output: the element-wise copies around the kernel cost three times its own time (8 prompts of 512 tokens, 32
 // heads of 128, per layer: six copies of 21 us and 35 -> 52 in all; without a table, against torch's attention and its
@@ -45,19 +49,14 @@ namespace sq {
 
 namespace {
 
+// What a workgroup needs after its first request (of the table) is out.
 struct LutAttnArgs {
-    const half_t* q;
-    const half_t* k;
-    const half_t* v;
     half_t* o;
     half_t* kc;       // caches that receive the K and V rows, or null
     half_t* vc;
-    const void* lut;  // null: every block (causal: up to the diagonal)
     LutAttnStrides st;
-    int lut_is_64, H, S, nblk, nnz, nvisit;
     float qk_scale;  // sm_scale * log2(e)
     float lazy;      // log2 of how far a score may exceed the reference maximum
-    int causal, total_wg;
 };
 
 // Chunk permutations inside a tile row of D halves (D / 8 chunks of 16 bytes).
@@ -78,14 +77,20 @@ __device__ __forceinline__ short4_t lds_read_tr(const uint8_t* p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p));
 }
 
-template <int D>
-__global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
+// KG = 1: two waves, steps of 32 keys.  KG = 2: four waves, steps of 64 keys, wave (qg, kg) on keys 32 kg .. + 31 of each
+// with a softmax state of its own; the two states of a query meet at the end.
+template <int D, int KG>
+__global__ __launch_bounds__(128 * KG, 2) void lut_attn_kernel(
+    const void* __restrict__ lut, int lut_is_64, int nblk, int nnz, int nvisit, int H, int S, int causal, int total_wg,
+    const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v, LutAttnArgs a) {
+    // (the scalars and q, k, v arrive in registers with the wave; a structure has to be fetched)
     constexpr int ROW = D * 2;              // bytes of a tile row
-    constexpr int TILE = 32 * ROW;          // K or V of one step: 32 keys
+    constexpr int STEP = 32 * KG;           // keys of a step
+    constexpr int TILE = STEP * ROW;        // K or V of one step
     constexpr int SB = 2 * TILE;            // a stage: K tile, V tile
     constexpr int NK = D / 16;              // matrix steps of S^T
     constexpr int DT = D / 32;              // 32-row tiles of O^T
-    constexpr int NL = TILE / 1024 / 2;     // direct loads per wave, operand and stage
+    constexpr int NL = 16 * ROW / 1024;     // direct loads per wave, operand and stage
     constexpr int RPL = 1024 / ROW;         // tile rows per load
     __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * SB];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
@@ -95,56 +100,65 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ln = lane & 31;
     const int lc = lane >> 5;
+    const int qg = wave / KG;
+    const int kg = wave % KG;
     // Workgroups are handed to the eight XCDs round-robin by their linear id, and every XCD has its own L2.
     // The id is therefore re-read as (XCD, slot): XCD x works through the x-th eighth of the (head, query block)
     // list, so that all query blocks of a head, which visit the same K and V rows, share one L2
     // instead of pulling those rows into all eight.  Causal: the long rows first.
-    const int per_xcd = (a.total_wg + 7) >> 3;
+    const int per_xcd = (total_wg + 7) >> 3;
     const int work = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (work >= a.total_wg) return;
-    const int zh = work / a.nblk;
-    const int qr = work - zh * a.nblk;
-    const int qb = a.causal ? a.nblk - 1 - qr : qr;
-    const int h = zh % a.H;
-    const int S = a.S;
-    const int z = zh / a.H;
-    const half_t* kz = a.k + z * a.st.kv[0] + h * a.st.kv[1];
-    const half_t* vz = a.v + z * a.st.kv[0] + h * a.st.kv[1];
+    if (work >= total_wg) return;
+    const int zh = work / nblk;
+    const int qr = work - zh * nblk;
+    const int qb = causal ? nblk - 1 - qr : qr;
+    const int h = zh % H;
+    const int z = zh / H;
+    const half_t* kz = k + z * a.st.kv[0] + h * a.st.kv[1];
+    const half_t* vz = v + z * a.st.kv[0] + h * a.st.kv[1];
     const int kv_row = (int)a.st.kv[2] * 2;  // bytes
-    const int m = qb * 64 + 32 * wave + ln;  // this lane's query
-
-    half8_t qf[NK];
-    {
-        const half_t* qp = a.q + z * a.st.q[0] + h * a.st.q[1] + imin(m, S - 1) * a.st.q[2] + 8 * lc;
-#pragma unroll
-        for (int s = 0; s < NK; s++) qf[s] = *(const half8_t*)(qp + 16 * s);
-    }
+    const int m = qb * 64 + 32 * qg + ln;  // this lane's query
 
     // The visited blocks, 64 table entries at a time: lane j holds entry j, `todo` has a bit for each that is visited.
-    const long lut_row = ((long)h * a.nblk + qb) * a.nnz;
-    const int nvisit = a.lut ? a.nvisit : (a.causal ? qb + 1 : a.nblk);
+    const long lut_row = ((long)h * nblk + qb) * nnz;
+    const int entries = lut ? nvisit : (causal ? qb + 1 : nblk);
     int entry = 0, jbase = 0, last = -1;
     uint64_t todo = 0;
+    auto table = [&](int j) {
+        int blk = -1;
+        if (j < entries) {
+            blk = j;
+            if (lut) blk = lut_is_64 ? (int)((const long long*)lut)[lut_row + j] : ((const int*)lut)[lut_row + j];
+        }
+        return blk;
+    };
+    auto take = [&](int blk) {
+        const int up = __shfl_up(blk, 1);
+        const int prev = lane == 0 ? last : up;
+        todo = __builtin_amdgcn_ballot_w64(blk != prev && blk >= 0 && (long)blk * 64 < S);
+        entry = blk;
+        last = __builtin_amdgcn_readlane(blk, 63);
+        jbase += 64;
+    };
     auto next_block = [&]() {  // its first key, or -1
         while (todo == 0) {
-            if (jbase >= nvisit) return -1;
-            const int j = jbase + lane;
-            int blk = -1;
-            if (j < nvisit) {
-                blk = j;
-                if (a.lut) blk = a.lut_is_64 ? (int)((const long long*)a.lut)[lut_row + j] : ((const int*)a.lut)[lut_row + j];
-            }
-            const int up = __shfl_up(blk, 1);
-            const int prev = lane == 0 ? last : up;
-            todo = __builtin_amdgcn_ballot_w64(blk != prev && blk >= 0 && (long)blk * 64 < S);
-            entry = blk;
-            last = __builtin_amdgcn_readlane(blk, 63);
-            jbase += 64;
+            if (jbase >= entries) return -1;
+            take(table(jbase + lane));
         }
         const int j = __builtin_ctzll(todo);
         todo &= todo - 1;
         return __builtin_amdgcn_readlane(entry, j) * 64;
     };
+    const int first = table(lane);  // requested ahead of the queries
+
+    half8_t qf[NK];
+    {
+        const half_t* qp = q + z * a.st.q[0] + h * a.st.q[1] + imin(m, S - 1) * a.st.q[2] + 8 * lc;
+#pragma unroll
+        for (int s = 0; s < NK; s++) qf[s] = *(const half8_t*)(qp + 16 * s);
+    }
+
+    take(first);
     int n0 = next_block();
 
     // Byte offsets of this wave's loads inside a step; load j covers tile rows RPL * (NL * wave + j) .. + RPL - 1.
@@ -158,14 +172,14 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
     uint32_t koff[NL], voff[NL];
 #pragma unroll
     for (int j = 0; j < NL; j++) {
-        koff[j] = lane_offset(j, 31, false);
-        voff[j] = lane_offset(j, 31, true);
+        koff[j] = lane_offset(j, STEP - 1, false);
+        voff[j] = lane_offset(j, STEP - 1, true);
     }
     auto issue = [&](int n, int slot) {
         const uint8_t* kb = (const uint8_t*)(kz + n * a.st.kv[2]);
         const uint8_t* vb = (const uint8_t*)(vz + n * a.st.kv[2]);
         const uint32_t l0 = lds0 + slot * SB + wave * (NL * 1024);
-        if (n + 32 <= S) {
+        if (n + STEP <= S) {
 #pragma unroll
             for (int j = 0; j < NL; j++) load_to_lds_x4(kb, koff[j], l0 + j * 1024);
 #pragma unroll
@@ -182,12 +196,12 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
     // LDS byte offsets of the operand reads.
     int kread[NK], vread[DT];
 #pragma unroll
-    for (int s = 0; s < NK; s++) kread[s] = ln * ROW + (((2 * s + lc) ^ k_swz<D>(ln)) * 16);
+    for (int s = 0; s < NK; s++) kread[s] = (32 * kg + ln) * ROW + (((2 * s + lc) ^ k_swz<D>(ln)) * 16);
     {
-        const int key = 4 * lc + ((lane & 15) >> 2);  // + 16 s + 8 i, which leave v_swz unchanged
+        const int key = 4 * lc + ((lane & 15) >> 2);  // + 32 kg + 16 s + 8 i, which leave v_swz unchanged
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
-            vread[dt] = TILE + key * ROW + (((4 * dt + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ v_swz<D>(key)) * 16) +
+            vread[dt] = TILE + (32 * kg + key) * ROW + (((4 * dt + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ v_swz<D>(key)) * 16) +
                         8 * (lane & 1);
     }
 
@@ -231,11 +245,12 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; v++) st[v] = __builtin_fmaf(st[v], a.qk_scale, -ref);
         // Masks (only where the step touches the end of the sequence or the causal diagonal; the test is uniform).
-        if (n + 32 > S || (a.causal && n + 31 > qb * 64 + 32 * wave)) {
+        const int nk = n + 32 * kg;
+        if (nk + 32 > S || (causal && nk + 31 > qb * 64 + 32 * qg)) {
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                const int key = n + 8 * (v >> 2) + 4 * lc + (v & 3);
-                const bool keep = (key < S) && (!a.causal || key <= m);
+                const int key = nk + 8 * (v >> 2) + 4 * lc + (v & 3);
+                const bool keep = (key < S) && (!causal || key <= m);
                 st[v] = keep ? st[v] : -INFINITY;
             }
         }
@@ -286,7 +301,7 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
             }
     };
 
-    // One barrier per step: behind it this step's tiles have landed for both waves and nobody reads the other slot any
+    // One barrier per step: behind it this step's tiles have landed for every wave and nobody reads the other slot any
     // more, which the next step's loads may then fill.
     auto landed = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
     // The query operands are waited for here, together with the first tiles: left to the loop, the compiler's wait for
@@ -297,41 +312,100 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
         asm volatile("" : "+v"(t));
         qf[s] = bit_cast<half8_t>(t);
     }
-    while (n0 >= 0) {
-        const int n1 = next_block();
-        const bool whole = n0 + 32 < S;  // the block has a second half
-        landed();
-        visit(n0, std::integral_constant<int, 0>{}, whole ? n0 + 32 : -1);
-        landed();
-        if (whole)
-            visit(n0 + 32, std::integral_constant<int, 1>{}, n1);
-        else if (n1 >= 0)
-            issue(n1, 0);
-        n0 = n1;
+    if constexpr (KG == 1) {
+        while (n0 >= 0) {
+            const int n1 = next_block();
+            const bool whole = n0 + 32 < S;  // the block has a second half
+            landed();
+            visit(n0, std::integral_constant<int, 0>{}, whole ? n0 + 32 : -1);
+            landed();
+            if (whole)
+                visit(n0 + 32, std::integral_constant<int, 1>{}, n1);
+            else if (n1 >= 0)
+                issue(n1, 0);
+            n0 = n1;
+        }
+    } else {
+        while (n0 >= 0) {
+            const int n1 = next_block();
+            landed();
+            visit(n0, std::integral_constant<int, 0>{}, n1);
+            if (n1 < 0) break;
+            n0 = next_block();
+            landed();
+            visit(n1, std::integral_constant<int, 1>{}, n0);
+        }
     }
 
     // The row sum of a query is split over its two lanes.  A query row without any visible key has l = 0 and acc = 0:
     // 0 * inf = NaN, which is also what the reference's running sums produce for such a row.
-    const float inv = 1.f / (l_i + __shfl_xor(l_i, 32));
-    // The wave's 32 x D outputs leave through its part of LDS (16-byte chunks permuted like K's) as whole rows: a lane
+    // The 32 x D outputs of a query group leave through LDS (16-byte chunks permuted like K's) as whole rows: a lane
     // holds four columns at a time, and 8-byte stores would cost the L2 eight times the write requests.
+    l_i += __shfl_xor(l_i, 32);
     __syncthreads();
-    uint8_t* out = lds + wave * TILE;
+    uint8_t* out = lds + qg * (32 * ROW);
+    auto park = [&](int dt, int i, half4_t o) {
+        *(half4_t*)(out + ln * ROW + (((4 * dt + i) ^ k_swz<D>(ln)) * 16) + 8 * lc) = o;
+    };
+    if constexpr (KG == 1) {
+        const float inv = 1.f / l_i;
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++)
+        for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            half4_t o;
+            for (int i = 0; i < 4; i++) {
+                half4_t o;
 #pragma unroll
-            for (int j = 0; j < 4; j++) o[j] = (half_t)(acc[dt][4 * i + j] * inv);
-            *(half4_t*)(out + ln * ROW + (((4 * dt + i) ^ k_swz<D>(ln)) * 16) + 8 * lc) = o;
-        }
-    __builtin_amdgcn_wave_barrier();
+                for (int j = 0; j < 4; j++) o[j] = (half_t)(acc[dt][4 * i + j] * inv);
+                park(dt, i, o);
+            }
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        // Each wave hands half of its output columns to the other key half's wave, with its reference maximum and row
+        // sum, and finishes the others.
+        constexpr int HALF = DT / 2;
+        float4_t* red = reinterpret_cast<float4_t*>(lds + 64 * ROW);                // [wave][HALF][4][64]
+        float2* stat = reinterpret_cast<float2*>(lds + 64 * ROW + 4 * HALF * 4096);  // [wave][64]
+        static_assert(64 * ROW + 4 * HALF * 4096 + 4 * 512 <= 2 * SB, "fits");
+        const float m_i = limit == -INFINITY ? -INFINITY : ref;
 #pragma unroll
-    for (int j = 0; j < TILE / 1024; j++) {
-        const int row = RPL * j + lrow;
+        for (int d = 0; d < HALF; d++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float4_t t;
+#pragma unroll
+                for (int j = 0; j < 4; j++) t[j] = kg == 0 ? acc[HALF + d][4 * i + j] : acc[d][4 * i + j];
+                red[((wave * HALF + d) * 4 + i) * 64 + lane] = t;
+            }
+        stat[wave * 64 + lane] = make_float2(m_i, l_i);
+        __syncthreads();
+        const int peer = wave ^ 1;
+        const float2 ps = stat[peer * 64 + lane];
+        const float mm = fmaxf(m_i, ps.x);
+        const float f_own = (m_i == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_i - mm);
+        const float f_peer = (ps.x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ps.x - mm);
+        const float inv = 1.f / (l_i * f_own + ps.y * f_peer);
+        const float w_own = f_own * inv, w_peer = f_peer * inv;
+#pragma unroll
+        for (int d = 0; d < HALF; d++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float4_t t = red[((peer * HALF + d) * 4 + i) * 64 + lane];
+                half4_t o;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float mine = kg == 0 ? acc[d][4 * i + j] : acc[HALF + d][4 * i + j];
+                    o[j] = (half_t)(mine * w_own + t[j] * w_peer);
+                }
+                park(d + (kg ? HALF : 0), i, o);
+            }
+        __syncthreads();
+    }
+    constexpr int PASSES = 32 * ROW / 1024 / KG;  // 1 KB of whole rows per wave and pass
+#pragma unroll
+    for (int j = 0; j < PASSES; j++) {
+        const int row = RPL * (PASSES * kg + j) + lrow;
         const u32x4_t t = *(const u32x4_t*)(out + row * ROW + ((lchunk ^ k_swz<D>(row)) * 16));
-        const int mr = qb * 64 + 32 * wave + row;
+        const int mr = qb * 64 + 32 * qg + row;
         if (mr < S) *(u32x4_t*)(a.o + z * a.st.o[0] + h * a.st.o[1] + mr * a.st.o[2] + 8 * lchunk) = t;
     }
     // The workgroup's own 64 rows of K and V go to the caches (their lines are in this XCD's L2).
@@ -339,8 +413,8 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
         half_t* kcz = a.kc + z * a.st.c[0] + h * a.st.c[1];
         half_t* vcz = a.vc + z * a.st.c[0] + h * a.st.c[1];
 #pragma unroll
-        for (int j = 0; j < TILE / 1024; j++) {
-            const int mr = qb * 64 + 32 * wave + RPL * j + lrow;
+        for (int j = 0; j < PASSES; j++) {
+            const int mr = qb * 64 + 32 * qg + RPL * (PASSES * kg + j) + lrow;
             if (mr < S) {
                 *(u32x4_t*)(kcz + mr * a.st.c[2] + 8 * lchunk) = *(const u32x4_t*)(kz + mr * a.st.kv[2] + 8 * lchunk);
                 *(u32x4_t*)(vcz + mr * a.st.c[2] + 8 * lchunk) = *(const u32x4_t*)(vz + mr * a.st.kv[2] + 8 * lchunk);
@@ -349,38 +423,43 @@ __global__ __launch_bounds__(128, 2) void lut_attn_kernel(LutAttnArgs a) {
     }
 }
 
+// Workgroups up to which the four-wave form is launched: two of them per CU, so that all are resident at once and what
+// counts is how soon each is through its own blocks.  Two against four waves (us): 16 heads x 1674 x 128, 432 workgroups,
+// 23.7 / 18.6; 2 x 12 x 1138 x 64, 432, 9.9 / 8.2; 12 x 128 x 64, 24, 4.6 / 4.2; 5 x 32 x 145 x 64 with one block per
+// row, 480, 5.5 / 5.7; beyond: 6 x 32 x 159 x 128, 576, 9.4 / 11.9; 2 x 16 x 1669 x 128, 864, 21.2 / 24.5.
+constexpr int SPLIT_WGS = 512;
+
 }  // namespace
 
 hipError_t launch_lut_attention(const void* q, const void* k, const void* v, void* o, void* k_cache, void* v_cache,
                                 const void* lut, int lut_elem_bytes, int Z, int H, int S, int D, int nnz,
                                 const LutAttnStrides& strides, float sm_scale, int causal, hipStream_t st) {
     LutAttnArgs a;
-    a.q = (const half_t*)q;
-    a.k = (const half_t*)k;
-    a.v = (const half_t*)v;
     a.o = (half_t*)o;
     a.kc = (half_t*)k_cache;
     a.vc = (half_t*)v_cache;
-    a.lut = lut;
     a.st = strides;
-    a.lut_is_64 = lut_elem_bytes == 8;
-    a.H = H;
-    a.S = S;
-    a.nblk = (S + 63) / 64;
-    a.nnz = nnz;
-    a.nvisit = nnz < a.nblk ? nnz : a.nblk;  // the reference clamps NNZ to ceil(S / 64) as well (the row pitch stays nnz)
     a.qk_scale = sm_scale * 1.44269504f;
     // Without a table the reference is the running maximum itself, whose probability 1 is exact in fp16: the error of a
     // dense softmax with it (2.43e-4 of the result at 512 keys, 2.51e-4 with the lazy one) at the price of more rescaling
     // (8 x 32 heads x 512 x 128: 51 -> 59 us).
     a.lazy = lut ? 8.f : 0.f;
-    a.causal = causal;
-    a.total_wg = a.nblk * Z * H;
-    const dim3 grid(((a.total_wg + 7) / 8) * 8);
-    if (D == 64)
-        hipLaunchKernelGGL((lut_attn_kernel<64>), grid, dim3(128), 0, st, a);
-    else
-        hipLaunchKernelGGL((lut_attn_kernel<128>), grid, dim3(128), 0, st, a);
+    const int nblk = (S + 63) / 64;
+    const int nvisit = lut && nnz < nblk ? nnz : nblk;  // the reference clamps NNZ to ceil(S / 64) as well (the row pitch stays nnz)
+    const int total_wg = nblk * Z * H;
+    const dim3 grid(((total_wg + 7) / 8) * 8);
+    const bool split = total_wg <= SPLIT_WGS;
+#define SQ_ATTN_LAUNCH(D_, KG_)                                                                                          \
+    hipLaunchKernelGGL((lut_attn_kernel<D_, KG_>), grid, dim3(128 * KG_), 0, st, lut, (int)(lut_elem_bytes == 8), nblk, nnz, \
+                       nvisit, H, S, causal, total_wg, (const half_t*)q, (const half_t*)k, (const half_t*)v, a)
+    if (D == 64) {
+        if (split) SQ_ATTN_LAUNCH(64, 2);
+        else SQ_ATTN_LAUNCH(64, 1);
+    } else {
+        if (split) SQ_ATTN_LAUNCH(128, 2);
+        else SQ_ATTN_LAUNCH(128, 1);
+    }
+#undef SQ_ATTN_LAUNCH
     return hipGetLastError();
 }
 

@@ -242,3 +242,30 @@ def test_strided_attention_refuses_what_it_cannot_address(capi):
     assert not capi.lut_attention_strided_ok(q, q, q.contiguous())                # k and v laid out differently
     assert not capi.lut_attention_strided_ok(q, q, q, q[:, :, :8], q[:, :, :8])   # a cache shorter than the prompt
     assert not capi.lut_attention_strided_ok(q.float(), q, q)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("z,h,s,causal", [(3, 171, 64, True), (1, 171, 161, False), (2, 86, 161, True), (1, 257, 97, True),
+                                           (1, 513, 33, False), (1, 128, 256, True), (1, 129, 250, False)])
+def test_both_forms_at_the_edges_of_a_step(capi, z, h, s, causal, d):
+    """Around 512 workgroups, up to which four waves share a step: 513, 513, 516, 514 and 513 are beyond it, the last two
+    are 512 and 516."""
+    rng = np.random.default_rng(h + s)
+    q, k, v = (rng.normal(size=(z, h, s, d)).astype(np.float16) for _ in range(3))
+    lut = att.layout_to_lut(att.synth_layout(h, (s + 63) // 64, 0.6, causal, seed=s))
+    _assert_close_fp16(capi, q, k, v, lut, d ** -0.5, causal)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_strided_attention_beyond_512_workgroups(capi, d):
+    z, h, s = 2, 100, 161
+    gen = torch.Generator(device="cuda").manual_seed(s + d)
+    qkv = torch.randn((z, s, 3, h, d), device="cuda", generator=gen).half()
+    q, k, v = (qkv[:, :, j].transpose(1, 2) for j in range(3))
+    lut = torch.from_numpy(att.layout_to_lut(att.synth_layout(h, (s + 63) // 64, 0.6, True, seed=s))).cuda()
+    ref = capi.lut_attention(q.contiguous(), k.contiguous(), v.contiguous(), lut, 0.1, True)
+    kc, vc = (torch.full((z, h, s + 3, d), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+    out = capi.lut_attention_strided(q, k, v, lut, 0.1, True, kc, vc, rows_first=True)
+    assert torch.equal(out.transpose(1, 2), ref)
+    assert torch.equal(kc[:, :, :s], k) and torch.equal(vc[:, :, :s], v)
+    assert bool((kc[:, :, s:] == 7).all()) and bool((vc[:, :, s:] == 7).all())
