@@ -172,8 +172,10 @@ class OPTDecoder(nn.Module):
         for layer, (kc, vc) in zip(self.layers, cache):
             x = layer(x, kc, vc, pos0)
         x = _layernorm(self.final_ln, x[:, -1:])
-        if b <= 8 and self.hidden % 512 == 0 and 512 <= self.hidden <= 8192:  # what sq_f16_gemv takes
-            return capi.f16_gemv(x, self.lm_head).view(b, 1, -1)
+        w = self.lm_head
+        if b <= 8 and self.hidden % 512 == 0 and self.hidden <= 8192 and w.dtype == torch.float16 and w.is_contiguous() \
+                and w.data_ptr() % 16 == 0:  # what sq_f16_gemv takes
+            return capi.f16_gemv(x, w).view(b, 1, -1)
         return torch.matmul(x, self.lm_head.t())  # [B, 1, vocab]
 
     @torch.no_grad()
