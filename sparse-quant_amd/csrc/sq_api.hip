@@ -323,6 +323,7 @@ static int autotune_candidates(int M, int K, int g, bool has_ws, int* out, int c
             for (int rest = 0; rest <= (has_ws ? 1 : 0); rest++)
                 for (int ks = rest ? 2 : 1; ks <= (has_ws ? 8 : 1); ks += ks < 4 ? 1 : 2)
                     add(SQ_ALGO_RING, shape | (rest ? 0x10 : 0) | (ks << 8));
+    if (M > 128) add(SQ_ALGO_RING, 9 | (1 << 8));  // 256 x 256 tiles: never ahead when split
     return n;
 }
 
