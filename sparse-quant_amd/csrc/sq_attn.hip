@@ -29,11 +29,13 @@
 // softmax and first loads run beside another's products.  Where there are too few workgroups for that, four waves take
 // steps of 64 keys and split them (SPLIT_WGS below).
 // Measured (us; before: 16 queries per wave, K through registers, V transposed by vector instructions):
-//   32 heads x 4096 x 128, causal, 26 % of the blocks   125 -> 87 (matrix pipes busy 0.39 of the cycles)
+//   32 heads x 4096 x 128, causal, 26 % of the blocks   125 -> 85 (matrix pipes busy 0.39 of the cycles)
 //   8 x 16 heads x 4096 x 64, 25 %                       225 -> 188
-//   8 x 32 heads x 512 x 128, causal, 26 %               38.5 -> 35 (134 MB to move: 22 at the rate of a copy)
-//   8 x 16 heads x 512 x 64, 25 %                        10.2 -> 9.0
-//   16 heads x 1674 x 128, causal, 42 %                  26.4 -> 18.6;   12 heads x 128 x 64  4.2 -> 4.2
+//   8 x 32 heads x 512 x 128, causal, 26 %               38.5 -> 34 (134 MB to move: 22 at the rate of a copy)
+//   8 x 16 heads x 512 x 64, 25 %                        10.2 -> 8.1
+//   16 heads x 1674 x 128, causal, 42 %                  26.4 -> 18.0;   12 heads x 128 x 64  4.2 -> 4.2
+// Outputs and cache rows are nontemporal stores: they are not read here again, and as ordinary ones they push K and V
+// rows out of the L2s (5 x 32 heads x 365 x 128 15.1 -> 13.8, 8 x 16 x 512 x 64 8.8 -> 8.1).
 // Of a small call's time 0.5 us was the fetch of the kernel's arguments in front of the first request: those that the
 // request of the table needs are scalars now, which arrive with the wave.
 // A model's prompt reads q, k and v where the fused projection left them and stores the cache rows and a [batch, row,
@@ -406,7 +408,8 @@ __global__ __launch_bounds__(128 * KG, 2) void lut_attn_kernel(
         const int row = RPL * (PASSES * kg + j) + lrow;
         const u32x4_t t = *(const u32x4_t*)(out + row * ROW + ((lchunk ^ k_swz<D>(row)) * 16));
         const int mr = qb * 64 + 32 * qg + row;
-        if (mr < S) *(u32x4_t*)(a.o + z * a.st.o[0] + h * a.st.o[1] + mr * a.st.o[2] + 8 * lchunk) = t;
+        if (mr < S)
+            __builtin_nontemporal_store(t, (u32x4_t*)(a.o + z * a.st.o[0] + h * a.st.o[1] + mr * a.st.o[2] + 8 * lchunk));
     }
     // The workgroup's own 64 rows of K and V go to the caches (their lines are in this XCD's L2).
     if (a.kc) {
@@ -416,8 +419,10 @@ __global__ __launch_bounds__(128 * KG, 2) void lut_attn_kernel(
         for (int j = 0; j < PASSES; j++) {
             const int mr = qb * 64 + 32 * qg + RPL * (PASSES * kg + j) + lrow;
             if (mr < S) {
-                *(u32x4_t*)(kcz + mr * a.st.c[2] + 8 * lchunk) = *(const u32x4_t*)(kz + mr * a.st.kv[2] + 8 * lchunk);
-                *(u32x4_t*)(vcz + mr * a.st.c[2] + 8 * lchunk) = *(const u32x4_t*)(vz + mr * a.st.kv[2] + 8 * lchunk);
+                const u32x4_t kr = *(const u32x4_t*)(kz + mr * a.st.kv[2] + 8 * lchunk);
+                const u32x4_t vr = *(const u32x4_t*)(vz + mr * a.st.kv[2] + 8 * lchunk);
+                __builtin_nontemporal_store(kr, (u32x4_t*)(kcz + mr * a.st.c[2] + 8 * lchunk));
+                __builtin_nontemporal_store(vr, (u32x4_t*)(vcz + mr * a.st.c[2] + 8 * lchunk));
             }
         }
     }
