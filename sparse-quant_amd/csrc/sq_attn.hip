@@ -30,7 +30,7 @@
 // steps of 64 keys and split them (SPLIT_WGS below).
 // Measured (us; before: 16 queries per wave, K through registers, V transposed by vector instructions):
 //   32 heads x 4096 x 128, causal, 26 % of the blocks   125 -> 85 (matrix pipes busy 0.39 of the cycles)
-//   8 x 16 heads x 4096 x 64, 25 %                       225 -> 188
+//   8 x 16 heads x 4096 x 64, 25 %                       225 -> 181
 //   8 x 32 heads x 512 x 128, causal, 26 %               38.5 -> 34 (134 MB to move: 22 at the rate of a copy)
 //   8 x 16 heads x 512 x 64, 25 %                        10.2 -> 8.1
 //   16 heads x 1674 x 128, causal, 42 %                  26.4 -> 18.0;   12 heads x 128 x 64  4.2 -> 4.2
@@ -81,8 +81,9 @@ __device__ __forceinline__ short4_t lds_read_tr(const uint8_t* p) {
 
 // KG = 1: two waves, steps of 32 keys.  KG = 2: four waves, steps of 64 keys, wave (qg, kg) on keys 32 kg .. + 31 of each
 // with a softmax state of its own; the two states of a query meet at the end.
-template <int D, int KG>
-__global__ __launch_bounds__(128 * KG, 2) void lut_attn_kernel(
+// WPS: waves per SIMD the registers are limited to.
+template <int D, int KG, int WPS>
+__global__ __launch_bounds__(128 * KG, WPS) void lut_attn_kernel(
     const void* __restrict__ lut, int lut_is_64, int nblk, int nnz, int nvisit, int H, int S, int causal, int total_wg,
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v, LutAttnArgs a) {
     // (the scalars and q, k, v arrive in registers with the wave; a structure has to be fetched)
@@ -433,6 +434,11 @@ __global__ __launch_bounds__(128 * KG, 2) void lut_attn_kernel(
 // 23.7 / 18.6; 2 x 12 x 1138 x 64, 432, 9.9 / 8.2; 12 x 128 x 64, 24, 4.6 / 4.2; 5 x 32 x 145 x 64 with one block per
 // row, 480, 5.5 / 5.7; beyond: 6 x 32 x 159 x 128, 576, 9.4 / 11.9; 2 x 16 x 1669 x 128, 864, 21.2 / 24.5.
 constexpr int SPLIT_WGS = 512;
+// D = 64 takes 132 registers left to itself: three waves per SIMD, 1536 workgroups on the chip at once.  Four (128
+// registers, 2048 workgroups) are a little slower where three hold the whole grid and save the second round beyond (us,
+// three / four): 8 x 16 heads x 640, 1280 workgroups, 9.7 / 10.0; 4 x 32 x 768, 1536, 17.8 / 19.5; 8 x 16 x 1024, 2048,
+// 22.4 / 19.1; 4 x 16 x 2048, 2048, 32.5 / 28.6; 8 x 16 x 1536, 3072, 39.1 / 39.2; 8 x 16 x 4096, 8192, 188 / 181.
+constexpr int THREE_WAVE_WGS = 1536;
 
 }  // namespace
 
@@ -454,15 +460,16 @@ hipError_t launch_lut_attention(const void* q, const void* k, const void* v, voi
     const int total_wg = nblk * Z * H;
     const dim3 grid(((total_wg + 7) / 8) * 8);
     const bool split = total_wg <= SPLIT_WGS;
-#define SQ_ATTN_LAUNCH(D_, KG_)                                                                                          \
-    hipLaunchKernelGGL((lut_attn_kernel<D_, KG_>), grid, dim3(128 * KG_), 0, st, lut, (int)(lut_elem_bytes == 8), nblk, nnz, \
-                       nvisit, H, S, causal, total_wg, (const half_t*)q, (const half_t*)k, (const half_t*)v, a)
+#define SQ_ATTN_LAUNCH(D_, KG_, WPS_)                                                                                    \
+    hipLaunchKernelGGL((lut_attn_kernel<D_, KG_, WPS_>), grid, dim3(128 * KG_), 0, st, lut, (int)(lut_elem_bytes == 8), nblk, \
+                       nnz, nvisit, H, S, causal, total_wg, (const half_t*)q, (const half_t*)k, (const half_t*)v, a)
     if (D == 64) {
-        if (split) SQ_ATTN_LAUNCH(64, 2);
-        else SQ_ATTN_LAUNCH(64, 1);
+        if (split) SQ_ATTN_LAUNCH(64, 2, 2);
+        else if (total_wg <= THREE_WAVE_WGS) SQ_ATTN_LAUNCH(64, 1, 2);
+        else SQ_ATTN_LAUNCH(64, 1, 4);
     } else {
-        if (split) SQ_ATTN_LAUNCH(128, 2);
-        else SQ_ATTN_LAUNCH(128, 1);
+        if (split) SQ_ATTN_LAUNCH(128, 2, 2);
+        else SQ_ATTN_LAUNCH(128, 1, 2);
     }
 #undef SQ_ATTN_LAUNCH
     return hipGetLastError();

@@ -246,10 +246,11 @@ def test_strided_attention_refuses_what_it_cannot_address(capi):
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("z,h,s,causal", [(3, 171, 64, True), (1, 171, 161, False), (2, 86, 161, True), (1, 257, 97, True),
-                                           (1, 513, 33, False), (1, 128, 256, True), (1, 129, 250, False)])
+                                           (1, 513, 33, False), (1, 128, 256, True), (1, 129, 250, False),
+                                           (4, 384, 64, True), (4, 385, 50, False), (1, 513, 129, True)])
 def test_both_forms_at_the_edges_of_a_step(capi, z, h, s, causal, d):
-    """Around 512 workgroups, up to which four waves share a step: 513, 513, 516, 514 and 513 are beyond it, the last two
-    are 512 and 516."""
+    """Around 512 workgroups, up to which four waves share a step (513, 513, 516, 514, 513, then 512 and 516), and around
+    1536, beyond which head dimension 64 runs with fewer registers (1536, 1540, 1539)."""
     rng = np.random.default_rng(h + s)
     q, k, v = (rng.normal(size=(z, h, s, d)).astype(np.float16) for _ in range(3))
     lut = att.layout_to_lut(att.synth_layout(h, (s + 63) // 64, 0.6, causal, seed=s))
