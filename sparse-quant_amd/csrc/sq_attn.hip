@@ -33,7 +33,7 @@
 //   8 x 16 heads x 4096 x 64, 25 %                       225 -> 181
 //   8 x 32 heads x 512 x 128, causal, 26 %               38.5 -> 34 (134 MB to move: 22 at the rate of a copy)
 //   8 x 16 heads x 512 x 64, 25 %                        10.2 -> 8.1
-//   16 heads x 1674 x 128, causal, 42 %                  26.4 -> 18.0;   12 heads x 128 x 64  4.2 -> 4.2
+//   16 heads x 1674 x 128, causal, 42 %                  26.6 -> 17.3;   12 heads x 128 x 64  4.2 -> 4.2
 // Outputs and cache rows are nontemporal stores: they are not read here again, and as ordinary ones they push K and V
 // rows out of the L2s (5 x 32 heads x 365 x 128 15.1 -> 13.8, 8 x 16 x 512 x 64 8.8 -> 8.1).
 // Of a small call's time 0.5 us was the fetch of the kernel's arguments in front of the first request: those that the
@@ -436,8 +436,8 @@ __global__ __launch_bounds__(128 * KG, WPS) void lut_attn_kernel(
 
 // Workgroups up to which the four-wave form is launched: two of them per CU, so that all are resident at once and what
 // counts is how soon each is through its own blocks.  Two against four waves (us): 16 heads x 1674 x 128, 432 workgroups,
-// 23.7 / 18.6; 2 x 12 x 1138 x 64, 432, 9.9 / 8.2; 12 x 128 x 64, 24, 4.6 / 4.2; 5 x 32 x 145 x 64 with one block per
-// row, 480, 5.5 / 5.7; beyond: 6 x 32 x 159 x 128, 576, 9.4 / 11.9; 2 x 16 x 1669 x 128, 864, 21.2 / 24.5.
+// 22.3 / 17.3; 2 x 12 x 1138 x 64, 432, 9.5 / 7.8; 12 x 128 x 64, 24, 4.7 / 4.2; 5 x 32 x 145 x 64 with one block per
+// row, 480, 5.3 / 5.4; beyond: 6 x 32 x 159 x 128, 576, 8.7 / 11.2; 2 x 16 x 1669 x 128, 864, 19.6 / 23.2.
 constexpr int SPLIT_WGS = 512;
 // D = 64 takes 132 registers left to itself: three waves per SIMD, 1536 workgroups on the chip at once.  Four (128
 // registers, 2048 workgroups) are a little slower where three hold the whole grid and save the second round beyond (us,

@@ -166,9 +166,13 @@ class OPTDecoder(nn.Module):
     @torch.no_grad()
     def forward(self, ids, cache, pos0, pos_ids=None):
         b, t = ids.shape
-        if pos_ids is None:
-            pos_ids = torch.arange(pos0, pos0 + t, device=ids.device) + 2
-        x = self.embed[ids] + self.pos[pos_ids]
+        if pos_ids is None and isinstance(pos0, int) and 0 <= pos0 and pos0 + t + 2 <= self.pos.shape[0] \
+                and self.pos.dtype == self.embed.dtype:
+            x = self.embed[ids].add_(self.pos[pos0 + 2:pos0 + t + 2])  # consecutive positions: a slice of the table
+        else:
+            if pos_ids is None:
+                pos_ids = torch.arange(pos0, pos0 + t, device=ids.device) + 2
+            x = self.embed[ids] + self.pos[pos_ids]
         for layer, (kc, vc) in zip(self.layers, cache):
             x = layer(x, kc, vc, pos0)
         x = _layernorm(self.final_ln, x[:, -1:])
