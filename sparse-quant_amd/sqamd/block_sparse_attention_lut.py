@@ -4,9 +4,9 @@ Same entry point and argument meaning as
 sparse-attention/nvidia/playground/kernels/block_sparse_attention_lut.py:246-309
 (`sparse_attention(q, k, v, sm_scale, lut, LT, BLOCK_M, BLOCK_N, attention_mask,
 attention_dropout)`): prefill (q_len == kv_len) runs the HIP kernel behind
-sq_lut_attention_fwd; decode (q_len < kv_len, q_len == 1) is dense attention over
+sq_lut_attention_strided (through `quant.lut_attention`); decode (q_len < kv_len, q_len == 1) is dense attention over
 the whole KV cache, the same quantity the reference computes with two matmuls and a softmax,
-here in one kernel behind sq_decode_attention.
+here in one kernel behind sq_decode_attention (through `quant.decode_attention`).
 """
 import torch
 
