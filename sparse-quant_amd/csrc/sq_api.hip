@@ -113,8 +113,14 @@ const ChoiceRule kChoiceRules[] = {
     // 5..16 tokens where a K range of the streaming kernel would leave its chunk slots part empty, and at group size 32
     {5, 16, P_LARGE | P_G128_64 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
      "8 / 16 tokens: 15360x5120 13.9 vs 16.0 / 19.0 (streaming kernel), 13696x5120 13.4 vs 15.7 / 19.3"},
-    {5, 16, P_OVER_16M | P_RING, P_G128_64, SQ_ALGO_RING,
+    {9, 16, P_OVER_16M | P_RING, P_G128_64, SQ_ALGO_RING,
      "16 tokens, group size 32: 5120x5120 10.3 vs 19.2, 12288x4096 12.2 vs 15.4, 4096x11008 13.0 vs 15.4; 4096x4096 8.6 vs 8.4"},
+    // (5..8 tokens: what the GEMV below does not take.  The GEMV applies the scale to its sums in fp32)
+    {5, 8, P_LARGE | P_WS | P_RING, P_G128_64, SQ_ALGO_RING,
+     "8 tokens, group size 32: 12288x4096 11.7 vs 14.7 (split-K kernel) and 15.2 (GEMV), 4096x11008 12.6 vs 14.9 / 13.7, "
+     "4096x8192 10.8 vs 12.3 / 10.9, 4096x16384 14.9 vs 17.5 / 18.8"},
+    {5, 8, P_OVER_16M | P_RING, P_G128_64 | P_K_LE_8192, SQ_ALGO_RING,
+     "8 tokens, group size 32: 2048x11008 10.3 vs 12.2 (split-K kernel), 1536x16384 10.7 vs 12.1"},
     // the streaming decode kernel, 5..16 tokens (3..4 on large weights); K beyond 4096 is split through the workspace
     {5, 16, P_G128_64 | P_K128 | P_K_LE_4096, 0, SQ_ALGO_STREAM,
      "8 tokens: fc1 10.0 vs 13.3 (split-K kernel), q/k/v in one launch 8.6 vs 12.1, 4096x4096 4.9 vs 6.5 (GEMV)"},
@@ -171,6 +177,11 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
     return SQ_ALGO_GEMM;
 }
 
+// At group size 128 the decode kernels (up to 64 tokens) apply the scale to their sums in fp32, and so does the ring kernel
+// there: W_hat would round every weight to fp16 (error against (q - z) s as real numbers, 32 tokens x 4096 columns: 2.1e-4
+// with the scale on the sums, which is the rounding of the output, 2.9e-4 with W_hat).
+int ring_tune(int M, int g) { return g == 128 && M <= 64 ? sq::RING_SUMS : 0; }
+
 int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int group_size,
                   int layout, int algo, sq::Epilogue epi, void* workspace, size_t workspace_bytes, void* stream) {
     if (M < 0) return SQ_ERR_BAD_SHAPE;
@@ -199,6 +210,7 @@ int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, 
                            workspace_bytes >= sq::skinny2_workspace_bytes(M > 32 ? 32 : M, N, K) &&
                            (N + 63) / 64 <= 16384;
         kernel = builtin_choice(M, N, K, group_size, ws_ok);
+        if (kernel == SQ_ALGO_RING) tune = ring_tune(M, group_size);
     }
     switch (kernel) {
         case SQ_ALGO_GEMV:
@@ -224,7 +236,7 @@ int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, 
                                      workspace_bytes >= sq::skinny2_workspace_bytes(M, N, K);
                 if (!sq::skinny3_wide_applies(N, K, ws_fits) || !sq::gemm_ring_applies(M, N, K)) return SQ_ERR_WORKSPACE;
                 return launch_code(sq::launch_gemm_ring(x, w, zs, y, aligned16(workspace) ? workspace : nullptr,
-                                                        workspace_bytes, M, N, K, group_size, 0, epi, st));
+                                                        workspace_bytes, M, N, K, group_size, ring_tune(M, group_size), epi, st));
             }
             if (M > 16 || (group_size != 128 && group_size != 64)) return SQ_ERR_BAD_ALGO;
             const bool ws_fits = workspace && aligned16(workspace) &&
@@ -318,11 +330,12 @@ static int autotune_candidates(int M, int K, int g, bool has_ws, int* out, int c
         if (M > 64)
             for (int v = 8; v <= 10; v++) add(SQ_ALGO_GEMM, v);
     }
+    const int sums = ring_tune(M, g);  // (shapes that cannot put the scale on the sums are refused)
     if (M > 4)
         for (int shape = 1; shape <= 8; shape++)
             for (int rest = 0; rest <= (has_ws ? 1 : 0); rest++)
                 for (int ks = rest ? 2 : 1; ks <= (has_ws ? 8 : 1); ks += ks < 4 ? 1 : 2)
-                    add(SQ_ALGO_RING, shape | (rest ? 0x10 : 0) | (ks << 8));
+                    add(SQ_ALGO_RING, shape | (rest ? 0x10 : 0) | sums | (ks << 8));
     if (M > 128) add(SQ_ALGO_RING, 9 | (1 << 8));  // 256 x 256 tiles: never ahead when split
     return n;
 }

@@ -72,6 +72,18 @@ __device__ __forceinline__ half8_t dequant8(uint32_t w, half2_t z64, half2_t s, 
     return bit_cast<half8_t>(r);
 }
 
+// The same without the scale: the integers q - z, exact in fp16.
+__device__ __forceinline__ half8_t integers8(uint32_t w, half2_t z64, const NibbleMasks& nm) {
+    const half2_t z1024 = z64 + (half2_t){(half_t)960.f, (half_t)960.f};
+    const uint32_t t = w >> 8;
+    u32x4_t r;
+    r.x = bit_cast<uint32_t>(bit_cast<half2_t>((w & nm.lo) | 0x64006400u) - z1024);
+    r.y = bit_cast<uint32_t>(bit_cast<half2_t>((w & nm.hi) | 0x54005400u) - z64);
+    r.z = bit_cast<uint32_t>(bit_cast<half2_t>((t & nm.lo) | 0x64006400u) - z1024);
+    r.w = bit_cast<uint32_t>(bit_cast<half2_t>((t & nm.hi) | 0x54005400u) - z64);
+    return bit_cast<half8_t>(r);
+}
+
 // Word -> 8 fp16 holding 64 + q (no zero / scale applied).
 __device__ __forceinline__ half8_t unpack8_raw(uint32_t w, const NibbleMasks& nm) {
     uint32_t h[4];

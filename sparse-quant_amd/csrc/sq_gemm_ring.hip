@@ -146,7 +146,12 @@ __device__ __forceinline__ void load_to_lds_x1_masked(const void* base, uint32_t
                  : "memory");
 }
 
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST>
+// SUMS: the matrix instructions see the integers q - z and the scale meets the sums of a stage (64 k of one group) in
+// fp32, as in the decode kernels at group size 128; without it they see W_hat.  Sixteen vector instructions per 64 k and
+// column tile go and sixteen per row tile come: the same count with one row tile, more with two.  Measured (us, W_hat / sums):
+// 32 tokens 12288x4096 11.96 / 12.03, 5120x13696 16.3 / 16.4; 48 tokens 12288x4096 16.4 / 16.1, 5120x13696 20.6 / 21.1;
+// 64 tokens 4096x11008 16.6 / 16.6, 15360x5120 20.4 / 21.0.
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(
     const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS, const half_t* __restrict__ X, half_t* __restrict__ Y,
     int M, int N, int K, int mtiles, int tiles, int nfull, int ksplit, Epilogue epi, float* part, unsigned* counters) {
@@ -154,6 +159,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     constexpr int BM = S::BM, BN = S::BN, KS = S::KS, SB = S::SB, XI = S::XI, WI = S::WI, ZI = S::ZI, ZL = S::ZL, PER = S::PER, P = S::P;
     constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = S::XB + S::WB;
     constexpr int H = MI > 3 || MI * NI > 4 ? 2 : 4, PH = 4 / H;  // 16-wide k slices per phase, phases per stage
+    static_assert(!SUMS || (PH == 1 && GS == 7), "a phase lies in one group");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S::LDS];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
@@ -288,10 +294,38 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     half8_t a[H][MI], b[H][NI];
     half2_t zs[NI];
     uint32_t q[NI][H];
+    float16_t part_sum[SUMS ? MI : 1][SUMS ? NI : 1];  // of the stage before, and its scales
+    float part_scale[SUMS ? NI : 1];
+    if constexpr (SUMS) {
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            part_scale[ni] = 0.f;
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) part_sum[mi][ni][v] = 0.f;
+        }
+    }
+    // (pinned, so that the wait for the matrix instructions' results is not moved in front of the barrier)
+    auto fold = [&]() {
+        if constexpr (SUMS) {
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++) {
+                    asm volatile("" : "+v"(part_sum[mi][ni]));
+#pragma unroll
+                    for (int v = 0; v < 16; v++)
+                        acc[mi][ni][v] = __builtin_fmaf(part_sum[mi][ni][v], part_scale[ni], acc[mi][ni][v]);
+                }
+        }
+    };
     auto dequantise = [&](int t) {
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++)
-            b[t][ni] = dequant8(q[ni][t], (half2_t){zs[ni].x, zs[ni].x}, (half2_t){zs[ni].y, zs[ni].y}, nm);
+        for (int ni = 0; ni < NI; ni++) {
+            const half2_t z = {zs[ni].x, zs[ni].x};
+            b[t][ni] = SUMS ? integers8(q[ni][t], z, nm) : dequant8(q[ni][t], z, (half2_t){zs[ni].y, zs[ni].y}, nm);
+        }
     };
     // Phase h of stage it (slot c): the wave's operands into registers, weights dequantised.
     auto fetch = [&](int it, int c, auto h_) {
@@ -324,6 +358,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     };
     // the first half of the phase's weights, finished in front of the barrier that follows
     auto dequantise_first = [&]() {
+        fold();
 #pragma unroll
         for (int t = 0; t < H / 2; t++) {
             dequantise(t);
@@ -349,9 +384,18 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-                for (int ni = 0; ni < NI; ni++)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t][mi], b[t][ni], acc[mi][ni], 0, 0, 0);
-        constexpr int MF = H / 2 * MI * NI, VA = (14 * NI * (H / 2) + MF - 1) / MF;
+                for (int ni = 0; ni < NI; ni++) {
+                    if constexpr (SUMS)
+                        part_sum[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            a[t][mi], b[t][ni], t == 0 ? (float16_t){} : part_sum[mi][ni], 0, 0, 0);
+                    else
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t][mi], b[t][ni], acc[mi][ni], 0, 0, 0);
+                }
+        if constexpr (SUMS) {
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) part_scale[ni] = (float)zs[ni].y;
+        }
+        constexpr int MF = H / 2 * MI * NI, VA = ((SUMS ? 10 : 14) * NI * (H / 2) + MF - 1) / MF;
 #pragma unroll
         for (int i = 0; i < MF; i++) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
@@ -465,6 +509,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                 turn();
             }
         }
+        fold();
     }
 
     // The K groups' sums meet in LDS, one 32-row slice of every row group at a time, and leave row-major, EV consecutive
@@ -572,12 +617,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 }  // namespace
 
 // The shapes that are built: {MI, NI, WM, WN, WK, stages}, i.e. a (32 MI WM) x (32 NI WN) tile and 64 WK columns of K
-// per stage.  LDS holds three or four stages.
-#define SQ_RING_SHAPES(X_)                                                                                             \
-    X_(1, 1, 2, 1, 1, 8, 3) X_(2, 1, 2, 1, 2, 4, 4) X_(3, 2, 2, 1, 2, 4, 3) X_(4, 3, 1, 1, 4, 2, 4) X_(5, 2, 2, 1, 4, 2, 4) \
-        X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3) X_(8, 4, 2, 1, 4, 2, 3) X_(9, 4, 2, 2, 4, 1, 3)
+// per stage.  LDS holds three or four stages.  Tiles of 32 and 64 rows also with the scale on the sums.
+#define SQ_RING_LOW_SHAPES(X_) \
+    X_(1, 1, 2, 1, 1, 8, 3) X_(2, 1, 2, 1, 2, 4, 4) X_(3, 2, 2, 1, 2, 4, 3) X_(5, 2, 2, 1, 4, 2, 4)
+#define SQ_RING_SHAPES(X_)                                                                               \
+    SQ_RING_LOW_SHAPES(X_) X_(4, 3, 1, 1, 4, 2, 4) X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3)        \
+        X_(8, 4, 2, 1, 4, 2, 3) X_(9, 4, 2, 2, 4, 1, 3)
 
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST>
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
 static hipError_t launch_shape(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int nfull,
                                int ksplit, Epilogue epi, void* ws, hipStream_t st) {
     using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
@@ -585,7 +632,7 @@ static hipError_t launch_shape(const void* x, const void* w, const void* zs, voi
     const int tiles = mt * ((N + S::BN - 1) / S::BN);
     if (ksplit == 1) nfull = tiles;
     const int grid = ksplit == 1 ? (tiles + 7) / 8 * 8 : nfull + ((tiles - nfull) * ksplit + 7) / 8 * 8;
-    hipLaunchKernelGGL((gemm_ring_kernel<MI, NI, WM, WN, WK, GS, ST>), dim3(grid), dim3(S::NT), 0, st, (const uint8_t*)w,
+    hipLaunchKernelGGL((gemm_ring_kernel<MI, NI, WM, WN, WK, GS, ST, SUMS>), dim3(grid), dim3(S::NT), 0, st, (const uint8_t*)w,
                        (const half2_t*)zs, (const half_t*)x, (half_t*)y, M, N, K, mt, tiles, nfull, ksplit, epi,
                        ws ? (float*)((char*)ws + RING_COUNTER_BYTES) : nullptr, (unsigned*)ws);
     return hipGetLastError();
@@ -638,7 +685,8 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes) {
     for (int s = 0; s < RING_SHAPES; s++) {
         const RingTile& t = kRingTiles[s];
         const int mt = (M + t.bm - 1) / t.bm;
-        if (t.bm > 64 && mt * t.bm * 2 > rows32 * 3) continue;  // a third of the matrix work would be padding
+        // a third of the matrix work would be padding; up to 64 rows the others are the ones with the scale on the sums
+        if (t.bm > 64 && (M <= 64 || mt * t.bm * 2 > rows32 * 3)) continue;
         const long tiles = (long)mt * ((N + t.bn - 1) / t.bn);
         const int stages = (K + t.ks - 1) / t.ks;
         const int full = (int)(tiles >> 8), rest = (int)(tiles & 255);
@@ -674,7 +722,8 @@ size_t gemm_ring_workspace_bytes(int M, int N, int K) {
 }
 
 // tune = 0 for the cost model's choice, else shape id | 0x10: only the tiles of the last, part-filled round of 256
-// workgroups split K | K split << 8.  hipErrorInvalidValue: not applicable (or the workspace is missing or too small).
+// workgroups split K | K split << 8; RING_SUMS: the scale on the sums (also with the model's choice; group size 128, tiles
+// of 32 and 64 rows).  hipErrorInvalidValue: not applicable (or the workspace is missing or too small).
 hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,
                             int K, int g, int tune, Epilogue epi, hipStream_t st) {
     if (!gemm_ring_applies(M, N, K)) return hipErrorInvalidValue;
@@ -695,16 +744,29 @@ hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* 
                 return hipErrorInvalidValue;
         }
     }
+#define SQ_RING_LAUNCH(MI, NI, WM, WN, WK, GS, ST, SUMS) \
+    launch_shape<MI, NI, WM, WN, WK, GS, ST, SUMS>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st)
+    if (tune & RING_SUMS) {
+        if (g != 128) return hipErrorInvalidValue;
+        switch (p.shape) {
+#define X_(id, MI, NI, WM, WN, WK, ST) \
+    case id:                           \
+        return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 7, ST, true);
+            SQ_RING_LOW_SHAPES(X_)
+#undef X_
+        }
+        return hipErrorInvalidValue;
+    }
     switch (p.shape) {
-#define X_(id, MI, NI, WM, WN, WK, ST)                                                                                    \
-    case id:                                                                                                              \
-        if (g == 128)                                                                                                     \
-            return launch_shape<MI, NI, WM, WN, WK, 7, ST>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st);         \
-        if (g == 64) return launch_shape<MI, NI, WM, WN, WK, 6, ST>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st); \
-        return launch_shape<MI, NI, WM, WN, WK, 5, ST>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st);
+#define X_(id, MI, NI, WM, WN, WK, ST)                                              \
+    case id:                                                                        \
+        if (g == 128) return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 7, ST, false);      \
+        if (g == 64) return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 6, ST, false);       \
+        return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 5, ST, false);
         SQ_RING_SHAPES(X_)
 #undef X_
     }
+#undef SQ_RING_LAUNCH
     return hipErrorInvalidValue;
 }
 

@@ -91,7 +91,9 @@ hipError_t launch_gemm_tuned(const void* x, const void* w, const void* zs, void*
                              int N, int K, int g, int tune, Epilogue epi, hipStream_t st);
 
 // sq_gemm_ring.hip: any M, the choice from 17 tokens up.  tune = 0: the cost model's plan within ws_bytes (ws may be
-// null: K is not split over workgroups).
+// null: K is not split over workgroups).  RING_SUMS in tune: the scale on the sums in fp32 instead of W_hat (group size
+// 128, up to 64-row tiles).
+constexpr int RING_SUMS = 0x20;
 bool gemm_ring_applies(int M, int N, int K);
 size_t gemm_ring_workspace_bytes(int M, int N, int K);
 hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,

@@ -1,4 +1,5 @@
-"""The ring kernel (17 tokens up): every tile shape, K split and group size on ragged M, N and K against the oracle."""
+"""The ring kernel (17 tokens up): every tile shape, K split and group size on ragged M, N and K against the oracle; with
+the scale on the sums, as few tokens take it, against (q - z) s in float64."""
 import numpy as np
 import pytest
 import torch
@@ -66,3 +67,61 @@ def test_ring_parity(capi, shape, m, n, k, g):
 def test_ring_parity_of_256_row_tiles(capi, m, n, k, g):
     """Two rows of waves over the same weight columns: the second row of tiles full, ragged and absent."""
     test_ring_parity(capi, 9, m, n, k, g)
+
+
+SUMS = 0x20  # tune word: the scale on the sums (shapes of 32 and 64 rows, group size 128)
+
+
+def real_weight(d, g):
+    """(q - z) s without a rounding."""
+    return (d["q"].astype(np.float64) - np.repeat(d["z"], g, 1)) * np.repeat(d["s"].astype(np.float64), g, 1)
+
+
+@pytest.mark.parametrize("m,n,k,g", [(1, 64, 128, 128), (33, 136, 640, 128), (64, 264, 1408, 128), (16, 72, 6144, 128),
+                                     (31, 5128, 384, 128)])
+@pytest.mark.parametrize("shape", [1, 2, 3, 5])
+def test_ring_parity_with_the_scale_on_the_sums(capi, shape, m, n, k, g):
+    d = orc.synth_linear(n, k, g, seed=7 * n + k)
+    w64, x = real_weight(d, g), orc.synth_x(m, k, seed=m)
+    x64 = x.astype(np.float64)
+    ref = x64 @ w64.T
+    # one rounding to fp16 and K fp32 additions of the products' magnitudes
+    bound = 2.0 ** -11 * np.abs(ref) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T) + 2.0 ** -24
+    w, zs, xd = to_dev(d["w_l1"]), to_dev(d["zs_l1"]), to_dev(x)
+    ws = torch.zeros(65536 + (96 << 20), dtype=torch.uint8, device=DEV)
+    ks_max = -(-k // {1: 512, 2: 256, 3: 256, 5: 128}[shape])
+    for ks in (1, 2, 3, 8):
+        if ks > ks_max:
+            continue
+        y = torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV)
+        algo = capi.SQ_ALGO_RING | ((shape | SUMS | (ks << 8)) << 8)
+        capi.gemm_ws(xd, w, zs, n, k, g, out=y, algo=algo, ws=ws)
+        got = y.cpu().numpy().astype(np.float64)
+        assert np.all(np.abs(got - ref) <= bound), (ks, np.max(np.abs(got - ref) / bound))
+        assert torch.equal(y, capi.gemm_ws(xd, w, zs, n, k, g, algo=algo, ws=ws))
+        assert capi.workspace_is_clean(ws)
+
+
+def test_ring_has_the_scale_on_the_sums_where_it_says(capi):
+    d = orc.synth_linear(64, 128, 32, seed=1)
+    x, w, zs = to_dev(orc.synth_x(8, 128)), to_dev(d["w_l1"]), to_dev(d["zs_l1"])
+    with pytest.raises(capi.SqError):  # another group size
+        capi.gemm(x, w, zs, 64, 128, 32, algo=capi.SQ_ALGO_RING | ((1 | SUMS) << 8))
+    with pytest.raises(capi.SqError):  # a shape of 96 rows
+        capi.gemm(x, w, zs[:, :2].contiguous(), 64, 128, 128, algo=capi.SQ_ALGO_RING | ((4 | SUMS) << 8))
+
+
+@pytest.mark.parametrize("use_ws", [True, False])
+@pytest.mark.parametrize("m,n,k,g", [(5, 5120, 5120, 32), (8, 5120, 5120, 32), (8, 6656, 5120, 128), (16, 6656, 5120, 128),
+                                     (17, 4096, 4096, 128), (32, 4096, 4096, 128), (32, 1000, 11008, 128),
+                                     (40, 2048, 1408, 128), (48, 2560, 13696, 128), (64, 2048, 1536, 128)])
+def test_few_tokens_round_no_weight_to_half(capi, m, n, k, g, use_ws):
+    """Where decode kernels keep the scale in fp32 the automatic choice does so whichever kernel it names: the result is
+    as far from (q - z) s in float64 as its one rounding to fp16 puts it (W_hat is 1.4 times as far, and fp32 sums add
+    a part in 2^24 of sums no more than some hundred times the result)."""
+    d = orc.synth_linear(n, k, g, seed=k)
+    x = orc.synth_x(m, k, seed=m)
+    ref = torch.from_numpy(x).to(DEV).double() @ torch.from_numpy(real_weight(d, g)).to(DEV).t()
+    y = capi.gemm_fused(to_dev(x), to_dev(d["w_l1"]), to_dev(d["zs_l1"]), n, k, g, use_workspace=use_ws)
+    rounding = (ref.half().double() - ref).norm()
+    assert (y.double() - ref).norm() <= 1.1 * rounding
