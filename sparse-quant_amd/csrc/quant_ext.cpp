@@ -18,6 +18,7 @@
 
 #include <map>
 #include <mutex>
+#include <sstream>
 #include <stdexcept>
 #include <string>
 #include <unordered_map>
@@ -403,7 +404,13 @@ c10::optional<at::Tensor> lut_attention(const at::Tensor& q, const at::Tensor& k
     if (lut.scalar_type() != at::kInt && lut.scalar_type() != at::kLong) return c10::nullopt;
     const int64_t Z = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
     const int64_t nnz = lut.size(-1);
-    if (S >= (1LL << 31) || nnz >= (1LL << 31) || Z * H > 65535) return c10::nullopt;
+    if (S >= (1LL << 31) || nnz >= (1LL << 31) || Z * H > 65535 || (D != 64 && D != 128)) return c10::nullopt;
+    const int64_t nblk = (S + 63) / 64;
+    if (lut.numel() < H * nblk * nnz || (lut.dim() >= 3 && lut.size(-2) != nblk)) {  // the kernel's row pitch, and its last row
+        std::ostringstream msg;
+        msg << "a look-up table of shape " << lut.sizes() << " for " << H << " heads of " << nblk << " query blocks";
+        throw std::invalid_argument(msg.str());
+    }
     at::NoGradGuard no_grad;
     c10::DeviceGuard guard(q.device());
     at::Tensor out = at::empty({Z, H, S, D}, q.options());

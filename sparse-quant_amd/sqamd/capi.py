@@ -411,9 +411,20 @@ def l2_convert_2bit_to_4bit(w2, stream=None):
     return out
 
 
+def _check_table(lut, heads, s):
+    """The kernel reads entry ((head * ceil(s / 64)) + block) * nnz + j: a table made for another prompt length has its
+    rows elsewhere, one with fewer rows ends before the last of them."""
+    nblk = (s + 63) // 64
+    if lut.numel() < heads * nblk * lut.shape[-1] or (lut.dim() >= 3 and lut.shape[-2] != nblk):
+        raise ValueError("a look-up table of shape %s for %d heads of %d query blocks (%d rows of q)"
+                         % (tuple(lut.shape), heads, nblk, s))
+
+
 def lut_attention(q, k, v, lut, sm_scale, causal, stream=None):
     """q, k, v fp16 [Z,H,S,D] contiguous; lut int32/int64 [H, ceil(S/64), nnz] -> out fp16 [Z,H,S,D]."""
     z, h, s, d = q.shape
+    if d in (64, 128):  # (another head dimension is refused below)
+        _check_table(lut, h, s)
     out = torch.empty_like(q)
     _check(lib().sq_lut_attention_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lut), lut.element_size(), z, h, s, d,
                                       lut.shape[-1], float(sm_scale), int(bool(causal)), _stream(stream)),
@@ -445,6 +456,10 @@ def lut_attention_strided(q, k, v, lut, sm_scale, causal, k_cache=None, v_cache=
     z, h, s, d = q.shape
     if not lut_attention_strided_ok(q, k, v, k_cache, v_cache):
         raise ValueError("lut_attention_strided: unsupported dtype, shape or strides")
+    if lut is not None:
+        if lut.dtype not in (torch.int32, torch.int64) or not lut.is_contiguous() or lut.device != q.device:
+            raise ValueError("lut_attention_strided: the table must be int32 or int64, contiguous and on the device of q")
+        _check_table(lut, h, s)
     if rows_first:
         out = torch.empty((z, s, h, d), dtype=q.dtype, device=q.device)
         o_st = (s * h * d, d, h * d)

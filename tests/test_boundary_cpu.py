@@ -186,3 +186,12 @@ def test_host_packers_match_oracle():
     q2i = q2.reshape(32, 32, 4, 2).transpose(0, 1, 3, 2).reshape(32, 256)
     assert np.array_equal(qw2.numpy(), orc.pack_2bit_l1(q2i))
     assert np.array_equal(orc.convert_2bit_to_4bit_l1(qw2.numpy()), orc.pack_l1(q2))
+
+
+@pytest.mark.parametrize("shape", [(2, 1, 2), (1, 2, 2), (2, 4, 2), (3, 2)])
+def test_attention_table_is_checked_before_any_launch(built_lib, shape):
+    """Two heads of two query blocks: a table for another prompt length or for fewer heads is a ValueError."""
+    from sqamd import capi
+    q = torch.zeros((1, 2, 65, 64), dtype=torch.float16)
+    with pytest.raises(ValueError, match="look-up table"):
+        capi.lut_attention(q, q, q, torch.zeros(shape, dtype=torch.int64), 0.125, True)

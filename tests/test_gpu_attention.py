@@ -270,3 +270,38 @@ def test_strided_attention_beyond_512_workgroups(capi, d):
     assert torch.equal(out.transpose(1, 2), ref)
     assert torch.equal(kc[:, :, :s], k) and torch.equal(vc[:, :, :s], v)
     assert bool((kc[:, :, s:] == 7).all()) and bool((vc[:, :, s:] == 7).all())
+
+
+def test_tables_of_another_prompt_are_refused(capi):
+    """The kernel addresses the table by the heads and the length of q: a table for fewer blocks or heads would be read
+    past its end, one for more blocks at the wrong rows.  Rows beyond the heads of q, and a table flattened to rows, are
+    what the addressing makes of them."""
+    import quant
+    from sqamd.block_sparse_attention_lut import sparse_attention
+    q = torch.randn((1, 2, 65, 64), device="cuda").half()
+    lut = torch.tensor([[[0, 0], [0, 1]]] * 2, device="cuda")
+    ref = sparse_attention(q, q, q, 0.125, lut)
+    for good in (torch.cat([lut, lut]), lut.view(4, 2), lut[None].contiguous()):
+        assert torch.equal(sparse_attention(q, q, q, 0.125, good), ref)
+        assert torch.equal(capi.lut_attention(q, q, q, good, 0.125, True), ref)
+        assert torch.equal(capi.lut_attention_strided(q, q, q, good, 0.125, True), ref)
+    for bad in (lut[:, :1].contiguous(), lut[:1].contiguous(), torch.cat([lut, lut], 1), lut.view(4, 2)[:3].contiguous()):
+        for call in (lambda: quant.lut_attention(q, q, q, bad, 0.125, True), lambda: sparse_attention(q, q, q, 0.125, bad),
+                     lambda: sparse_attention(q, q, q, 0.125, bad.cpu()), lambda: capi.lut_attention(q, q, q, bad, 0.125, True),
+                     lambda: capi.lut_attention_strided(q, q, q, bad, 0.125, True)):
+            with pytest.raises(ValueError):
+                call()
+    for bad in (lut.float(), lut.cpu(), torch.cat([lut, lut], 2)[..., ::2]):
+        with pytest.raises(ValueError):
+            capi.lut_attention_strided(q, q, q, bad, 0.125, True)
+
+
+def test_a_prompt_longer_than_its_table_is_refused(capi):
+    from sqamd.opt_decode import OPTDecoder
+    model = OPTDecoder(layers=1, hidden=512, heads=4, ffn=512, vocab=64, max_pos=256, dev="cuda")
+    model.set_prefill_lut(64, 0.5)
+    cache = model.new_cache(1, 130)
+    ids = torch.zeros((1, 65), dtype=torch.long, device="cuda")
+    assert torch.isfinite(model(ids[:, :64], cache, 0)).all()
+    with pytest.raises(ValueError):
+        model(ids, cache, 0)
