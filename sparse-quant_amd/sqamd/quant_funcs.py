@@ -76,6 +76,8 @@ def _one_launch(weight, n_bit, group_size, layout):
     """Whether the packing kernel takes this weight: a plain fp16 [N, K] device tensor, dense and 16-byte aligned, with a
     group size the kernel is built for, and nothing that has to see the torch operations (autograd, function transforms,
     tracing).  Everything else is packed by the torch operations below, which also raise what a bad call raises."""
+    if torch.jit.is_tracing():  # (the kernel's outputs would be constants of the trace)
+        return False
     if type(weight) not in (torch.Tensor, torch.nn.Parameter) or weight.dtype != torch.float16 or weight.dim() != 2:
         return False
     if not weight.is_cuda or weight.numel() == 0 or not weight.is_contiguous():

@@ -73,3 +73,13 @@ def test_from_float_and_the_weights_the_kernel_leaves_alone(built_lib):
     for other in (shifted, w.float(), w.bfloat16(), w.clone().requires_grad_(), w.cpu()):
         assert not qf._one_launch(other, 4, 128, capi.SQ_LAYOUT_L1)
     assert not qf._one_launch(w, 4, 16, capi.SQ_LAYOUT_L1) and not qf._one_launch(w[:8], 4, 128, capi.SQ_LAYOUT_L2)
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+def test_a_trace_of_the_packer_follows_its_input(built_lib):
+    pack = lambda w: qf.quant_muxi(w, 256, 64, group_size=128)
+    traced = torch.jit.trace(pack, (weight(64, 256, 0),), check_trace=False)
+    other = (torch.randn((64, 256), device=DEV) * 0.02).half()
+    assert qf._one_launch(other, 4, 128, capi.SQ_LAYOUT_L1)
+    for a, b in zip(traced(other), pack(other)):
+        assert torch.equal(a, b)
