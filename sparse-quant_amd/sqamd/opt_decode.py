@@ -179,7 +179,7 @@ class OPTDecoder(nn.Module):
         w = self.lm_head
         if b <= 8 and self.hidden % 512 == 0 and self.hidden <= 8192 and w.dtype == torch.float16 and w.is_contiguous() \
                 and w.data_ptr() % 16 == 0:  # what sq_f16_gemv takes
-            return capi.f16_gemv(x, w).view(b, 1, -1)
+            return capi.f16_gemv(x, w).view(*x.shape[:-1], w.shape[0])  # (a prompt of no tokens has no row either)
         return torch.matmul(x, self.lm_head.t())  # [B, 1, vocab]
 
     @torch.no_grad()

@@ -114,3 +114,12 @@ def test_lut_attention_routes_agree(mods):
     with pytest.raises(capi.SqError) as e:
         bsa.sparse_attention(x, x, x, 0.125, lut)
     assert e.value.code == capi.SQ_ERR_BAD_SHAPE
+
+
+@pytest.mark.parametrize("b,t,rows", [(2, 0, 0), (2, 1, 1), (3, 5, 1), (9, 2, 1)])
+def test_logits_have_a_row_per_last_token(built_lib, b, t, rows):
+    """With the logits' own kernel (up to 8 sequences) as with the library's product (9)."""
+    from sqamd.opt_decode import OPTDecoder
+    model = OPTDecoder(layers=1, hidden=512, heads=4, ffn=512, vocab=64, max_pos=64, dev=DEV)
+    logits = model(torch.zeros((b, t), dtype=torch.long, device=DEV), model.new_cache(b, 8), 0)
+    assert logits.shape == (b, rows, 64)
