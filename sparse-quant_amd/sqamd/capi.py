@@ -441,7 +441,8 @@ def _rows_readable(*tensors):
 def lut_attention_strided_ok(q, k, v, k_cache=None, v_cache=None):
     """Whether lut_attention_strided takes these tensors."""
     caches = () if k_cache is None else (k_cache, v_cache)
-    return (all(t.dtype == torch.float16 and t.is_cuda for t in (q, k, v) + caches) and q.shape[3] in (64, 128)
+    return (all(t.dtype == torch.float16 and t.is_cuda and t.device == q.device for t in (q, k, v) + caches)
+            and q.shape[3] in (64, 128)
             and q.shape == k.shape == v.shape and k.stride() == v.stride() and k.stride(2) < 1 << 24
             and _rows_readable(q, k, v, *caches)
             and (k_cache is None or (k_cache.stride() == v_cache.stride() and k_cache.shape == v_cache.shape
@@ -468,10 +469,11 @@ def lut_attention_strided(q, k, v, lut, sm_scale, causal, k_cache=None, v_cache=
         o_st = (h * s * d, s * d, d)
     c_st = (0, 0, 0) if k_cache is None else k_cache.stride()[:3]
     strides = (ctypes.c_long * 12)(*q.stride()[:3], *k.stride()[:3], *o_st, *c_st)
-    _check(lib().sq_lut_attention_strided(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(k_cache), _ptr(v_cache), _ptr(lut),
-                                          0 if lut is None else lut.element_size(), z, h, s, d,
-                                          0 if lut is None else lut.shape[-1], strides, float(sm_scale),
-                                          int(bool(causal)), _stream(stream)), "sq_lut_attention_strided")
+    with torch.cuda.device(q.device):  # as the torch operations it stands for, whatever device is current
+        _check(lib().sq_lut_attention_strided(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(k_cache), _ptr(v_cache), _ptr(lut),
+                                              0 if lut is None else lut.element_size(), z, h, s, d,
+                                              0 if lut is None else lut.shape[-1], strides, float(sm_scale),
+                                              int(bool(causal)), _stream(stream)), "sq_lut_attention_strided")
     return out
 
 

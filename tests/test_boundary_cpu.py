@@ -195,3 +195,40 @@ def test_attention_table_is_checked_before_any_launch(built_lib, shape):
     q = torch.zeros((1, 2, 65, 64), dtype=torch.float16)
     with pytest.raises(ValueError, match="look-up table"):
         capi.lut_attention(q, q, q, torch.zeros(shape, dtype=torch.int64), 0.125, True)
+
+
+def test_attention_that_fills_a_cache_stays_on_one_device(built_lib, monkeypatch):
+    """Tensors of two devices are left to the torch operations, and the kernel runs on the device of q whichever is
+    current (tensors that only claim to be on a device: nothing is launched)."""
+    import contextlib
+    from types import SimpleNamespace
+
+    from sqamd import capi
+
+    def on(index):
+        t = torch.zeros((1, 2, 65, 64), dtype=torch.float16)
+        return SimpleNamespace(dtype=t.dtype, is_cuda=True, device=torch.device("cuda", index), shape=t.shape,
+                               stride=lambda *a: t.stride(*a), data_ptr=lambda: 4096)
+
+    q, far = on(1), on(0)
+    assert capi.lut_attention_strided_ok(q, q, q, q, q)
+    for at in range(5):
+        args = [q] * 5
+        args[at] = far
+        assert not capi.lut_attention_strided_ok(*args)
+
+    current, launched = [0], []
+
+    @contextlib.contextmanager
+    def device(dev):
+        before, current[0] = current[0], torch.device(dev).index
+        yield
+        current[0] = before
+
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: q)
+    monkeypatch.setattr(capi, "_stream", lambda stream=None: None)
+    monkeypatch.setattr(capi, "lib", lambda: SimpleNamespace(
+        sq_lut_attention_strided=lambda *a: launched.append(current[0]) or capi.SQ_OK))
+    capi.lut_attention_strided(q, q, q, None, 0.125, True, q, q)
+    assert launched == [1] and current == [0]
