@@ -348,11 +348,10 @@ int sq_w4a16_autotune(const void* x, const void* w, const void* zs, void* y, int
     if (copies > 1 && (w_stride % 16 != 0 || zs_stride % 16 != 0 || w_stride < (size_t)N * K / 2)) return SQ_ERR_MISALIGNED;
     const sq::Epilogue none{nullptr, nullptr, 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // A recorded word has to fit every workspace that counts as full later on: no candidate sees more than that.
     const bool has_ws = full_workspace(workspace, workspace_bytes, M, N, K);
-    if (!has_ws) {
-        workspace = nullptr;
-        workspace_bytes = 0;
-    }
+    if (!has_ws) workspace = nullptr;
+    workspace_bytes = has_ws ? sq_w4a16_workspace_bytes(M, N, K) : 0;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
         if (e0) (void)hipEventDestroy(e0);

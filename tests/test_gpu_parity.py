@@ -886,6 +886,25 @@ def test_measured_kernel_choice_is_recorded_and_used(capi):
     assert capi.autotune_clear() == 0
 
 
+@pytest.mark.parametrize("m,n,k,g", [(8, 1024, 8192, 128), (16, 512, 4096, 32), (40, 256, 4096, 128), (300, 264, 2048, 64)])
+def test_picker_stays_within_the_workspace_a_later_call_may_have(capi, m, n, k, g):
+    """A recorded choice is used with any workspace of sq_w4a16_workspace_bytes or more: whatever the picker is handed, its
+    candidates touch no more than that, and a call with just that runs."""
+    need = capi.lib().sq_w4a16_workspace_bytes(m, n, k)
+    d = orc.synth_linear(n, k, g, seed=k)
+    x, w, zs = to_dev(orc.synth_x(m, k, seed=m)), to_dev(d["w_l1"]), to_dev(d["zs_l1"])
+    ws = torch.zeros(need + (96 << 20), dtype=torch.uint8, device=DEV)
+    ws[need:] = 0x5A
+    capi.autotune_clear()
+    y = torch.empty((m, n), dtype=torch.float16, device=DEV)
+    capi.autotune(x, w, zs, n, k, g, ws=ws, reps=2, out=y)
+    torch.cuda.synchronize()
+    touched = int((ws[need:] != 0x5A).sum())
+    assert touched == 0
+    assert torch.equal(y, capi.gemm_ws(x, w, zs, n, k, g, ws=torch.zeros(need, dtype=torch.uint8, device=DEV)))
+    capi.autotune_clear()
+
+
 # ------------------------------------------------------------------ seeded random shapes through the built-in choice
 @pytest.mark.parametrize("seed", [11, 12, 13])
 def test_random_shapes_fused_auto_dispatch(capi, seed):
