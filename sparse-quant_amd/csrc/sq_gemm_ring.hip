@@ -229,7 +229,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         zlane[j] = (uint32_t)((long)imin(n0 + d / P, N - 1) * groups * 4) + (d % P) * 4;
     }
     // All loads of stage it into slot c.  EDGE: the last stage of a K that ends inside it; what is missing re-reads the
-    // end of the row (and meets a scale of 0).
+    // end of the row (see clip).
     auto issue = [&](int it, int c, auto EDGE_) {
         constexpr bool EDGE = decltype(EDGE_)::value;
         const int k0 = it * KS, left = K - k0;
@@ -349,11 +349,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int mi = 0; mi < MI; mi++) a[t][mi] = *(const half8_t*)(l + xoff[h * H + t] + mi * 4096);
     };
-    // Weights past the end of K get the scale 0 (only the last stage can hold any).
+    // Past the end of K (only the last stage can hold any of it) weights get the scale 0 and activations become 0: what was
+    // read there is the end of the row, and an infinity times 0 would be a NaN in every column.
     auto clip = [&](int it) {
         if (it * KS + 64 * kg + (GS == 5 ? 32 * lc : 0) >= K) {
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) zs[ni].y = (half_t)0.f;
+#pragma unroll
+            for (int t = 0; t < H; t++)
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++) a[t][mi] = (half8_t){};
         }
     };
     // the first half of the phase's weights, finished in front of the barrier that follows

@@ -125,3 +125,25 @@ def test_few_tokens_round_no_weight_to_half(capi, m, n, k, g, use_ws):
     y = capi.gemm_fused(to_dev(x), to_dev(d["w_l1"]), to_dev(d["zs_l1"]), n, k, g, use_workspace=use_ws)
     rounding = (ref.half().double() - ref).norm()
     assert (y.double() - ref).norm() <= 1.1 * rounding
+
+
+@pytest.mark.parametrize("m,n,k,g", [(1, 72, 640, 128), (33, 136, 1408, 128), (70, 72, 416, 32), (20, 72, 960, 64)])
+@pytest.mark.parametrize("shape", range(10))
+def test_ring_keeps_an_infinite_activation_to_its_row(capi, shape, m, n, k, g):
+    """An infinity in the last column of one row, K ending inside a stage: infinities of the weights' signs in that row,
+    the other rows as without it (a shape of 0: the automatic choice of shape)."""
+    d = orc.synth_linear(n, k, g, seed=k)
+    d["q"][:, -1] = np.where(d["z"][:, -1] == 0, 15, 0)  # no weight of 0 in that column
+    w, zs = to_dev(orc.pack_l1(d["q"])), to_dev(d["zs_l1"])
+    x = orc.synth_x(m, k, seed=m)
+    ws = torch.zeros(65536 + (96 << 20), dtype=torch.uint8, device=DEV)
+    words = [shape] + ([shape | SUMS] if g == 128 and m <= 64 and shape in (0, 1, 2, 3, 5) else [])
+    for tune in words:
+        run = lambda: capi.gemm_ws(to_dev(x), w, zs, n, k, g, algo=capi.SQ_ALGO_RING | (tune << 8), ws=ws).cpu().numpy()
+        x[m // 2, -1] = 0.5
+        plain = run()
+        x[m // 2, -1] = np.inf
+        got = run()
+        assert np.array_equal(got[m // 2], np.where(d["q"][:, -1] > 0, np.inf, -np.inf).astype(np.float16)), hex(tune)
+        got[m // 2] = plain[m // 2]
+        assert np.array_equal(got, plain), hex(tune)
