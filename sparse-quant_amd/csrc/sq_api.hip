@@ -513,16 +513,22 @@ static size_t sequence_splitk_bytes(const sq_linear_desc* linears, int count, in
     if (!linears || count <= 0 || count > SQ_SEQUENCE_MAX || M <= 2) return base;
     // more than 2 tokens: what sq_w4a16_gemm_ws wants for the largest run of linears that may share a launch
     // (their rows concatenated, each rounded up to a 64-row block) and for every single linear
+    // (the ring kernel splits K of a narrow weight further than that of a wide one: one linear can want more than the run)
     long rows = 0;
     int kmax = 0;
+    size_t need = base;
     for (int l = 0; l < count; l++) {
         if (linears[l].N <= 0 || linears[l].K <= 0) return base;
         rows += ((long)linears[l].N + 63) / 64 * 64;
         if (linears[l].K > kmax) kmax = linears[l].K;
     }
     if (rows > (1L << 30)) return base;
-    const size_t a = (sq_w4a16_workspace_bytes(M, (int)rows, kmax) + 255) & ~(size_t)255;
-    return a > base ? a : base;
+    for (int l = -1; l < count; l++) {
+        const size_t a = l < 0 ? sq_w4a16_workspace_bytes(M, (int)rows, kmax)
+                               : sq_w4a16_workspace_bytes(M, linears[l].N, linears[l].K);
+        if (a > need) need = a;
+    }
+    return (need + 255) & ~(size_t)255;
 }
 
 size_t sq_w4a16_gemv_sequence_workspace_bytes(const sq_linear_desc* linears, int count, int M) {
@@ -652,8 +658,14 @@ int sq_w4a16_gemv_sequence(const sq_linear_desc* linears, int count, int M, int 
                 const sq::SeqProblem& q = probs[l];
                 const sq::Epilogue epi{static_cast<const sq::half_t*>(q.bias), static_cast<const sq::half_t*>(q.residual),
                                        q.act};
+                // no more than it needs: behind that may lie the one-launch mode's region (see sequence_splitk_bytes)
+                size_t bytes = 0;
+                if (M > 2 && workspace) {
+                    bytes = sq_w4a16_workspace_bytes(M, q.N, q.K);
+                    if (workspace_bytes < bytes) bytes = workspace_bytes;
+                }
                 const int rc = gemm_dispatch(q.x, q.w, q.zs, q.y, M, q.N, q.K, q.group_size, layout, SQ_ALGO_AUTO, epi,
-                                             M > 2 ? workspace : nullptr, M > 2 ? workspace_bytes : 0, stream);
+                                             bytes ? workspace : nullptr, bytes, stream);
                 if (rc != SQ_OK) return rc;
             }
         }

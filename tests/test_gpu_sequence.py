@@ -391,3 +391,21 @@ def test_sequence_rejections(capi):
     descs[0].act = 7
     assert call(2, 1) == capi.SQ_ERR_BAD_ALGO
     assert L.sq_w4a16_gemv_sequence(None, 2, 1, 1, 0, ws, 256, None) == capi.SQ_ERR_NULL_POINTER
+
+
+def test_k_split_of_a_lone_linear_leaves_the_one_launch_region_alone(capi):
+    """8 tokens: the first linear alone would split its K further than the workspace of the list is laid out for.  With
+    more bytes behind that it must not run into the words that sq_w4a16_gemv_sequence_status reads."""
+    m, lin, refs = 8, [], []
+    for i, (n, k, g) in enumerate([(2048, 16384, 32), (64, 256, 128)]):
+        d, x = make_linear(n, k, g, seed=400 + i), orc.synth_x(m, k, seed=410 + i)
+        refs.append(oracle_linear(x, d))
+        lin.append(dict(x=to_dev(x), w=d["w_dev"], zs=d["zs_dev"], n=n, k=k, group_size=g,
+                        y=torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV)))
+    seq = capi.LinearSequence(lin, m, DEV)
+    seq.ws = torch.zeros(seq.ws.numel() + (4 << 20), dtype=torch.uint8, device=DEV)
+    seq.run()
+    torch.cuda.synchronize()
+    for l, ref in zip(lin, refs):
+        assert rel_err(l["y"].float().cpu().numpy(), ref) <= TOL
+    assert seq.error_flag() == 0 and capi.workspace_is_clean(seq.ws)
