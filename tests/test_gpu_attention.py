@@ -305,3 +305,39 @@ def test_a_prompt_longer_than_its_table_is_refused(capi):
     assert torch.isfinite(model(ids[:, :64], cache, 0)).all()
     with pytest.raises(ValueError):
         model(ids, cache, 0)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("z,h,s", [(1, 2, 161), (3, 171, 97)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(capi, bad, z, h, s, d):
+    """Causal, every block visited, in both forms (up to 512 workgroups and beyond).  A query that is not finite spoils its
+    own row; a key the rows behind it and its own, and nothing in front of it; a value, whose product with a masked
+    probability of 0 is a NaN, the rows from the start of its block of 64 on."""
+    gen = torch.Generator(device="cuda").manual_seed(s + d)
+    q, k, v = (torch.randn((z, h, s, d), device="cuda", generator=gen).half() for _ in range(3))
+    nb = (s + 63) // 64
+    rows = torch.arange(nb, device="cuda")
+    lut = torch.minimum(rows.expand(h, nb, nb), rows.view(1, nb, 1)).contiguous()
+    plain = capi.lut_attention(q, k, v, lut, d ** -0.5, True)
+    zi, hi, j = z - 1, h - 1, 75
+
+    def spoilt(which):
+        t = [q.clone(), k.clone(), v.clone()]
+        t[which][zi, hi, j, 3] = bad
+        out = capi.lut_attention(*t, lut, d ** -0.5, True)
+        touched = (out != plain).any(-1)
+        mine = touched[zi, hi].clone()
+        touched[zi, hi] = False
+        assert not bool(touched.any())  # other heads
+        return out[zi, hi], mine
+
+    out, mine = spoilt(0)
+    assert mine.nonzero().flatten().tolist() == [j] and not bool(out[j].isfinite().all())
+    out, mine = spoilt(1)
+    assert not bool(mine[:j].any())
+    if bad != bad:
+        assert bool(out[j:].isnan().all())
+    out, mine = spoilt(2)
+    assert not bool(mine[:64].any())
+    assert not bool(out[j:, 3].isfinite().any()) and bool(out[:, :3].isfinite().all()) and bool(out[:, 4:].isfinite().all())

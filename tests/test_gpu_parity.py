@@ -951,9 +951,9 @@ def test_random_shapes_fused_auto_dispatch(capi, seed):
 @pytest.mark.parametrize("m,n,k,g", [(32, 13824, 5120, 128), (17, 13824, 5120, 128), (24, 5120, 13824, 128),
                                      (32, 8192, 4352, 64), (20, 8192, 4352, 32)])
 def test_large_weights_17_to_32_tokens_auto_dispatch(capi, m, n, k, g):
-    """Large weights whose K is no multiple of 4096 at 17..32 tokens, which the automatic choice serves with the tiled
-    GEMM's 32-row tiles and a K split through the workspace: every output element against the oracle with bias,
-    ReLU and residual in the store, and against the split-K decode kernel asked for by name on the same operands."""
+    """Large weights whose K is no multiple of 4096 at 17..32 tokens, with and without a workspace (the automatic choice
+    is the ring kernel): every output element against the oracle with bias, ReLU and residual in the store, and the
+    split-K decode kernel asked for by name on the same operands."""
     d = orc.synth_linear(n, k, g, seed=n + k + m)
     w_hat = orc.dequant_l1(d["w_l1"], d["zs_l1"], g)
     x = orc.synth_x(m, k, seed=m + 3)

@@ -22,7 +22,7 @@ def to_dev(a):
 
 
 # (M, N, K, g): one row; a row past a tile; K shorter than a stage, ending inside one, inside 64 columns (group size 32);
-# N inside the first tile, one chunk past a tile; tiles beyond one round of 256 (the last case)
+# N inside the first tile, one chunk past a tile; several hundred tiles of the smallest shapes (the last case)
 CASES = [(1, 64, 128, 128), (33, 136, 640, 128), (97, 264, 1408, 128), (128, 256, 2048, 64), (100, 520, 960, 64),
          (65, 72, 416, 32), (40, 392, 1056, 32), (300, 5128, 384, 128)]
 
@@ -69,6 +69,7 @@ def test_ring_parity_of_256_row_tiles(capi, m, n, k, g):
     test_ring_parity(capi, 9, m, n, k, g)
 
 
+REST = 0x10  # tune word: only the tiles of the last round of 256 split K
 SUMS = 0x20  # tune word: the scale on the sums (shapes of 32 and 64 rows, group size 128)
 
 
@@ -147,3 +148,34 @@ def test_ring_keeps_an_infinite_activation_to_its_row(capi, shape, m, n, k, g):
         assert np.array_equal(got[m // 2], np.where(d["q"][:, -1] > 0, np.inf, -np.inf).astype(np.float16)), hex(tune)
         got[m // 2] = plain[m // 2]
         assert np.array_equal(got, plain), hex(tune)
+
+
+@pytest.mark.parametrize("shape,bm,bn,stage", [(1, 32, 64, 512), (2, 32, 128, 256), (3, 64, 128, 256), (4, 96, 128, 128),
+                                               (5, 64, 256, 128), (6, 96, 256, 128), (7, 128, 128, 128),
+                                               (8, 128, 256, 128), (9, 256, 256, 64)])
+def test_ring_whole_tiles_beside_split_ones(capi, shape, bm, bn, stage):
+    """260 tiles, ragged at both ends: 256 by one workgroup each and the last four in up to eight parts of K, in one
+    launch; nine stages, the last one part-filled.  Every word has to run."""
+    m, n, k, g = 2 * bm - 5, 129 * bn + 8, 8 * stage + 128, 128
+    gen = torch.Generator(device=DEV).manual_seed(shape)
+    w = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=gen)
+    z = torch.randint(64, 80, (n, k // g), device=DEV, generator=gen).half()
+    sc = (torch.rand((n, k // g), device=DEV, generator=gen) * 0.01 + 0.001).half()
+    pairs = lambda s: torch.stack([z, s], -1).reshape(n, -1).contiguous()
+    zs, x = pairs(sc), torch.randn((m, k), device=DEV, generator=gen).half()
+    ws = torch.zeros(65536 + 4 * 8 * bm * bn * 4, dtype=torch.uint8, device=DEV)
+    x64 = x.double()
+    for flag in (0, SUMS) if shape in (1, 2, 3, 5) else (0,):
+        if flag:  # (q - z) s without a rounding: the integers times the scales
+            w64 = capi.dequant(w, pairs(torch.ones_like(sc)), n, k, g).double() * sc.double().repeat_interleave(g, 1)
+        else:
+            w64 = capi.dequant(w, zs, n, k, g).double()
+        ref = x64 @ w64.t()
+        # one rounding to fp16 and K fp32 additions of the products' magnitudes
+        bound = 2.0 ** -11 * ref.abs() + k * 2.0 ** -24 * (x64.abs() @ w64.abs().t()) + 2.0 ** -24
+        for ks in (2, 3, 4, 6, 8):
+            y = torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV)
+            capi.gemm_ws(x, w, zs, n, k, g, out=y, algo=capi.SQ_ALGO_RING | ((shape | REST | flag | (ks << 8)) << 8), ws=ws)
+            worst = float(((y.double() - ref).abs() / bound).nan_to_num(nan=9.0).max())
+            assert worst <= 1.0, (ks, flag)
+            assert capi.workspace_is_clean(ws)

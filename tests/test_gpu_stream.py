@@ -152,9 +152,9 @@ def test_stream_is_the_automatic_choice_at_full_size(capi, n, k, m):
 @pytest.mark.parametrize("n,k", [(8192, 1024), (8200, 3200), (16384, 4096), (4096, 16384), (4096, 11008)])
 @pytest.mark.parametrize("m", [17, 24, 31, 32])
 def test_stream_two_token_tiles(capi, n, k, m):
-    """17..32 tokens: two token tiles per weight word, every wave moving the activations of its own chunks into LDS
-    (short K ranges leave chunk slots empty, long ones are split through the workspace, ragged N and K); explicit
-    kernel id and automatic dispatch against the oracle on sampled rows, with bias, ReLU and residual on the way out."""
+    """17..32 tokens on weights that the two-tile streaming kernel takes in grouped launches (see the next test): for one
+    linear its id and the automatic choice both run the ring kernel, with equal bits.  Short and long K, ragged N and K
+    against the oracle on sampled rows, with bias, ReLU and residual on the way out."""
     d = linear(n, k, seed=95)
     rng = np.random.default_rng(96 + m)
     x = orc.synth_x(m, k, seed=97 + m)
@@ -176,6 +176,44 @@ def test_stream_two_token_tiles(capi, n, k, m):
     # fixed summation order: the same bits on a second call, counters back at zero
     assert torch.equal(y, capi.gemm_fused(xd, d["w_dev"], d["zs_dev"], n, k, G, bias=bd, residual=rd, act=1, ws=ws))
     assert capi.workspace_is_clean(ws)
+
+
+@pytest.mark.parametrize("k,ns", [(3200, (8200, 136)), (11008, (2752, 200)), (16384, (2056, 72, 64))])
+@pytest.mark.parametrize("m", [17, 24, 31, 32])
+def test_grouped_two_token_tiles(capi, m, k, ns):
+    """17..32 tokens, several linears of equal K in one launch: two token tiles per weight word, every wave moving the
+    activations of its own chunks into LDS.  Rows enough for 128 workgroups or more, which is what the kernel asks for;
+    K in one range with empty chunk slots, and in three and four ranges through the workspace; ragged N; against the
+    oracle on sampled rows, with bias, ReLU and residual, each linear with its own."""
+    assert sum(-(-n // 64) for n in ns) * -(-k // 4096) >= 128
+    rng = np.random.default_rng(m + k)
+    lin, refs = [], []
+    for i, n in enumerate(ns):
+        d = linear(n, k, seed=300 + i)
+        rows = np.sort(rng.choice(n, size=min(n, 192), replace=False))
+        rows[0], rows[-1] = 0, n - 1
+        x = orc.synth_x(m, k, seed=310 + i)
+        bias = rng.normal(0, 1.0, size=n).astype(np.float16)
+        res = rng.normal(0, 1.0, size=(m, n)).astype(np.float16)
+        plain = orc.gemm_ref(x, d["w_hat"][rows]).astype(np.float64)
+        ref = plain + bias[rows].astype(np.float64)[None, :]
+        if i % 2:
+            ref = np.maximum(ref, 0.0)
+        refs.append((rows, ref + res[:, rows].astype(np.float64), np.max(np.abs(plain))))
+        lin.append(dict(x=to_dev(x), w=d["w_dev"], zs=d["zs_dev"], bias=to_dev(bias), residual=to_dev(res),
+                        y=torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV), n=n, k=k, group_size=G,
+                        act=i % 2, depends=False))
+    seq = capi.LinearSequence(lin, m, torch.device(DEV))
+    seq.run()
+    torch.cuda.synchronize()
+    for l, (rows, ref, scale) in zip(lin, refs):
+        got = l["y"].float().cpu().numpy()
+        assert np.all(np.isfinite(got))
+        assert np.max(np.abs(got[:, rows] - ref)) <= TOL * scale
+    first = [l["y"].clone() for l in lin]
+    seq.run()  # fixed summation order: the same bits, counters back at zero
+    assert all(torch.equal(a, l["y"]) for a, l in zip(first, lin))
+    assert capi.workspace_is_clean(seq.ws)
 
 
 def test_stream_properties(capi):
