@@ -133,14 +133,14 @@ int sq_w4a16_autotune_clear(void);
 /* sq_w4a16_gemm_ws for callers that cannot allocate device memory: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the
  * reference.  Same product, same kernels and the same automatic kernel choice, bit-identical
- * results; the workspace is a buffer of SQ_STATIC_WS_BYTES (16 MiB + 64 KiB) that lives inside
- * the library's device code, one copy per GPU for the life of the process, so the call
+ * results; the workspace is a buffer that lives inside the library's device code (37.6 MiB, what the
+ * ring kernel can want at most), one copy per GPU for the life of the process, so the call
  * allocates and frees nothing.  The caller still passes inputs and the output.
- * Limit: a call whose kernels would take more than SQ_STATIC_WS_BYTES from a workspace is rejected
- * with SQ_ERR_STATIC_WS and nothing is launched: the split-K decode kernels at 3..32 tokens (every
- * such batch with N <= 16384 fits) and the K splits of the tiled GEMM beyond 16 tokens.  One or two
- * tokens, and a GEMM whose grid fills the chip without a K split, use no workspace and are never
- * rejected, whatever N is.
+ * Limit: a call for which the split-K decode kernels at 3..32 tokens (every such batch with
+ * N <= 16384 fits) or the K splits of the tiled GEMM beyond 32 tokens are laid out to take more than
+ * SQ_STATIC_WS_BYTES (16 MiB + 64 KiB) is rejected with SQ_ERR_STATIC_WS and nothing is launched.
+ * One or two tokens, and a GEMM whose grid fills the chip without a K split, use no workspace and are
+ * never rejected, whatever N is.
  * The first call on a device looks the buffer's address up (hipGetSymbolAddress); nothing is
  * cleared, the array is zero when the library is loaded and every kernel leaves its counters zero.
  * Every call on a GPU shares that GPU's buffer: calls that overlap in time on one GPU (two

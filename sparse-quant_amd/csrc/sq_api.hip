@@ -11,7 +11,9 @@
 // call allocates nothing.  Every GPU the library runs on holds its own copy of the array until the
 // process ends; the name below is only the host-side handle of the symbol, the device address is
 // looked up once per device with hipGetSymbolAddress and that pointer is what the kernels get.
-static __device__ __align__(256) unsigned char scratch[SQ_STATIC_WS_BYTES];
+// It holds every plan of the ring kernel: within less, that kernel would split K otherwise than with a caller's workspace.
+constexpr size_t SCRATCH_BYTES = sq::RING_WORKSPACE_MAX > SQ_STATIC_WS_BYTES ? sq::RING_WORKSPACE_MAX : SQ_STATIC_WS_BYTES;
+static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 
 namespace {
 
@@ -461,7 +463,7 @@ int sq_w4a16_gemm_static_ws(const void* x, const void* w, const void* zs, void* 
     if (layout != SQ_LAYOUT_L1) return SQ_ERR_BAD_LAYOUT;
     // What the kernels of this token count would take from a workspace: nothing up to 2 tokens (the GEMV has
     // no workspace form), the split-K decode kernels' counters and partial tiles up to 32, the tiled GEMM's K
-    // split beyond (the ring kernel plans within whatever it is given).  A shape that wants more than the static
+    // split beyond (the ring kernel's always fits).  A shape that wants more than the static
     // buffer is refused rather than served by a slower workspace-free kernel behind the caller's back.
     const size_t need = M <= 2 ? 0 : (M <= 32 ? sq::skinny2_workspace_bytes(M, N, K) : sq::gemm_workspace_bytes(M, N, K));
     if (need > (size_t)SQ_STATIC_WS_BYTES) return SQ_ERR_STATIC_WS;
@@ -471,7 +473,7 @@ int sq_w4a16_gemm_static_ws(const void* x, const void* w, const void* zs, void* 
     void* ws = static_workspace();
     if (!ws) return SQ_ERR_LAUNCH;
     return gemm_dispatch(x, w, zs, y, M, N, K, group_size, layout, algo, sq::Epilogue{nullptr, nullptr, 0}, ws,
-                         (size_t)SQ_STATIC_WS_BYTES, stream);
+                         SCRATCH_BYTES, stream);
 }
 
 int sq_workspace_reset(void* workspace, size_t bytes, void* stream) {

@@ -710,7 +710,7 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes) {
         static const int splits[5] = {2, 3, 4, 6, 8};
         for (int ks : splits) {
             const long w = (long)rest * ks;
-            if (ks > stages || w > 300) break;
+            if (ks > stages || w > RING_PARTS_MAX) break;
             const int st = (stages + ks - 1) / ks;
             const float ex = t.ex0 + t.ex1 * ks + t.exmb * (4e-6f * w * t.bm * t.bn);
             const int r = (int)(w >> 8), last = (int)(w & 255);

@@ -94,6 +94,8 @@ hipError_t launch_gemm_tuned(const void* x, const void* w, const void* zs, void*
 // null: K is not split over workgroups).  RING_SUMS in tune: the scale on the sums in fp32 instead of W_hat (group size
 // 128, up to 64-row tiles).
 constexpr int RING_SUMS = 0x20;
+constexpr int RING_PARTS_MAX = 300;  // workgroups that share tiles of a plan, each with a partial tile of up to 128 x 256
+constexpr size_t RING_WORKSPACE_MAX = 65536 + (size_t)RING_PARTS_MAX * 128 * 256 * 4;
 bool gemm_ring_applies(int M, int N, int K);
 size_t gemm_ring_workspace_bytes(int M, int N, int K);
 hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,
