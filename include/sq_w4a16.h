@@ -50,12 +50,17 @@ extern "C" {
 #define SQ_ALGO_GEMM 4           /* any M: LDS-tiled MFMA GEMM */
 #define SQ_ALGO_SKINNY_WS 5      /* M <= 32: 64-row tiles, K split over workgroups through a workspace
                                     (sq_w4a16_gemm_ws only) */
-#define SQ_ALGO_STREAM 6         /* M <= 16 at group size 128 or 64, M <= 32 at group size 128: weight loads a fixed
-                                  * distance ahead of the arithmetic, activations staged in LDS first; K beyond 4096
-                                  * is split through the workspace */
-
-#define SQ_ALGO_RING 7           /* any M: 32 .. 128-row tiles, eight waves in two alternating groups, K split inside
-                                  * the workgroup (and over workgroups through the workspace) */
+#define SQ_ALGO_STREAM 6         /* M <= 16 at group size 128 or 64: weight loads a fixed distance ahead of the
+                                  * arithmetic, activations staged in LDS first; K beyond 4096 is split through the
+                                  * workspace.  17 <= M <= 32 at group size 128: the two-tile form of that kernel
+                                  * serves grouped launches only (sq_w4a16_gemv_sequence); for one linear the id is
+                                  * taken on the same weights (64-row blocks x ceil(K / 4096) of 128 or more, with a
+                                  * workspace where K > 4096) and runs SQ_ALGO_RING as the automatic choice does */
+#define SQ_ALGO_RING 7           /* any M: 32 .. 256-row tiles, eight waves in two alternating groups, K split inside
+                                  * the workgroup (and over workgroups through the workspace).  Tuning: 0 = planned,
+                                  * or tile shape 1..9 | 0x10 (only the last round of tiles splits K) | parts << 8;
+                                  * 0x20: the scale on the sums in fp32 instead of W_hat (group size 128, tiles of 32
+                                  * and 64 rows; the automatic choice up to 64 tokens at group size 128) */
 
 /* Library version (major*10000 + minor*100 + patch). */
 int sq_version(void);
@@ -88,15 +93,14 @@ int sq_w4a16_gemm_ex(const void* x, const void* w, const void* zs, void* y,
  * first 64 KiB zeroed before the first call (every call leaves them zero); calls that
  * share a workspace must not overlap in time.  With SQ_ALGO_AUTO the split is taken
  * where it is the fastest: the streaming decode kernel for 3..16 tokens at group size
- * 128 when K exceeds 4096 (a shorter K needs no split and no workspace), the split-K
- * decode kernel for 5..32 tokens otherwise on weights of 2^25 elements or more or with
- * K > 8192 and for 17..32 tokens on any weight, the same kernel in two blocks for 33..48
- * tokens on such weights, and a K split of the tiled GEMM for larger M whose grid would
- * leave most CUs idle and for 17..32 tokens on weights of 2^25 elements or more that the
- * two-tile streaming kernel would serve in part-empty rounds of workgroups (K a multiple
- * of 256; at group size 64 and 32, N >= 8192).  A workspace that is NULL, misaligned or too small is ignored under
- * SQ_ALGO_AUTO (the workspace-free kernels run); an explicit SQ_ALGO_SKINNY_WS then
- * returns SQ_ERR_WORKSPACE. */
+ * 128 or 64 when K exceeds 4096 (a shorter K needs no split and no workspace); the ring
+ * kernel, whose last, part-filled round of tiles is split, from 17 tokens on, and from 5
+ * on large weights whose K would leave the streaming kernel's workgroups part empty and
+ * at group size 32 on weights of more than 2^24 elements; the split-K decode kernel for
+ * what is left at 5..16 tokens on weights of 2^25 elements or more or with K > 8192.  A
+ * workspace that is NULL or misaligned is ignored under SQ_ALGO_AUTO, as is one too small
+ * for the decode kernels (the ring kernel splits K as far as it fits); an explicit
+ * SQ_ALGO_SKINNY_WS then returns SQ_ERR_WORKSPACE. */
 int sq_w4a16_gemm_ws(const void* x, const void* w, const void* zs, void* y,
                      int M, int N, int K, int group_size, int layout, int algo,
                      void* workspace, size_t workspace_bytes, void* stream);
@@ -108,7 +112,8 @@ int sq_w4a16_gemm_ws(const void* x, const void* w, const void* zs, void* y,
  * sq_w4a16_autotune runs the product x * W_hat^T with every kernel family and tuning that can
  * serve (M, N, K, group_size) -- the decode GEMV's workgroup shapes, the streaming kernel's row
  * blocks and K splits, the split-K kernel's splits, the tiled GEMM's tile heights, K splits and
- * staging variants -- `reps` launches each between two HIP events on `stream`, and records the
+ * staging variants, the ring kernel's shapes and K splits, within sq_w4a16_workspace_bytes(M, N, K)
+ * bytes of the workspace -- `reps` launches each between two HIP events on `stream`, and records the
  * fastest in a process-wide table that SQ_ALGO_AUTO consults first from then on, for exactly
  * this (M, N, K, group_size) and workspace situation (a workspace of at least
  * sq_w4a16_workspace_bytes(M, N, K) bytes present or not).  This is the one GEMM entry point

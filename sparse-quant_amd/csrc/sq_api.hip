@@ -320,7 +320,7 @@ static int autotune_candidates(int M, int K, int g, bool has_ws, int* out, int c
             for (int ks = 1; ks <= 8; ks *= 2)
                 if (ks == 1 ? K <= 4096 : (has_ws && K / ks >= 1024 && K / ks <= 4096)) add(SQ_ALGO_STREAM, rows[r] | (ks << 4));
     }
-        if (M > 2 && M <= 32 && has_ws)
+    if (M > 2 && M <= 32 && has_ws)
         for (int ks = 1; ks <= 8; ks *= 2) add(SQ_ALGO_SKINNY_WS, ks);
     if (M > 2 && M <= 64) add(SQ_ALGO_SKINNY, 0);
     if (M > 16) {
@@ -643,8 +643,11 @@ int sq_w4a16_gemv_sequence(const sq_linear_desc* linears, int count, int M, int 
                 return SQ_ERR_LAUNCH;
         }
         if (!done && l1 - l0 > 1 && M > 4 && M <= 32 && workspace && aligned16(workspace)) {
-            // the split-K decode kernel on the concatenated row blocks, where it is what one linear of the
-            // group's total size would get (large weight, more than 16 tokens, or long K)
+            // the split-K decode kernel on the concatenated row blocks: large weights, more than 16 tokens, or long K
+            // (17..32 tokens, the grouped launches against a launch of the ring kernel each, us at 32 tokens and group
+            // size 128: q/k/v of 4096x4096 14.9 / 27.4, 5120 + 1024 + 1024 rows of 5120 16.5 / 27.7, three of 1024x1024
+            // 7.3 / 23.8; two of 11008x4096 26.7 / 24.0.  One weight of their rows through the ring kernel: 12.1, 11.2,
+            // 8.0, 18.7)
             long elems = 0;
             for (int l = l0; l < l1; l++) elems += (long)probs[l].N * probs[l].K;
             if (elems >= (1L << 25) || M > 16 || probs[l0].K > 8192) {

@@ -29,7 +29,7 @@
 // softmax and first loads run beside another's products.  Where there are too few workgroups for that, four waves take
 // steps of 64 keys and split them (SPLIT_WGS below).
 // Measured (us; before: 16 queries per wave, K through registers, V transposed by vector instructions):
-//   32 heads x 4096 x 128, causal, 26 % of the blocks   125 -> 85 (matrix pipes busy 0.39 of the cycles)
+//   32 heads x 4096 x 128, causal, 26 % of the blocks   125 -> 85 (matrix pipes busy 0.41 of the cycles)
 //   8 x 16 heads x 4096 x 64, 25 %                       225 -> 181
 //   8 x 32 heads x 512 x 128, causal, 26 %               38.5 -> 34 (134 MB to move: 22 at the rate of a copy)
 //   8 x 16 heads x 512 x 64, 25 %                        10.2 -> 8.1
@@ -40,7 +40,7 @@
 // request of the table needs are scalars now, which arrive with the wave.
 // A model's prompt reads q, k and v where the fused projection left them and stores the cache rows and a [batch, row,
 // hidden] output: the element-wise copies around the kernel cost three times its own time (8 prompts of 512 tokens, 32
-// heads of 128, per layer: six copies of 21 us and 35 -> 52 in all; without a table, against torch's attention and its
+// heads of 128, per layer: six copies of 21 us and 35 -> 42 in all; without a table, against torch's attention and its
 // copies, 157 -> 59).
 #include "sq_common.h"
 #include "sq_kernels.h"

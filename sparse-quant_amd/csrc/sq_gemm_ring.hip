@@ -33,7 +33,7 @@
 //
 // Operand mapping as in sq_gemm.hip: D = X W^T with activations as A (lane = row) and weights as B (lane = column);
 // lane (ln, lc) of a wave holds k = 32 lc + 8 t .. + 7 of its 64 for slice t, one packed word of the weight row per
-// slice; W_hat = fp16((q - z) * s) bit for bit.
+// slice; W_hat = fp16((q - z) * s) bit for bit, or with SUMS the integers q - z.
 // (replaces w4a16_gemm_wmma_kernel, reference: quantization/muxi/backend/w4a16_gemm.cuh:466-600, and the role of
 // turbomind::GemmS4F16, quantization/nvidia/kernel/gemm_s4_f16/gemm_template.h:358-450)
 #include "sq_common.h"

@@ -194,7 +194,7 @@ def workspace_is_clean(ws, nbytes=65536, stream=None):
 
 
 def gemm_ws(x, w, zs, n, k, group_size, algo=SQ_ALGO_AUTO, out=None, stream=None, ws=None):
-    """x fp16 [M,K] -> y fp16 [M,N] through sq_w4a16_gemm_ws (workspace-backed split-K for 5 <= M <= 32)."""
+    """x fp16 [M,K] -> y fp16 [M,N] through sq_w4a16_gemm_ws (K split over workgroups through the workspace)."""
     m = x.numel() // k
     if out is None:
         out = torch.empty((m, n), dtype=torch.float16, device=x.device)
