@@ -103,7 +103,8 @@ enum : unsigned {
     P_OVER_16M = 1u << 8,     // N * K > 2^24 elements
     P_CHUNK_FILL = 1u << 9,   // the least K split of the streaming kernel fills 3/4 or more of a workgroup's 32 chunks
     P_RING = 1u << 10,        // the ring kernel can address the operands
-    P_SHORT_ROUNDS = 1u << 11,  // many rounds of 128 x 256 tiles over a short K (see builtin_choice)
+    P_SMALL_K2048 = 1u << 11,   // N * K <= 2^22 elements and K <= 2048
+    P_SHORT_ROUNDS = 1u << 12,  // many rounds of 128 x 256 tiles over a short K (see builtin_choice)
 };
 struct ChoiceRule {
     int m_lo, m_hi;
@@ -116,7 +117,9 @@ const ChoiceRule kChoiceRules[] = {
     {5, 16, P_LARGE | P_G128_64 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
      "8 / 16 tokens: 15360x5120 13.9 vs 16.0 / 19.0 (streaming kernel), 13696x5120 13.4 vs 15.7 / 19.3"},
     {9, 16, P_OVER_16M | P_RING, P_G128_64, SQ_ALGO_RING,
-     "16 tokens, group size 32: 5120x5120 10.3 vs 19.2, 12288x4096 12.2 vs 15.4, 4096x11008 13.0 vs 15.4; 4096x4096 8.6 vs 8.4"},
+     "16 tokens, group size 32: 5120x5120 10.3 vs 19.2, 12288x4096 12.2 vs 15.4, 4096x11008 13.0 vs 15.4; 4096x4096 8.6 vs 8.4; "
+     "9 tokens: 5120x4096 9.4 vs 11.8 (16-column kernel), 16000x2048 8.2 vs 11.3, 6144x3072 8.6 vs 9.6; the other way where that "
+     "kernel's N / 16 workgroups just fill their rounds: 8192x2176 8.6 vs 7.1, 4096x4608 9.0 vs 7.5"},
     // (5..8 tokens: what the GEMV below does not take.  The GEMV applies the scale to its sums in fp32)
     {5, 8, P_LARGE | P_WS | P_RING, P_G128_64, SQ_ALGO_RING,
      "8 tokens, group size 32: 12288x4096 11.7 vs 14.7 (split-K kernel) and 15.2 (GEMV), 4096x11008 12.6 vs 14.9 / 13.7, "
@@ -132,6 +135,10 @@ const ChoiceRule kChoiceRules[] = {
      "4 tokens: fc2 11.9 vs 13.6 (GEMV); 13824x5120, whose K ranges fill 20 of a workgroup's 32 chunks: 14.6 vs 13.9 (GEMV)"},
     // small weights at 17..32 tokens: the 16-column kernel (one launch, no exchange between workgroups)
     {17, 32, P_SMALL, 0, SQ_ALGO_SKINNY, "24 tokens: 3072x1024 4.9 vs 5.2 (ring kernel); 2048x2048 at 32 tokens 7.4 vs 6.8"},
+    {17, 28, P_SMALL_K2048, 0, SQ_ALGO_SKINNY,
+     "2048x1664 at 17 / 24 / 28 / 32 tokens 5.1 / 5.9 / 6.3 / 6.7 vs 7.2 / 7.2 / 7.3 / 7.3 (ring kernel, four stages of K); 1536x1792 "
+     "5.2 / 5.8 / 6.2 / 6.8 vs 6.8 / 6.9 / 6.9 / 6.9; 2048x2048 5.9 / 6.4 / 6.7 / 7.0 vs 7.2 / 7.2 / 7.2 / 7.1; 1024x2048 at 28 "
+     "tokens and group size 64 6.6 vs 6.5"},
     // everything else from 17 tokens up
     {17, 1 << 30, P_RING, P_SHORT_ROUNDS, SQ_ALGO_RING,
      "see sq_gemm_ring.hip: 1.25x at 24..32 tokens, 1.4x at 40..160, 1.2x at 256..700, 1.1x at 1024..2048 (geometric means over 18 weights)"},
@@ -155,6 +162,7 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
     if (g == 128 || g == 64) p |= P_G128_64;
     if (K % 128 == 0) p |= P_K128;
     if (nk <= (1L << 22) && K <= 1536) p |= P_SMALL;
+    if (nk <= (1L << 22) && K <= 2048) p |= P_SMALL_K2048;
     {
         const int chunks = K / 128, ks0 = (chunks + 31) / 32;
         if (ks0 > 0 && chunks * 4 >= ks0 * 32 * 3) p |= P_CHUNK_FILL;
