@@ -56,7 +56,7 @@ extern "C" {
                                   * serves grouped launches only (sq_w4a16_gemv_sequence); for one linear the id is
                                   * taken on the same weights (64-row blocks x ceil(K / 4096) of 128 or more, with a
                                   * workspace where K > 4096) and runs SQ_ALGO_RING as the automatic choice does */
-#define SQ_ALGO_RING 7           /* any M: 32 .. 256-row tiles, eight waves in two alternating groups, K split inside
+#define SQ_ALGO_RING 7           /* any M: 32 .. 256-row tiles, operands through a ring of direct loads, K split inside
                                   * the workgroup (and over workgroups through the workspace).  Tuning: 0 = planned,
                                   * or tile shape 1..9 | 0x10 (only the last round of tiles splits K) | parts << 8;
                                   * 0x20: the scale on the sums in fp32 instead of W_hat (group size 128, tiles of 32

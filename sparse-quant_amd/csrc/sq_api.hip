@@ -171,16 +171,16 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
     if (K <= 8192) p |= P_K_LE_8192;
     if (K <= 32768) p |= P_K_LE_32768;
     if (sq::gemm_ring_applies(M, N, K)) p |= P_RING;
-    if (M > 1024 && K <= 4096 && K % 256 == 0 && g >= 64) {
+    if (M > 1024 && K <= 2048 && K % 256 == 0 && g >= 64) {
         // One workgroup per CU pays its first loads and its stores in full every round, two per CU hide them behind each
         // other; the ring kernel's 256 x 256 tiles make that up where they fill their last round (us, two per CU against
-        // the ring kernel: 6144x1536 at 4096 tokens, 384 of its tiles, 84 against 93; 8192x1024 at 5000, 640 tiles, 94
-        // against 103; 13312x4096 at 5000, 1040 tiles, 564 against 578; but 8192x2048 at 4096, 512 tiles, 141 against 135,
-        // 16384x4096 at 4096, 1024 tiles, 527 against 508, and 6144x1536 at 2048, 192 tiles, 52 against 46).  With fewer
-        // rounds of 128 x 256 or a longer K the ring kernel is ahead whatever they fill.
+        // the ring kernel: 6144x1536 at 4096 tokens, 384 of its tiles, 85 against 96; 8192x1024 at 5000, 640 tiles, 97
+        // against 116; 24576x1024 at 5000, 1920 tiles, 273 against 287; but 5120x2048 at 3000, 240 tiles, 71 against 63).
+        // With fewer rounds or a longer K the ring kernel is ahead whatever they fill (13312x4096 at 5000, 1040 tiles, 545
+        // against 533; 16384x3072 at 3000 291 against 269).
         const long tiles = (long)((N + 255) / 256) * ((M + 127) / 128);
         const long wide = (long)((N + 255) / 256) * ((M + 255) / 256), rounds = (wide + 255) / 256;
-        if (tiles >= (K <= 2048 ? 384 : 1500) && rounds > 1 && wide * 20 < rounds * 256 * 17) p |= P_SHORT_ROUNDS;
+        if (tiles >= 384 && rounds > 1 && wide * 20 < rounds * 256 * 17) p |= P_SHORT_ROUNDS;
     }
     for (const ChoiceRule& r : kChoiceRules)
         if (M >= r.m_lo && M <= r.m_hi && (p & r.need) == r.need && (p & r.forbid) == 0) return r.kernel;

@@ -2,19 +2,22 @@
 // contraction, and the contraction itself until many rounds of short K favour the two-workgroups-per-CU kernel of
 // sq_gemm.hip.
 //
-// What bounds it.  At 32..600 tokens neither HBM nor the matrix cores are full; what a CU can issue is: about five
-// vector instructions fit beside a v_mfma_f32_32x32x16_f16 (32 cycles), each further one costs five cycles or more,
-// and dequantising eight weights takes thirteen.  A workgroup with one wave per SIMD (the kernel this one replaces)
-// leaves the matrix pipe idle through every barrier, LDS trip and load issue.  Hence:
-//   * eight waves, two per SIMD, in two groups that alternate: while waves 0..3 issue the matrix instructions of a
-//     phase from registers, waves 4..7 read their operands from LDS, dequantise and request the next loads, then the
-//     groups swap at a barrier.  (Measured on a loop of the same instruction mix: both groups in step 1790 cycles per
-//     64 k of a 64-row tile, alternating 1520, matrix instructions alone 1040.)  Part of the dequantisation sits
-//     between the matrix instructions of the phase before it is needed.
+// What bounds it.  At 32..600 tokens neither HBM nor the matrix cores are full; what a CU can issue is: a
+// v_mfma_f32_32x32x16_f16 takes 32 cycles and hides vector instructions of the other wave of its SIMD completely, but a
+// wave gets one out every 5..6 cycles, and dequantising eight weights takes thirteen.  Beyond, the clock: with the matrix
+// pipes 0.9 busy it falls to 1.5 GHz (2.4 with the same loads and no matrix instruction), so that every instruction that
+// goes is time.  Hence:
+//   * all waves in step, one barrier per stage (64 k of a wave), everything one slice (16 k) or two ahead in registers:
+//     beside the matrix instructions of a slice stand the dequantisation of the next one's weights, the LDS reads of the
+//     activations of the one after that and the stage's requests, one by one, because four waves that send theirs
+//     together wait 350 cycles for the address unit.  (Two groups of waves that alternate between matrix instructions and
+//     everything else, as the SUMS loop below still does: the other half, LDS trip, requests and half the
+//     dequantisation one after the other, takes 1050 cycles a phase against 660 of matrix instructions.  Loop cycles
+//     100 tokens x 15360x5120 42400 -> 38500, 333 x 12288x4096 83300 -> 63000, 2048 x 16384x4096 172600 -> 149500.)
 //   * K is split over the waves of the workgroup (WK groups of 64 consecutive k each per stage of KS = 64 WK), so that
 //     a weight row is read in 64..256-byte pieces, a stage holds 40..50 KB, and narrow weights fill the chip without
 //     partial tiles in memory.  The groups' sums meet in LDS at the end.
-//   * every operand goes global -> LDS by direct loads, ST - 1 stages ahead (three or four stages of a ring); rows past
+//   * every operand goes global -> LDS by direct loads, up to ST stages ahead (three or four stages of a ring); rows past
 //     M are never requested (their lanes are masked, their LDS rows are zero), so padding costs no memory traffic.
 //   * where the tiles leave CUs idle, the tiles of the last, part-filled round split K over workgroups through the
 //     caller's workspace.
@@ -23,13 +26,16 @@
 //   100 tokens  4096x4096 15.9 -> 11.0, 15360x5120 37.3 -> 28.8, 5120x13696 54.0 -> 30.2
 //   333 tokens  4096x4096 27.0 -> 20.2, 12288x4096 65.1 -> 47.5, 5120x13696 90.3 -> 65.0
 //   1024 tokens 4096x4096 46.0 -> 41, 5120x13696 202 -> 152; 2048 tokens 4096x16384 269 -> 243 (1.13 PFLOP/s)
-// Tiles of 256 x 256 (two rows of waves that share the weight columns, no K groups to add up at the end, a quarter less
-// to load per product) where they fill the chip: 12288x4096 at 1024 tokens 118 -> 105, 16384x4096 at 2048 tokens
-// 269 -> 259, at 4096 tokens 537 -> 512, 15360x5120 at 4096 tokens 647 -> 610 (1.06 PFLOP/s on a box where the smaller
-// tiles reach 1.00).
-// Tried and dropped: all waves in one group with software-pipelined operands (8..15 % slower), stages of 32 k per wave
-// with twice the bytes in flight (10 % slower: a barrier per 8 matrix instructions), the group sums handed over in
-// registers' order instead of row-major slices (1..4 % slower below 256 tokens).
+//   in step     100 tokens 15360x5120 28.2 -> 26.9, 192 12288x4096 31.1 -> 29.8, 333 12288x4096 at group size 64
+//   45.9 -> 42.7, 2048 4096x16384 246 -> 235
+// Tiles of 256 x 256 with four waves of 256 x 64 (one wave per SIMD, 256 accumulation registers), which dequantise every
+// weight once where eight waves of 128 x 64 did it twice, at the same loop cycles a clock of 1550 instead of 1450 MHz:
+// 16384x4096 at 2048 tokens 249 -> 238, and no K groups to add up at the end.
+// Tried and dropped: eight waves in step without the scheduling (8..15 % slower than alternating groups; the waits for
+// LDS were not counted then, since the compiler does not see a wait in inline assembly), 32 k per wave and stage (half the
+// LDS reads, no faster), four waves of 128 x 128 (250 where 256 x 64 take 238), requests between the matrix instructions
+// of alternating groups (5..15 % slower), the group sums handed over in registers' order instead of row-major slices
+// (1..4 % slower below 256 tokens).
 //
 // Operand mapping as in sq_gemm.hip: D = X W^T with activations as A (lane = row) and weights as B (lane = column);
 // lane (ln, lc) of a wave holds k = 32 lc + 8 t .. + 7 of its 64 for slice t, one packed word of the weight row per
@@ -85,7 +91,7 @@ struct RingShape {
     static constexpr int PER = XI + WI + ZI;
     static constexpr int LDS = ST * SB;
     static constexpr int TAIL = NW * 32 * 32 * NI * 4;  // one 32-row slice of every wave's sums
-    static_assert(XI * NW * 1024 == XB && WI * NW * 1024 == WB && ZI * ZL * NW == BN * P && NW == 8, "loads divide over the waves");
+    static_assert(XI * NW * 1024 == XB && WI * NW * 1024 == WB && ZI * ZL * NW == BN * P && (NW == 8 || NW == 4), "loads divide over the waves");
     static_assert(LDS <= 163840 && TAIL <= LDS, "fits");
 };
 
@@ -150,16 +156,17 @@ __device__ __forceinline__ void load_to_lds_x1_masked(const void* base, uint32_t
 // fp32, as in the decode kernels at group size 128; without it they see W_hat.  Sixteen vector instructions per 64 k and
 // column tile go and sixteen per row tile come: the same count with one row tile, more with two.  Measured (us, W_hat / sums):
 // 32 tokens 12288x4096 11.96 / 12.03, 5120x13696 16.3 / 16.4; 48 tokens 12288x4096 16.4 / 16.1, 5120x13696 20.6 / 21.1;
-// 64 tokens 4096x11008 16.6 / 16.6, 15360x5120 20.4 / 21.0.
+// 64 tokens 4096x11008 16.6 / 16.6, 15360x5120 20.4 / 21.0.  Its loop keeps the two alternating groups of waves (0..3 fetch
+// phase p + 1 while 4..7 compute phase p): in step it would need a second set of sums.
 template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
-__global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(
+__global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4))) void gemm_ring_kernel(
     const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS, const half_t* __restrict__ X, half_t* __restrict__ Y,
     int M, int N, int K, int mtiles, int tiles, int nfull, int ksplit, Epilogue epi, float* part, unsigned* counters) {
     using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
     constexpr int BM = S::BM, BN = S::BN, KS = S::KS, SB = S::SB, XI = S::XI, WI = S::WI, ZI = S::ZI, ZL = S::ZL, PER = S::PER, P = S::P;
     constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = S::XB + S::WB;
-    constexpr int H = MI > 3 || MI * NI > 4 ? 2 : 4, PH = 4 / H;  // 16-wide k slices per phase, phases per stage
-    static_assert(!SUMS || (PH == 1 && GS == 7), "a phase lies in one group");
+    constexpr int H = 4;  // 16-wide k slices per stage and wave
+    static_assert(!SUMS || (MI * NI <= 4 && GS == 7 && S::NW == 8), "a stage of a wave lies in one group, and the registers suffice");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S::LDS];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
@@ -228,11 +235,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         const int d = (wave * ZI + j) * ZL + (lane & (ZL - 1));
         zlane[j] = (uint32_t)((long)imin(n0 + d / P, N - 1) * groups * 4) + (d % P) * 4;
     }
-    // All loads of stage it into slot c.  EDGE: the last stage of a K that ends inside it; weights that are missing re-read
+    // Loads of stage it into slot c.  EDGE: the last stage of a K that ends inside it; weights that are missing re-read
     // the end of the row (and meet a scale of 0), activations are zeros in LDS (an infinity at the end of a row, re-read,
     // would be a NaN in every column.  Clearing the operands in the last stages' registers instead cost the 256 x 256 tiles
     // 0.9 % whatever K was: 16384x4096 at 4096 tokens 493 -> 498 us).
-    auto issue = [&](int it, int c, auto EDGE_) {
+    auto issue = [&](int it, int c, auto EDGE_, int lo = 0, int hi = 1 << 20) __attribute__((always_inline)) {  // requests lo .. hi - 1
         constexpr bool EDGE = decltype(EDGE_)::value;
         const int k0 = it * KS, left = K - k0;
         const uint8_t* xb = (const uint8_t*)X + (long)k0 * 2;
@@ -241,6 +248,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         const uint32_t l0 = lds0 + c * SB;
 #pragma unroll
         for (int j = 0; j < ZI; j++) {
+            if (j < lo || j >= hi) continue;
             uint32_t o = zlane[j];
             if constexpr (EDGE) {
                 const int p = ((wave * ZI + j) * ZL + (lane & (ZL - 1))) % P;
@@ -250,6 +258,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
 #pragma unroll
         for (int j = 0; j < WI; j++) {
+            if (ZI + j < lo || ZI + j >= hi) continue;
             uint32_t o = wlane[j];
             if constexpr (EDGE) {
                 const int R = (wave * WI + j) * (32 / WK) + lane / (2 * WK);
@@ -260,6 +269,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
 #pragma unroll
         for (int j = 0; j < XI; j++) {
+            if (ZI + WI + j < lo || ZI + WI + j >= hi) continue;
             uint64_t mask = xmask[j];
             if constexpr (EDGE) {
                 const int ii = wave * XI + j;
@@ -294,12 +304,196 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[mi][ni][v] = 0.f;
 
-    half8_t a[H][MI], b[H][NI];
-    half2_t zs[NI];
-    uint32_t q[NI][H];
-    float16_t part_sum[SUMS ? MI : 1][SUMS ? NI : 1];  // of the stage before, and its scales
-    float part_scale[SUMS ? NI : 1];
-    if constexpr (SUMS) {
+    auto wait_lds = []() { __builtin_amdgcn_s_waitcnt(0xC07F); };  // lgkmcnt(0), where the compiler sees it: later waits stay counted
+    if constexpr (!SUMS) {
+        half8_t a[4][MI], b[2][NI];               // activations of slice t in a[t], weights of slice t in b[t & 1]
+        uint32_t q[NI][4], q3[NI], qn[NI][4];     // packed words of the stage (the last one apart), and of the next stage
+        half2_t zs[NI], zn[NI], z1024[NI];
+        uint32_t hi8[NI];
+        auto read_weights = [&](int c) {
+            const uint8_t* l = lds + c * SB;
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) {
+                zn[ni] = *(const half2_t*)(l + zoff + ni * (32 * P * 4));
+                const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (32 * 32 * WK));
+#pragma unroll
+                for (int t = 0; t < 4; t++) qn[ni][t] = v[t];
+            }
+        };
+        auto read_rows = [&](int c, int t, int lo, int hi) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = lo; r < hi; r++) a[t][r] = *(const half8_t*)(lds + c * SB + xoff[t] + r * 4096);
+        };
+        // Weights past the end of K get the scale 0 (only the last stage can hold any).
+        auto clip = [&](int it) {
+            if (it * KS + 64 * kg + (GS == 5 ? 32 * lc : 0) >= K) {
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++) zn[ni].y = (half_t)0.f;
+            }
+        };
+        // Pair j of a word, i.e. two of its eight weights, as dequant8 gives them.
+        auto dequantise_pair = [&](int slot, int ni, int j, uint32_t w, half2_t z) __attribute__((always_inline)) {
+            const half2_t z64 = {z.x, z.x}, sc = {z.y, z.y};
+            if (j == 0) z1024[ni] = z64 + (half2_t){(half_t)960.f, (half_t)960.f};
+            if (j == 2) hi8[ni] = w >> 8;
+            const uint32_t src = j < 2 ? w : hi8[ni];
+            u32x4_t v = bit_cast<u32x4_t>(b[slot][ni]);
+            v[j] = (j & 1) ? dequant_pair((src & nm.hi) | 0x54005400u, z64, sc)
+                           : dequant_pair((src & nm.lo) | 0x64006400u, z1024[ni], sc);
+            b[slot][ni] = bit_cast<half8_t>(v);
+        };
+        // The next stage becomes readable in the middle of a stage, in front of row block BAR of slice 2: by then the last
+        // rows of the stage, requested from LDS in slice 1, have arrived without a wait, and its slot is free.
+        constexpr int BAR = MI >= 4 ? 1 : 0;
+        constexpr int PAIRS = 4 * NI;  // of a slice
+        constexpr int NB = 4 * MI;     // row blocks of a stage, counted from slice 2 for the requests
+        // Slice t of the stage in slot c, row block by row block: matrix instructions, beside them a share of the next
+        // slice's dequantisation and (AHEAD) of the rows of the slice after that (from slot cn past the middle);
+        // behind them the requests(row block).
+        auto slice = [&](auto t_, auto ahead_, int c, int cn, auto middle, auto requests) __attribute__((always_inline)) {
+            constexpr int t = decltype(t_)::value;
+            constexpr bool AHEAD = decltype(ahead_)::value;
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) {
+                if (t == 2 && mi == BAR) middle();
+                if constexpr (AHEAD) {
+                    constexpr int first = t == 2 ? BAR : 0, n = MI - first;
+                    if (mi >= first) read_rows(t < 2 ? c : cn, (t + 2) & 3, (mi - first) * MI / n, (mi - first + 1) * MI / n);
+                }
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t][mi], b[t & 1][ni], acc[mi][ni], 0, 0, 0);
+#pragma unroll
+                for (int k = mi * PAIRS / MI; k < (mi + 1) * PAIRS / MI; k++) {
+                    const int ni = k / 4;
+                    if constexpr (t < 2)
+                        dequantise_pair((t + 1) & 1, ni, k & 3, q[ni][t + 1], zs[ni]);
+                    else if constexpr (t == 2)
+                        dequantise_pair(1, ni, k & 3, mi < BAR ? q[ni][3] : q3[ni], zs[ni]);
+                    else
+                        dequantise_pair(0, ni, k & 3, qn[ni][0], zn[ni]);
+                }
+                constexpr int VA = (14 * NI + MI * NI - 1) / (MI * NI);
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, VA, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                requests(((t + 2) & 3) * MI + mi);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) {  // finished here, not where the matrix instructions want it
+                u32x4_t v = bit_cast<u32x4_t>(b[(t + 1) & 1][ni]);
+                asm volatile("" : "+v"(v));
+                b[(t + 1) & 1][ni] = bit_cast<half8_t>(v);
+            }
+        };
+        auto keep_last_word = [&]() {
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) q3[ni] = q[ni][3];
+        };
+        auto take = [&]() {
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) {
+                zs[ni] = zn[ni];
+#pragma unroll
+                for (int t = 0; t < 4; t++) q[ni][t] = qn[ni][t];
+            }
+        };
+        // Middle of a stage: the next one has landed (full: all but the ST - 2 younger ones), and every wave has read this one.
+        auto landed = [&](bool full) {
+            wait_lds();
+            if (full)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        };
+        using T0 = std::integral_constant<int, 0>;
+        using T1 = std::integral_constant<int, 1>;
+        using T2 = std::integral_constant<int, 2>;
+        using T3 = std::integral_constant<int, 3>;
+        using Yes = std::true_type;
+        using No = std::false_type;
+        if (it0 < it1) {
+            // The first stage's loads of all waves before any wave's second, and the last slot's behind the first reads.
+#pragma unroll
+            for (int s = 0; s < ST - 1; s++) {
+                if (it0 + s < it1) issue_any(it0 + s, s);
+                if (s == 0) __builtin_amdgcn_s_barrier();
+            }
+            landed(it0 + ST - 1 <= it1);
+            read_weights(0);
+            read_rows(0, 0, 0, MI);
+            read_rows(0, 1, 0, MI);
+            if (it0 + ST - 1 < it1) issue_any(it0 + ST - 1, ST - 1);
+            clip(it0);
+#pragma unroll
+            for (int k = 0; k < PAIRS; k++) dequantise_pair(0, k / 4, k & 3, qn[k / 4][0], zn[k / 4]);
+            take();
+            int c = 0, cp = ST - 1, it = it0;
+            auto nothing = []() {};
+            auto no_requests = [](int) {};
+            // A stage that requests stage it + ST, a whole one, into its own slot from the middle on, the rest of it in the
+            // stage after (FIRST: none of it is left from the stage before).  No branch inside: the waits for LDS stay counted.
+            const int plain = it1 * KS > K ? it1 - 1 : it1;
+            auto stage = [&](auto first_) {
+                constexpr bool FIRST = decltype(first_)::value;
+                const int cn = c == ST - 1 ? 0 : c + 1;
+                auto rest = [&](int o) __attribute__((always_inline)) {
+                    if constexpr (!FIRST) issue(it + ST - 1, cp, std::false_type{}, o * PER / NB, (o + 1) * PER / NB);
+                };
+                auto begin = [&](int o) __attribute__((always_inline)) {
+                    if (o >= BAR) issue(it + ST, c, std::false_type{}, o == BAR ? 0 : o * PER / NB, (o + 1) * PER / NB);
+                };
+                auto middle = [&]() {
+                    keep_last_word();
+                    landed(true);
+                    read_weights(cn);
+                };
+                slice(T0{}, Yes{}, c, cn, nothing, rest);
+                slice(T1{}, Yes{}, c, cn, nothing, rest);
+                slice(T2{}, Yes{}, c, cn, middle, begin);
+                slice(T3{}, Yes{}, c, cn, nothing, begin);
+                take();
+                cp = c;
+                c = cn;
+                it++;
+            };
+            if (it + ST < plain) {
+                stage(Yes{});
+                while (it + ST < plain) stage(No{});
+                issue(it + ST - 1, cp, std::false_type{}, 2 * MI * PER / NB, PER);
+            }
+            // the last ST stages, and one more where K ends inside the last
+            for (; it < it1; it++) {
+                const int cn = c == ST - 1 ? 0 : c + 1;
+                auto middle = [&]() {
+                    keep_last_word();
+                    landed(it + ST - 1 < it1);
+                    if (it + 1 < it1) {
+                        read_weights(cn);
+                        read_rows(cn, 0, 0, MI);
+                        read_rows(cn, 1, 0, MI);
+                        clip(it + 1);
+                    }
+                    if (it + ST < it1) issue_any(it + ST, c);
+                };
+                slice(T0{}, Yes{}, c, cn, nothing, no_requests);
+                slice(T1{}, Yes{}, c, cn, nothing, no_requests);
+                slice(T2{}, No{}, c, cn, middle, no_requests);
+                slice(T3{}, No{}, c, cn, nothing, no_requests);
+                take();
+                c = cn;
+            }
+        }
+    } else {
+        half8_t a[H][MI], b[H][NI];
+        half2_t zs[NI];
+        uint32_t q[NI][H];
+        float16_t part_sum[MI][NI];  // of the stage before, and its scales
+        float part_scale[NI];
 #pragma unroll
         for (int ni = 0; ni < NI; ni++) {
             part_scale[ni] = 0.f;
@@ -308,10 +502,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
                 for (int v = 0; v < 16; v++) part_sum[mi][ni][v] = 0.f;
         }
-    }
-    // (pinned, so that the wait for the matrix instructions' results is not moved in front of the barrier)
-    auto fold = [&]() {
-        if constexpr (SUMS) {
+        // (pinned, so that the wait for the matrix instructions' results is not moved in front of the barrier)
+        auto fold = [&]() {
 #pragma unroll
             for (int mi = 0; mi < MI; mi++)
 #pragma unroll
@@ -321,198 +513,186 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                     for (int v = 0; v < 16; v++)
                         acc[mi][ni][v] = __builtin_fmaf(part_sum[mi][ni][v], part_scale[ni], acc[mi][ni][v]);
                 }
-        }
-    };
-    auto dequantise = [&](int t) {
+        };
+        auto unpack = [&](int t) {
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++) {
-            const half2_t z = {zs[ni].x, zs[ni].x};
-            b[t][ni] = SUMS ? integers8(q[ni][t], z, nm) : dequant8(q[ni][t], z, (half2_t){zs[ni].y, zs[ni].y}, nm);
-        }
-    };
-    // Phase h of stage it (slot c): the wave's operands into registers, weights dequantised.
-    auto fetch = [&](int it, int c, auto h_) {
-        constexpr int h = decltype(h_)::value;
-        const uint8_t* l = lds + c * SB;
+            for (int ni = 0; ni < NI; ni++) b[t][ni] = integers8(q[ni][t], (half2_t){zs[ni].x, zs[ni].x}, nm);
+        };
+        // The wave's operands of the stage in slot c into registers.
+        auto fetch = [&](int c) {
+            const uint8_t* l = lds + c * SB;
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++) {
-            zs[ni] = *(const half2_t*)(l + zoff + ni * (32 * P * 4));
-            if constexpr (H == 4) {
+            for (int ni = 0; ni < NI; ni++) {
+                zs[ni] = *(const half2_t*)(l + zoff + ni * (32 * P * 4));
                 const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (32 * 32 * WK));
 #pragma unroll
                 for (int t = 0; t < 4; t++) q[ni][t] = v[t];
-            } else {
-                const u32x2_t v = *(const u32x2_t*)(l + woff + 8 * h + ni * (32 * 32 * WK));
-                q[ni][0] = v.x;
-                q[ni][1] = v.y;
             }
-        }
 #pragma unroll
-        for (int t = 0; t < H; t++)
+            for (int t = 0; t < H; t++)
 #pragma unroll
-            for (int mi = 0; mi < MI; mi++) a[t][mi] = *(const half8_t*)(l + xoff[h * H + t] + mi * 4096);
-    };
-    // Weights past the end of K get the scale 0 (only the last stage can hold any).
-    auto clip = [&](int it) {
-        if (it * KS + 64 * kg + (GS == 5 ? 32 * lc : 0) >= K) {
+                for (int mi = 0; mi < MI; mi++) a[t][mi] = *(const half8_t*)(l + xoff[t] + mi * 4096);
+        };
+        // Weights past the end of K get the scale 0 (only the last stage can hold any).
+        auto clip = [&](int it) {
+            if (it * KS + 64 * kg >= K) {
 #pragma unroll
-            for (int ni = 0; ni < NI; ni++) zs[ni].y = (half_t)0.f;
-        }
-    };
-    // the first half of the phase's weights, finished in front of the barrier that follows
-    auto dequantise_first = [&]() {
-        fold();
-#pragma unroll
-        for (int t = 0; t < H / 2; t++) {
-            dequantise(t);
-#pragma unroll
-            for (int ni = 0; ni < NI; ni++) {
-                u32x4_t v = bit_cast<u32x4_t>(b[t][ni]);
-                asm volatile("" : "+v"(v));
-                b[t][ni] = bit_cast<half8_t>(v);
+                for (int ni = 0; ni < NI; ni++) zs[ni].y = (half_t)0.f;
             }
-        }
-    };
-    // Matrix instructions of the phase; those of its first half hide the dequantisation of the second.
-    auto compute = [&]() {
+        };
+        // the first half of the stage's weights, finished in front of the barrier that follows
+        auto unpack_first = [&]() {
+            fold();
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++)
-#pragma unroll
-            for (int t = H / 2; t < H; t++) asm volatile("" : "+v"(q[ni][t]));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int t = H / 2; t < H; t++) dequantise(t);
-#pragma unroll
-        for (int t = 0; t < H; t++)
-#pragma unroll
-            for (int mi = 0; mi < MI; mi++)
+            for (int t = 0; t < H / 2; t++) {
+                unpack(t);
 #pragma unroll
                 for (int ni = 0; ni < NI; ni++) {
-                    if constexpr (SUMS)
+                    u32x4_t v = bit_cast<u32x4_t>(b[t][ni]);
+                    asm volatile("" : "+v"(v));
+                    b[t][ni] = bit_cast<half8_t>(v);
+                }
+            }
+        };
+        // Matrix instructions of the stage; those of its first half hide the unpacking of the second.
+        auto compute = [&]() {
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                for (int t = H / 2; t < H; t++) asm volatile("" : "+v"(q[ni][t]));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = H / 2; t < H; t++) unpack(t);
+#pragma unroll
+            for (int t = 0; t < H; t++)
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                    for (int ni = 0; ni < NI; ni++)
                         part_sum[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
                             a[t][mi], b[t][ni], t == 0 ? (float16_t){} : part_sum[mi][ni], 0, 0, 0);
-                    else
-                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t][mi], b[t][ni], acc[mi][ni], 0, 0, 0);
-                }
-        if constexpr (SUMS) {
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) part_scale[ni] = (float)zs[ni].y;
-        }
-        constexpr int MF = H / 2 * MI * NI, VA = ((SUMS ? 10 : 14) * NI * (H / 2) + MF - 1) / MF;
+            constexpr int MF = H / 2 * MI * NI, VA = (10 * NI * (H / 2) + MF - 1) / MF;
 #pragma unroll
-        for (int i = 0; i < MF; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x2, VA, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x8, MF, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    if (it0 < it1) {
-#pragma unroll
-        for (int s = 0; s < ST - 1; s++)
-            if (it0 + s < it1) issue_any(it0 + s, s);
-        if (it0 + ST - 1 <= it1)
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        using H0 = std::integral_constant<int, 0>;
-        using H1 = std::integral_constant<int, PH - 1>;
-        // Stage it + 1 has landed: all but the loads of the younger stages are done.
-        auto landed_full = []() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory"); };
-        auto landed_all = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-        auto turn = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-        int c = 0, cp = ST - 1, it = it0;
-        auto next = [&]() {
-            cp = c;
-            c = c == ST - 1 ? 0 : c + 1;
+            for (int i = 0; i < MF; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, VA, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x8, MF, 0);
+            __builtin_amdgcn_sched_barrier(0);
         };
-        const int full = it1 - (ST - 1);  // stages below it still have a stage to request
-        // Both branches pass the same barriers, two per phase: waves 0..3 fetch phase p + 1 while waves 4..7 compute
-        // phase p.  A stage's first fetch also requests stage it + ST - 1 into the slot of stage it - 1, which both
-        // groups have read by then.
-        if (wave < 4) {
-            if (it < full) {
-                fetch(it, 0, H0{});
-                issue_any(it + ST - 1, ST - 1);
-                dequantise_first();
+        if (it0 < it1) {
+#pragma unroll
+            for (int s = 0; s < ST - 1; s++)
+                if (it0 + s < it1) issue_any(it0 + s, s);
+            // Stage it + 1 has landed: all but the loads of the younger stages are done.
+            auto landed_full = []() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory"); };
+            auto landed_all = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+            auto turn = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+            if (it0 + ST - 1 <= it1)
+                landed_full();
+            else
+                landed_all();
+            int c = 0, cp = ST - 1, it = it0;
+            auto next = [&]() {
+                cp = c;
+                c = c == ST - 1 ? 0 : c + 1;
+            };
+            const int full = it1 - (ST - 1);  // stages below it still have a stage to request
+            // Both branches pass the same barriers, two per stage: waves 0..3 fetch stage it + 1 while waves 4..7 compute
+            // stage it.  A fetch also requests stage it + ST - 1 into the slot of stage it - 1, which both groups have
+            // read by then.
+            if (wave < 4) {
+                fetch(0);
+                if (it < full)
+                    issue_any(it + ST - 1, ST - 1);
+                else
+                    clip(it);
+                unpack_first();
+                turn();
+                for (; it + 1 < full; it++) {
+                    compute();
+                    landed_full();
+                    next();
+                    fetch(c);
+                    issue_any(it + ST, cp);
+                    unpack_first();
+                    turn();
+                }
+                for (; it < it1; it++) {
+                    compute();
+                    landed_all();
+                    next();
+                    if (it + 1 < it1) {
+                        fetch(c);
+                        clip(it + 1);
+                        unpack_first();
+                    }
+                    turn();
+                }
             } else {
-                fetch(it, 0, H0{});
-                clip(it);
-                dequantise_first();
-            }
-            turn();
-            for (; it + 1 < full; it++) {
-                compute();
-                if constexpr (PH == 2) {
-                    turn();
-                    fetch(it, c, H1{});
-                    dequantise_first();
-                    turn();
-                    compute();
-                }
-                landed_full();
-                next();
-                fetch(it + 1, c, H0{});
-                issue_any(it + ST, cp);
-                dequantise_first();
                 turn();
-            }
-            for (; it < it1; it++) {
-                compute();
-                if constexpr (PH == 2) {
+                for (; it < full; it++) {
+                    fetch(c);
+                    issue_any(it + ST - 1, cp);
+                    unpack_first();
+                    landed_full();
+                    compute();
+                    next();
                     turn();
-                    fetch(it, c, H1{});
+                }
+                for (; it < it1; it++) {
+                    fetch(c);
                     clip(it);
-                    dequantise_first();
-                    turn();
+                    unpack_first();
+                    landed_all();
                     compute();
+                    next();
+                    turn();
                 }
-                landed_all();
-                next();
-                if (it + 1 < it1) {
-                    fetch(it + 1, c, H0{});
-                    clip(it + 1);
-                    dequantise_first();
-                }
-                turn();
             }
-        } else {
-            turn();
-            for (; it < full; it++) {
-                fetch(it, c, H0{});
-                issue_any(it + ST - 1, cp);
-                dequantise_first();
-                if constexpr (PH == 2) {
-                    turn();
-                    compute();
-                    turn();
-                    fetch(it, c, H1{});
-                    dequantise_first();
-                }
-                landed_full();
-                compute();
-                next();
-                turn();
-            }
-            for (; it < it1; it++) {
-                fetch(it, c, H0{});
-                clip(it);
-                dequantise_first();
-                if constexpr (PH == 2) {
-                    turn();
-                    compute();
-                    turn();
-                    fetch(it, c, H1{});
-                    clip(it);
-                    dequantise_first();
-                }
-                landed_all();
-                compute();
-                next();
-                turn();
-            }
+            fold();
         }
-        fold();
+    }
+
+    if constexpr (WK == 1) {
+        if (ks == 1) {
+            // No sums to add: every wave turns its own half slices (16 rows) row-major through a region of its own, two in
+            // turn, so that nothing waits for another wave.
+            constexpr int HC = 32 * NI;               // columns of a wave
+            constexpr int CH = HC / 8, RP = 64 / CH;  // chunks of a row, rows per pass
+            static_assert(S::NW * 2 * 16 * HC * 4 <= S::LDS && 16 % RP == 0, "fits");
+            float* own = reinterpret_cast<float*>(lds) + wave * (2 * 16 * HC);
+            float v[2][16 / RP][8];
+            auto turn_over = [&](int hs) __attribute__((always_inline)) {
+                float* o = own + (hs & 1) * (16 * HC);
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        o[(8 * (e >> 2) + 4 * lc + (e & 3)) * HC + 32 * ni + ln] = acc[hs >> 1][ni][8 * (hs & 1) + e];
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int g = 0; g < 16 / RP; g++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[hs & 1][g][e] = o[(g * RP + lane / CH) * HC + (lane % CH) * 8 + e];
+                asm volatile("" ::: "memory");
+            };
+            const int n = n0 + wn * HC + (lane % CH) * 8;
+            __syncthreads();
+            turn_over(0);
+#pragma unroll
+            for (int hs = 0; hs < 2 * MI; hs++) {
+                if (hs + 1 < 2 * MI) turn_over(hs + 1);
+#pragma unroll
+                for (int g = 0; g < 16 / RP; g++) {
+                    const int m = m0 + wm * (32 * MI) + 16 * hs + g * RP + lane / CH;
+                    if (m < M && n < N) finish_cols<8>(v[hs & 1][g], Y, m, n, N, epi);
+                }
+            }
+            return;
+        }
     }
 
     // The K groups' sums meet in LDS, one 32-row slice of every row group at a time, and leave row-major, EV consecutive
@@ -532,26 +712,32 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         const int n = n0 + cc * EV;
         if (m < M && n < N) finish_cols<EV>(v, Y, m, n, N, epi);
     };
+    constexpr int SL = S::LDS / S::TAIL < MI ? S::LDS / S::TAIL : MI;  // slices at once
+    constexpr int SF = S::TAIL / 4;
 #pragma unroll
     for (int mi = 0; mi < MI; mi++) {
-        __syncthreads();
+        if (mi % SL == 0) {
+            __syncthreads();
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++)
+            for (int sl = 0; sl < SL && mi + sl < MI; sl++)
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                red[((kg * WM + wm) * 32 + 8 * (v >> 2) + 4 * lc + (v & 3)) * BN + wcol + 32 * ni] = acc[mi][ni][v];
-        __syncthreads();
+                for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++)
+                        red[sl * SF + ((kg * WM + wm) * 32 + 8 * (v >> 2) + 4 * lc + (v & 3)) * BN + wcol + 32 * ni] = acc[mi + sl][ni][v];
+            __syncthreads();
+        }
 #pragma unroll
         for (int g = 0; g < G; g++) {
             const int ch = tid + g * S::NT;
             const int r = ch / CPR, cc = ch % CPR;  // r: row of the WM * 32 of this slice
             float v[EV];
 #pragma unroll
-            for (int e = 0; e < EV; e++) v[e] = red[r * BN + cc * EV + e];
+            for (int e = 0; e < EV; e++) v[e] = red[mi % SL * SF + r * BN + cc * EV + e];
 #pragma unroll
             for (int q = 1; q < WK; q++)
 #pragma unroll
-                for (int e = 0; e < EV; e++) v[e] += red[(q * WM * 32 + r) * BN + cc * EV + e];
+                for (int e = 0; e < EV; e++) v[e] += red[mi % SL * SF + (q * WM * 32 + r) * BN + cc * EV + e];
             if (ks == 1) {
                 finish(mi, g, v);
             } else {
@@ -625,7 +811,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     X_(1, 1, 2, 1, 1, 8, 3) X_(2, 1, 2, 1, 2, 4, 4) X_(3, 2, 2, 1, 2, 4, 3) X_(5, 2, 2, 1, 4, 2, 4)
 #define SQ_RING_SHAPES(X_)                                                                               \
     SQ_RING_LOW_SHAPES(X_) X_(4, 3, 1, 1, 4, 2, 4) X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3)        \
-        X_(8, 4, 2, 1, 4, 2, 3) X_(9, 4, 2, 2, 4, 1, 3)
+        X_(8, 4, 2, 1, 4, 2, 3) X_(9, 8, 2, 1, 4, 1, 3)
 
 template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
 static hipError_t launch_shape(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int nfull,
@@ -644,8 +830,11 @@ static hipError_t launch_shape(const void* x, const void* w, const void* zs, voi
 // What a shape costs, in us: a workgroup takes `step0 + step1 * a` per stage of K and `fixed` besides (first loads, sums,
 // stores), a = the share of the 256 CUs that its round keeps busy (memory and clock are shared); a K split adds the
 // exchange of the partial tiles, `ex0 + ex1 * parts + exmb` per MB of them.  One workgroup fills a CU.  Least-squares
-// fits to 9000 timings of 18 weights (3072 x 1024 .. 28672 x 8192) x 23 token counts (12 .. 4096) x all shapes and
-// splits: rms error 5..7 %, the choice within 0.5 % of the best in the geometric mean, 11 % at worst.
+// fits: tiles of 32 rows to 9000 timings of 18 weights (3072 x 1024 .. 28672 x 8192) x 23 token counts (12 .. 4096), the
+// others, with the loop in step, to 4400 timings of 14 weights (3072 x 1024 .. 24576 x 8192) x 19 token counts (20 ..
+// 4096), all shapes and splits: rms error 3..7 %, the choice within 0.7 % of the best in the geometric mean (1.8 % with the
+// constants of the alternating loop, which left the 128 x 128 tiles out: 224 tokens x 15360x5120 52 where they take 43),
+// 17 % at worst (80 tokens x 4096x16384).
 struct RingTile {
     int bm, bn, ks;
     float fixed, step0, step1, ex0, ex1, exmb;
@@ -653,13 +842,19 @@ struct RingTile {
 static const RingTile kRingTiles[] = {
     {32, 64, 512, 1.723f, 0.829f, 0.160f, 0.301f, 0.226f, 0.861f},
     {32, 128, 256, 1.498f, 0.754f, 0.096f, 0.448f, 0.304f, 0.649f},
-    {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f},
-    {96, 128, 128, 2.993f, 0.625f, 0.206f, 0.534f, 0.521f, 0.308f},
-    {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f},
-    {96, 256, 128, 4.305f, 1.017f, 0.410f, 0.106f, 1.298f, 0.243f},
-    {128, 128, 128, 3.276f, 0.802f, 0.268f, 0.000f, 0.967f, 0.278f},
-    {128, 256, 128, 4.931f, 1.142f, 0.611f, 0.100f, 1.663f, 0.230f},
-    {256, 256, 64, 5.673f, 0.778f, 0.907f, 0.f, 0.f, 0.f},  // never split, see plan_ring
+    {64, 128, 256, 2.477f, 0.758f, 0.383f, 0.349f, 0.557f, 0.414f},
+    {96, 128, 128, 3.023f, 0.456f, 0.375f, 0.311f, 0.719f, 0.278f},
+    {64, 256, 128, 2.321f, 0.788f, 0.289f, 1.297f, 0.832f, 0.357f},
+    {96, 256, 128, 4.394f, 0.724f, 0.637f, 0.267f, 1.403f, 0.188f},
+    {128, 128, 128, 2.849f, 0.506f, 0.482f, 0.000f, 1.028f, 0.301f},
+    {128, 256, 128, 5.724f, 0.883f, 0.792f, 0.986f, 1.489f, 0.180f},
+    {256, 256, 64, 8.358f, 0.930f, 0.669f, 0.f, 0.f, 0.f},  // never split, see plan_ring
+};
+// The same with the scale on the sums (up to 64 tokens), where other constants hold: shapes 1..5, of which the fourth is
+// not built for it.
+static const RingTile kRingSumsTiles[] = {
+    kRingTiles[0], kRingTiles[1], {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f},
+    kRingTiles[3], {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f},
 };
 constexpr int RING_SHAPES = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
 #define X_(id, MI, NI, WM, WN, WK, ST)                                                                              \
@@ -681,12 +876,12 @@ static size_t ring_bytes(const RingPlan& p, int M, int N) {
 
 // The cheapest shape and K split whose partial tiles fit `ws_bytes`.  Where the tiles come in full rounds of 256 and a
 // rest, only the rest splits K.
-static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes) {
+static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes, bool sums) {
     RingPlan best{1, 0, 1};
     float best_us = 3.4e38f;
     const int rows32 = (M + 31) / 32 * 32;
     for (int s = 0; s < RING_SHAPES; s++) {
-        const RingTile& t = kRingTiles[s];
+        const RingTile& t = sums && s < 5 ? kRingSumsTiles[s] : kRingTiles[s];
         const int mt = (M + t.bm - 1) / t.bm;
         // a third of the matrix work would be padding; up to 64 rows the others are the ones with the scale on the sums
         if (t.bm > 64 && (M <= 64 || mt * t.bm * 2 > rows32 * 3)) continue;
@@ -721,7 +916,10 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes) {
 }
 
 size_t gemm_ring_workspace_bytes(int M, int N, int K) {
-    return gemm_ring_applies(M, N, K) ? ring_bytes(plan_ring(M, N, K, (size_t)64 << 20), M, N) : 0;
+    if (!gemm_ring_applies(M, N, K)) return 0;
+    const size_t b = ring_bytes(plan_ring(M, N, K, (size_t)64 << 20, false), M, N);
+    const size_t sums = M <= 64 ? ring_bytes(plan_ring(M, N, K, (size_t)64 << 20, true), M, N) : 0;
+    return b > sums ? b : sums;
 }
 
 // tune = 0 for the cost model's choice, else shape id | 0x10: only the tiles of the last, part-filled round of 256
@@ -732,7 +930,7 @@ hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* 
     if (!gemm_ring_applies(M, N, K)) return hipErrorInvalidValue;
     RingPlan p{tune & 0xF, 0, (tune >> 8) & 0xFF};
     if (p.shape == 0) {
-        p = plan_ring(M, N, K, ws ? ws_bytes : 0);
+        p = plan_ring(M, N, K, ws ? ws_bytes : 0, (tune & RING_SUMS) != 0);
     } else {
         if (p.shape > RING_SHAPES || p.ksplit > 8) return hipErrorInvalidValue;
         const RingTile& t = kRingTiles[p.shape - 1];

@@ -65,8 +65,29 @@ def test_ring_parity(capi, shape, m, n, k, g):
 
 @pytest.mark.parametrize("m,n,k,g", CASES + [(257, 264, 320, 64), (520, 136, 1056, 32)])
 def test_ring_parity_of_256_row_tiles(capi, m, n, k, g):
-    """Two rows of waves over the same weight columns: the second row of tiles full, ragged and absent."""
+    """Four waves of 256 x 64: the second row of tiles full, ragged and absent."""
     test_ring_parity(capi, 9, m, n, k, g)
+
+
+@pytest.mark.parametrize("shape,stage", [(1, 512), (2, 256), (3, 256), (4, 128), (5, 128), (6, 128), (7, 128), (8, 128), (9, 64)])
+@pytest.mark.parametrize("short", [0, 32])
+def test_ring_every_count_of_stages(capi, shape, stage, short):
+    """Fewer stages than the ring has slots, as many, one and several more; the last one whole and ending early."""
+    m, n, g = 37, 136, 32
+    ws = torch.zeros(65536 + (8 << 20), dtype=torch.uint8, device=DEV)
+    for stages in range(1, 8):
+        k = stage * stages - short
+        d = orc.synth_linear(n, k, g, seed=k)
+        x = orc.synth_x(m, k, seed=shape)
+        x64, w64 = x.astype(np.float64), orc.dequant_l1(d["w_l1"], d["zs_l1"], g).astype(np.float64)
+        ref = x64 @ w64.T
+        # one rounding to fp16 and K fp32 additions, as above
+        bound = 2.0 ** -11 * np.abs(ref) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T) + 2.0 ** -24
+        w, zs, xd = to_dev(d["w_l1"]), to_dev(d["zs_l1"]), to_dev(x)
+        for parts in (1, 2) if stages > 1 else (1,):
+            y = capi.gemm_fused(xd, w, zs, n, k, g, algo=capi.SQ_ALGO_RING | ((shape | (parts << 8)) << 8), ws=ws)
+            got = y.cpu().numpy().astype(np.float64)
+            assert np.all(np.abs(got - ref) <= bound), (stages, parts, np.max(np.abs(got - ref) / bound))
 
 
 REST = 0x10  # tune word: only the tiles of the last round of 256 split K
