@@ -198,10 +198,12 @@ int sq_w4a16_gemm_fused(const void* x, const void* w, const void* zs, const void
                         int layout, int act, int algo, void* workspace, size_t workspace_bytes,
                         void* stream);
 
-/* Front half of a gated MLP: Y = silu(X * W_gate_hat^T) .* (X * W_up_hat^T), two launches: the up
- * projection into up_scratch (fp16 [M, N], caller-allocated, must not overlap y; holds the up
- * projection afterwards), then the gate projection, whose store applies SiLU to the fp32
- * accumulator and multiplies by up_scratch before the one rounding of Y.  Both weights are [N, K]
+/* Front half of a gated MLP: Y = silu(X * W_gate_hat^T) .* (X * W_up_hat^T).  Up to 16
+ * tokens two launches: the up projection into up_scratch (fp16 [M, N], caller-allocated, must not
+ * overlap y; holds the up projection afterwards), then the gate projection, whose store applies SiLU
+ * to the fp32 accumulator and multiplies by up_scratch before the one rounding of Y.  Where
+ * SQ_ALGO_RING is the automatic choice one launch, which multiplies the fp32 sums and stores the up
+ * projection beside Y.  Both weights are [N, K]
  * with their own zeros/scales; for a packed weight cat(W_gate, W_up) in layout L1 pass the two
  * row slices (w_up = w + N * K / 2 bytes, zs_up = zs + N * (K / g) * 4 bytes).  workspace as for
  * sq_w4a16_gemm_ws (may be NULL).  In the role of gemm_awq_silu_dot_ut, which the reference's
@@ -212,6 +214,12 @@ int sq_w4a16_gemm_silu_dot(const void* x, const void* w_gate, const void* zs_gat
                            const void* zs_up, void* y, void* up_scratch, int M, int N, int K,
                            int group_size, int layout, void* workspace, size_t workspace_bytes,
                            void* stream);
+
+/* The same without up_scratch, in one launch; SQ_ERR_BAD_ALGO, with nothing launched, where two would
+ * be needed.  algo: SQ_ALGO_AUTO, or SQ_ALGO_RING with a tuning word (of the 2 N columns of both). */
+int sq_w4a16_gemm_silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, const void* w_up,
+                               const void* zs_up, void* y, int M, int N, int K, int group_size, int layout,
+                               int algo, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Up to SQ_SEQUENCE_MAX decode linears (1..4 tokens) with one call:
  *     for l in 0 .. count-1:  y_l = act_l(x_l * W_hat_l^T + bias_l) + residual_l

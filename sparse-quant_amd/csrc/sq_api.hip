@@ -697,12 +697,55 @@ int sq_w4a16_gemm_fused(const void* x, const void* w, const void* zs, const void
     return gemm_dispatch(x, w, zs, y, M, N, K, group_size, layout, algo, epi, workspace, workspace_bytes, stream);
 }
 
+// Both products in one launch where the ring kernel is the choice for each and no measured choice of the shape says
+// otherwise; SQ_ERR_BAD_ALGO, with nothing launched, where it is not.
+static int silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, const void* w_up, const void* zs_up, void* y,
+                        void* up, int M, int N, int K, int group_size, int layout, int algo, void* workspace,
+                        size_t workspace_bytes, void* stream) {
+    if (M < 0) return SQ_ERR_BAD_SHAPE;
+    const int rc = check_weight(N, K, group_size, layout);
+    if (rc != SQ_OK) return rc;
+    if (layout != SQ_LAYOUT_L1) return SQ_ERR_BAD_LAYOUT;
+    if (M == 0) return SQ_OK;
+    if (!x || !w_gate || !zs_gate || !w_up || !zs_up || !y) return SQ_ERR_NULL_POINTER;
+    if (!aligned16(x) || !aligned16(w_gate) || !aligned16(zs_gate) || !aligned16(w_up) || !aligned16(zs_up) || !aligned16(y))
+        return SQ_ERR_MISALIGNED;
+    if (N > (1 << 29)) return SQ_ERR_BAD_ALGO;
+    const bool ws_ok = workspace && aligned16(workspace);
+    int tune = ring_tune(M, group_size);
+    if (algo == SQ_ALGO_AUTO) {
+        if (M <= 16) return SQ_ERR_BAD_ALGO;
+        if (g_tuned_count.load(std::memory_order_relaxed) > 0 &&
+            tuned_lookup(M, N, K, group_size, full_workspace(workspace, workspace_bytes, M, N, K)) != 0)
+            return SQ_ERR_BAD_ALGO;
+        if (builtin_choice(M, N, K, group_size, ws_ok) != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
+    } else {
+        if ((algo & 0xFF) != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
+        tune = (algo >> 8) & 0xFFFF;
+    }
+    const hipError_t e = sq::launch_gemm_ring_pair(x, w_gate, zs_gate, w_up, zs_up, y, up, ws_ok ? workspace : nullptr,
+                                                   workspace_bytes, M, N, K, group_size, tune, static_cast<hipStream_t>(stream));
+    return e == hipErrorInvalidValue ? SQ_ERR_BAD_ALGO : launch_code(e);
+}
+
+int sq_w4a16_gemm_silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, const void* w_up, const void* zs_up,
+                               void* y, int M, int N, int K, int group_size, int layout, int algo, void* workspace,
+                               size_t workspace_bytes, void* stream) {
+    return silu_dot_one(x, w_gate, zs_gate, w_up, zs_up, y, nullptr, M, N, K, group_size, layout, algo, workspace,
+                        workspace_bytes, stream);
+}
+
 int sq_w4a16_gemm_silu_dot(const void* x, const void* w_gate, const void* zs_gate, const void* w_up, const void* zs_up,
                            void* y, void* up_scratch, int M, int N, int K, int group_size, int layout, void* workspace,
                            size_t workspace_bytes, void* stream) {
     if (M > 0 && (!up_scratch || !w_up || !zs_up)) return SQ_ERR_NULL_POINTER;
     if (M > 0 && !aligned16(up_scratch)) return SQ_ERR_MISALIGNED;
     if (M > 0 && up_scratch == y) return SQ_ERR_BAD_SHAPE;
+    if (M > 16) {
+        const int rc = silu_dot_one(x, w_gate, zs_gate, w_up, zs_up, y, up_scratch, M, N, K, group_size, layout, SQ_ALGO_AUTO,
+                                    workspace, workspace_bytes, stream);
+        if (rc != SQ_ERR_BAD_ALGO) return rc;
+    }
     // the up projection first, rounded to fp16 once; the gate projection multiplies it into its store
     const int rc = gemm_dispatch(x, w_up, zs_up, up_scratch, M, N, K, group_size, layout, SQ_ALGO_AUTO,
                                  sq::Epilogue{nullptr, nullptr, SQ_ACT_NONE}, workspace, workspace_bytes, stream);

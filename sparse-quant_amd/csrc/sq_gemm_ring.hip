@@ -138,6 +138,22 @@ __device__ __forceinline__ void finish_cols(float (&v)[EV], half_t* __restrict__
     *(hv_t*)(Y + idx) = h;
 }
 
+// silu(v[e]) * v[EO + e] for EO outputs; U (may be null) receives v[EO + e].
+template <int EO>
+__device__ __forceinline__ void finish_pair(const float (&v)[2 * EO], half_t* __restrict__ Y, half_t* __restrict__ U, int m, int n,
+                                            int N) {
+    typedef _Float16 hv_t __attribute__((ext_vector_type(EO)));
+    hv_t h;
+    if (U) {
+#pragma unroll
+        for (int e = 0; e < EO; e++) h[e] = (half_t)v[EO + e];
+        *(hv_t*)(U + (long)m * N + n) = h;
+    }
+#pragma unroll
+    for (int e = 0; e < EO; e++) h[e] = (half_t)(v[e] * __builtin_amdgcn_rcpf(1.f + __expf(-v[e])) * v[EO + e]);
+    *(hv_t*)(Y + (long)m * N + n) = h;
+}
+
 // Direct loads by part of a wave's lanes (mask): the instruction is issued whatever the mask, so that the counted waits
 // hold for every wave.  The wave runs with all lanes active around it.
 __device__ __forceinline__ void load_to_lds_x4_masked(const void* base, uint32_t lane_byte, uint32_t lds_byte, uint64_t mask) {
@@ -158,10 +174,16 @@ __device__ __forceinline__ void load_to_lds_x1_masked(const void* base, uint32_t
 // 32 tokens 12288x4096 11.96 / 12.03, 5120x13696 16.3 / 16.4; 48 tokens 12288x4096 16.4 / 16.1, 5120x13696 20.6 / 21.1;
 // 64 tokens 4096x11008 16.6 / 16.6, 15360x5120 20.4 / 21.0.  Its loop keeps the two alternating groups of waves (0..3 fetch
 // phase p + 1 while 4..7 compute phase p): in step it would need a second set of sums.
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
+//
+// PAIR: silu(X W^T) * (X W2^T), both weights [N, K], in one launch: half of a tile's columns are W's and half W2's, the same
+// outputs' in the same workgroup, so that the product is formed in the store and the tiles of both fill the chip's rounds
+// together (us, two launches / one: 11008x4096 at 32 tokens 25.1 / 19.5, at 333 and group size 64 101 / 80.0; 13696x5120 at
+// 100 62.7 / 43.4; 11008x4096 at 2048 396 / 329).  Nothing is rounded between the products.
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool PAIR>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4))) void gemm_ring_kernel(
     const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS, const half_t* __restrict__ X, half_t* __restrict__ Y,
-    int M, int N, int K, int mtiles, int tiles, int nfull, int ksplit, Epilogue epi, float* part, unsigned* counters) {
+    int M, int N, int K, int mtiles, int tiles, int nfull, int ksplit, Epilogue epi, float* part, unsigned* counters,
+    const uint8_t* __restrict__ W2, const half2_t* __restrict__ ZS2, half_t* __restrict__ U) {
     using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
     constexpr int BM = S::BM, BN = S::BN, KS = S::KS, SB = S::SB, XI = S::XI, WI = S::WI, ZI = S::ZI, ZL = S::ZL, PER = S::PER, P = S::P;
     constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = S::XB + S::WB;
@@ -202,7 +224,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     }
     const int nt = tile / mtiles;
     const int m0 = (tile - nt * mtiles) * BM;
-    const int n0 = nt * BN;
+    // PAIR: rows 0 .. BN / 2 - 1 of the stage's weights are W's, the others W2's, for outputs n0 .. n0 + BN / 2 - 1.
+    constexpr int BO = PAIR ? BN / 2 : BN;
+    const int n0 = nt * BO;
+    const bool second = PAIR && wave >= S::NW / 2;  // this wave loads W2
+    const uint8_t* const Wl = second ? W2 : W;
+    const half2_t* const Zl = second ? ZS2 : ZS;
     const int groups = K >> GS;
     const int nst = (K + KS - 1) / KS;
     const int spz = (nst + ks - 1) / ks;
@@ -228,12 +255,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
     for (int j = 0; j < WI; j++) {
         const int R = (wave * WI + j) * (32 / WK) + lane / (2 * WK);
-        wlane[j] = (uint32_t)((long)imin(n0 + R, N - 1) * (K >> 1)) + (((lane % (2 * WK)) ^ wswz<WK>(R)) * 16);
+        wlane[j] = (uint32_t)((long)imin(n0 + R % BO, N - 1) * (K >> 1)) + (((lane % (2 * WK)) ^ wswz<WK>(R)) * 16);
     }
 #pragma unroll
     for (int j = 0; j < ZI; j++) {
         const int d = (wave * ZI + j) * ZL + (lane & (ZL - 1));
-        zlane[j] = (uint32_t)((long)imin(n0 + d / P, N - 1) * groups * 4) + (d % P) * 4;
+        zlane[j] = (uint32_t)((long)imin(n0 + d / P % BO, N - 1) * groups * 4) + (d % P) * 4;
     }
     // Loads of stage it into slot c.  EDGE: the last stage of a K that ends inside it; weights that are missing re-read
     // the end of the row (and meet a scale of 0), activations are zeros in LDS (an infinity at the end of a row, re-read,
@@ -243,8 +270,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         constexpr bool EDGE = decltype(EDGE_)::value;
         const int k0 = it * KS, left = K - k0;
         const uint8_t* xb = (const uint8_t*)X + (long)k0 * 2;
-        const uint8_t* wb = W + (k0 >> 1);
-        const uint8_t* zb = (const uint8_t*)ZS + (k0 >> GS) * 4;
+        const uint8_t* wb = Wl + (k0 >> 1);
+        const uint8_t* zb = (const uint8_t*)Zl + (k0 >> GS) * 4;
         const uint32_t l0 = lds0 + c * SB;
 #pragma unroll
         for (int j = 0; j < ZI; j++) {
@@ -292,7 +319,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     int xoff[4];
 #pragma unroll
     for (int t = 0; t < 4; t++) xoff[t] = xrow + (((4 * lc + t) ^ swz8(ln)) * 16);
-    const int wcol = wn * 32 * NI + ln;
+    // Row of the stage's weights (and column of the sums on their way out) of the wave's first 32 columns; CN to the next 32.
+    constexpr int CN = PAIR ? BO : 32;
+    const int wcol = (PAIR ? (NI == 2 ? 32 * wn : (wn & 1) * BO + 32 * (wn >> 1)) : wn * 32 * NI) + ln;
+    static_assert(!PAIR || NI == 2 || (NI == 1 && WN % 2 == 0), "both weights of an output column in one wave or in neighbours");
     const int woff = W_OFF + wcol * (32 * WK) + (((2 * kg + lc) ^ wswz<WK>(ln)) * 16);
     const int zoff = Z_OFF + (wcol * P + ((64 * kg + (GS == 5 ? 32 * lc : 0)) >> GS)) * 4;
 
@@ -314,8 +344,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             const uint8_t* l = lds + c * SB;
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) {
-                zn[ni] = *(const half2_t*)(l + zoff + ni * (32 * P * 4));
-                const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (32 * 32 * WK));
+                zn[ni] = *(const half2_t*)(l + zoff + ni * (CN * P * 4));
+                const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (CN * 32 * WK));
 #pragma unroll
                 for (int t = 0; t < 4; t++) qn[ni][t] = v[t];
             }
@@ -523,8 +553,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             const uint8_t* l = lds + c * SB;
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) {
-                zs[ni] = *(const half2_t*)(l + zoff + ni * (32 * P * 4));
-                const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (32 * 32 * WK));
+                zs[ni] = *(const half2_t*)(l + zoff + ni * (CN * P * 4));
+                const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (CN * 32 * WK));
 #pragma unroll
                 for (int t = 0; t < 4; t++) q[ni][t] = v[t];
             }
@@ -660,11 +690,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         if (ks == 1) {
             // No sums to add: every wave turns its own half slices (16 rows) row-major through a region of its own, two in
             // turn, so that nothing waits for another wave.
-            constexpr int HC = 32 * NI;               // columns of a wave
-            constexpr int CH = HC / 8, RP = 64 / CH;  // chunks of a row, rows per pass
+            constexpr int HC = 32 * NI;                             // columns of a wave, PAIR: of 32 outputs
+            constexpr int CH = HC / (PAIR ? 16 : 8), RP = 64 / CH;  // chunks of a row, rows per pass
+            constexpr int EO = PAIR ? 16 : 8;                       // sums of a chunk
             static_assert(S::NW * 2 * 16 * HC * 4 <= S::LDS && 16 % RP == 0, "fits");
             float* own = reinterpret_cast<float*>(lds) + wave * (2 * 16 * HC);
-            float v[2][16 / RP][8];
+            float v[2][16 / RP][EO];
             auto turn_over = [&](int hs) __attribute__((always_inline)) {
                 float* o = own + (hs & 1) * (16 * HC);
 #pragma unroll
@@ -676,10 +707,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
                 for (int g = 0; g < 16 / RP; g++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++) v[hs & 1][g][e] = o[(g * RP + lane / CH) * HC + (lane % CH) * 8 + e];
+                    for (int e = 0; e < EO; e++)
+                        v[hs & 1][g][e] = o[(g * RP + lane / CH) * HC + (lane % CH) * 8 + (e & 7) + (e >> 3) * 32];
                 asm volatile("" ::: "memory");
             };
-            const int n = n0 + wn * HC + (lane % CH) * 8;
+            const int n = n0 + wn * (PAIR ? 32 : HC) + (lane % CH) * 8;
             __syncthreads();
             turn_over(0);
 #pragma unroll
@@ -688,7 +720,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
                 for (int g = 0; g < 16 / RP; g++) {
                     const int m = m0 + wm * (32 * MI) + 16 * hs + g * RP + lane / CH;
-                    if (m < M && n < N) finish_cols<8>(v[hs & 1][g], Y, m, n, N, epi);
+                    if (m < M && n < N) {
+                        if constexpr (PAIR)
+                            finish_pair<8>(v[hs & 1][g], Y, U, m, n, N);
+                        else
+                            finish_cols<8>(v[hs & 1][g], Y, m, n, N, epi);
+                    }
                 }
             }
             return;
@@ -698,9 +735,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     // The K groups' sums meet in LDS, one 32-row slice of every row group at a time, and leave row-major, EV consecutive
     // columns per thread.
     constexpr int PT = 16 * NI / WK;     // sums per thread and slice
-    constexpr int EV = PT < 8 ? PT : 8;
+    constexpr int EO = PAIR ? (PT < 16 ? PT / 2 : 8) : (PT < 8 ? PT : 8);  // outputs of a chunk
+    constexpr int EV = PAIR ? 2 * EO : EO;                                 // its sums
     constexpr int G = PT / EV;
-    constexpr int CPR = BN / EV;         // column chunks per row
+    constexpr int CPR = BN / EV;         // chunks per row
     constexpr int L = MI * PT / 4;       // float4 per thread
     float* red = reinterpret_cast<float*>(lds);
     const long tsz = (long)BM * BN;
@@ -709,9 +747,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         const int ch = tid + g * S::NT;
         const int r = ch / CPR, cc = ch % CPR;
         const int m = m0 + (r >> 5) * (32 * MI) + 32 * mi + (r & 31);
-        const int n = n0 + cc * EV;
-        if (m < M && n < N) finish_cols<EV>(v, Y, m, n, N, epi);
+        const int n = n0 + cc * EO;
+        if (m < M && n < N) {
+            if constexpr (PAIR)
+                finish_pair<EO>(v, Y, U, m, n, N);
+            else
+                finish_cols<EV>(v, Y, m, n, N, epi);
+        }
     };
+    auto column = [](int cc, int e) __attribute__((always_inline)) { return cc * EO + e % EO + (e / EO) * BO; };
     constexpr int SL = S::LDS / S::TAIL < MI ? S::LDS / S::TAIL : MI;  // slices at once
     constexpr int SF = S::TAIL / 4;
 #pragma unroll
@@ -724,7 +768,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                 for (int ni = 0; ni < NI; ni++)
 #pragma unroll
                     for (int v = 0; v < 16; v++)
-                        red[sl * SF + ((kg * WM + wm) * 32 + 8 * (v >> 2) + 4 * lc + (v & 3)) * BN + wcol + 32 * ni] = acc[mi + sl][ni][v];
+                        red[sl * SF + ((kg * WM + wm) * 32 + 8 * (v >> 2) + 4 * lc + (v & 3)) * BN + wcol + CN * ni] = acc[mi + sl][ni][v];
             __syncthreads();
         }
 #pragma unroll
@@ -733,11 +777,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             const int r = ch / CPR, cc = ch % CPR;  // r: row of the WM * 32 of this slice
             float v[EV];
 #pragma unroll
-            for (int e = 0; e < EV; e++) v[e] = red[mi % SL * SF + r * BN + cc * EV + e];
+            for (int e = 0; e < EV; e++) v[e] = red[mi % SL * SF + r * BN + column(cc, e)];
 #pragma unroll
             for (int q = 1; q < WK; q++)
 #pragma unroll
-                for (int e = 0; e < EV; e++) v[e] += red[mi % SL * SF + (q * WM * 32 + r) * BN + cc * EV + e];
+                for (int e = 0; e < EV; e++) v[e] += red[mi % SL * SF + (q * WM * 32 + r) * BN + column(cc, e)];
             if (ks == 1) {
                 finish(mi, g, v);
             } else {
@@ -813,17 +857,19 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     SQ_RING_LOW_SHAPES(X_) X_(4, 3, 1, 1, 4, 2, 4) X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3)        \
         X_(8, 4, 2, 1, 4, 2, 3) X_(9, 8, 2, 1, 4, 1, 3)
 
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
-static hipError_t launch_shape(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int nfull,
-                               int ksplit, Epilogue epi, void* ws, hipStream_t st) {
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool PAIR>
+static hipError_t launch_shape(const void* x, const void* w, const void* zs, const void* w2, const void* zs2, void* y, void* u, int M,
+                               int N, int K, int nfull, int ksplit, Epilogue epi, void* ws, hipStream_t st) {
     using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
     const int mt = (M + S::BM - 1) / S::BM;
-    const int tiles = mt * ((N + S::BN - 1) / S::BN);
+    constexpr int BO = PAIR ? S::BN / 2 : S::BN;
+    const int tiles = mt * ((N + BO - 1) / BO);
     if (ksplit == 1) nfull = tiles;
     const int grid = ksplit == 1 ? (tiles + 7) / 8 * 8 : nfull + ((tiles - nfull) * ksplit + 7) / 8 * 8;
-    hipLaunchKernelGGL((gemm_ring_kernel<MI, NI, WM, WN, WK, GS, ST, SUMS>), dim3(grid), dim3(S::NT), 0, st, (const uint8_t*)w,
+    hipLaunchKernelGGL((gemm_ring_kernel<MI, NI, WM, WN, WK, GS, ST, SUMS, PAIR>), dim3(grid), dim3(S::NT), 0, st, (const uint8_t*)w,
                        (const half2_t*)zs, (const half_t*)x, (half_t*)y, M, N, K, mt, tiles, nfull, ksplit, epi,
-                       ws ? (float*)((char*)ws + RING_COUNTER_BYTES) : nullptr, (unsigned*)ws);
+                       ws ? (float*)((char*)ws + RING_COUNTER_BYTES) : nullptr, (unsigned*)ws, (const uint8_t*)w2,
+                       (const half2_t*)zs2, (half_t*)u);
     return hipGetLastError();
 }
 
@@ -925,28 +971,31 @@ size_t gemm_ring_workspace_bytes(int M, int N, int K) {
 // tune = 0 for the cost model's choice, else shape id | 0x10: only the tiles of the last, part-filled round of 256
 // workgroups split K | K split << 8; RING_SUMS: the scale on the sums (also with the model's choice; group size 128, tiles
 // of 32 and 64 rows).  hipErrorInvalidValue: not applicable (or the workspace is missing or too small).
-hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,
-                            int K, int g, int tune, Epilogue epi, hipStream_t st) {
-    if (!gemm_ring_applies(M, N, K)) return hipErrorInvalidValue;
+// PAIR: N outputs of two weights, planned as 2 N columns.
+template <bool PAIR>
+static hipError_t launch_ring(const void* x, const void* w, const void* zs, const void* w2, const void* zs2, void* y, void* u, void* ws,
+                              size_t ws_bytes, int M, int N, int K, int g, int tune, Epilogue epi, hipStream_t st) {
+    const int cols = PAIR ? 2 * N : N;
+    if ((PAIR && N > (1 << 29)) || !gemm_ring_applies(M, cols, K)) return hipErrorInvalidValue;
     RingPlan p{tune & 0xF, 0, (tune >> 8) & 0xFF};
     if (p.shape == 0) {
-        p = plan_ring(M, N, K, ws ? ws_bytes : 0, (tune & RING_SUMS) != 0);
+        p = plan_ring(M, cols, K, ws ? ws_bytes : 0, (tune & RING_SUMS) != 0);
     } else {
         if (p.shape > RING_SHAPES || p.ksplit > 8) return hipErrorInvalidValue;
         const RingTile& t = kRingTiles[p.shape - 1];
-        const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const long tiles = (long)((M + t.bm - 1) / t.bm) * ((cols + t.bn - 1) / t.bn);
         if (tiles > (1L << 24)) return hipErrorInvalidValue;
         if (p.ksplit < 1) p.ksplit = 1;
         if (tune & 0x10) p.nfull = (int)(tiles / 256 * 256);
         if (p.ksplit > 1) {
-            const size_t need = ring_bytes(p, M, N);
+            const size_t need = ring_bytes(p, M, cols);
             if (tiles == p.nfull || tiles - p.nfull > (long)(RING_COUNTER_BYTES / 4) || p.ksplit > (K + t.ks - 1) / t.ks ||
                 need - RING_COUNTER_BYTES >= 0x7FFFFFFFu || !ws || ws_bytes < need)
                 return hipErrorInvalidValue;
         }
     }
 #define SQ_RING_LAUNCH(MI, NI, WM, WN, WK, GS, ST, SUMS) \
-    launch_shape<MI, NI, WM, WN, WK, GS, ST, SUMS>(x, w, zs, y, M, N, K, p.nfull, p.ksplit, epi, ws, st)
+    launch_shape<MI, NI, WM, WN, WK, GS, ST, SUMS, PAIR>(x, w, zs, w2, zs2, y, u, M, N, K, p.nfull, p.ksplit, epi, ws, st)
     if (tune & RING_SUMS) {
         if (g != 128) return hipErrorInvalidValue;
         switch (p.shape) {
@@ -969,6 +1018,17 @@ hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* 
     }
 #undef SQ_RING_LAUNCH
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,
+                            int K, int g, int tune, Epilogue epi, hipStream_t st) {
+    return launch_ring<false>(x, w, zs, nullptr, nullptr, y, nullptr, ws, ws_bytes, M, N, K, g, tune, epi, st);
+}
+
+hipError_t launch_gemm_ring_pair(const void* x, const void* w_gate, const void* zs_gate, const void* w_up, const void* zs_up,
+                                 void* y, void* up, void* ws, size_t ws_bytes, int M, int N, int K, int g, int tune, hipStream_t st) {
+    return launch_ring<true>(x, w_gate, zs_gate, w_up, zs_up, y, up, ws, ws_bytes, M, N, K, g, tune, Epilogue{nullptr, nullptr, 0},
+                             st);
 }
 
 }  // namespace sq

@@ -101,6 +101,11 @@ size_t gemm_ring_workspace_bytes(int M, int N, int K);
 hipError_t launch_gemm_ring(const void* x, const void* w, const void* zs, void* y, void* ws, size_t ws_bytes, int M, int N,
                             int K, int g, int tune, Epilogue epi, hipStream_t st);
 
+// silu(x w_gate^T) * (x w_up^T), both weights [N, K], in one launch of the same kernel, planned as 2 N columns; up (may be
+// null) receives x w_up^T.
+hipError_t launch_gemm_ring_pair(const void* x, const void* w_gate, const void* zs_gate, const void* w_up, const void* zs_up,
+                                 void* y, void* up, void* ws, size_t ws_bytes, int M, int N, int K, int g, int tune, hipStream_t st);
+
 // sq_gemm2.hip: software-pipelined 128 x 256 tile variant for M > 64.
 hipError_t launch_gemm_pipe(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int g,
                             int variant, Epilogue epi, hipStream_t st);

@@ -30,6 +30,7 @@ SIGNATURES = {
     "sq_w4a16_gemm_static_ws": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp]),
     "sq_w4a16_gemm_fused": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t, _vp]),
     "sq_w4a16_gemm_silu_dot": (_i, [_vp] * 7 + [_i] * 5 + [_vp, ctypes.c_size_t, _vp]),
+    "sq_w4a16_gemm_silu_dot_one": (_i, [_vp] * 6 + [_i] * 6 + [_vp, ctypes.c_size_t, _vp]),
     "sq_w4a16_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i]),
     "sq_w4a16_autotune": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t, _i, ctypes.c_size_t,
                                ctypes.c_size_t, _i, _vp, ctypes.POINTER(_i), ctypes.POINTER(ctypes.c_float),

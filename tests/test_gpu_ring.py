@@ -90,6 +90,49 @@ def test_ring_every_count_of_stages(capi, shape, stage, short):
             assert np.all(np.abs(got - ref) <= bound), (stages, parts, np.max(np.abs(got - ref) / bound))
 
 
+@pytest.mark.parametrize("m,n,k,g", [(17, 8, 128, 128), (33, 72, 640, 128), (70, 200, 960, 64), (300, 136, 416, 32),
+                                     (100, 1160, 384, 128)])
+def test_ring_gate_and_up_in_one_launch(capi, m, n, k, g):
+    """silu(gate) * up with both weights in every tile: outputs that end inside a tile's half, every shape, K split, and the
+    sums scaled; the up projection where it is asked for."""
+    d = [orc.synth_linear(n, k, g, seed=s) for s in (n, n + 1)]
+    x = orc.synth_x(m, k, seed=m)
+    x64 = x.astype(np.float64)
+    dev = [(to_dev(i["w_l1"]), to_dev(i["zs_l1"])) for i in d]
+    xd = to_dev(x)
+    ws = torch.zeros(65536 + (32 << 20), dtype=torch.uint8, device=DEV)
+    L, p = capi.lib(), lambda t: t.data_ptr()
+
+    def check(y, weights, what):
+        gate, up = (x64 @ w.T for w in weights)
+        s = 1 / (1 + np.exp(-gate))
+        ref = gate * s * up
+        # errors of the sums (K fp32 additions) through d silu <= 1.1 and the product, those of exp and rcp (4 ulp of
+        # fp32), one rounding to fp16
+        eg, eu = (k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w).T) for w in weights)
+        bound = (2.0 ** -11 + 2.0 ** -20) * np.abs(ref) + 1.1 * eg * np.abs(up) + np.abs(gate * s) * eu + eg * eu + 2.0 ** -24
+        err = np.abs(y.cpu().numpy().astype(np.float64) - ref)
+        assert np.all(err <= bound), (what, np.max(err / bound))
+
+    w_hat = [orc.dequant_l1(i["w_l1"], i["zs_l1"], g).astype(np.float64) for i in d]
+    for shape in range(1, 10):
+        for sums in (0, 0x20) if g == 128 and shape in (1, 2, 3, 5) else (0,):
+            for parts in (1, 2):
+                y = torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV)
+                rc = L.sq_w4a16_gemm_silu_dot_one(p(xd), *(p(t) for w in dev for t in w), p(y), m, n, k, g, capi.SQ_LAYOUT_L1,
+                                                  capi.SQ_ALGO_RING | ((shape | sums | (parts << 8)) << 8), p(ws), ws.numel(),
+                                                  capi._stream(None))
+                assert rc == 0 or (parts > 1 and rc == capi.SQ_ERR_BAD_ALGO)
+                if rc == 0:
+                    check(y, [real_weight(i, g) for i in d] if sums else w_hat, (shape, sums, parts))
+                assert capi.workspace_is_clean(ws)
+    y, up = capi.gemm_silu_dot(xd, *(t for w in dev for t in w), n, k, g)
+    scaled = g == 128 and m <= 64
+    check(y, [real_weight(i, g) for i in d] if scaled else w_hat, "automatic")
+    ref = x64 @ (real_weight(d[1], g) if scaled else w_hat[1]).T
+    assert np.all(np.abs(up.cpu().numpy() - ref) <= 2.0 ** -11 * np.abs(ref) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w_hat[1]).T) * 2 + 2.0 ** -24)
+
+
 REST = 0x10  # tune word: only the tiles of the last round of 256 split K
 SUMS = 0x20  # tune word: the scale on the sums (shapes of 32 and 64 rows, group size 128)
 
