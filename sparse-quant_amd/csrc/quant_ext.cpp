@@ -341,13 +341,13 @@ at::Tensor gemm_awq_silu_dot_ut(at::Tensor I, c10::optional<at::Tensor> W1, c10:
     size_t ws_bytes = 0;
     at::Tensor ws;
     if (rows > 2 && rows <= 1024) {
-        // (both weights share a launch from 17 tokens up)
+        // (both weights can share a launch)
         ws = workspace_for(I, stream, std::max(sq_w4a16_workspace_bytes((int)rows, N, (int)Kin),
-                                               rows > 16 && N < (1 << 29) ? sq_w4a16_workspace_bytes((int)rows, 2 * N, (int)Kin) : 0));
+                                               N < (1 << 29) ? sq_w4a16_workspace_bytes((int)rows, 2 * N, (int)Kin) : 0));
         ws_ptr = ws.data_ptr();
         ws_bytes = (size_t)ws.numel();
     }
-    if (rows > 16) {
+    {
         const int rc = sq_w4a16_gemm_silu_dot_one(I.data_ptr(), gate.first.data_ptr(), gate.second.data_ptr(), up.first.data_ptr(),
                                                   up.second.data_ptr(), O.data_ptr(), (int)rows, N, (int)Kin, group_size,
                                                   SQ_LAYOUT_L1, SQ_ALGO_AUTO, ws_ptr, ws_bytes, stream);
