@@ -202,8 +202,8 @@ int sq_w4a16_gemm_fused(const void* x, const void* w, const void* zs, const void
  * two launches: the up projection into up_scratch (fp16 [M, N], caller-allocated, must not
  * overlap y; holds the up projection afterwards), then the gate projection, whose store applies SiLU
  * to the fp32 accumulator and multiplies by up_scratch before the one rounding of Y.  Or, from
- * 17 tokens up where SQ_ALGO_RING is the automatic choice and on the weights of fewer tokens where it
- * measures ahead (group size 128), one launch, which multiplies the fp32 sums and stores the up
+ * 17 tokens up where SQ_ALGO_RING is the automatic choice and at fewer tokens on the weights where it
+ * measures ahead, one launch, which multiplies the fp32 sums and stores the up
  * projection beside Y.  Both weights are [N, K]
  * with their own zeros/scales; for a packed weight cat(W_gate, W_up) in layout L1 pass the two
  * row slices (w_up = w + N * K / 2 bytes, zs_up = zs + N * (K / g) * 4 bytes).  workspace as for

@@ -192,16 +192,18 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
 // with the scale on the sums, which is the rounding of the output, 2.9e-4 with W_hat).
 int ring_tune(int M, int g) { return g == 128 && M <= 64 ? sq::RING_SUMS : 0; }
 
-// Gate and up of a gated MLP in one ring launch at up to 16 tokens (group size 128, the scale on the sums as in the kernels
-// of the two launches), us, two launches / one:
+// Gate and up of a gated MLP in one ring launch at up to 16 tokens, us, two launches / one.  Group size 64, 5 tokens up, where
+// the two would be the streaming kernel's (W_hat there as here): 7680x2560 17.6 / 9.9, 2816x1024 6.3 / 5.7, 13824x4608
+// 29.2 / 22.8, 12288x4096 20.4 / 19.8; 4096x4096 10.3 / 10.3.  Group size 128 (the scale on the sums here as there):
 //   the streaming kernel's K ranges leave its chunk slots part empty: 13696x5120 at 8 tokens 30.7 / 25.3, 5632x2048 8.7 / 7.6,
 //   2816x1024 6.3 / 5.8, 28672x5120 52.6 / 47.6; with more tiles than a round and a short K 24576x2048 20.7 / 21.1 at 5
 //   they fill them: one launch where its 32 x 128 tiles do not leave half the chip or nearly a round idle: 8192x4096 16.4 /
 //   13.1, 14336x4096 20.4 / 20.0, 16384x4096 22.1 / 20.8; but 11008x4096 17.6 / 19.3 (172 tiles), 2048x4096 8.7 / 8.8 (32)
 //   1 and 2 tokens (the GEMV): 8192x5120 17.8 / 15.7, 15360x5120 29.0 / 24.5; but 7680x3072 10.5 / 10.8
-bool pair_at_few_tokens(int M, int N, int K, int g) {
-    if (g != 128) return false;
+bool pair_at_few_tokens(int M, int N, int K, int g, bool ws_ok) {
     const long tiles = (2L * N + 127) / 128;
+    if (g == 64) return M >= 5 && (tiles <= 256 || K > 4096) && builtin_choice(M, N, K, g, ws_ok) == SQ_ALGO_STREAM;
+    if (g != 128) return false;
     const int chunks = K / 128, parts = (chunks + 31) / 32;
     const bool filled = chunks * 4 >= parts * 32 * 3;
     if (M <= 2) return !filled && K > 4096 && tiles >= 128 && tiles <= 256;
@@ -731,7 +733,7 @@ static int silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, 
     const bool ws_ok = workspace && aligned16(workspace);
     int tune = ring_tune(M, group_size);
     if (algo == SQ_ALGO_AUTO) {
-        if (M <= 16 && !pair_at_few_tokens(M, N, K, group_size)) return SQ_ERR_BAD_ALGO;
+        if (M <= 16 && !pair_at_few_tokens(M, N, K, group_size, ws_ok)) return SQ_ERR_BAD_ALGO;
         if (g_tuned_count.load(std::memory_order_relaxed) > 0 &&
             tuned_lookup(M, N, K, group_size, full_workspace(workspace, workspace_bytes, M, N, K)) != 0)
             return SQ_ERR_BAD_ALGO;

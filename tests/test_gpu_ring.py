@@ -91,7 +91,7 @@ def test_ring_every_count_of_stages(capi, shape, stage, short):
 
 
 @pytest.mark.parametrize("m,n,k,g", [(17, 8, 128, 128), (33, 72, 640, 128), (70, 200, 960, 64), (300, 136, 416, 32),
-                                     (100, 1160, 384, 128)])
+                                     (100, 1160, 384, 128), (9, 72, 640, 64), (3, 40, 256, 128)])
 def test_ring_gate_and_up_in_one_launch(capi, m, n, k, g):
     """silu(gate) * up with both weights in every tile: outputs that end inside a tile's half, every shape, K split, and the
     sums scaled; the up projection where it is asked for."""
