@@ -104,6 +104,9 @@ enum : unsigned {
     P_CHUNK_FILL = 1u << 9,   // the least K split of the streaming kernel fills 3/4 or more of a workgroup's 32 chunks
     P_RING = 1u << 10,        // the ring kernel can address the operands
     P_SMALL_K2048 = 1u << 11,   // N * K <= 2^22 elements and K <= 2048
+    P_G64 = 1u << 13,           // group size 64
+    P_SPILL = 1u << 14,         // the streaming kernel's 64-row workgroups times K ranges come to 257..400: a second round, part empty
+    P_PARTS4 = 1u << 15,        // four K ranges of the streaming kernel or more
     P_SHORT_ROUNDS = 1u << 12,  // many rounds of 128 x 256 tiles over a short K (see builtin_choice)
 };
 struct ChoiceRule {
@@ -116,6 +119,18 @@ const ChoiceRule kChoiceRules[] = {
     // 5..16 tokens where a K range of the streaming kernel would leave its chunk slots part empty, and at group size 32
     {5, 16, P_LARGE | P_G128_64 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
      "8 / 16 tokens: 15360x5120 13.9 vs 16.0 / 19.0 (streaming kernel), 13696x5120 13.4 vs 15.7 / 19.3"},
+    {5, 16, P_OVER_16M | P_G64 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
+     "group size 64, 8 / 16 tokens: 4608x4608 9.3 / 9.6 vs 10.2 / 11.2 (streaming kernel), 5120x5120 10.3 / 10.7 vs 10.4 / 11.3; at "
+     "group size 128 5120x5120 10.4 / 10.5 vs 9.9 / 10.4"},
+    // K ranges and row blocks that make a second round of few workgroups
+    {5, 16, P_G64 | P_SPILL | P_PARTS4 | P_RING, P_K_LE_4096, SQ_ALGO_RING,
+     "group size 64, 8 / 16 tokens: 4352x17408 16.5 / 17.6 vs 19.8 / 21.1 (streaming kernel), 5120x13824 14.6 / 15.2 vs 15.4 / 19.8"},
+    {9, 16, P_G128_64 | P_SPILL | P_PARTS4 | P_RING, P_K_LE_4096, SQ_ALGO_RING,
+     "16 tokens: 4352x17408 17.3 vs 19.4 (streaming kernel), 5120x13824 14.6 vs 15.9, 5120x16384 17.0 vs 17.4; 8 tokens 5120x20480 "
+     "18.7 vs 18.0"},
+    {9, 16, P_G64 | P_SPILL | P_RING, P_K_LE_4096, SQ_ALGO_RING,
+     "16 tokens, group size 64: 10240x8192 17.6 vs 21.0 (streaming kernel), 6144x12288 17.9 vs 19.9; at group size 128 17.4 vs 16.9, "
+     "17.7 vs 16.2"},
     {9, 16, P_OVER_16M | P_RING, P_G128_64, SQ_ALGO_RING,
      "16 tokens, group size 32: 5120x5120 10.3 vs 19.2, 12288x4096 12.2 vs 15.4, 4096x11008 13.0 vs 15.4; 4096x4096 8.6 vs 8.4; "
      "9 tokens: 5120x4096 9.4 vs 11.8 (16-column kernel), 16000x2048 8.2 vs 11.3, 6144x3072 8.6 vs 9.6; the other way where that "
@@ -160,12 +175,16 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
     if (nk > (1L << 24)) p |= P_OVER_16M;
     if (ws_ok) p |= P_WS;
     if (g == 128 || g == 64) p |= P_G128_64;
+    if (g == 64) p |= P_G64;
     if (K % 128 == 0) p |= P_K128;
     if (nk <= (1L << 22) && K <= 1536) p |= P_SMALL;
     if (nk <= (1L << 22) && K <= 2048) p |= P_SMALL_K2048;
     {
         const int chunks = K / 128, ks0 = (chunks + 31) / 32;
         if (ks0 > 0 && chunks * 4 >= ks0 * 32 * 3) p |= P_CHUNK_FILL;
+        const long wgs = (long)((N + 63) / 64) * ks0;
+        if (wgs > 256 && wgs <= 400) p |= P_SPILL;
+        if (ks0 >= 4) p |= P_PARTS4;
     }
     if (K <= 4096) p |= P_K_LE_4096;
     if (K <= 8192) p |= P_K_LE_8192;
@@ -193,7 +212,7 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
 int ring_tune(int M, int g) { return g == 128 && M <= 64 ? sq::RING_SUMS : 0; }
 
 // Gate and up of a gated MLP in one ring launch at up to 16 tokens, us, two launches / one.  Group size 64, 5 tokens up, where
-// the two would be the streaming kernel's (W_hat there as here): 7680x2560 17.6 / 9.9, 2816x1024 6.3 / 5.7, 13824x4608
+// the two would be the streaming or the ring kernel's (W_hat there as here): 7680x2560 17.6 / 9.9, 2816x1024 6.3 / 5.7, 13824x4608
 // 29.2 / 22.8, 12288x4096 20.4 / 19.8; 4096x4096 10.3 / 10.3.  Group size 128 (the scale on the sums here as there):
 //   the streaming kernel's K ranges leave its chunk slots part empty: 13696x5120 at 8 tokens 30.7 / 25.3, 5632x2048 8.7 / 7.6,
 //   2816x1024 6.3 / 5.8, 28672x5120 52.6 / 47.6; with more tiles than a round and a short K 24576x2048 20.7 / 21.1 at 5
@@ -202,7 +221,10 @@ int ring_tune(int M, int g) { return g == 128 && M <= 64 ? sq::RING_SUMS : 0; }
 //   1 and 2 tokens (the GEMV): 8192x5120 17.8 / 15.7, 15360x5120 29.0 / 24.5; but 7680x3072 10.5 / 10.8
 bool pair_at_few_tokens(int M, int N, int K, int g, bool ws_ok) {
     const long tiles = (2L * N + 127) / 128;
-    if (g == 64) return M >= 5 && (tiles <= 256 || K > 4096) && builtin_choice(M, N, K, g, ws_ok) == SQ_ALGO_STREAM;
+    if (g == 64) {
+        const int each = builtin_choice(M, N, K, g, ws_ok);
+        return M >= 5 && (tiles <= 256 || K > 4096) && (each == SQ_ALGO_STREAM || each == SQ_ALGO_RING);
+    }
     if (g != 128) return false;
     const int chunks = K / 128, parts = (chunks + 31) / 32;
     const bool filled = chunks * 4 >= parts * 32 * 3;
