@@ -919,32 +919,33 @@ static hipError_t launch_shape(const void* x, const void* w, const void* zs, con
 
 // What a shape costs, in us: a workgroup takes `step0 + step1 * a` per stage of K and `fixed` besides (first loads, sums,
 // stores), a = the share of the 256 CUs that its round keeps busy (memory and clock are shared); a K split adds the
-// exchange of the partial tiles, `ex0 + ex1 * parts + exmb` per MB of them.  One workgroup fills a CU.  Least-squares
+// exchange of the partial tiles, `ex0 + ex1 * parts + exmb` per MB of them, and every round of 256 after the first `round`.
+// One workgroup fills a CU.  Least-squares
 // fits: tiles of 32 rows to 9000 timings of 18 weights (3072 x 1024 .. 28672 x 8192) x 23 token counts (12 .. 4096), the
-// others, with the loop in step, to 4400 timings of 14 weights (3072 x 1024 .. 24576 x 8192) x 19 token counts (20 ..
-// 4096), all shapes and splits: rms error 3..7 %, the choice within 0.7 % of the best in the geometric mean (1.8 % with the
-// constants of the alternating loop, which left the 128 x 128 tiles out: 224 tokens x 15360x5120 52 where they take 43),
-// 17 % at worst (80 tokens x 4096x16384).
+// others, with the loop in step, to 7300 timings of 26 weights (1536 x 6144 .. 24576 x 8192) x 34 token counts (20 .. 4096),
+// all shapes and splits, then adjusted for the choice (rms error 6..7 %): within 0.5 % of the best in the geometric mean
+// (1.8 % with the constants of the alternating loop, which left the 128 x 128 tiles out: 224 tokens x 15360x5120 52 where
+// they take 43), 19 % at worst (512 tokens x 8192x1024).
 struct RingTile {
     int bm, bn, ks;
-    float fixed, step0, step1, ex0, ex1, exmb;
+    float fixed, step0, step1, ex0, ex1, exmb, round;
 };
 static const RingTile kRingTiles[] = {
-    {32, 64, 512, 1.723f, 0.829f, 0.160f, 0.301f, 0.226f, 0.861f},
-    {32, 128, 256, 1.498f, 0.754f, 0.096f, 0.448f, 0.304f, 0.649f},
-    {64, 128, 256, 2.477f, 0.758f, 0.383f, 0.349f, 0.557f, 0.414f},
-    {96, 128, 128, 3.023f, 0.456f, 0.375f, 0.311f, 0.719f, 0.278f},
-    {64, 256, 128, 2.321f, 0.788f, 0.289f, 1.297f, 0.832f, 0.357f},
-    {96, 256, 128, 4.394f, 0.724f, 0.637f, 0.267f, 1.403f, 0.188f},
-    {128, 128, 128, 2.849f, 0.506f, 0.482f, 0.000f, 1.028f, 0.301f},
-    {128, 256, 128, 5.724f, 0.883f, 0.792f, 0.986f, 1.489f, 0.180f},
-    {256, 256, 64, 8.358f, 0.930f, 0.669f, 0.f, 0.f, 0.f},  // never split, see plan_ring
+    {32, 64, 512, 1.723f, 0.829f, 0.160f, 0.301f, 0.226f, 0.861f, 0.f},
+    {32, 128, 256, 1.498f, 0.754f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f},
+    {64, 128, 256, 2.575f, 0.763f, 0.379f, 0.745f, 0.539f, 0.391f, 1.281f},
+    {96, 128, 128, 2.852f, 0.474f, 0.337f, 1.205f, 0.592f, 0.286f, 1.910f},
+    {64, 256, 128, 2.544f, 0.820f, 0.309f, 1.556f, 0.799f, 0.335f, 1.349f},
+    {96, 256, 128, 4.013f, 0.701f, 0.595f, 1.206f, 1.294f, 0.195f, 2.135f},
+    {128, 128, 128, 2.534f, 0.521f, 0.427f, 0.491f, 0.920f, 0.316f, 2.287f},
+    {128, 256, 128, 6.570f, 0.884f, 0.773f, 2.005f, 1.435f, 0.167f, 2.126f},
+    {256, 256, 64, 9.097f, 0.833f, 0.671f, 0.f, 0.f, 0.f, 2.701f},  // never split, see plan_ring
 };
 // The same with the scale on the sums (up to 64 tokens), where other constants hold: shapes 1..5, of which the fourth is
 // not built for it.
 static const RingTile kRingSumsTiles[] = {
-    kRingTiles[0], kRingTiles[1], {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f},
-    kRingTiles[3], {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f},
+    kRingTiles[0], kRingTiles[1], {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f, 0.f},
+    kRingTiles[3], {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f, 0.f},
 };
 constexpr int RING_SHAPES = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
 #define X_(id, MI, NI, WM, WN, WK, ST)                                                                              \
@@ -980,14 +981,15 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes, bool sums) {
         const int full = (int)(tiles >> 8), rest = (int)(tiles & 255);
         const float one = stages * (t.step0 + t.step1) + t.fixed;
         const float base = 2.f + full * one;
-        auto consider = [&](float us, int nfull, int ks) {
+        auto consider = [&](float us, int rounds, int nfull, int ks) {
+            if (rounds > 1) us += (rounds - 1) * t.round;
             if (us >= best_us) return;
             const RingPlan p{s + 1, nfull, ks};
             if (ks > 1 && ring_bytes(p, M, N) > ws_bytes) return;
             best_us = us;
             best = p;
         };
-        consider(base + (rest ? stages * (t.step0 + t.step1 * rest * (1.f / 256)) + t.fixed : 0.f), 0, 1);
+        consider(base + (rest ? stages * (t.step0 + t.step1 * rest * (1.f / 256)) + t.fixed : 0.f), full + (rest != 0), 0, 1);
         // (256 x 256 tiles split over K were behind smaller tiles wherever they were timed: partial tiles of 256 KB)
         if (ws_bytes == 0 || rest == 0 || t.bm == 256) continue;
         static const int splits[5] = {2, 3, 4, 6, 8};
@@ -999,7 +1001,7 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes, bool sums) {
             const int r = (int)(w >> 8), last = (int)(w & 255);
             consider(base + r * (st * (t.step0 + t.step1) + t.fixed) +
                          (last ? st * (t.step0 + t.step1 * last * (1.f / 256)) + t.fixed : 0.f) + ex,
-                     full * 256, ks);
+                     full + r + (last != 0), full * 256, ks);
         }
     }
     return best;
