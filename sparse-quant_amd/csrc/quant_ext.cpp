@@ -398,6 +398,29 @@ at::Tensor walinear_forward(const at::Tensor& x, const at::Tensor& W, const at::
                      act_code(act), with_ln ? &ln : nullptr, true);
 }
 
+// One fp16 weight [N, K] quantised and packed in one launch: codes, zeros_scales, and (layout L2, want_fake) the
+// fake-quantised weight.  Which weights come here quant_funcs decides; the C ABI checks what it is given.
+std::tuple<at::Tensor, at::Tensor, c10::optional<at::Tensor>> quantise(const at::Tensor& w, const int group_size, const int n_bit,
+                                                                       const int layout, const bool want_fake) {
+    SQ_CHECK_DEVICE(w);
+    SQ_CHECK_CONTIGUOUS(w);
+    SQ_CHECK_DTYPE(w, at::kHalf);
+    SQ_CHECK_DIMS(w, 2);
+    const int64_t n = w.size(0), k = w.size(1);
+    TORCH_CHECK(n < (1LL << 31) && k < (1LL << 31) && group_size > 0, "problem too large");
+    at::NoGradGuard no_grad;
+    c10::DeviceGuard guard(w.device());
+    const bool l1 = layout == SQ_LAYOUT_L1;
+    at::Tensor q = l1 ? at::empty({n, k * n_bit / 8}, w.options().dtype(at::kByte)) : at::empty({k, n / 8}, w.options().dtype(at::kInt));
+    at::Tensor zs = l1 ? at::empty({n, 2 * (k / group_size)}, w.options()) : at::empty({k / group_size, 2 * n}, w.options());
+    c10::optional<at::Tensor> fake;
+    if (want_fake) fake = at::empty({n, k}, w.options());
+    raise_if_error(sq_w4a16_quantise(w.data_ptr(), q.data_ptr(), zs.data_ptr(), want_fake ? fake->data_ptr() : nullptr, (int)n, (int)k,
+                                     group_size, n_bit, layout, current_stream(w)),
+                   "quantise");
+    return {q, zs, fake};
+}
+
 // The two branches of sparse_attention on tensors that need no conversion (12.4 and 19.2 us of host time a call from
 // Python, 7.1 and 6.3 here: 8 x 16 heads x 512 x 64 at 25 % took 11.1 us and takes 8.7); anything else returns nothing
 // and takes the general path in Python, which copies or refuses it.
@@ -635,6 +658,7 @@ PYBIND11_MODULE(quant, m) {
           py::arg("W2") = py::none(), py::arg("ZS1") = py::none(), py::arg("ZS2") = py::none(),
           py::arg("W13") = py::none(), py::arg("ZS13") = py::none(), py::arg("M"), py::arg("N"), py::arg("K"),
           py::arg("group_size"));
+    m.def("quantise", &quantise);
     m.def("convert_2bit_to_4bit", &convert_2bit_to_4bit);
     m.def("convert_4bit_to_2bit", &convert_4bit_to_2bit);
     m.def("clear_repack_cache", &clear_repack_cache);

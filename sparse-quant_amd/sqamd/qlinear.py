@@ -21,17 +21,7 @@ class WALinear(nn.Module):
     def __init__(self, in_features, out_features, w_config=None, a_config=None, w_bit=4, a_bit=16,
                  group_size=None, bias=True, quantize_output=False, dev="cuda", dtype=None, layout="l1"):
         super().__init__()
-        if layout not in ("l1", "l2"):
-            raise ValueError("layout must be 'l1' or 'l2'")
-        self.in_features = in_features
-        self.out_features = out_features
-        self.w_config = w_config
-        self.a_config = a_config
-        self.w_bit = w_bit
-        self.a_bit = a_bit
-        self.layout = layout
-        self.group_size = group_size if group_size is not None else (64 if layout == "l1" else 128)
-        self.quantize_output = quantize_output
+        self._describe(in_features, out_features, w_config, a_config, w_bit, a_bit, group_size, quantize_output, layout)
         g = self.group_size
         if layout == "l1":
             self.register_buffer("zeros_scales", torch.zeros(out_features, in_features * 2 // g,
@@ -47,6 +37,14 @@ class WALinear(nn.Module):
             self.register_buffer("bias", torch.zeros((1, out_features), dtype=torch.float16, device=dev))
         else:
             self.register_buffer("bias", None)
+
+    def _describe(self, in_features, out_features, w_config, a_config, w_bit, a_bit, group_size, quantize_output, layout):
+        if layout not in ("l1", "l2"):
+            raise ValueError("layout must be 'l1' or 'l2'")
+        # (plain values: nn.Module's attribute hook has nothing to sort them into and costs a microsecond each)
+        self.__dict__.update(in_features=in_features, out_features=out_features, w_config=w_config, a_config=a_config,
+                             w_bit=w_bit, a_bit=a_bit, layout=layout, quantize_output=quantize_output,
+                             group_size=group_size if group_size is not None else (64 if layout == "l1" else 128))
 
     def forward(self, x, residual=None, act="none", pre_ln=None):
         """y = act(x W_hat^T + bias) + residual.  With the defaults this is the reference's
@@ -86,17 +84,20 @@ class WALinear(nn.Module):
     def from_float(module, w_config, a_config=None, quantize_output=False, layout="l1"):
         assert isinstance(module, nn.Linear)
         n_bit, g = w_config["n_bit"], w_config["group_size"]
-        # every buffer is replaced below: on the meta device the constructor's zeros cost no fills
-        new = WALinear(module.in_features, module.out_features, w_config, a_config, w_bit=n_bit, group_size=g,
-                       bias=module.bias is not None, quantize_output=quantize_output, dev="meta", layout=layout)
+        # The buffers are registered as they will be, not as the constructor's zeros: those, on the meta device, and
+        # replacing them took most of the call's host time (1280 x 1472: 46 -> 16 us a call with the packer in the extension).
+        new = WALinear.__new__(WALinear)
+        nn.Module.__init__(new)
+        new._describe(module.in_features, module.out_features, w_config, a_config, n_bit, 16, g, quantize_output, layout)
         if layout == "l1":
-            new.weight, new.zeros_scales = quant_funcs.quant_muxi(module.weight.data, module.in_features,
-                                                                  module.out_features, n_bit=n_bit, group_size=g)
+            weight, zeros_scales = quant_funcs.quant_muxi(module.weight.data, module.in_features, module.out_features,
+                                                          n_bit=n_bit, group_size=g)
         else:
-            new.weight, new.zeros_scales, _ = quant_funcs._lmdeploy(module.weight.data, module.in_features,
-                                                                    module.out_features, g, n_bit, want_fake=False)
-        if module.bias is not None:
-            new.bias = module.bias.data.half().unsqueeze(0)
+            weight, zeros_scales, _ = quant_funcs._lmdeploy(module.weight.data, module.in_features, module.out_features, g,
+                                                            n_bit, want_fake=False)
+        new.register_buffer("zeros_scales", zeros_scales)
+        new.register_buffer("weight", weight)
+        new.register_buffer("bias", None if module.bias is None else module.bias.data.half().unsqueeze(0))
         return new
 
     def __repr__(self):

@@ -101,7 +101,9 @@ def quant_muxi(weight, input_features, output_features, n_bit=4, group_size=64, 
     """
     assert weight.shape == (output_features, input_features)
     if compute_dtype in (None, torch.float16) and _one_launch(weight, n_bit, group_size, capi.SQ_LAYOUT_L1):
-        return capi.quantise(weight, group_size, n_bit)[:2]
+        import quant
+
+        return quant.quantise(weight, group_size, n_bit, capi.SQ_LAYOUT_L1, False)[:2]
     q, scales, zeros = quantize_tensor(_as(weight, compute_dtype), n_bit, group_size)
     q = interleave_k(q)
     if n_bit == 4:
@@ -146,7 +148,7 @@ def _lmdeploy(weight, input_features, output_features, group_size, n_bit, comput
         raise ValueError("n_bit must be 2 or 4")
     if compute_dtype in (None, torch.float16) and weight.shape == (output_features, input_features) and \
             _one_launch(weight, n_bit, group_size, capi.SQ_LAYOUT_L2):
-        qweight, zeros_scales, w_fp16 = capi.quantise(weight, group_size, n_bit, capi.SQ_LAYOUT_L2, want_fake)
+        qweight, zeros_scales, w_fp16 = quant.quantise(weight, group_size, n_bit, capi.SQ_LAYOUT_L2, want_fake)
         return (convert_4bit_to_2bit(qweight) if n_bit == 2 else qweight), zeros_scales, w_fp16
     w = _as(weight, compute_dtype)
     q, scales, zeros = quantize_tensor(w, n_bit, group_size)
