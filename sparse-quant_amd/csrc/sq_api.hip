@@ -108,6 +108,8 @@ enum : unsigned {
     P_SPILL = 1u << 14,         // the streaming kernel's 64-row workgroups times K ranges come to 257..400: a second round, part empty
     P_PARTS4 = 1u << 15,        // four K ranges of the streaming kernel or more
     P_SHORT_ROUNDS = 1u << 12,  // many rounds of 128 x 256 tiles over a short K (see builtin_choice)
+    // what the streaming kernel needs of a K that it splits
+    P_STREAM_SPLIT = P_G128_64 | P_K128 | P_WS | P_K_LE_32768,
 };
 struct ChoiceRule {
     int m_lo, m_hi;
@@ -119,16 +121,19 @@ const ChoiceRule kChoiceRules[] = {
     // 5..16 tokens where a K range of the streaming kernel would leave its chunk slots part empty, and at group size 32
     {5, 16, P_LARGE | P_G128_64 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
      "8 / 16 tokens: 15360x5120 13.9 vs 16.0 / 19.0 (streaming kernel), 13696x5120 13.4 vs 15.7 / 19.3"},
-    {5, 16, P_OVER_16M | P_G64 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
+    // (in place of the streaming kernel alone: where that does not run, the GEMV keeps the scale in fp32 at 5..8 tokens and
+    // group size 64, and without a workspace the ring kernel leaves most of the chip idle: 3136x5888 at 9 tokens 13.5 vs 8.3
+    // (16-column kernel), 4672x6016 at 8 14.1 vs 10.7 (GEMV))
+    {5, 16, P_OVER_16M | P_G64 | P_STREAM_SPLIT | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
      "group size 64, 8 / 16 tokens: 4608x4608 9.3 / 9.6 vs 10.2 / 11.2 (streaming kernel), 5120x5120 10.3 / 10.7 vs 10.4 / 11.3; at "
      "group size 128 5120x5120 10.4 / 10.5 vs 9.9 / 10.4"},
     // K ranges and row blocks that make a second round of few workgroups
-    {5, 16, P_G64 | P_SPILL | P_PARTS4 | P_RING, P_K_LE_4096, SQ_ALGO_RING,
+    {5, 16, P_G64 | P_SPILL | P_PARTS4 | P_STREAM_SPLIT | P_RING, P_K_LE_4096, SQ_ALGO_RING,
      "group size 64, 8 / 16 tokens: 4352x17408 16.5 / 17.6 vs 19.8 / 21.1 (streaming kernel), 5120x13824 14.6 / 15.2 vs 15.4 / 19.8"},
-    {9, 16, P_G128_64 | P_SPILL | P_PARTS4 | P_RING, P_K_LE_4096, SQ_ALGO_RING,
+    {9, 16, P_SPILL | P_PARTS4 | P_STREAM_SPLIT | P_RING, P_K_LE_4096, SQ_ALGO_RING,
      "16 tokens: 4352x17408 17.3 vs 19.4 (streaming kernel), 5120x13824 14.6 vs 15.9, 5120x16384 17.0 vs 17.4; 8 tokens 5120x20480 "
      "18.7 vs 18.0"},
-    {9, 16, P_G64 | P_SPILL | P_RING, P_K_LE_4096, SQ_ALGO_RING,
+    {9, 16, P_G64 | P_SPILL | P_STREAM_SPLIT | P_RING, P_K_LE_4096, SQ_ALGO_RING,
      "16 tokens, group size 64: 10240x8192 17.6 vs 21.0 (streaming kernel), 6144x12288 17.9 vs 19.9; at group size 128 17.4 vs 16.9, "
      "17.7 vs 16.2"},
     {9, 16, P_OVER_16M | P_RING, P_G128_64, SQ_ALGO_RING,
@@ -144,7 +149,7 @@ const ChoiceRule kChoiceRules[] = {
     // the streaming decode kernel, 5..16 tokens (3..4 on large weights); K beyond 4096 is split through the workspace
     {5, 16, P_G128_64 | P_K128 | P_K_LE_4096, 0, SQ_ALGO_STREAM,
      "8 tokens: fc1 10.0 vs 13.3 (split-K kernel), q/k/v in one launch 8.6 vs 12.1, 4096x4096 4.9 vs 6.5 (GEMV)"},
-    {5, 16, P_G128_64 | P_K128 | P_WS | P_K_LE_32768, 0, SQ_ALGO_STREAM, "8 tokens: fc2 12.7 vs 14.6 (split-K kernel)"},
+    {5, 16, P_STREAM_SPLIT, 0, SQ_ALGO_STREAM, "8 tokens: fc2 12.7 vs 14.6 (split-K kernel)"},
     {3, 4, P_LARGE | P_G128_64 | P_K128 | P_K_LE_4096, 0, SQ_ALGO_STREAM, "4 tokens: fc1 9.7 vs 10.7 (GEMV)"},
     {3, 4, P_LARGE | P_G128_64 | P_K128 | P_WS | P_K_LE_32768 | P_CHUNK_FILL, 0, SQ_ALGO_STREAM,
      "4 tokens: fc2 11.9 vs 13.6 (GEMV); 13824x5120, whose K ranges fill 20 of a workgroup's 32 chunks: 14.6 vs 13.9 (GEMV)"},

@@ -179,7 +179,8 @@ def test_ring_has_the_scale_on_the_sums_where_it_says(capi):
 @pytest.mark.parametrize("use_ws", [True, False])
 @pytest.mark.parametrize("m,n,k,g", [(5, 5120, 5120, 32), (8, 5120, 5120, 32), (8, 6656, 5120, 128), (16, 6656, 5120, 128),
                                      (17, 4096, 4096, 128), (32, 4096, 4096, 128), (32, 1000, 11008, 128),
-                                     (40, 2048, 1408, 128), (48, 2560, 13696, 128), (64, 2048, 1536, 128)])
+                                     (40, 2048, 1408, 128), (48, 2560, 13696, 128), (64, 2048, 1536, 128),
+                                     (5, 2816, 6080, 64), (8, 4096, 4672, 64)])
 def test_few_tokens_round_no_weight_to_half(capi, m, n, k, g, use_ws):
     """Where decode kernels keep the scale in fp32 the automatic choice does so whichever kernel it names: the result is
     as far from (q - z) s in float64 as its one rounding to fp16 puts it (W_hat is 1.4 times as far, and fp32 sums add
@@ -190,6 +191,11 @@ def test_few_tokens_round_no_weight_to_half(capi, m, n, k, g, use_ws):
     y = capi.gemm_fused(to_dev(x), to_dev(d["w_l1"]), to_dev(d["zs_l1"]), n, k, g, use_workspace=use_ws)
     rounding = (ref.half().double() - ref).norm()
     assert (y.double() - ref).norm() <= 1.1 * rounding
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 3328, 5120), (8, 5120, 5120), (6, 4096, 4672)])
+def test_few_tokens_round_no_weight_to_half_without_a_workspace_at_group_size_64(capi, m, n, k):
+    test_few_tokens_round_no_weight_to_half(capi, m, n, k, 64, False)
 
 
 @pytest.mark.parametrize("m,n,k,g", [(1, 72, 640, 128), (33, 136, 1408, 128), (70, 72, 416, 32), (20, 72, 960, 64)])
