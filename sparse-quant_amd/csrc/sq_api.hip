@@ -78,6 +78,12 @@ inline bool full_workspace(const void* workspace, size_t workspace_bytes, int M,
            workspace_bytes >= sq_w4a16_workspace_bytes(M, N, K);
 }
 
+// Whether the decode kernels can split K through this workspace.
+inline bool decode_workspace(const void* workspace, size_t workspace_bytes, int M, int N, int K) {
+    return workspace && aligned16(workspace) && workspace_bytes >= sq::skinny2_workspace_bytes(M > 32 ? 32 : M, N, K) &&
+           (N + 63) / 64 <= 16384;
+}
+
 int tuned_lookup(int M, int N, int K, int g, bool has_ws) {
     const int n = g_tuned_count.load(std::memory_order_acquire);
     for (int i = n - 1; i >= 0; i--) {  // the latest measurement of a shape wins
@@ -262,10 +268,7 @@ int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, 
         }
     }
     if (kernel == SQ_ALGO_AUTO) {
-        const bool ws_ok = workspace && aligned16(workspace) &&
-                           workspace_bytes >= sq::skinny2_workspace_bytes(M > 32 ? 32 : M, N, K) &&
-                           (N + 63) / 64 <= 16384;
-        kernel = builtin_choice(M, N, K, group_size, ws_ok);
+        kernel = builtin_choice(M, N, K, group_size, decode_workspace(workspace, workspace_bytes, M, N, K));
         if (kernel == SQ_ALGO_RING) tune = ring_tune(M, group_size);
     }
     switch (kernel) {
@@ -757,7 +760,7 @@ static int silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, 
     if (!aligned16(x) || !aligned16(w_gate) || !aligned16(zs_gate) || !aligned16(w_up) || !aligned16(zs_up) || !aligned16(y))
         return SQ_ERR_MISALIGNED;
     if (N > (1 << 29)) return SQ_ERR_BAD_ALGO;
-    const bool ws_ok = workspace && aligned16(workspace);
+    const bool ws_ok = decode_workspace(workspace, workspace_bytes, M, N, K);
     int tune = ring_tune(M, group_size);
     if (algo == SQ_ALGO_AUTO) {
         if (M <= 16 && !pair_at_few_tokens(M, N, K, group_size, ws_ok)) return SQ_ERR_BAD_ALGO;
@@ -769,8 +772,9 @@ static int silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, 
         if ((algo & 0xFF) != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
         tune = (algo >> 8) & 0xFFFF;
     }
-    const hipError_t e = sq::launch_gemm_ring_pair(x, w_gate, zs_gate, w_up, zs_up, y, up, ws_ok ? workspace : nullptr,
-                                                   workspace_bytes, M, N, K, group_size, tune, static_cast<hipStream_t>(stream));
+    const hipError_t e = sq::launch_gemm_ring_pair(x, w_gate, zs_gate, w_up, zs_up, y, up,
+                                                   aligned16(workspace) ? workspace : nullptr, workspace_bytes, M, N, K,
+                                                   group_size, tune, static_cast<hipStream_t>(stream));
     return e == hipErrorInvalidValue ? SQ_ERR_BAD_ALGO : launch_code(e);
 }
 

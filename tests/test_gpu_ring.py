@@ -198,6 +198,18 @@ def test_few_tokens_round_no_weight_to_half_without_a_workspace_at_group_size_64
     test_few_tokens_round_no_weight_to_half(capi, m, n, k, 64, False)
 
 
+def test_gate_and_up_with_little_workspace_round_no_weight_to_half(capi):
+    """Less than the streaming kernel wants: the GEMV twice, with its scale in fp32."""
+    m, n, k, g = 8, 2560, 5120, 64
+    d = orc.synth_linear(n, k, g, seed=k)
+    x, w, zs = orc.synth_x(m, k, seed=m), to_dev(d["w_l1"]), to_dev(d["zs_l1"])
+    ws = torch.zeros(1 << 20, dtype=torch.uint8, device=DEV)
+    assert ws.numel() < capi.lib().sq_w4a16_workspace_bytes(m, n, k)
+    _, up = capi.gemm_silu_dot(to_dev(x), w, zs, w, zs, n, k, g, ws=ws)
+    ref = torch.from_numpy(x).to(DEV).double() @ torch.from_numpy(real_weight(d, g)).to(DEV).t()
+    assert (up.double() - ref).norm() <= 1.1 * (ref.half().double() - ref).norm()
+
+
 @pytest.mark.parametrize("m,n,k,g", [(1, 72, 640, 128), (33, 136, 1408, 128), (70, 72, 416, 32), (20, 72, 960, 64)])
 @pytest.mark.parametrize("shape", range(10))
 def test_ring_keeps_an_infinite_activation_to_its_row(capi, shape, m, n, k, g):
