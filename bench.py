@@ -885,7 +885,7 @@ def gated_mlp_leg(torch, capi, g, dev, gen, stream, n=11008, k=4096, tokens=(1, 
         b = torch.empty((m, n), dtype=torch.float16, device=dev)
         torch.cuda.synchronize()
         with torch.cuda.stream(stream):
-            ws = capi.workspace(m, n, k, dev, stream) if 2 < m <= 1024 else None
+            ws = capi.workspace(m, n, k, dev, stream, gated=True) if 2 < m <= 1024 else None
 
             def fused():
                 for (wg, zg), (wu, zu) in pool:

@@ -207,7 +207,8 @@ int sq_w4a16_gemm_fused(const void* x, const void* w, const void* zs, const void
  * projection beside Y.  Both weights are [N, K]
  * with their own zeros/scales; for a packed weight cat(W_gate, W_up) in layout L1 pass the two
  * row slices (w_up = w + N * K / 2 bytes, zs_up = zs + N * (K / g) * 4 bytes).  workspace as for
- * sq_w4a16_gemm_ws (may be NULL).  In the role of gemm_awq_silu_dot_ut, which the reference's
+ * sq_w4a16_gemm_ws (may be NULL), of sq_w4a16_gemm_silu_dot_workspace_bytes(M, N, K) bytes (the one
+ * launch splits K as far as the workspace holds its partial tiles).  In the role of gemm_awq_silu_dot_ut, which the reference's
  * kernel test imports from a package that is not part of it; the expected value and tolerance
  * are that test's: silu(x W1^T) * (x W2^T) within atol = rtol = 2e-2 (reference:
  * quantization/nvidia/script/gemm_awq_test.py:50-56,66-72,105). */
@@ -215,6 +216,10 @@ int sq_w4a16_gemm_silu_dot(const void* x, const void* w_gate, const void* zs_gat
                            const void* zs_up, void* y, void* up_scratch, int M, int N, int K,
                            int group_size, int layout, void* workspace, size_t workspace_bytes,
                            void* stream);
+
+/* Bytes for both gated entry points: sq_w4a16_workspace_bytes(M, N, K) or, if that is more, what the one
+ * launch can use.  Host arithmetic, no GPU needed. */
+size_t sq_w4a16_gemm_silu_dot_workspace_bytes(int M, int N, int K);
 
 /* The same without up_scratch, in one launch; SQ_ERR_BAD_ALGO, with nothing launched, where two would
  * be needed.  algo: SQ_ALGO_AUTO, or SQ_ALGO_RING with a tuning word (of the 2 N columns of both). */

@@ -341,9 +341,7 @@ at::Tensor gemm_awq_silu_dot_ut(at::Tensor I, c10::optional<at::Tensor> W1, c10:
     size_t ws_bytes = 0;
     at::Tensor ws;
     if (rows > 2 && rows <= 1024) {
-        // (both weights can share a launch)
-        ws = workspace_for(I, stream, std::max(sq_w4a16_workspace_bytes((int)rows, N, (int)Kin),
-                                               N < (1 << 29) ? sq_w4a16_workspace_bytes((int)rows, 2 * N, (int)Kin) : 0));
+        ws = workspace_for(I, stream, sq_w4a16_gemm_silu_dot_workspace_bytes((int)rows, N, (int)Kin));
         ws_ptr = ws.data_ptr();
         ws_bytes = (size_t)ws.numel();
     }

@@ -354,6 +354,13 @@ size_t sq_w4a16_workspace_bytes(int M, int N, int K) {
     return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
+size_t sq_w4a16_gemm_silu_dot_workspace_bytes(int M, int N, int K) {
+    const size_t each = sq_w4a16_workspace_bytes(M, N, K);
+    if (each == 0 || N > (1 << 29)) return each;
+    const size_t both = sq::gemm_ring_workspace_bytes(M, 2 * N, K);  // (the one launch is always the ring kernel's)
+    return each > both ? each : both;
+}
+
 int sq_w4a16_gemm_ws(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int group_size,
                      int layout, int algo, void* workspace, size_t workspace_bytes, void* stream) {
     return gemm_dispatch(x, w, zs, y, M, N, K, group_size, layout, algo, sq::Epilogue{nullptr, nullptr, 0}, workspace,

@@ -31,6 +31,7 @@ SIGNATURES = {
     "sq_w4a16_gemm_fused": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t, _vp]),
     "sq_w4a16_gemm_silu_dot": (_i, [_vp] * 7 + [_i] * 5 + [_vp, ctypes.c_size_t, _vp]),
     "sq_w4a16_gemm_silu_dot_one": (_i, [_vp] * 6 + [_i] * 6 + [_vp, ctypes.c_size_t, _vp]),
+    "sq_w4a16_gemm_silu_dot_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i]),
     "sq_w4a16_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i]),
     "sq_w4a16_autotune": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t, _i, ctypes.c_size_t,
                                ctypes.c_size_t, _i, _vp, ctypes.POINTER(_i), ctypes.POINTER(ctypes.c_float),
@@ -173,9 +174,10 @@ def _cached_workspace(key, need, device):
     return ws
 
 
-def workspace(m, n, k, device, stream=None):
-    """A zero-initialised workspace tensor, cached per (device, stream) and grown on demand."""
-    need = lib().sq_w4a16_workspace_bytes(m, n, k)
+def workspace(m, n, k, device, stream=None, gated=False):
+    """A zero-initialised workspace tensor, cached per (device, stream) and grown on demand (gated: for gate and up,
+    [n, k] each)."""
+    need = (lib().sq_w4a16_gemm_silu_dot_workspace_bytes if gated else lib().sq_w4a16_workspace_bytes)(m, n, k)
     key = (str(device), (stream or torch.cuda.current_stream()).cuda_stream)
     return _cached_workspace(key, max(need, 1 << 20), device)
 
@@ -265,7 +267,7 @@ def gemm_silu_dot(x, w_gate, zs_gate, w_up, zs_up, n, k, group_size, out=None, s
         out = torch.empty((m, n), dtype=torch.float16, device=x.device)
     up = up_out if up_out is not None else torch.empty((m, n), dtype=torch.float16, device=x.device)
     if ws is None and use_workspace and 2 < m <= 1024:
-        ws = workspace(m, n, k, x.device, stream)
+        ws = workspace(m, n, k, x.device, stream, gated=True)
     _check(lib().sq_w4a16_gemm_silu_dot(_ptr(x), _ptr(w_gate), _ptr(zs_gate), _ptr(w_up), _ptr(zs_up), _ptr(out), _ptr(up),
                                         m, n, k, group_size, SQ_LAYOUT_L1, _ptr(ws), 0 if ws is None else ws.numel(),
                                         _stream(stream)), "sq_w4a16_gemm_silu_dot")

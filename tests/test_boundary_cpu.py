@@ -120,6 +120,11 @@ def test_host_side_queries_need_no_gpu(built_lib):
     assert L.sq_w4a16_workspace_bytes(0, 4096, 4096) == 0
     sizes = [L.sq_w4a16_workspace_bytes(m, 4096, 16384) for m in (1, 16, 17, 32, 33, 64, 512, 1024)]
     assert all(b >= counters for b in sizes) and sizes[0] <= sizes[1] <= sizes[2] == sizes[3]
+    # gate and up: never more than one weight's or the ring kernel's largest plan (300 partial tiles of 128 x 256)
+    for m, n, k in ((3, 11008, 4096), (32, 11008, 4096), (333, 11008, 4096), (1024, 13696, 5120)):
+        one, both = L.sq_w4a16_workspace_bytes(m, n, k), L.sq_w4a16_gemm_silu_dot_workspace_bytes(m, n, k)
+        assert one <= both <= max(one, counters + 300 * 128 * 256 * 4), (m, n, k)
+    assert L.sq_w4a16_gemm_silu_dot_workspace_bytes(0, 4096, 4096) == 0
     fus = L.sq_w4a16_ln_fusable
     assert fus(8, 16384, 4096, 128, capi.SQ_LAYOUT_L1) == 1 and fus(1, 12288, 4096, 128, capi.SQ_LAYOUT_L1) == 1
     for bad in ((9, 16384, 4096, 128, capi.SQ_LAYOUT_L1), (8, 16384, 2048, 128, capi.SQ_LAYOUT_L1),

@@ -133,6 +133,23 @@ def test_ring_gate_and_up_in_one_launch(capi, m, n, k, g):
     assert np.all(np.abs(up.cpu().numpy() - ref) <= 2.0 ** -11 * np.abs(ref) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w_hat[1]).T) * 2 + 2.0 ** -24)
 
 
+def test_gate_and_up_hold_no_more_than_the_ring_kernel_can_use(capi):
+    """The extension keeps its workspace per stream: 40 MB for 11008 x 4096 at 333 tokens, not the 135 MB that the tiled GEMM
+    would want for a weight of 2 x 11008 rows."""
+    import quant
+    m, n, k, g = 333, 11008, 4096, 64
+    w = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV)
+    zs = torch.full((n, 2 * (k // g)), 65.0, dtype=torch.float16, device=DEV)
+    x = torch.randn((1, m, k), device=DEV).half()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        before = torch.cuda.memory_allocated()
+        y = quant.gemm_awq_silu_dot_ut(x, w, w, zs, zs, None, None, m, n, k, g)
+        torch.cuda.synchronize()
+        held = torch.cuda.memory_allocated() - before - y.numel() * 2
+    assert held <= capi.lib().sq_w4a16_gemm_silu_dot_workspace_bytes(m, n, k) + (1 << 20) <= 40 << 20
+
+
 REST = 0x10  # tune word: only the tiles of the last round of 256 split K
 SUMS = 0x20  # tune word: the scale on the sums (shapes of 32 and 64 rows, group size 128)
 
