@@ -230,12 +230,9 @@ int ring_tune(int M, int g) { return g == 128 && M <= 64 ? sq::RING_SUMS : 0; }
 //   they fill them: one launch where its 32 x 128 tiles do not leave half the chip or nearly a round idle: 8192x4096 16.4 /
 //   13.1, 14336x4096 20.4 / 20.0, 16384x4096 22.1 / 20.8; but 11008x4096 17.6 / 19.3 (172 tiles), 2048x4096 8.7 / 8.8 (32)
 //   1 and 2 tokens (the GEMV): 8192x5120 17.8 / 15.7, 15360x5120 29.0 / 24.5; but 7680x3072 10.5 / 10.8
-bool pair_at_few_tokens(int M, int N, int K, int g, bool ws_ok) {
+bool pair_at_few_tokens(int M, int N, int K, int g, int each) {  // each: the kernel of the two launches
     const long tiles = (2L * N + 127) / 128;
-    if (g == 64) {
-        const int each = builtin_choice(M, N, K, g, ws_ok);
-        return M >= 5 && (tiles <= 256 || K > 4096) && (each == SQ_ALGO_STREAM || each == SQ_ALGO_RING);
-    }
+    if (g == 64) return M >= 5 && (tiles <= 256 || K > 4096) && (each == SQ_ALGO_STREAM || each == SQ_ALGO_RING);
     if (g != 128) return false;
     const int chunks = K / 128, parts = (chunks + 31) / 32;
     const bool filled = chunks * 4 >= parts * 32 * 3;
@@ -754,7 +751,7 @@ int sq_w4a16_gemm_fused(const void* x, const void* w, const void* zs, const void
 }
 
 // Both products in one launch where the ring kernel is the choice for each, or pair_at_few_tokens says so, and no measured
-// choice of the shape says otherwise; SQ_ERR_BAD_ALGO, with nothing launched, where it is not.
+// choice of the shape names a third kernel; SQ_ERR_BAD_ALGO, with nothing launched, where it is not.
 static int silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, const void* w_up, const void* zs_up, void* y,
                         void* up, int M, int N, int K, int group_size, int layout, int algo, void* workspace,
                         size_t workspace_bytes, void* stream) {
@@ -767,14 +764,16 @@ static int silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, 
     if (!aligned16(x) || !aligned16(w_gate) || !aligned16(zs_gate) || !aligned16(w_up) || !aligned16(zs_up) || !aligned16(y))
         return SQ_ERR_MISALIGNED;
     if (N > (1 << 29)) return SQ_ERR_BAD_ALGO;
-    const bool ws_ok = decode_workspace(workspace, workspace_bytes, M, N, K);
     int tune = ring_tune(M, group_size);
     if (algo == SQ_ALGO_AUTO) {
-        if (M <= 16 && !pair_at_few_tokens(M, N, K, group_size, ws_ok)) return SQ_ERR_BAD_ALGO;
-        if (g_tuned_count.load(std::memory_order_relaxed) > 0 &&
-            tuned_lookup(M, N, K, group_size, full_workspace(workspace, workspace_bytes, M, N, K)) != 0)
-            return SQ_ERR_BAD_ALGO;
-        if (M > 16 && builtin_choice(M, N, K, group_size, ws_ok) != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
+        const int each = builtin_choice(M, N, K, group_size, decode_workspace(workspace, workspace_bytes, M, N, K));
+        if (M <= 16 ? !pair_at_few_tokens(M, N, K, group_size, each) : each != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
+        if (g_tuned_count.load(std::memory_order_relaxed) > 0) {
+            // A measured choice is one linear's.  Another shape of the ring kernel, or another form of the kernel that the
+            // one launch is ahead of, is no measurement against it; any other kernel is.
+            const int measured = tuned_lookup(M, N, K, group_size, full_workspace(workspace, workspace_bytes, M, N, K)) & 0xFF;
+            if (measured != SQ_ALGO_AUTO && measured != SQ_ALGO_RING && measured != each) return SQ_ERR_BAD_ALGO;
+        }
     } else {
         if ((algo & 0xFF) != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
         tune = (algo >> 8) & 0xFFFF;

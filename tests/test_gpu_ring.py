@@ -150,6 +150,30 @@ def test_gate_and_up_hold_no_more_than_the_ring_kernel_can_use(capi):
     assert held <= capi.lib().sq_w4a16_gemm_silu_dot_workspace_bytes(m, n, k) + (1 << 20) <= 40 << 20
 
 
+def test_gate_and_up_of_a_measured_shape(capi):
+    """The picker measures single linears: what it records for a shape leaves the one launch of gate and up in place where it
+    names the ring kernel, and takes it away where it names another one than the built-in choice (the ring kernel here)."""
+    g, seen = 64, set()
+    L, p = capi.lib(), lambda t: t.data_ptr()
+    capi.autotune_clear()
+    for m, n, k in [(m, n, k) for m in (20, 40, 72, 104, 136, 200) for n, k in ((1536, 1024), (2816, 2048), (4096, 2560))]:
+        w = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV)
+        zs = torch.full((n, 2 * (k // g)), 65.0, dtype=torch.float16, device=DEV)
+        x, y = torch.randn((m, k), device=DEV).half(), torch.empty((m, n), dtype=torch.float16, device=DEV)
+        ws = capi.workspace(m, n, k, DEV, gated=True)
+        one = lambda: L.sq_w4a16_gemm_silu_dot_one(p(x), p(w), p(zs), p(w), p(zs), p(y), m, n, k, g, capi.SQ_LAYOUT_L1,
+                                                   capi.SQ_ALGO_AUTO, p(ws), ws.numel(), capi._stream(None))
+        before = one()
+        word = capi.autotune(x, w, zs, n, k, g, ws=ws, reps=3)[0] & 0xFF
+        assert one() == (before if word in (0, capi.SQ_ALGO_RING) else capi.SQ_ERR_BAD_ALGO), (m, n, k, word)
+        if before == 0 and word == capi.SQ_ALGO_RING:
+            seen.add((m, n, k))
+    torch.cuda.synchronize()
+    capi.autotune_clear()
+    if not seen:
+        pytest.skip("the picker confirmed the built-in plan of every shape")
+
+
 REST = 0x10  # tune word: only the tiles of the last round of 256 split K
 SUMS = 0x20  # tune word: the scale on the sums (shapes of 32 and 64 rows, group size 128)
 
