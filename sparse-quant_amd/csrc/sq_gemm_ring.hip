@@ -388,18 +388,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         constexpr int PAIRS = 4 * NI;  // of a slice
         constexpr int NB = 4 * MI;     // row blocks of a stage, counted from slice 2 for the requests
         // Slice t of the stage in slot c, row block by row block: matrix instructions, beside them a share of the next
-        // slice's dequantisation and (AHEAD) of the rows of the slice after that (from slot cn past the middle);
-        // behind them the requests(row block).
-        auto slice = [&](auto t_, auto ahead_, int c, int cn, auto middle, auto requests) __attribute__((always_inline)) {
+        // slice's dequantisation and of the rows of the slice after that (from slot cn past the middle); behind them the
+        // requests(row block).
+        auto slice = [&](auto t_, int c, int cn, auto middle, auto requests) __attribute__((always_inline)) {
             constexpr int t = decltype(t_)::value;
-            constexpr bool AHEAD = decltype(ahead_)::value;
 #pragma unroll
             for (int mi = 0; mi < MI; mi++) {
                 if (t == 2 && mi == BAR) middle();
-                if constexpr (AHEAD) {
-                    constexpr int first = t == 2 ? BAR : 0, n = MI - first;
-                    if (mi >= first) read_rows(t < 2 ? c : cn, (t + 2) & 3, (mi - first) * MI / n, (mi - first + 1) * MI / n);
-                }
+                constexpr int first = t == 2 ? BAR : 0, n = MI - first;
+                if (mi >= first) read_rows(t < 2 ? c : cn, (t + 2) & 3, (mi - first) * MI / n, (mi - first + 1) * MI / n);
 #pragma unroll
                 for (int ni = 0; ni < NI; ni++)
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t][mi], b[t & 1][ni], acc[mi][ni], 0, 0, 0);
@@ -492,10 +489,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                     landed(true);
                     read_weights(cn);
                 };
-                slice(T0{}, Yes{}, c, cn, nothing, rest);
-                slice(T1{}, Yes{}, c, cn, nothing, rest);
-                slice(T2{}, Yes{}, c, cn, middle, begin);
-                slice(T3{}, Yes{}, c, cn, nothing, begin);
+                slice(T0{}, c, cn, nothing, rest);
+                slice(T1{}, c, cn, nothing, rest);
+                slice(T2{}, c, cn, middle, begin);
+                slice(T3{}, c, cn, nothing, begin);
                 take();
                 cp = c;
                 c = cn;
@@ -506,24 +503,23 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                 while (it + ST < plain) stage(No{});
                 issue(it + ST - 1, cp, std::false_type{}, 2 * MI * PER / NB, PER);
             }
-            // the last ST stages, and one more where K ends inside the last
+            // The last ST stages, and one more where K ends inside the last: nothing left to request but that one.  The slices
+            // are those of the loop above, so the last stage reads a slot that nobody multiplies.  (Where a workgroup has no
+            // more stages than these, reading the next stage's operands all at once behind the barrier is time: 256 x 256
+            // tiles with 9..16 stages 1.5 % of the launch, 96 x 128 and 128 x 128 with 8 or fewer 1 %.)
             for (; it < it1; it++) {
                 const int cn = c == ST - 1 ? 0 : c + 1;
                 auto middle = [&]() {
                     keep_last_word();
                     landed(it + ST - 1 < it1);
-                    if (it + 1 < it1) {
-                        read_weights(cn);
-                        read_rows(cn, 0, 0, MI);
-                        read_rows(cn, 1, 0, MI);
-                        clip(it + 1);
-                    }
                     if (it + ST < it1) issue_any(it + ST, c);
+                    read_weights(cn);
                 };
-                slice(T0{}, Yes{}, c, cn, nothing, no_requests);
-                slice(T1{}, Yes{}, c, cn, nothing, no_requests);
-                slice(T2{}, No{}, c, cn, middle, no_requests);
-                slice(T3{}, No{}, c, cn, nothing, no_requests);
+                slice(T0{}, c, cn, nothing, no_requests);
+                slice(T1{}, c, cn, nothing, no_requests);
+                slice(T2{}, c, cn, middle, no_requests);
+                clip(it + 1);
+                slice(T3{}, c, cn, nothing, no_requests);
                 take();
                 c = cn;
             }
