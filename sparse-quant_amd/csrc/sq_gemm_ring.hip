@@ -10,10 +10,14 @@
 //   * all waves in step, one barrier per stage (64 k of a wave), everything one slice (16 k) or two ahead in registers:
 //     beside the matrix instructions of a slice stand the dequantisation of the next one's weights, the LDS reads of the
 //     activations of the one after that and the stage's requests, one by one, because four waves that send theirs
-//     together wait 350 cycles for the address unit.  (Two groups of waves that alternate between matrix instructions and
-//     everything else, as the SUMS loop below still does: the other half, LDS trip, requests and half the
-//     dequantisation one after the other, takes 1050 cycles a phase against 660 of matrix instructions.  Loop cycles
-//     100 tokens x 15360x5120 42400 -> 38500, 333 x 12288x4096 83300 -> 63000, 2048 x 16384x4096 172600 -> 149500.)
+//     together wait 350 cycles for the address unit.  (With two groups of waves that alternate between matrix instructions
+//     and everything else, the other half, LDS trip, requests and half the dequantisation one after the other, takes 1050
+//     cycles a phase against 660 of matrix instructions.  Loop cycles, alternating -> in step: 100 tokens x 15360x5120
+//     42400 -> 38500, 333 x 12288x4096 83300 -> 63000, 2048 x 16384x4096 172600 -> 149500.)
+//   * tiles of 32 rows alternate all the same: their two matrix instructions per slice hide no LDS trip (in step
+//     against alternating, geometric means over 200 weights and token counts: 32 x 128 tiles 4.5 % slower with up to 4
+//     stages, 4 % with 5..8, 2.5 % with 9..32; 32 x 64 tiles 2.5 % slower, level, 1 % faster.  800 tokens x 1024x1024 6.6 /
+//     7.2 us, 32 x 8192x2048 at group size 64 8.1 / 8.5).  So does the scale on the sums (SUMS below).
 //   * K is split over the waves of the workgroup (WK groups of 64 consecutive k each per stage of KS = 64 WK), so that
 //     a weight row is read in 64..256-byte pieces, a stage holds 40..50 KB, and narrow weights fill the chip without
 //     partial tiles in memory.  The groups' sums meet in LDS at the end.
@@ -198,6 +202,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     constexpr int BM = S::BM, BN = S::BN, KS = S::KS, SB = S::SB, XI = S::XI, WI = S::WI, ZI = S::ZI, ZL = S::ZL, PER = S::PER, P = S::P;
     constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = S::XB + S::WB;
     constexpr int H = 4;  // 16-wide k slices per stage and wave
+    constexpr bool ALTERNATE = SUMS || MI == 1;  // two groups of waves in turn (see the head of this file)
+    static_assert(!ALTERNATE || S::NW == 8, "waves 0..3 and 4..7");
     static_assert(!SUMS || (MI * NI <= 4 && GS == 7 && S::NW == 8), "a stage of a wave lies in one group, and the registers suffice");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S::LDS];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
@@ -345,7 +351,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             for (int v = 0; v < 16; v++) acc[mi][ni][v] = 0.f;
 
     auto wait_lds = []() { __builtin_amdgcn_s_waitcnt(0xC07F); };  // lgkmcnt(0), where the compiler sees it: later waits stay counted
-    if constexpr (!SUMS) {
+    if constexpr (!ALTERNATE) {
         half8_t a[4][MI], b[2][NI];               // activations of slice t in a[t], weights of slice t in b[t & 1]
         uint32_t q[NI][4], q3[NI], qn[NI][4];     // packed words of the stage (the last one apart), and of the next stage
         half2_t zs[NI], zn[NI], z1024[NI];
@@ -528,31 +534,38 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         half8_t a[H][MI], b[H][NI];
         half2_t zs[NI];
         uint32_t q[NI][H];
-        float16_t part_sum[MI][NI];  // of the stage before, and its scales
-        float part_scale[NI];
+        float16_t part_sum[SUMS ? MI : 1][SUMS ? NI : 1];  // of the stage before, and its scales
+        float part_scale[SUMS ? NI : 1];
+        if constexpr (SUMS) {
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++) {
-            part_scale[ni] = 0.f;
+            for (int ni = 0; ni < NI; ni++) {
+                part_scale[ni] = 0.f;
 #pragma unroll
-            for (int mi = 0; mi < MI; mi++)
+                for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) part_sum[mi][ni][v] = 0.f;
+                    for (int v = 0; v < 16; v++) part_sum[mi][ni][v] = 0.f;
+            }
         }
         // (pinned, so that the wait for the matrix instructions' results is not moved in front of the barrier)
         auto fold = [&]() {
+            if constexpr (SUMS) {
 #pragma unroll
-            for (int mi = 0; mi < MI; mi++)
+                for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-                for (int ni = 0; ni < NI; ni++) {
-                    asm volatile("" : "+v"(part_sum[mi][ni]));
+                    for (int ni = 0; ni < NI; ni++) {
+                        asm volatile("" : "+v"(part_sum[mi][ni]));
 #pragma unroll
-                    for (int v = 0; v < 16; v++)
-                        acc[mi][ni][v] = __builtin_fmaf(part_sum[mi][ni][v], part_scale[ni], acc[mi][ni][v]);
-                }
+                        for (int v = 0; v < 16; v++)
+                            acc[mi][ni][v] = __builtin_fmaf(part_sum[mi][ni][v], part_scale[ni], acc[mi][ni][v]);
+                    }
+            }
         };
         auto unpack = [&](int t) {
 #pragma unroll
-            for (int ni = 0; ni < NI; ni++) b[t][ni] = integers8(q[ni][t], (half2_t){zs[ni].x, zs[ni].x}, nm);
+            for (int ni = 0; ni < NI; ni++) {
+                const half2_t z = {zs[ni].x, zs[ni].x};
+                b[t][ni] = SUMS ? integers8(q[ni][t], z, nm) : dequant8(q[ni][t], z, (half2_t){zs[ni].y, zs[ni].y}, nm);
+            }
         };
         // The wave's operands of the stage in slot c into registers.
         auto fetch = [&](int c) {
@@ -571,7 +584,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         };
         // Weights past the end of K get the scale 0 (only the last stage can hold any).
         auto clip = [&](int it) {
-            if (it * KS + 64 * kg >= K) {
+            if (it * KS + 64 * kg + (GS == 5 ? 32 * lc : 0) >= K) {
 #pragma unroll
                 for (int ni = 0; ni < NI; ni++) zs[ni].y = (half_t)0.f;
             }
@@ -604,12 +617,18 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
                 for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-                    for (int ni = 0; ni < NI; ni++)
-                        part_sum[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                            a[t][mi], b[t][ni], t == 0 ? (float16_t){} : part_sum[mi][ni], 0, 0, 0);
+                    for (int ni = 0; ni < NI; ni++) {
+                        if constexpr (SUMS)
+                            part_sum[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                a[t][mi], b[t][ni], t == 0 ? (float16_t){} : part_sum[mi][ni], 0, 0, 0);
+                        else
+                            acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t][mi], b[t][ni], acc[mi][ni], 0, 0, 0);
+                    }
+            if constexpr (SUMS) {
 #pragma unroll
-            for (int ni = 0; ni < NI; ni++) part_scale[ni] = (float)zs[ni].y;
-            constexpr int MF = H / 2 * MI * NI, VA = (10 * NI * (H / 2) + MF - 1) / MF;
+                for (int ni = 0; ni < NI; ni++) part_scale[ni] = (float)zs[ni].y;
+            }
+            constexpr int MF = H / 2 * MI * NI, VA = ((SUMS ? 10 : 14) * NI * (H / 2) + MF - 1) / MF;
 #pragma unroll
             for (int i = 0; i < MF; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
