@@ -711,6 +711,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
     }
 
+    // One test in front of all requests of multiplicand and residual: a launch without them otherwise passes a branch for
+    // every chunk (256 x 256 tiles with 9..16 stages 4 % slower, 64 x 256 and 128 x 128 with up to four 2 %).
+    const bool extras = !PAIR && (epi.mul || epi.residual);
     if constexpr (WK == 1) {
         if (ks == 1) {
             // No sums to add: every wave turns its own half slices (16 rows) row-major through a region of its own, two in
@@ -749,13 +752,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                 }
             };
             if (!PAIR && epi.bias && n < N) bias = Cols<8>::load(epi.bias + n);
+            if (extras) {
 #pragma unroll
-            for (int hs = 0; hs < DEEP; hs++) request(hs);
+                for (int hs = 0; hs < DEEP; hs++) request(hs);
+            }
             __syncthreads();
             turn_over(0);
 #pragma unroll
             for (int hs = 0; hs < 2 * MI; hs++) {
-                if (hs + DEEP < 2 * MI) request(hs + DEEP);
+                if (extras && hs + DEEP < 2 * MI) request(hs + DEEP);
                 if (hs + 1 < 2 * MI) turn_over(hs + 1);
 #pragma unroll
                 for (int g = 0; g < 16 / RP; g++) {
@@ -804,13 +809,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
     };
     auto column = [](int cc, int e) __attribute__((always_inline)) { return cc * EO + e % EO + (e / EO) * BO; };
-    constexpr int SL = S::LDS / S::TAIL < MI ? S::LDS / S::TAIL : MI;  // slices at once
+    // Slices at once: several behind one barrier where a slice is one chunk a thread (tiles of 128 columns, 96 and 128 rows:
+    // one by one 0.5..1 % slower); else one, so that a slice's stores go out while the next one's sums are added (64 x 256
+    // tiles with up to 4 stages 2 % slower with all slices at once, 128 x 256 1 %).
+    constexpr int SL = NI > 1 || MI < 3 ? 1 : S::LDS / S::TAIL < MI ? S::LDS / S::TAIL : MI;
     constexpr int SF = S::TAIL / 4;
     Extra<EO> extra[SL][G];
 #pragma unroll
     for (int mi = 0; mi < MI; mi++) {
         if (mi % SL == 0) {
-            if (ks == 1) {
+            if (extras && ks == 1) {
 #pragma unroll
                 for (int sl = 0; sl < SL && mi + sl < MI; sl++)
 #pragma unroll
@@ -869,9 +877,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             for (int l0 = 0; l0 < L; l0 += U) {
                 u32x4_t pv[U][NZ];
                 Extra<EO> px[U / (EV / 4)];
+                if (extras) {
 #pragma unroll
-                for (int i0 = 0; i0 < U; i0 += EV / 4)
-                    request(px[i0 / (EV / 4)], (l0 + i0) / (EV / 4) / G, (l0 + i0) / (EV / 4) % G);
+                    for (int i0 = 0; i0 < U; i0 += EV / 4)
+                        request(px[i0 / (EV / 4)], (l0 + i0) / (EV / 4) / G, (l0 + i0) / (EV / 4) % G);
+                }
                 const uint32_t base = (uint32_t)(((long)tr * tsz + (long)l0 * (S::NT * 4) + tid * 4) * 4);
                 const uint32_t zstep = (uint32_t)((long)rest * tsz * 4);
 #pragma unroll
