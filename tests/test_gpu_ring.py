@@ -1,5 +1,7 @@
-"""The ring kernel (17 tokens up): every tile shape, K split and group size on ragged M, N and K against the oracle; with
+"""The ring kernel: every tile shape, K split and group size on ragged M, N and K against the oracle; with
 the scale on the sums, as few tokens take it, against (q - z) s in float64."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -131,6 +133,83 @@ def test_ring_gate_and_up_in_one_launch(capi, m, n, k, g):
     check(y, [real_weight(i, g) for i in d] if scaled else w_hat, "automatic")
     ref = x64 @ (real_weight(d[1], g) if scaled else w_hat[1]).T
     assert np.all(np.abs(up.cpu().numpy() - ref) <= 2.0 ** -11 * np.abs(ref) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w_hat[1]).T) * 2 + 2.0 ** -24)
+
+
+class _Epilogue(ctypes.Structure):
+    """sq::Epilogue of csrc/sq_kernels.h."""
+    _fields_ = [("bias", ctypes.c_void_p), ("residual", ctypes.c_void_p), ("act", ctypes.c_int), ("mul", ctypes.c_void_p)]
+
+
+@pytest.mark.parametrize("m,n,k,g", [(1, 64, 128, 128), (33, 136, 640, 128), (97, 264, 1408, 64), (40, 392, 1056, 32),
+                                     (300, 520, 384, 128)])
+@pytest.mark.parametrize("shape", range(1, 10))
+def test_ring_multiplicand(capi, shape, m, n, k, g):
+    """silu(x W^T + bias) * mul + residual by every tile shape, unsplit and with K split (the last round too).  The library's
+    entry points set a multiplicand only where gate and up take a launch each, which leaves the larger tiles to choices
+    that a timing makes: here the launcher itself is called."""
+    launch = getattr(capi.lib(), "_ZN2sq16launch_gemm_ringEPKvS1_S1_PvS2_miiiiiNS_8EpilogueEP12ihipStream_t")
+    v, i = ctypes.c_void_p, ctypes.c_int
+    launch.restype, launch.argtypes = i, [v] * 5 + [ctypes.c_size_t] + [i] * 5 + [_Epilogue, v]
+    d = orc.synth_linear(n, k, g, seed=n + k)
+    x = orc.synth_x(m, k, seed=m)
+    rng = np.random.default_rng(m)
+    bias, mul, res = (rng.normal(0, 1, s).astype(np.float16) for s in (n, (m, n), (m, n)))
+    x64, w64, b64, mul64, r64 = (a.astype(np.float64) for a in (x, orc.dequant_l1(d["w_l1"], d["zs_l1"], g), bias, mul, res))
+    t = x64 @ w64.T + b64
+    y64 = t / (1 + np.exp(-t)) * mul64
+    # errors of the sum (K fp32 additions) through d silu <= 1.1, those of exp, rcp and the products (8 ulp of fp32), one
+    # rounding to fp16
+    es = k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T + np.abs(b64))
+    xd, w, zs, bd, md, rd = (to_dev(a) for a in (x, d["w_l1"], d["zs_l1"], bias, mul, res))
+    ws = torch.zeros(65536 + (96 << 20), dtype=torch.uint8, device=DEV)
+    p = lambda a: None if a is None else a.data_ptr()
+    for residual in (None, rd):
+        ref = y64 + (0 if residual is None else r64)
+        bound = 2.0 ** -11 * np.abs(ref) + 1.1 * es * np.abs(mul64) + 2.0 ** -20 * (np.abs(y64) + np.abs(ref)) + 2.0 ** -24
+        ran = 0
+        for word in (shape, shape | (2 << 8), shape | REST | (3 << 8)):
+            y = torch.full((m, n), float("nan"), dtype=torch.float16, device=DEV)
+            rc = launch(p(xd), p(w), p(zs), p(y), p(ws), ws.numel(), m, n, k, g, word,
+                        _Epilogue(p(bd), p(residual), capi.SQ_ACT_SILU, p(md)), capi._stream(None))
+            assert rc == 0 or (word != shape and rc == 1)  # (hipErrorInvalidValue: fewer stages than parts)
+            if rc:
+                continue
+            ran += 1
+            err = np.abs(y.cpu().numpy().astype(np.float64) - ref)
+            assert np.all(err <= bound), (hex(word), np.max(err / bound))
+            assert capi.workspace_is_clean(ws)
+        assert ran >= 1
+
+
+def gated_operands(m, n, k, g, seed):
+    """x, then weight and zeros/scales of gate and of up, with their float64 products: of W_hat, and of (q - z) s unrounded."""
+    from sqamd import capi as c
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn((m, k), device=DEV, generator=gen).half()
+    dev, hat, real = [], [], []
+    for _ in range(2):
+        w = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=gen)
+        z = torch.randint(0, 16, (n, k // g), device=DEV, generator=gen).half()
+        s = (torch.rand((n, k // g), device=DEV, generator=gen) * 0.002 + 0.0002).half()
+        pairs = lambda v: torch.stack([z, v], -1).reshape(n, -1).contiguous()
+        dev += [w, pairs(s)]
+        hat.append(x.double() @ c.dequant(w, dev[-1], n, k, g).double().t())
+        real.append(x.double() @ (c.dequant(w, pairs(torch.ones_like(s)), n, k, g).double() * s.double().repeat_interleave(g, 1)).t())
+    return x, dev, hat, real
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 8192, 4096), (9, 5128, 5120), (16, 5128, 5120)])
+def test_gate_and_up_in_two_ring_launches(capi, m, n, k):
+    """Group size 32 at few tokens on large weights: each projection is the ring kernel's, the second multiplies the first
+    into its store."""
+    x, dev, (gate, up), _ = gated_operands(m, n, k, 32, seed=m)
+    ref = torch.nn.functional.silu(gate) * up
+    for ws in (None, capi.workspace(m, n, k, DEV, gated=True)):
+        y, u = capi.gemm_silu_dot(x, *dev, n, k, 32, ws=ws, use_workspace=False)
+        # the up projection is rounded to fp16 before the product (2^-11) and the product is (2^-11); the sums' fp32 errors
+        # are those of a result of norm-wise relative error k^(1/2) 2^-24 < 2^-17
+        assert (u.double() - up).norm() <= (2.0 ** -11 + 2.0 ** -17) * up.norm()
+        assert (y.double() - ref).norm() <= (2.0 ** -10 + 2.0 ** -15) * ref.norm()
 
 
 def test_gate_and_up_hold_no_more_than_the_ring_kernel_can_use(capi):
