@@ -222,23 +222,54 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
 // with the scale on the sums, which is the rounding of the output, 2.9e-4 with W_hat).
 int ring_tune(int M, int g) { return g == 128 && M <= 64 ? sq::RING_SUMS : 0; }
 
-// Gate and up of a gated MLP in one ring launch at up to 16 tokens, us, two launches / one.  Group size 64, 5 tokens up, where
-// the two would be the streaming or the ring kernel's (W_hat there as here): 7680x2560 17.6 / 9.9, 2816x1024 6.3 / 5.7, 13824x4608
-// 29.2 / 22.8, 12288x4096 20.4 / 19.8; 4096x4096 10.3 / 10.3.  Group size 128 (the scale on the sums here as there):
+// Gate and up of a gated MLP in one ring launch at up to 16 tokens, us, two launches / one.  The lines were drawn through a sweep
+// of 1200 weights (256..33000 rows, K 768..10500) x 1..16 tokens, with and without a workspace: where one launch is taken it takes
+// 0.8 of the two in the geometric mean, at worst 1.05.
+// Group size 64, 5 tokens up, where the two would be the streaming or the ring kernel's (W_hat there as here): 7680x2560 17.6 /
+// 9.9, 2816x1024 6.3 / 5.7, 13824x4608 29.2 / 22.8, 12288x4096 20.4 / 19.8; but 24576x2048 at 5 20.7 / 21.1, 8512x3968 17.0 / 18.1.
+// Group size 128 (the scale on the sums here as there):
 //   the streaming kernel's K ranges leave its chunk slots part empty: 13696x5120 at 8 tokens 30.7 / 25.3, 5632x2048 8.7 / 7.6,
-//   2816x1024 6.3 / 5.8, 28672x5120 52.6 / 47.6; with more tiles than a round and a short K 24576x2048 20.7 / 21.1 at 5
-//   they fill them: one launch where its 32 x 128 tiles do not leave half the chip or nearly a round idle: 8192x4096 16.4 /
-//   13.1, 14336x4096 20.4 / 20.0, 16384x4096 22.1 / 20.8; but 11008x4096 17.6 / 19.3 (172 tiles), 2048x4096 8.7 / 8.8 (32)
-//   1 and 2 tokens (the GEMV): 8192x5120 17.8 / 15.7, 15360x5120 29.0 / 24.5; but 7680x3072 10.5 / 10.8
-bool pair_at_few_tokens(int M, int N, int K, int g, int each) {  // each: the kernel of the two launches
+//   2816x1024 6.3 / 5.8, 28672x5120 52.6 / 47.6; but at 3 19072x4992 without a workspace 32.0 / 36.8, 26112x5504 42.7 / 48.2
+//   they fill them: one launch where its 32 x 128 tiles leave neither half the chip nor most of a round idle: 8192x4096 16.4 /
+//   13.1, 14336x4096 20.4 / 20.0, 16384x4096 22.1 / 20.8; but 8256x4096 14.2 / 17.5 (129 tiles), 11008x4096 17.6 / 19.3 (172),
+//   2048x4096 8.7 / 8.8 (32), and at 3 without a workspace 8384x10112 32.4 / 37.4
+//   1 and 2 tokens (the GEMV): 8192x5120 17.8 / 15.7, 15360x5120 29.0 / 24.5; but 7680x3072 10.5 / 10.8, and at 1 9856x5120 18.2 /
+//   20.2 (154 tiles), 12992x5248 21.5 / 22.9 (203)
+// With few tokens a last stage of K that is half empty (K % 256 != 0) is time: 11584x5760 at 3 22.3 / 24.7, 11200x3712 at 5 and
+// group size 64 17.5 / 18.4.
+// Up to 8 tokens and 64 tiles the latency of two decode launches stands against one ring launch's and the exchange of its K
+// ranges, or a K that is not split: 2048x2048 at 3 6.9 / 8.0, at 5 and group size 64 7.1 / 7.7; 1408x2304 at 3 7.2 / 8.0;
+// 4096x3328 at 5 and group size 64 9.9 / 10.9, without a workspace 512x3840 8.7 / 10.8; 3520x2944 at 5 8.9 / 9.5;
+// 3328x3712 at 16 and group size 64 without a workspace 11.3 / 12.2.
+bool pair_at_few_tokens(int M, int N, int K, int g, int each, bool ws_ok) {  // each: the kernel of the two launches
     const long tiles = (2L * N + 127) / 128;
-    if (g == 64) return M >= 5 && (tiles <= 256 || K > 4096) && (each == SQ_ALGO_STREAM || each == SQ_ALGO_RING);
+    const bool half_stage = K % 256 != 0;
+    if (g == 64) {
+        if (M < 5 || (tiles > 256 && K <= 4096) || (each != SQ_ALGO_STREAM && each != SQ_ALGO_RING)) return false;
+        if (K > 4096) return true;
+        if (M > 8) return tiles > 64 || K <= 3328 || ws_ok;
+        if (K > 3328 && half_stage) return false;
+        if (tiles > 64) return tiles <= 128 || tiles > 140 || K <= 3840;
+        return K <= 1024 || (K <= 1536 && tiles > 16) || (K > 2048 && (K <= 2560 || (ws_ok && tiles <= 32)));
+    }
     if (g != 128) return false;
     const int chunks = K / 128, parts = (chunks + 31) / 32;
-    const bool filled = chunks * 4 >= parts * 32 * 3;
-    if (M <= 2) return !filled && K > 4096 && tiles >= 128 && tiles <= 256;
-    if (!filled) return tiles <= 256 || K > 4096;
-    return (tiles > 64 && tiles <= 140) || (tiles >= 224 && tiles <= 256);
+    const bool filled = chunks * 100 >= parts * 32 * (parts == 1 && M > 4 && M <= 8 ? 70 : 75);
+    if (M <= 2) {
+        if (filled || K <= 4096 || tiles > 256 || (half_stage && tiles > 128)) return false;
+        return tiles == 128 || tiles >= (K <= 4608 ? (M == 1 ? 176 : 128) : (M == 1 ? 208 : 176));
+    }
+    if (filled) {
+        const bool spilled = K > 4096 ? M <= 4 && !ws_ok : K > (M <= 4 ? 3584 : 3328);  // tiles past 128 cost a round
+        const bool whole = !half_stage || M > 8 || K > 4096;
+        return (tiles > 64 && tiles <= (spilled || !whole ? 128 : 140)) || (whole && tiles >= 224 && tiles <= 256);
+    }
+    if (M <= 4 && K > 4096 && tiles > 128 && (half_stage || (!ws_ok && K > 5632))) return false;
+    if (tiles > 256) return K > 4096 && (M > 4 || (ws_ok && K <= 5120));
+    if (M > 8 || tiles > 64 || K <= 1024 || K > 4096) return M > 8 || tiles > 64 || K <= 8192 || ws_ok;
+    if (K <= 2048) return tiles == 64 && K <= 1536;
+    if (K <= 2560) return M > 4 || tiles > 31;
+    return ws_ok && (M <= 4 ? tiles > 48 : !half_stage || tiles <= 32);
 }
 
 int gemm_dispatch(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int group_size,
@@ -766,8 +797,9 @@ static int silu_dot_one(const void* x, const void* w_gate, const void* zs_gate, 
     if (N > (1 << 29)) return SQ_ERR_BAD_ALGO;
     int tune = ring_tune(M, group_size);
     if (algo == SQ_ALGO_AUTO) {
-        const int each = builtin_choice(M, N, K, group_size, decode_workspace(workspace, workspace_bytes, M, N, K));
-        if (M <= 16 ? !pair_at_few_tokens(M, N, K, group_size, each) : each != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
+        const bool ws_ok = decode_workspace(workspace, workspace_bytes, M, N, K);
+        const int each = builtin_choice(M, N, K, group_size, ws_ok);
+        if (M <= 16 ? !pair_at_few_tokens(M, N, K, group_size, each, ws_ok) : each != SQ_ALGO_RING) return SQ_ERR_BAD_ALGO;
         if (g_tuned_count.load(std::memory_order_relaxed) > 0) {
             // A measured choice is one linear's.  Another shape of the ring kernel, or another form of the kernel that the
             // one launch is ahead of, is no measurement against it; any other kernel is.

@@ -212,6 +212,30 @@ def test_gate_and_up_in_two_ring_launches(capi, m, n, k):
         assert (y.double() - ref).norm() <= (2.0 ** -10 + 2.0 ** -15) * ref.norm()
 
 
+@pytest.mark.parametrize("m,n,k,g,use_ws,one", [
+    (1, 8192, 5120, 128, False, True), (2, 8192, 5120, 128, False, True), (1, 8320, 5120, 128, False, False),
+    (3, 8192, 4096, 128, True, True), (3, 8256, 4096, 128, True, False), (16, 8256, 4096, 128, True, False),
+    (3, 2048, 2048, 128, True, False), (9, 2048, 2048, 128, True, True), (3, 1408, 2304, 128, True, False),
+    (5, 1408, 2304, 128, True, True), (5, 1408, 2688, 128, False, False), (5, 2048, 2048, 64, True, False),
+    (5, 4096, 3328, 64, True, False), (5, 512, 3840, 64, False, False), (5, 512, 3840, 64, True, True),
+    (3, 17920, 5120, 128, False, False), (3, 17920, 5120, 128, True, True), (5, 8512, 3968, 64, True, False),
+    (3, 11584, 5760, 128, True, False), (3, 11584, 5632, 128, True, True)])
+def test_gate_and_up_of_few_tokens_in_one_launch_where_it_is_faster(capi, m, n, k, g, use_ws, one):
+    """Both sides of the lines between one launch and two, and the result of the one that is chosen."""
+    x, dev, hat, real = gated_operands(m, n, k, g, seed=n)
+    ws = capi.workspace(m, n, k, DEV, gated=True) if use_ws else None
+    L, p = capi.lib(), lambda t: None if t is None else t.data_ptr()
+    y = torch.empty((m, n), dtype=torch.float16, device=DEV)
+    rc = L.sq_w4a16_gemm_silu_dot_one(p(x), *(p(t) for t in dev), p(y), m, n, k, g, capi.SQ_LAYOUT_L1, capi.SQ_ALGO_AUTO, p(ws),
+                                      0 if ws is None else ws.numel(), capi._stream(None))
+    assert rc == (capi.SQ_OK if one else capi.SQ_ERR_BAD_ALGO)
+    y = capi.gemm_silu_dot(x, *dev, n, k, g, out=y, ws=ws, use_workspace=False)[0]
+    # (two launches round the up projection and the product, the GEMV and the sums scaled neither weight; fp32 sums as above)
+    gate, up = real if g == 128 else hat
+    ref = torch.nn.functional.silu(gate) * up
+    assert (y.double() - ref).norm() <= (2.0 ** -10 + 2.0 ** -15) * ref.norm()
+
+
 def test_gate_and_up_hold_no_more_than_the_ring_kernel_can_use(capi):
     """The extension keeps its workspace per stream: 40 MB for 11008 x 4096 at 333 tokens, not the 135 MB that the tiled GEMM
     would want for a weight of 2 x 11008 rows."""
