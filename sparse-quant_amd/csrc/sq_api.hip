@@ -111,8 +111,13 @@ enum : unsigned {
     P_RING = 1u << 10,        // the ring kernel can address the operands
     P_SMALL_K2048 = 1u << 11,   // N * K <= 2^22 elements and K <= 2048
     P_G64 = 1u << 13,           // group size 64
-    P_SPILL = 1u << 14,         // the streaming kernel's 64-row workgroups times K ranges come to 257..400: a second round, part empty
+    // the streaming kernel's 64-row workgroups times K ranges come to 257..400 (336 with four K ranges: 42 tiles of 128 columns,
+    // the last that the ring kernel's six parts of K keep in one round): a second round, part empty
+    P_SPILL = 1u << 14,
     P_PARTS4 = 1u << 15,        // four K ranges of the streaming kernel or more
+    P_PARTS5 = 1u << 16,        // five
+    P_OVER_128 = 1u << 17,    // more than 128 of those workgroups
+    P_FEW_OVER = 1u << 18,      // at most 160 of them, or K ranges filled less than 0.6: two K ranges either way
     P_SHORT_ROUNDS = 1u << 12,  // many rounds of 128 x 256 tiles over a short K (see builtin_choice)
     // what the streaming kernel needs of a K that it splits
     P_STREAM_SPLIT = P_G128_64 | P_K128 | P_WS | P_K_LE_32768,
@@ -130,15 +135,19 @@ const ChoiceRule kChoiceRules[] = {
     // (in place of the streaming kernel alone: where that does not run, the GEMV keeps the scale in fp32 at 5..8 tokens and
     // group size 64, and without a workspace the ring kernel leaves most of the chip idle: 3136x5888 at 9 tokens 13.5 vs 8.3
     // (16-column kernel), 4672x6016 at 8 14.1 vs 10.7 (GEMV))
-    {5, 16, P_OVER_16M | P_G64 | P_STREAM_SPLIT | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
-     "group size 64, 8 / 16 tokens: 4608x4608 9.3 / 9.6 vs 10.2 / 11.2 (streaming kernel), 5120x5120 10.3 / 10.7 vs 10.4 / 11.3; at "
-     "group size 128 5120x5120 10.4 / 10.5 vs 9.9 / 10.4"},
+    {5, 8, P_OVER_16M | P_G64 | P_STREAM_SPLIT | P_OVER_128 | P_FEW_OVER | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
+     "group size 64, 8 tokens: 4608x4608 9.3 vs 10.2 (streaming kernel), 5120x5120 10.3 vs 10.4, 5376x4608 0.92 of it, 4736x5376 at 5 "
+     "0.95; but 3072x6016 1.16, 3008x5888 at 5 1.12, 5696x5888 at 6 1.06, 2432x8576 1.13; at group size 128 5120x5120 10.4 vs 9.9"},
+    {9, 16, P_OVER_16M | P_G64 | P_STREAM_SPLIT | P_OVER_128 | P_RING, P_CHUNK_FILL | P_K_LE_4096, SQ_ALGO_RING,
+     "group size 64, 16 tokens: 4608x4608 9.6 vs 11.2 (streaming kernel), 5120x5120 10.7 vs 11.3, 3200x8704 0.93 of it; but 3648x4992 "
+     "1.07, 2688x8576 1.08, 4096x6016 at 10 1.14; at group size 128 5120x5120 10.5 vs 10.4"},
     // K ranges and row blocks that make a second round of few workgroups
-    {5, 16, P_G64 | P_SPILL | P_PARTS4 | P_STREAM_SPLIT | P_RING, P_K_LE_4096, SQ_ALGO_RING,
-     "group size 64, 8 / 16 tokens: 4352x17408 16.5 / 17.6 vs 19.8 / 21.1 (streaming kernel), 5120x13824 14.6 / 15.2 vs 15.4 / 19.8"},
+    {5, 8, P_G64 | P_SPILL | P_PARTS5 | P_STREAM_SPLIT | P_RING, P_K_LE_4096, SQ_ALGO_RING,
+     "group size 64, 8 tokens: 4352x17408 16.5 vs 19.8 (streaming kernel), 15 weights of five ranges 0.78..0.94 of it; of four ranges "
+     "0.95..1.09 (5120x13824 14.6 vs 15.4, 4288x15872 at 6 16.7 vs 15.3)"},
     {9, 16, P_SPILL | P_PARTS4 | P_STREAM_SPLIT | P_RING, P_K_LE_4096, SQ_ALGO_RING,
-     "16 tokens: 4352x17408 17.3 vs 19.4 (streaming kernel), 5120x13824 14.6 vs 15.9, 5120x16384 17.0 vs 17.4; 8 tokens 5120x20480 "
-     "18.7 vs 18.0"},
+     "16 tokens: 4352x17408 17.3 vs 19.4 (streaming kernel), 5120x13824 14.6 vs 15.9, 5120x16384 17.0 vs 17.4; but 5504x15232 at 10 "
+     "1.22 of it, 5632x16000 at group size 64 21.6 vs 20.4; 8 tokens 5120x20480 18.7 vs 18.0"},
     {9, 16, P_G64 | P_SPILL | P_STREAM_SPLIT | P_RING, P_K_LE_4096, SQ_ALGO_RING,
      "16 tokens, group size 64: 10240x8192 17.6 vs 21.0 (streaming kernel), 6144x12288 17.9 vs 19.9; at group size 128 17.4 vs 16.9, "
      "17.7 vs 16.2"},
@@ -194,8 +203,11 @@ int builtin_choice(int M, int N, int K, int g, bool ws_ok) {
         const int chunks = K / 128, ks0 = (chunks + 31) / 32;
         if (ks0 > 0 && chunks * 4 >= ks0 * 32 * 3) p |= P_CHUNK_FILL;
         const long wgs = (long)((N + 63) / 64) * ks0;
-        if (wgs > 256 && wgs <= 400) p |= P_SPILL;
+        if (wgs > 256 && wgs <= (ks0 == 4 ? 336 : 400)) p |= P_SPILL;
         if (ks0 >= 4) p |= P_PARTS4;
+        if (ks0 >= 5) p |= P_PARTS5;
+        if (wgs > 128) p |= P_OVER_128;
+        if (ks0 <= 2 && (wgs <= 160 || chunks * 10 < ks0 * 32 * 6)) p |= P_FEW_OVER;
     }
     if (K <= 4096) p |= P_K_LE_4096;
     if (K <= 8192) p |= P_K_LE_8192;

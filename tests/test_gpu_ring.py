@@ -337,6 +337,23 @@ def test_few_tokens_round_no_weight_to_half(capi, m, n, k, g, use_ws):
     assert (y.double() - ref).norm() <= 1.1 * rounding
 
 
+@pytest.mark.parametrize("m,n,k,g,algo", [
+    (8, 4608, 4608, 64, "RING"), (8, 3072, 5888, 64, "STREAM"), (8, 5632, 5888, 64, "STREAM"), (7, 2560, 8704, 64, "STREAM"),
+    (12, 4736, 5376, 64, "RING"), (12, 3584, 5376, 64, "STREAM"), (8, 4352, 17408, 64, "RING"), (8, 5632, 15616, 64, "STREAM"),
+    (10, 4736, 14336, 128, "RING"), (10, 5504, 15232, 128, "STREAM")])
+def test_few_tokens_take_the_kernel_that_measures_ahead(capi, m, n, k, g, algo):
+    """Both sides of the lines between the streaming and the ring kernel where K is split; the two add in different orders."""
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    w = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=gen)
+    zs = (torch.rand((n, 2 * (k // g)), device=DEV, generator=gen) + 0.01).half()
+    x = torch.randn((m, k), device=DEV, generator=gen).half()
+    ws = capi.workspace(m, n, k, DEV)
+    word = {"STREAM": capi.SQ_ALGO_STREAM, "RING": capi.SQ_ALGO_RING | ((SUMS if g == 128 else 0) << 8)}
+    y, same = (capi.gemm_ws(x, w, zs, n, k, g, algo=a, ws=ws) for a in (capi.SQ_ALGO_AUTO, word.pop(algo)))
+    assert torch.equal(y, same)
+    assert not torch.equal(y, capi.gemm_ws(x, w, zs, n, k, g, algo=word.popitem()[1], ws=ws))
+
+
 @pytest.mark.parametrize("m,n,k", [(5, 3328, 5120), (8, 5120, 5120), (6, 4096, 4672)])
 def test_few_tokens_round_no_weight_to_half_without_a_workspace_at_group_size_64(capi, m, n, k):
     test_few_tokens_round_no_weight_to_half(capi, m, n, k, 64, False)
