@@ -943,14 +943,16 @@ static hipError_t launch_shape(const void* x, const void* w, const void* zs, con
 }
 
 // What a shape costs, in us: a workgroup takes `step0 + step1 * a` per stage of K and `fixed` besides (first loads, sums,
-// stores), a = the share of the 256 CUs that its round keeps busy (memory and clock are shared); a K split adds the
+// stores), a = the share of the 256 CUs that its round keeps busy (memory and clock are shared), and no less per stage than the
+// rows that the eight XCDs ask for take at 6.5 TB/s (consecutive tiles of a column are one XCD's, so that narrow weights at
+// thousands of tokens read the activations once for every column); a K split adds the
 // exchange of the partial tiles, `ex0 + ex1 * parts + exmb` per MB of them, and every round of 256 after the first `round`.
 // One workgroup fills a CU.  Least-squares
 // fits: tiles of 32 rows to 9000 timings of 18 weights (3072 x 1024 .. 28672 x 8192) x 23 token counts (12 .. 4096), the
-// others, with the loop in step, to 7300 timings of 26 weights (1536 x 6144 .. 24576 x 8192) x 34 token counts (20 .. 4096),
-// all shapes and splits, then adjusted for the choice (rms error 6..7 %): within 0.5 % of the best in the geometric mean
-// (1.8 % with the constants of the alternating loop, which left the 128 x 128 tiles out: 224 tokens x 15360x5120 52 where
-// they take 43), 19 % at worst (512 tokens x 8192x1024).
+// others then adjusted for the choice alone on all shapes and splits of 13500 weights (512 .. 20480 rows, K 768 .. 16384) with
+// a token count each (17 .. 4096): on 1350 that were kept back 0.25 % above the best in the geometric mean, 1.1 % of them by
+// more than 5 %, at worst 11 % (with constants fitted to 26 weights from 1536 rows up, and without the rate, 0.5 %, 3 % and
+// 30 %: 3272 tokens x 1024x1152 20.2 us where they take 14.5).
 struct RingTile {
     int bm, bn, ks;
     float fixed, step0, step1, ex0, ex1, exmb, round;
@@ -958,13 +960,13 @@ struct RingTile {
 static const RingTile kRingTiles[] = {
     {32, 64, 512, 1.723f, 0.829f, 0.160f, 0.301f, 0.226f, 0.861f, 0.f},
     {32, 128, 256, 1.498f, 0.754f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f},
-    {64, 128, 256, 2.575f, 0.763f, 0.379f, 0.745f, 0.539f, 0.391f, 1.281f},
-    {96, 128, 128, 2.852f, 0.474f, 0.337f, 1.205f, 0.592f, 0.286f, 1.910f},
-    {64, 256, 128, 2.544f, 0.820f, 0.309f, 1.556f, 0.799f, 0.335f, 1.349f},
-    {96, 256, 128, 4.013f, 0.701f, 0.595f, 1.206f, 1.294f, 0.195f, 2.135f},
-    {128, 128, 128, 2.534f, 0.521f, 0.427f, 0.491f, 0.920f, 0.316f, 2.287f},
-    {128, 256, 128, 6.570f, 0.884f, 0.773f, 2.005f, 1.435f, 0.167f, 2.126f},
-    {256, 256, 64, 9.097f, 0.833f, 0.671f, 0.f, 0.f, 0.f, 2.701f},  // never split, see plan_ring
+    {64, 128, 256, 2.774f, 0.734f, 0.380f, 0.702f, 0.545f, 0.299f, 0.747f},
+    {96, 128, 128, 2.255f, 0.472f, 0.337f, 1.219f, 0.605f, 0.272f, 2.082f},
+    {64, 256, 128, 2.615f, 0.799f, 0.277f, 1.381f, 0.949f, 0.188f, 1.770f},
+    {96, 256, 128, 4.013f, 0.701f, 0.594f, 1.226f, 1.557f, 0.188f, 1.946f},
+    {128, 128, 128, 2.247f, 0.548f, 0.340f, 0.853f, 1.153f, 0.353f, 3.134f},
+    {128, 256, 128, 4.966f, 0.881f, 0.734f, 2.088f, 1.086f, 0.201f, 2.056f},
+    {256, 256, 64, 9.097f, 0.833f, 0.661f, 0.f, 0.f, 0.f, 1.343f},  // never split, see plan_ring
 };
 // The same with the scale on the sums (up to 64 tokens), where other constants hold: shapes 1..5, of which the fourth is
 // not built for it.
@@ -1004,7 +1006,13 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes, bool sums) {
         const long tiles = (long)mt * ((N + t.bn - 1) / t.bn);
         const int stages = (K + t.ks - 1) / t.ks;
         const int full = (int)(tiles >> 8), rest = (int)(tiles & 255);
-        const float one = stages * (t.step0 + t.step1) + t.fixed;
+        auto step = [&](int wgs) {  // of a round of wgs workgroups
+            const float rows = 8.f * ((wgs + 7) / 8 < mt ? (wgs + 7) / 8 : mt) * (t.bm < M ? t.bm : M);
+            const float busy = t.step0 + t.step1 * wgs * (1.f / 256), read = rows * t.ks * (2e-6f / 6.5f);
+            return busy > read ? busy : read;
+        };
+        const float full_step = step(256);
+        const float one = stages * full_step + t.fixed;
         const float base = 2.f + full * one;
         auto consider = [&](float us, int rounds, int nfull, int ks) {
             if (rounds > 1) us += (rounds - 1) * t.round;
@@ -1014,7 +1022,7 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes, bool sums) {
             best_us = us;
             best = p;
         };
-        consider(base + (rest ? stages * (t.step0 + t.step1 * rest * (1.f / 256)) + t.fixed : 0.f), full + (rest != 0), 0, 1);
+        consider(base + (rest ? stages * step(rest) + t.fixed : 0.f), full + (rest != 0), 0, 1);
         // (256 x 256 tiles split over K were behind smaller tiles wherever they were timed: partial tiles of 256 KB)
         if (ws_bytes == 0 || rest == 0 || t.bm == 256) continue;
         static const int splits[5] = {2, 3, 4, 6, 8};
@@ -1024,9 +1032,8 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes, bool sums) {
             const int st = (stages + ks - 1) / ks;
             const float ex = t.ex0 + t.ex1 * ks + t.exmb * (4e-6f * w * t.bm * t.bn);
             const int r = (int)(w >> 8), last = (int)(w & 255);
-            consider(base + r * (st * (t.step0 + t.step1) + t.fixed) +
-                         (last ? st * (t.step0 + t.step1 * last * (1.f / 256)) + t.fixed : 0.f) + ex,
-                     full + r + (last != 0), full * 256, ks);
+            consider(base + r * (st * full_step + t.fixed) + (last ? st * step(last) + t.fixed : 0.f) + ex, full + r + (last != 0),
+                     full * 256, ks);
         }
     }
     return best;
