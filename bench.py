@@ -871,7 +871,7 @@ def ln_fused_leg(torch, capi, pool, shapes, g, dev, gen, stream, m=8):
 
 def gated_mlp_leg(torch, capi, g, dev, gen, stream, n=11008, k=4096, tokens=(1, 8, 2048), copies=8):
     """Front half of a Llama-7B MLP, silu(x W_gate^T) * (x W_up^T) with both weights 11008 x 4096: sq_w4a16_gemm_silu_dot
-    (two launches, SiLU and product in the second one's store) against two plain linears followed by torch's silu and
+    (two launches, SiLU and product in the second one's store, or one launch of the ring kernel) against two plain linears followed by torch's silu and
     multiply (four launches), cold weights (rotating pool), HIP-graph replay; parity against the oracle's float64
     formula on sampled output rows."""
     import numpy as np

@@ -95,8 +95,10 @@ int sq_w4a16_gemm_ex(const void* x, const void* w, const void* zs, void* y,
  * where it is the fastest: the streaming decode kernel for 3..16 tokens at group size
  * 128 or 64 when K exceeds 4096 (a shorter K needs no split and no workspace); the ring
  * kernel, whose last, part-filled round of tiles is split, from 17 tokens on, and from 5
- * on large weights whose K would leave the streaming kernel's workgroups part empty and
- * at group size 32 on weights of more than 2^24 elements; the split-K decode kernel for
+ * on large weights whose K would leave the streaming kernel's workgroups part empty (at
+ * group size 64 from 2^24 elements up where they are more than 128), on weights whose row
+ * blocks times K ranges would begin a second round with few of them (at group size 128 from
+ * 9), and at group size 32 on weights of more than 2^24 elements; the split-K decode kernel for
  * what is left at 5..16 tokens on weights of 2^25 elements or more or with K > 8192.  A
  * workspace that is NULL or misaligned is ignored under SQ_ALGO_AUTO, as is one too small
  * for the decode kernels (the ring kernel splits K as far as it fits); an explicit

@@ -233,8 +233,8 @@ __global__ __launch_bounds__(128 * KG, WPS) void lut_attn_kernel(
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (KG == 2) __builtin_amdgcn_s_setprio(0);
         // The products of S^T are a chain, and requests that go out one by one between them do not wait for the address unit
-        // (16 heads x 1674 x 128 18.5 -> 17.8 us).  With two waves per step another workgroup's waves fill that time (32 heads
-        // x 4096 x 128 86.9 -> 86.7).
+        // (together with the counted waits of `landed`: 16 heads x 1674 x 128 19.1 -> 18.6 us on one box, 18.9 -> 18.0 on another).
+        // With two waves per step another workgroup's waves fill that time (32 heads x 4096 x 128 86.9 -> 86.7).
         if (KG == 2 && next >= 0 && next + STEP <= S) {
             const uint8_t* kb = (const uint8_t*)(kz + next * a.st.kv[2]);
             const uint8_t* vb = (const uint8_t*)(vz + next * a.st.kv[2]);
@@ -267,8 +267,9 @@ __global__ __launch_bounds__(128 * KG, WPS) void lut_attn_kernel(
 #pragma unroll
                 for (int i = 0; i < 2; i++) vf[s][dt][i] = lds_read_tr(l + vread[dt] + (16 * s + 8 * i) * ROW);
         __builtin_amdgcn_sched_barrier(0);
-        // (the four waves of a step wait for each other: the one in its softmax goes first.  16 heads x 1674 x 128 17.8 ->
-        // 17.2 us, 2 x 16 x 567 x 128 8.6 -> 8.4; with two waves per step it changes nothing)
+        // (the four waves of a step wait for each other: the one in its softmax goes first.  By itself, before the requests
+        // went between the products: 16 heads x 1674 x 128 17.8 -> 17.2 us, 2 x 16 x 567 x 128 8.6 -> 8.4; with two waves per step
+        // it changes nothing)
         if constexpr (KG == 2) __builtin_amdgcn_s_setprio(1);
         // scores relative to the reference maximum, in units of log2
 #pragma unroll

@@ -1,6 +1,7 @@
 // GEMM for 17 tokens up (any group size, any K) with layout L1: the product between a weight stream and a matrix-core
 // contraction, and the contraction itself until many rounds of short K favour the two-workgroups-per-CU kernel of
-// sq_gemm.hip.
+// sq_gemm.hip.  At 5..16 tokens it takes the weights whose K the streaming kernel splits badly, and gate and up of a gated
+// MLP in one launch (PAIR) from one token where that measures ahead; both are rules of sq_api.hip.
 //
 // What bounds it.  At 32..600 tokens neither HBM nor the matrix cores are full; what a CU can issue is: a
 // v_mfma_f32_32x32x16_f16 takes 32 cycles and hides vector instructions of the other wave of its SIMD completely, but a
@@ -187,7 +188,8 @@ __device__ __forceinline__ void load_to_lds_x1_masked(const void* base, uint32_t
 // column tile go and sixteen per row tile come: the same count with one row tile, more with two.  Measured (us, W_hat / sums):
 // 32 tokens 12288x4096 11.96 / 12.03, 5120x13696 16.3 / 16.4; 48 tokens 12288x4096 16.4 / 16.1, 5120x13696 20.6 / 21.1;
 // 64 tokens 4096x11008 16.6 / 16.6, 15360x5120 20.4 / 21.0.  Its loop keeps the two alternating groups of waves (0..3 fetch
-// phase p + 1 while 4..7 compute phase p): in step it would need a second set of sums.
+// phase p + 1 while 4..7 compute phase p): in step it would need a second set of sums, which tiles of 64 rows (222..226 registers
+// of 256) have no room for, and tiles of 32 rows are slower in step as they are.
 //
 // PAIR: silu(X W^T) * (X W2^T), both weights [N, K], in one launch: half of a tile's columns are W's and half W2's, the same
 // outputs' in the same workgroup, so that the product is formed in the store and the tiles of both fill the chip's rounds

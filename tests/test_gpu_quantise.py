@@ -58,6 +58,17 @@ def test_quantise_parity(built_lib, monkeypatch, n, k, g, n_bit):
             assert a.dtype == b.dtype and same(a, b), (seed, a.shape)
 
 
+@pytest.mark.parametrize("layout", [capi.SQ_LAYOUT_L1, capi.SQ_LAYOUT_L2])
+def test_c_abi_packs_as_the_extension_does(built_lib, layout):
+    """sq_w4a16_quantise through the ctypes binding, with and without the fake-quantised weight."""
+    import quant
+    w = weight(64, 256, 1)
+    for fake in (False, True) if layout == capi.SQ_LAYOUT_L2 else (False,):
+        got, ref = capi.quantise(w, 64, 4, layout, fake), quant.quantise(w, 64, 4, layout, fake)
+        assert (got[2] is None) == (ref[2] is None) == (not fake)
+        assert all(a.dtype == b.dtype and same(a, b) for a, b in zip(got, ref) if a is not None)
+
+
 def test_from_float_and_the_weights_the_kernel_leaves_alone(built_lib):
     w = weight(64, 256, 0)
     lin = torch.nn.Linear(256, 64, device=DEV, dtype=torch.float16)
