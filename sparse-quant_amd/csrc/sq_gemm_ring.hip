@@ -83,21 +83,26 @@ constexpr int ring_trip(int l, int cap, int unit) {
     return u;
 }
 
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST>
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
 struct RingShape {
     static constexpr int NW = WM * WN * WK, NT = 64 * NW;
     static constexpr int BM = 32 * MI * WM, BN = 32 * NI * WN, KS = 64 * WK;
     static constexpr int XB = WK * BM * 128, WB = BN * WK * 32;
     static constexpr int P = (KS >> GS) ? (KS >> GS) : 1;  // zeros/scales pairs per column and stage
-    static constexpr int ZB = BN * P * 4;
-    static constexpr int SB = XB + WB + ZB;
+    // Zeros/scales: a stage's own with its other operands, or (SETS) those of ZN stages, ZD of a row, in two buffers behind
+    // the stages: see issue_set.
+    static constexpr bool SETS = SUMS && P <= 2;
+    static constexpr int ZD = SETS ? 8 : P, ZN = ZD / P;
+    static constexpr int ZB = BN * ZD * 4;
+    static constexpr int SB = XB + WB + (SETS ? 0 : ZB);
     static constexpr int XI = XB / 1024 / NW, WI = WB / 1024 / NW;
-    static constexpr int ZL = BN * P / NW < 64 ? BN * P / NW : 64, ZI = BN * P / NW / ZL;  // lanes and instructions of a wave
-    static constexpr int PER = XI + WI + ZI;
-    static constexpr int LDS = ST * SB;
+    static constexpr int ZL = BN * ZD / NW < 64 ? BN * ZD / NW : 64, ZI = BN * ZD / NW / ZL;  // lanes and instructions of a wave
+    static constexpr int PER = XI + WI + (SETS ? 0 : ZI);
+    static constexpr int LDS = ST * SB + (SETS ? 2 * ZB : 0);
     static constexpr int TAIL = NW * 32 * 32 * NI * 4;  // one 32-row slice of every wave's sums
-    static_assert(XI * NW * 1024 == XB && WI * NW * 1024 == WB && ZI * ZL * NW == BN * P && (NW == 8 || NW == 4), "loads divide over the waves");
+    static_assert(XI * NW * 1024 == XB && WI * NW * 1024 == WB && ZI * ZL * NW == BN * ZD && (NW == 8 || NW == 4), "loads divide over the waves");
     static_assert(LDS <= 163840 && TAIL <= LDS, "fits");
+    static_assert(!SETS || ZN >= ST - 1, "two buffers");
 };
 
 // EV consecutive columns of bias, multiplicand and residual, requested before the sums are there: their latency does not
@@ -200,9 +205,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS, const half_t* __restrict__ X, half_t* __restrict__ Y,
     int M, int N, int K, int mtiles, int tiles, int nfull, int ksplit, Epilogue epi, float* part, unsigned* counters,
     const uint8_t* __restrict__ W2, const half2_t* __restrict__ ZS2, half_t* __restrict__ U) {
-    using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
+    using S = RingShape<MI, NI, WM, WN, WK, GS, ST, SUMS>;
     constexpr int BM = S::BM, BN = S::BN, KS = S::KS, SB = S::SB, XI = S::XI, WI = S::WI, ZI = S::ZI, ZL = S::ZL, PER = S::PER, P = S::P;
-    constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = S::XB + S::WB;
+    constexpr bool SETS = S::SETS;
+    constexpr int ZD = S::ZD, ZN = S::ZN;
+    constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = SETS ? ST * SB : S::XB + S::WB;
     constexpr int H = 4;  // 16-wide k slices per stage and wave
     constexpr bool ALTERNATE = SUMS || MI == 1;  // two groups of waves in turn (see the head of this file)
     static_assert(!ALTERNATE || S::NW == 8, "waves 0..3 and 4..7");
@@ -278,8 +285,22 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
     for (int j = 0; j < ZI; j++) {
         const int d = (wave * ZI + j) * ZL + (lane & (ZL - 1));
-        zlane[j] = (uint32_t)((long)imin(n0 + d / P % BO, N - 1) * groups * 4) + (d % P) * 4;
+        zlane[j] = (uint32_t)((long)imin(n0 + d / ZD % BO, N - 1) * groups * 4) + (SETS ? 0 : d % P * 4);
     }
+    // A stage's own zeros/scales are 4 or 8 bytes of a row, each in a line of its own: with 32 rows per tile a third of the lines
+    // that a stage asks for, and the loads come back in order.  So 32 bytes of a row at once, in front of the first of the ZN
+    // stages that they serve (us: 64 tokens 12288x4096 in tiles of 64 x 128 23.2 -> 21.9, 64 x 256 split in two 26.5 -> 25.4; 32
+    // tokens 4096x11008 in tiles of 32 x 128 split in two 24.4 -> 22.7, gate and up of 11008x4096 19.4 -> 17.8).  Two buffers: set s
+    // goes out when all have read stage ZN s - ST, which is no earlier than the last one of set s - 2.  Not for the waves in step:
+    // the branch in their loop costs what it saves (100 tokens 15360x5120 in tiles of 96 x 128 32.3 -> 33.8, 200 12288x4096 in 96 x 256
+    // 34.9 -> 37.3, 333 at group size 64 41.4 -> 42.3).
+    auto issue_set = [&](int set) {
+        const int g = ((it0 * KS) >> GS) + set * ZD;
+#pragma unroll
+        for (int j = 0; j < ZI; j++)
+            load_to_lds_x1_masked(Zl, zlane[j] + imin(g + lane % ZD, groups - 1) * 4,
+                                  lds0 + Z_OFF + (set & 1) * S::ZB + (wave * ZI + j) * ZL * 4, zmask);
+    };
     // Loads of stage it into slot c.  EDGE: the last stage of a K that ends inside it; weights that are missing re-read
     // the end of the row (and meet a scale of 0), activations are zeros in LDS (an infinity at the end of a row, re-read,
     // would be a NaN in every column.  Clearing the operands in the last stages' registers instead cost the 256 x 256 tiles
@@ -291,8 +312,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         const uint8_t* wb = Wl + (k0 >> 1);
         const uint8_t* zb = (const uint8_t*)Zl + (k0 >> GS) * 4;
         const uint32_t l0 = lds0 + c * SB;
+        constexpr int ZP = SETS ? 0 : ZI;
 #pragma unroll
-        for (int j = 0; j < ZI; j++) {
+        for (int j = 0; j < (SETS ? 0 : ZI); j++) {
             if (j < lo || j >= hi) continue;
             uint32_t o = zlane[j];
             if constexpr (EDGE) {
@@ -303,7 +325,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
 #pragma unroll
         for (int j = 0; j < WI; j++) {
-            if (ZI + j < lo || ZI + j >= hi) continue;
+            if (ZP + j < lo || ZP + j >= hi) continue;
             uint32_t o = wlane[j];
             if constexpr (EDGE) {
                 const int R = (wave * WI + j) * (32 / WK) + lane / (2 * WK);
@@ -314,7 +336,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
 #pragma unroll
         for (int j = 0; j < XI; j++) {
-            if (ZI + WI + j < lo || ZI + WI + j >= hi) continue;
+            if (ZP + WI + j < lo || ZP + WI + j >= hi) continue;
             uint64_t mask = xmask[j];
             if constexpr (EDGE) {
                 const int ii = wave * XI + j;
@@ -327,6 +349,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
     };
     auto issue_any = [&](int it, int c) {
+        if constexpr (SETS) {
+            if ((it - it0) % ZN == 0) issue_set((it - it0) / ZN);
+        }
         if (it * KS + KS <= K)
             issue(it, c, std::false_type{});
         else
@@ -342,7 +367,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     const int wcol = (PAIR ? (NI == 2 ? 32 * wn : (wn & 1) * BO + 32 * (wn >> 1)) : wn * 32 * NI) + ln;
     static_assert(!PAIR || NI == 2 || (NI == 1 && WN % 2 == 0), "both weights of an output column in one wave or in neighbours");
     const int woff = W_OFF + wcol * (32 * WK) + (((2 * kg + lc) ^ wswz<WK>(ln)) * 16);
-    const int zoff = Z_OFF + (wcol * P + ((64 * kg + (GS == 5 ? 32 * lc : 0)) >> GS)) * 4;
+    const int zoff = Z_OFF + (wcol * ZD + ((64 * kg + (GS == 5 ? 32 * lc : 0)) >> GS)) * 4;
 
     float16_t acc[MI][NI];
 #pragma unroll
@@ -570,11 +595,13 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             }
         };
         // The wave's operands of the stage in slot c into registers.
-        auto fetch = [&](int c) {
+        auto fetch = [&](int it, int c) {
             const uint8_t* l = lds + c * SB;
+            const uint8_t* zl = l;
+            if constexpr (SETS) zl = lds + (it - it0) / ZN % 2 * S::ZB + (it - it0) % ZN * (P * 4);
 #pragma unroll
             for (int ni = 0; ni < NI; ni++) {
-                zs[ni] = *(const half2_t*)(l + zoff + ni * (CN * P * 4));
+                zs[ni] = *(const half2_t*)(zl + zoff + ni * (CN * ZD * 4));
                 const u32x4_t v = *(const u32x4_t*)(l + woff + ni * (CN * 32 * WK));
 #pragma unroll
                 for (int t = 0; t < 4; t++) q[ni][t] = v[t];
@@ -644,11 +671,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             for (int s = 0; s < ST - 1; s++)
                 if (it0 + s < it1) issue_any(it0 + s, s);
             // Stage it + 1 has landed: all but the loads of the younger stages are done.
-            auto landed_full = []() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory"); };
+            auto landed_full = [&](int it) {
+                if (SETS && (it - it0 + ST - 1) % ZN < ST - 2)  // a set went out with one of the younger ones
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER + ZI) : "memory");
+                else
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * PER) : "memory");
+            };
             auto landed_all = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
             auto turn = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
             if (it0 + ST - 1 <= it1)
-                landed_full();
+                landed_full(it0 - 1);
             else
                 landed_all();
             int c = 0, cp = ST - 1, it = it0;
@@ -661,7 +693,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             // stage it.  A fetch also requests stage it + ST - 1 into the slot of stage it - 1, which both groups have
             // read by then.
             if (wave < 4) {
-                fetch(0);
+                fetch(it, 0);
                 if (it < full)
                     issue_any(it + ST - 1, ST - 1);
                 else
@@ -670,9 +702,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                 turn();
                 for (; it + 1 < full; it++) {
                     compute();
-                    landed_full();
+                    landed_full(it);
                     next();
-                    fetch(c);
+                    fetch(it + 1, c);
                     issue_any(it + ST, cp);
                     unpack_first();
                     turn();
@@ -682,7 +714,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                     landed_all();
                     next();
                     if (it + 1 < it1) {
-                        fetch(c);
+                        fetch(it + 1, c);
                         clip(it + 1);
                         unpack_first();
                     }
@@ -691,16 +723,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             } else {
                 turn();
                 for (; it < full; it++) {
-                    fetch(c);
+                    fetch(it, c);
                     issue_any(it + ST - 1, cp);
                     unpack_first();
-                    landed_full();
+                    landed_full(it);
                     compute();
                     next();
                     turn();
                 }
                 for (; it < it1; it++) {
-                    fetch(c);
+                    fetch(it, c);
                     clip(it);
                     unpack_first();
                     landed_all();
@@ -933,7 +965,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool PAIR>
 static hipError_t launch_shape(const void* x, const void* w, const void* zs, const void* w2, const void* zs2, void* y, void* u, int M,
                                int N, int K, int nfull, int ksplit, Epilogue epi, void* ws, hipStream_t st) {
-    using S = RingShape<MI, NI, WM, WN, WK, GS, ST>;
+    using S = RingShape<MI, NI, WM, WN, WK, GS, ST, SUMS>;
     const int mt = (M + S::BM - 1) / S::BM;
     constexpr int BO = PAIR ? S::BN / 2 : S::BN;
     const int tiles = mt * ((N + BO - 1) / BO);
@@ -973,9 +1005,11 @@ static const RingTile kRingTiles[] = {
     {256, 256, 64, 9.097f, 0.833f, 0.661f, 0.f, 0.f, 0.f, 1.343f},  // never split, see plan_ring
 };
 // The same with the scale on the sums (up to 64 tokens), where other constants hold: shapes 1..5, of which the fourth is
-// not built for it.
+// not built for it.  Adjusted for the choice on 96 weights x token counts (768 .. 22016 rows, K 768 .. 16384, 17 .. 64 tokens) with
+// the zeros/scales of several stages at once: 0.3 % above the best in the geometric mean (0.5 with the constants before), at worst 6 %.
 static const RingTile kRingSumsTiles[] = {
-    kRingTiles[0], kRingTiles[1], {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f, 0.f},
+    kRingTiles[0], {32, 128, 256, 1.498f, 0.706f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f},
+    {64, 128, 256, 2.740f, 0.778f, 0.244f, 0.211f, 0.576f, 0.409f, 0.f},
     kRingTiles[3], {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f, 0.f},
 };
 constexpr int RING_SHAPES = sizeof(kRingTiles) / sizeof(kRingTiles[0]);

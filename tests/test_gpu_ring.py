@@ -311,6 +311,30 @@ def test_ring_parity_with_the_scale_on_the_sums(capi, shape, m, n, k, g):
         assert capi.workspace_is_clean(ws)
 
 
+@pytest.mark.parametrize("shape,stage", [(1, 512), (2, 256), (3, 256), (5, 128)])
+@pytest.mark.parametrize("short", [0, 128])
+def test_ring_sums_every_count_of_stages(capi, shape, stage, short):
+    """Zeros and scales come for four or eight stages at once: a last set that is whole, one stage long and ends early, a part
+    of K that begins inside what would be another part's set, and row ends of the last weight row."""
+    m, n, g = 19, 136, 128
+    ws = torch.zeros(65536 + (8 << 20), dtype=torch.uint8, device=DEV)
+    for stages in (1, 2, 3, 4, 5, 7, 8, 9, 12, 13, 16, 17, 18, 25) if stage < 512 else (1, 2, 3, 5):
+        k = stage * stages - (short if stage > 128 else 0)
+        d = orc.synth_linear(n, k, g, seed=k)
+        w64, x = real_weight(d, g), orc.synth_x(m, k, seed=shape)
+        x64 = x.astype(np.float64)
+        ref = x64 @ w64.T
+        # one rounding to fp16 and K fp32 additions of the products' magnitudes
+        bound = 2.0 ** -11 * np.abs(ref) + k * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T) + 2.0 ** -24
+        w, zs, xd = to_dev(d["w_l1"]), to_dev(d["zs_l1"]), to_dev(x)
+        for parts in (1, 2, 3):
+            if parts > stages:
+                continue
+            algo = capi.SQ_ALGO_RING | ((shape | SUMS | (parts << 8)) << 8)
+            got = capi.gemm_ws(xd, w, zs, n, k, g, algo=algo, ws=ws).cpu().numpy().astype(np.float64)
+            assert np.all(np.abs(got - ref) <= bound), (stages, parts, np.max(np.abs(got - ref) / bound))
+
+
 def test_ring_has_the_scale_on_the_sums_where_it_says(capi):
     d = orc.synth_linear(64, 128, 32, seed=1)
     x, w, zs = to_dev(orc.synth_x(8, 128)), to_dev(d["w_l1"]), to_dev(d["zs_l1"])
