@@ -29,29 +29,32 @@ namespace sq {
 
 constexpr int GEMM_BN = 256;
 constexpr int GEMM_BK = 64;
+constexpr int GEMM_COUNTER_BYTES = 65536;  // start of the workspace: one uint32 per output tile
 constexpr int GEMM_STAGES = 3;  // register stages; loads run GEMM_STAGES - 1 steps ahead
 
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
-// What follows the K loop in both tiled kernels: with K split over gridDim.z workgroups the
+// What follows the K loop in both tiled kernels: with K split over ksplit workgroups the
 // partial tiles meet in the workspace, then the epilogue and the fp16 stores (through `lds`, 32 KiB
 // of shared memory that the main loop no longer needs).
 template <int MI>
 __device__ __forceinline__ void gemm_tail(float16_t (&acc)[MI][2], half_t* __restrict__ Y, int M, int N, int m0, int n0,
-                                          const Epilogue& epi, float* part, unsigned* counters, float* lds) {
+                                          const Epilogue& epi, void* ws, int ksplit, float* lds) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int ln = lane & 31;
     const int lc = lane >> 5;
-    const int ksplit = gridDim.z;
     if (ksplit > 1) {
+        unsigned* const counters = (unsigned*)ws;
+        float* const part = (float*)((char*)ws + GEMM_COUNTER_BYTES);
         // Partial tiles meet in the workspace: 128-bit stores at the device-coherent cache level,
         // one counter per output tile; the workgroup that arrives last adds the partials in a
         // fixed order (bit-reproducible), stores the tile and resets the counter.
         __shared__ unsigned last_flag;
         constexpr int SLOTS = MI * 2 * 4;  // float4 per thread
-        const long tile = (long)blockIdx.y * gridDim.x + blockIdx.x;
-        const long ntile = (long)gridDim.x * gridDim.y;
+        const int ntiles = (N + GEMM_BN - 1) / GEMM_BN;
+        const long tile = (long)blockIdx.y * ntiles + blockIdx.x;
+        const long ntile = (long)ntiles * ((M + 32 * MI - 1) / (32 * MI));
         float* mine = part + ((long)blockIdx.z * ntile + tile) * (SLOTS * 256 * 4);
 #pragma unroll
         for (int mi = 0; mi < MI; mi++)
@@ -120,8 +123,8 @@ __device__ __forceinline__ void gemm_tail(float16_t (&acc)[MI][2], half_t* __res
 template <int MI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS,
                                                    const half_t* __restrict__ X, half_t* __restrict__ Y, int M,
-                                                   int N, int K, int gshift, Epilogue epi, float* part,
-                                                   unsigned* counters) {
+                                                   int N, int K, int gshift, int ksplit, Epilogue epi,
+                                                   void* ws) {
     constexpr int BM = 32 * MI;
     // Activation tile, two stages, row pitch 128 B (64 halves, no padding); the eight
     // 16-byte chunks of row R are stored at chunk position c ^ swz(R); 8 consecutive
@@ -140,8 +143,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     const int n0 = blockIdx.x * GEMM_BN + 64 * wave;
     const int groups = K >> gshift;
     const int nit = (K + GEMM_BK - 1) / GEMM_BK;
-    // K split over gridDim.z workgroups (1 = no split): this one runs steps it0 .. it1-1.
-    const int ksplit = gridDim.z;
+    // K split over ksplit workgroups (1 = no split): this one runs steps it0 .. it1-1.
     const int spz = (nit + ksplit - 1) / ksplit;
     const int it0 = blockIdx.z * spz;
     const int it1 = imin(it0 + spz, nit);
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         step(it + 5, std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
     }
 
-    gemm_tail<MI>(acc, Y, M, N, m0, n0, epi, part, counters, reinterpret_cast<float*>(&xs[0][0]));
+    gemm_tail<MI>(acc, Y, M, N, m0, n0, epi, ws, ksplit, reinterpret_cast<float*>(&xs[0][0]));
 }
 
 // Both operands through LDS, for group sizes 32, 64 and 128 and K a multiple of 256.  The kernels above hand
@@ -298,7 +300,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 template <int MI, int GS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_lds_kernel(
     const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS, const half_t* __restrict__ X, half_t* __restrict__ Y,
-    int M, int N, int K, Epilogue epi, float* part, unsigned* counters) {
+    int M, int N, int K, int ksplit, Epilogue epi, void* ws) {
     constexpr int BM = 32 * MI;
     constexpr int XB = BM * 128;  // bytes of an activation stage
     constexpr int WB = 256 * 32;  // bytes of a weight stage
@@ -324,7 +326,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     const int groups = K >> GS;
     const int nit = K / GEMM_BK;
     // K split in whole four-step groups
-    const int ksplit = gridDim.z;
     const int spz = ((nit + ksplit - 1) / ksplit + 3) & ~3;
     const int it0 = blockIdx.z * spz;
     const int it1 = imin(it0 + spz, nit);
@@ -448,33 +449,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         if constexpr (P == 4) zc ^= 1;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last two steps' loads ran ahead of the range
-    gemm_tail<MI>(acc, Y, M, N, m0, n0, epi, part, counters, reinterpret_cast<float*>(lds));
+    gemm_tail<MI>(acc, Y, M, N, m0, n0, epi, ws, ksplit, reinterpret_cast<float*>(lds));
 }
-
-constexpr int GEMM_COUNTER_BYTES = 65536;  // start of the workspace: one uint32 per output tile
 
 template <int MI>
 static hipError_t launch_mi(const void* x, const void* w, const void* zs, void* y, int M, int N, int K, int gshift,
                             Epilogue epi, void* ws, int ksplit, bool lds, hipStream_t st) {
     const dim3 grid((N + GEMM_BN - 1) / GEMM_BN, (M + 32 * MI - 1) / (32 * MI), ksplit);
-    unsigned* counters = (unsigned*)ws;
-    float* part = ws ? (float*)((char*)ws + GEMM_COUNTER_BYTES) : nullptr;
     // the LDS kernel addresses its operands with 32-bit byte offsets per lane
     const bool fits32 = (long)M * K * 2 < (1L << 32) && (long)N * (K / 2) < (1L << 32);
     if (lds && gshift >= 5 && gshift <= 7 && K % 256 == 0 && fits32) {
         if (gshift == 7)
             hipLaunchKernelGGL((gemm_lds_kernel<MI, 7>), grid, dim3(256), 0, st, (const uint8_t*)w, (const half2_t*)zs,
-                               (const half_t*)x, (half_t*)y, M, N, K, epi, part, counters);
+                               (const half_t*)x, (half_t*)y, M, N, K, ksplit, epi, ws);
         else if (gshift == 6)
             hipLaunchKernelGGL((gemm_lds_kernel<MI, 6>), grid, dim3(256), 0, st, (const uint8_t*)w, (const half2_t*)zs,
-                               (const half_t*)x, (half_t*)y, M, N, K, epi, part, counters);
+                               (const half_t*)x, (half_t*)y, M, N, K, ksplit, epi, ws);
         else
             hipLaunchKernelGGL((gemm_lds_kernel<MI, 5>), grid, dim3(256), 0, st, (const uint8_t*)w, (const half2_t*)zs,
-                               (const half_t*)x, (half_t*)y, M, N, K, epi, part, counters);
+                               (const half_t*)x, (half_t*)y, M, N, K, ksplit, epi, ws);
         return hipGetLastError();
     }
     hipLaunchKernelGGL((gemm_kernel<MI>), grid, dim3(256), 0, st, (const uint8_t*)w, (const half2_t*)zs,
-                       (const half_t*)x, (half_t*)y, M, N, K, gshift, epi, part, counters);
+                       (const half_t*)x, (half_t*)y, M, N, K, gshift, ksplit, epi, ws);
     return hipGetLastError();
 }
 

@@ -311,14 +311,16 @@ __device__ __forceinline__ void skinny2_body(const uint8_t* __restrict__ W, cons
     if (tid == 0) __hip_atomic_store(&counters[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+__device__ __forceinline__ float* sk2_part(void* ws) { return (float*)((char*)ws + SK2_COUNTER_BYTES); }
+
 template <int MT, int NWV, int S, int RT, bool FIXUP>
 __global__ __launch_bounds__(64 * NWV) void skinny2_kernel(const uint8_t* __restrict__ W,
                                                            const half2_t* __restrict__ ZS,
                                                            const half_t* __restrict__ X, half_t* __restrict__ Y,
-                                                           float* part, unsigned* counters, int M, int N, int K,
-                                                           int gshift, int ksplit, Epilogue epi) {
-    skinny2_body<MT, NWV, S, RT, FIXUP>(W, ZS, X, Y, part, counters, M, N, K, gshift, ksplit, epi, blockIdx.x, blockIdx.x,
-                                        gridDim.x);
+                                                           void* ws, int M, int N, int K, int gshift, int ksplit,
+                                                           Epilogue epi) {
+    skinny2_body<MT, NWV, S, RT, FIXUP>(W, ZS, X, Y, sk2_part(ws), (unsigned*)ws, M, N, K, gshift, ksplit, epi, blockIdx.x,
+                                        blockIdx.x, (N + 16 * RT - 1) / (16 * RT));
 }
 
 // Up to four linears that do not depend on each other and share M, K and the group size in one launch: the
@@ -332,21 +334,21 @@ struct Skinny2Group {
     const half_t* residual[GEMV_GROUP_MAX];
     int N[GEMV_GROUP_MAX];
     int act[GEMV_GROUP_MAX];
-    int blk_end[GEMV_GROUP_MAX];  // first row block behind linear p
+    int blk_end[GEMV_GROUP_MAX];  // first row block behind linear p; the last one: of the whole launch
     int count;
 };
 
 template <int MT, int NWV, int S, int RT, bool FIXUP>
-__global__ __launch_bounds__(64 * NWV) void skinny2_group_kernel(const Skinny2Group grp, float* part, unsigned* counters,
-                                                                 int M, int K, int gshift, int ksplit) {
+__global__ __launch_bounds__(64 * NWV) void skinny2_group_kernel(const Skinny2Group grp, void* ws, int M, int K,
+                                                                 int gshift, int ksplit) {
     int p = 0;
 #pragma unroll
     for (int q = 0; q < GEMV_GROUP_MAX - 1; q++)
         if (q + 1 < grp.count && (int)blockIdx.x >= grp.blk_end[q]) p = q + 1;
     const int rb = blockIdx.x - (p > 0 ? grp.blk_end[p - 1] : 0);
     const Epilogue epi{grp.bias[p], grp.residual[p], grp.act[p]};
-    skinny2_body<MT, NWV, S, RT, FIXUP>(grp.W[p], grp.ZS[p], grp.X[p], grp.Y[p], part, counters, M, grp.N[p], K, gshift,
-                                        ksplit, epi, rb, blockIdx.x, gridDim.x);
+    skinny2_body<MT, NWV, S, RT, FIXUP>(grp.W[p], grp.ZS[p], grp.X[p], grp.Y[p], sk2_part(ws), (unsigned*)ws, M, grp.N[p], K,
+                                        gshift, ksplit, epi, rb, blockIdx.x, grp.blk_end[GEMV_GROUP_MAX - 1]);
 }
 
 size_t skinny2_workspace_bytes(int M, int N, int K) {
@@ -359,14 +361,12 @@ template <int MT, int NWV, int S, int RT>
 static hipError_t launch_cfg(const void* x, const void* w, const void* zs, void* y, void* ws, int M, int N, int K,
                              int gshift, bool fixup, int ksplit, Epilogue epi, hipStream_t st) {
     const dim3 grid((N + 16 * RT - 1) / (16 * RT), ksplit);
-    unsigned* counters = (unsigned*)ws;
-    float* part = (float*)((char*)ws + SK2_COUNTER_BYTES);
     if (fixup)
         hipLaunchKernelGGL((skinny2_kernel<MT, NWV, S, RT, true>), grid, dim3(64 * NWV), 0, st, (const uint8_t*)w,
-                           (const half2_t*)zs, (const half_t*)x, (half_t*)y, part, counters, M, N, K, gshift, ksplit, epi);
+                           (const half2_t*)zs, (const half_t*)x, (half_t*)y, ws, M, N, K, gshift, ksplit, epi);
     else
         hipLaunchKernelGGL((skinny2_kernel<MT, NWV, S, RT, false>), grid, dim3(64 * NWV), 0, st, (const uint8_t*)w,
-                           (const half2_t*)zs, (const half_t*)x, (half_t*)y, part, counters, M, N, K, gshift, ksplit, epi);
+                           (const half2_t*)zs, (const half_t*)x, (half_t*)y, ws, M, N, K, gshift, ksplit, epi);
     return hipGetLastError();
 }
 
@@ -425,10 +425,8 @@ static hipError_t launch_group_cfg(const SeqProblem* probs, int count, void* ws,
         g.blk_end[p] = blocks;
     }
     g.count = count;
-    unsigned* counters = (unsigned*)ws;
-    float* part = (float*)((char*)ws + SK2_COUNTER_BYTES);
-    hipLaunchKernelGGL((skinny2_group_kernel<MT, NWV, 2, 4, true>), dim3(blocks, ksplit), dim3(64 * NWV), 0, st, g, part,
-                       counters, M, K, gshift, ksplit);
+    hipLaunchKernelGGL((skinny2_group_kernel<MT, NWV, 2, 4, true>), dim3(blocks, ksplit), dim3(64 * NWV), 0, st, g, ws,
+                       M, K, gshift, ksplit);
     return hipGetLastError();
 }
 

@@ -714,13 +714,14 @@ __device__ __forceinline__ void skinny3_wide_body(const uint8_t* __restrict__ W,
     if (tid == 0) __hip_atomic_store(&counters[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+__device__ __forceinline__ float* sk3_part(void* ws) { return (float*)((char*)ws + SK3_COUNTER_BYTES); }
+
 template <int MROWS, int RT, int CH, bool LN, int GPC>
 __global__ __launch_bounds__(SK3_NT) void skinny3_kernel(const uint8_t* __restrict__ W, const uint32_t* __restrict__ ZS,
-                                                         const half_t* __restrict__ X, half_t* __restrict__ Y,
-                                                         float* part, unsigned* counters, int M, int N, int K,
-                                                         int ksplit, Epilogue epi, LnPre ln) {
-    skinny3_body<MROWS, RT, CH, SK3_DEPTH, LN, GPC>(W, ZS, X, Y, part, counters, M, N, K, ksplit, epi, ln, blockIdx.x, blockIdx.x,
-                                               gridDim.x);
+                                                         const half_t* __restrict__ X, half_t* __restrict__ Y, void* ws,
+                                                         int M, int N, int K, int ksplit, Epilogue epi, LnPre ln) {
+    skinny3_body<MROWS, RT, CH, SK3_DEPTH, LN, GPC>(W, ZS, X, Y, sk3_part(ws), (unsigned*)ws, M, N, K, ksplit, epi, ln,
+                                                    blockIdx.x, blockIdx.x, (N + 16 * RT - 1) / (16 * RT));
 }
 
 struct Skinny3Group {
@@ -732,34 +733,35 @@ struct Skinny3Group {
     const half_t* residual[GEMV_GROUP_MAX];
     int N[GEMV_GROUP_MAX];
     int act[GEMV_GROUP_MAX];
-    int blk_end[GEMV_GROUP_MAX];  // first row block behind linear p
+    int blk_end[GEMV_GROUP_MAX];  // first row block behind linear p; the last one: of the whole launch
     int count;
 };
 
 template <int MROWS, int RT, int CH>
-__global__ __launch_bounds__(SK3_NT) void skinny3_group_kernel(const Skinny3Group grp, float* part, unsigned* counters,
-                                                               int M, int K, int ksplit) {
+__global__ __launch_bounds__(SK3_NT) void skinny3_group_kernel(const Skinny3Group grp, void* ws, int M, int K,
+                                                               int ksplit) {
     int p = 0;
 #pragma unroll
     for (int q = 0; q < GEMV_GROUP_MAX - 1; q++)
         if (q + 1 < grp.count && (int)blockIdx.x >= grp.blk_end[q]) p = q + 1;
     const int rb = blockIdx.x - (p > 0 ? grp.blk_end[p - 1] : 0);
     const Epilogue epi{grp.bias[p], grp.residual[p], grp.act[p]};
-    skinny3_body<MROWS, RT, CH, SK3_DEPTH, false, 1>(grp.W[p], grp.ZS[p], grp.X[p], grp.Y[p], part, counters, M, grp.N[p], K,
-                                                  ksplit, epi, LnPre{nullptr, nullptr, 0.f}, rb, blockIdx.x, gridDim.x);
+    skinny3_body<MROWS, RT, CH, SK3_DEPTH, false, 1>(grp.W[p], grp.ZS[p], grp.X[p], grp.Y[p], sk3_part(ws), (unsigned*)ws, M,
+                                                     grp.N[p], K, ksplit, epi, LnPre{nullptr, nullptr, 0.f}, rb, blockIdx.x,
+                                                     grp.blk_end[GEMV_GROUP_MAX - 1]);
 }
 
 template <int RT, int CH>
-__global__ __launch_bounds__(SK3_NT) void skinny3_wide_group_kernel(const Skinny3Group grp, float* part,
-                                                                    unsigned* counters, int M, int K, int ksplit) {
+__global__ __launch_bounds__(SK3_NT) void skinny3_wide_group_kernel(const Skinny3Group grp, void* ws, int M, int K,
+                                                                    int ksplit) {
     int p = 0;
 #pragma unroll
     for (int q = 0; q < GEMV_GROUP_MAX - 1; q++)
         if (q + 1 < grp.count && (int)blockIdx.x >= grp.blk_end[q]) p = q + 1;
     const int rb = blockIdx.x - (p > 0 ? grp.blk_end[p - 1] : 0);
     const Epilogue epi{grp.bias[p], grp.residual[p], grp.act[p]};
-    skinny3_wide_body<RT, CH>(grp.W[p], grp.ZS[p], grp.X[p], grp.Y[p], part, counters, M, grp.N[p], K, ksplit, epi, rb,
-                              blockIdx.x, gridDim.x);
+    skinny3_wide_body<RT, CH>(grp.W[p], grp.ZS[p], grp.X[p], grp.Y[p], sk3_part(ws), (unsigned*)ws, M, grp.N[p], K, ksplit,
+                              epi, rb, blockIdx.x, grp.blk_end[GEMV_GROUP_MAX - 1]);
 }
 
 template <typename Kern>
@@ -784,8 +786,7 @@ hipError_t launch_cfg(const void* x, const void* w, const void* zs, void* y, voi
     if (e != hipSuccess) return e;
     const dim3 grid((N + 16 * RT - 1) / (16 * RT), ksplit);
     hipLaunchKernelGGL((skinny3_kernel<MROWS, RT, CH, LN, GPC>), grid, dim3(SK3_NT), lds, st, (const uint8_t*)w,
-                       (const uint32_t*)zs, (const half_t*)x, (half_t*)y,
-                       ws ? (float*)((char*)ws + SK3_COUNTER_BYTES) : nullptr, (unsigned*)ws, M, N, K, ksplit, epi, ln);
+                       (const uint32_t*)zs, (const half_t*)x, (half_t*)y, ws, M, N, K, ksplit, epi, ln);
     return hipGetLastError();
 }
 
@@ -812,7 +813,7 @@ hipError_t launch_group_cfg(const SeqProblem* probs, int count, void* ws, int M,
     }
     g.count = count;
     hipLaunchKernelGGL((skinny3_group_kernel<MROWS, RT, CH>), dim3(blocks, ksplit), dim3(SK3_NT), lds, st, g,
-                       ws ? (float*)((char*)ws + SK3_COUNTER_BYTES) : nullptr, (unsigned*)ws, M, K, ksplit);
+                       ws, M, K, ksplit);
     return hipGetLastError();
 }
 
@@ -1004,7 +1005,7 @@ hipError_t launch_skinny3_wide_group(const SeqProblem* probs, int count, int M, 
     const hipError_t e = allow_lds(skinny3_wide_group_kernel<4, 4>, lds, allowed);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((skinny3_wide_group_kernel<4, 4>), dim3(blocks, ksplit), dim3(SK3_NT), lds, st, g,
-                       ws ? (float*)((char*)ws + SK3_COUNTER_BYTES) : nullptr, (unsigned*)ws, M, K, ksplit);
+                       ws, M, K, ksplit);
     return hipGetLastError();
 }
 
