@@ -402,7 +402,7 @@ int sq_lut_attention_strided(const void* q, const void* k, const void* v, void* 
  *              (every call leaves them zero), so one workspace serves calls with different B*H.  The kernel
  *              runs one workgroup per (batch, head); with fewer than 256 of them and a workspace
  *              the cache rows of a head are shared among up to 16 workgroups whose partial
- *              softmax states meet in the workspace (batch 1, 32 heads, 640 rows: 4 workgroups
+ *              softmax states meet in the workspace (batch 1, 32 heads of 128, 640 rows: 5 workgroups
  *              per head).  Calls that share a workspace must be ordered (same stream).
  * D in {64, 128}; all strides in elements and multiples of 8; pointers 16-byte aligned.  A fully
  * masked row gives NaN, as in the reference. */

@@ -27,8 +27,27 @@ namespace sq {
 
 namespace {
 
+typedef float float2_t __attribute__((ext_vector_type(2)));
+
 constexpr int DA_WAVES = 8;
 constexpr int DA_U = 4;  // rows of a batch per row slot: 128-bit loads per wave and operand in one request (6 and 8: no faster)
+
+// Rows that the eight waves of a workgroup request at once: a pass.
+__host__ __device__ constexpr int pass_rows(int D) { return DA_WAVES * (64 / (D / 8)) * DA_U; }
+
+// Shares of a head's rows, at most `most`: one pass each where there are enough.  A pass costs 1 to 1.3 us after the first and
+// the meeting of the shares 2.2 us (stores, counter and loads through the level that the eight L2s share), so the rows are
+// shared only where that saves two passes.  us, by two passes' worth of rows as it was / so: 1 x 32 heads x 256 rows x 128
+// 6.7 / 5.8, x 501 8.2 / 6.9; 4 x 32 x 301 x 128 8.7 / 6.8; 8 x 12 x 501 x 64 7.5 / 6.2; 1 x 32 x 401 x 64 6.5 / 5.5.
+__host__ __device__ inline int shares_of(int rows, int most, int D) {
+    const int passes = (rows + pass_rows(D) - 1) / pass_rows(D);
+    const int shares = passes < most ? passes : most;
+    return shares > 1 && passes - (passes + shares - 1) / shares >= 2 ? shares : 1;
+}
+
+// Workgroups up to which heads are shared: one per CU.  Two per CU were slower for caches of up to 1000 rows (8 x 12 heads x
+// 301 x 128 6.5 / 8.4 us) and hardly faster beyond (x 2001 19.6 / 19.3).
+constexpr int DA_WGS = 256;
 
 struct DecodeAttnArgs {
     const half_t* q;
@@ -45,9 +64,8 @@ struct DecodeAttnArgs {
     int H, Lmax, cache_len;
     const long long* cache_len_dev;
     float scale;
-    // Split of the cache rows over gridDim.y workgroups per (batch, head), for launches with too few
-    // heads to fill the chip: partial softmax states (m, l, D outputs) meet in `part`, one counter
-    // per head in `counters` (zero between calls), the last arriver merges.
+    // Shares of a head's cache rows, one workgroup each (grid y), for launches with too few heads to fill the chip: the
+    // partial softmax states meet in `part`, one counter per head in `counters` (zero between calls), the last arriver merges.
     float* part;
     unsigned* counters;
 };
@@ -58,10 +76,13 @@ template <int D, bool MASK>
 __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnArgs a) {
     constexpr int LPR = D / 8;    // lanes per cache row
     constexpr int RPI = 64 / LPR; // rows per load instruction
-    constexpr int STEP = DA_WAVES * RPI * DA_U;
+    constexpr int STEP = pass_rows(D);
+    static_assert(STEP == DA_WAVES * RPI * DA_U);
     __shared__ float mred[DA_WAVES];
     __shared__ float lred[DA_WAVES];
-    __shared__ float ored[DA_WAVES][D];
+    __shared__ __attribute__((aligned(16))) float ored[DECODE_ATTN_MAX_SPLIT][D];  // outputs of the waves, then of the shares
+    __shared__ float2_t weight[DECODE_ATTN_MAX_SPLIT];  // of a share's outputs, and its sum
+    static_assert(DA_WAVES <= DECODE_ATTN_MAX_SPLIT && DECODE_ATTN_MAX_SPLIT <= 16 && 64 * DA_WAVES * 4 >= 16 * D);
     __shared__ unsigned last_flag;
 
     const int tid = threadIdx.x;
@@ -77,10 +98,13 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     const int n0max = a.Lmax - (append ? 1 : 0);
     n0 = n0 < 0 ? 0 : (n0 > n0max ? n0max : n0);
     const int L = n0 + (append ? 1 : 0);  // rows attended; the appended row is row n0
-    // This workgroup's share of the rows: [r0, r1).
-    const int nsplit = gridDim.y;
+    // This workgroup's share of the rows: [r0, r1).  The launch is sized for the whole cache where only the device knows the
+    // length: the workgroups that the rows are too few for leave (64 rows of a cache of 1024, 1 x 32 heads x 128: 9.8 -> 3.4 us).
+    const int slots = gridDim.y, share = blockIdx.y;
+    const int nsplit = shares_of(L, slots, D);
+    if (share >= nsplit) return;
     const int rows_per = (L + nsplit - 1) / nsplit;
-    const int r0 = imin(blockIdx.y * rows_per, L);
+    const int r0 = imin(share * rows_per, L);
     const int r1 = imin(r0 + rows_per, L);
 
     half_t* kbase = a.kc + (long)b * a.c_bs + (long)h * a.c_hs + 8 * c;
@@ -219,14 +243,14 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
         if (tid < D) a.o[(long)blockIdx.x * D + tid] = (half_t)(o / lsum);  // nothing visible: 0 / 0 = NaN, as the reference
         return;
     }
-    // Partial state of this share: [m, l, o[0..D)], exchanged at the device-coherent level (relaxed
+    // Partial states of a head: [share][D] outputs, then [share] (m, l), exchanged at the device-coherent level (relaxed
     // agent-scope accesses, ordered by the wait below and the counter; no device-wide fence).
-    float* mine = a.part + ((long)blockIdx.x * nsplit + blockIdx.y) * (D + 2);
-    if (tid < D) __hip_atomic_store(mine + 2 + tid, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid == 0) {
-        __hip_atomic_store(mine, mb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(mine + 1, lsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    float* const outs = a.part + (long)blockIdx.x * slots * (D + 2);
+    unsigned long long* const states = (unsigned long long*)(outs + slots * D);
+    if (tid < D) __hip_atomic_store(outs + share * D + tid, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0)
+        __hip_atomic_store(states + share, bit_cast<unsigned long long>((float2_t){mb, lsum}), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
@@ -235,17 +259,37 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     }
     __syncthreads();
     if (!last_flag) return;
+    // Everything is asked for at once: four outputs of a share per thread, and in every wave lane s the state of share s
+    // (unused ones count as empty).  Each thread walking over the shares for its output took a round trip per share, twice:
+    // 1 x 32 heads x 128 (us) x 2001 rows 13.9 -> 10.4, x 4001 18.2 -> 14.7; 1 x 12 x 4001 x 64 16.9 -> 8.5.
+    // The sums run over the shares in their order: bit-reproducible.
+    constexpr int QD = D / 4;
+    const int sp = tid / QD, d4 = tid % QD * 4;
+    unsigned long long v01 = 0, v23 = 0, ml = bit_cast<unsigned long long>((float2_t){-INFINITY, 0.f});
+    if (sp < nsplit) {
+        const unsigned long long* src = (const unsigned long long*)(outs + sp * D + d4);
+        v01 = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        v23 = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (lane < nsplit) ml = __hip_atomic_load(states + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float2_t state = bit_cast<float2_t>(ml);
+    float mg = state.x;
+#pragma unroll
+    for (int x = 1; x < DECODE_ATTN_MAX_SPLIT; x <<= 1) mg = fmaxf(mg, __shfl_xor(mg, x, 64));
+    const float f = (state.x == -INFINITY) ? 0.f : __expf(state.x - mg);
+    if (tid < DECODE_ATTN_MAX_SPLIT) weight[tid] = (float2_t){f, state.y};
+    if (sp < DECODE_ATTN_MAX_SPLIT) {
+        *(unsigned long long*)&ored[sp][d4] = v01;
+        *(unsigned long long*)&ored[sp][d4 + 2] = v23;
+    }
+    __syncthreads();
     if (tid < D) {
-        const float* all = a.part + (long)blockIdx.x * nsplit * (D + 2);
-        float mg = -INFINITY;
-        for (int sp = 0; sp < nsplit; sp++)
-            mg = fmaxf(mg, __hip_atomic_load(all + sp * (D + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         float lg = 0.f, og = 0.f;
-        for (int sp = 0; sp < nsplit; sp++) {  // fixed order: bit-reproducible
-            const float ms = __hip_atomic_load(all + sp * (D + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const float f = (ms == -INFINITY) ? 0.f : __expf(ms - mg);
-            lg += __hip_atomic_load(all + sp * (D + 2) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * f;
-            og += __hip_atomic_load(all + sp * (D + 2) + 2 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * f;
+#pragma unroll
+        for (int s = 0; s < DECODE_ATTN_MAX_SPLIT; s++) {
+            const float2_t w = weight[s];
+            lg += w.y * w.x;
+            og += ored[s][tid] * w.x;
         }
         a.o[(long)blockIdx.x * D + tid] = (half_t)(og / lg);
     }
@@ -277,14 +321,14 @@ hipError_t launch_decode_attention(const void* q, const void* k_new, const void*
                                    long n_bs, long n_hs, long c_bs, long c_hs, long m_bs, int cache_len,
                                    const long long* cache_len_dev, float sm_scale, void* workspace,
                                    size_t workspace_bytes, hipStream_t st) {
-    // Shares per head: enough workgroups for the 256 CUs, at least 128 rows each (what one pass of
-    // the eight waves covers), only with a workspace that holds the partial states.
+    // Heads are shared only with a workspace that holds the partial states.
     int nsplit = 1;
     const long heads = (long)B * H;
     if (workspace && heads < 256) {
         const int rows = cache_len_dev ? Lmax : cache_len + (k_new ? 1 : 0);
-        while (nsplit < DECODE_ATTN_MAX_SPLIT && heads * nsplit * 2 <= 256 && rows / (nsplit * 2) >= 128) nsplit *= 2;
-        if (workspace_bytes < decode_attention_workspace_bytes(B, H, D)) nsplit = 1;
+        const int most = (int)(DA_WGS / heads);
+        if (workspace_bytes >= decode_attention_workspace_bytes(B, H, D))
+            nsplit = shares_of(rows, most < DECODE_ATTN_MAX_SPLIT ? most : DECODE_ATTN_MAX_SPLIT, D);
     }
     DecodeAttnArgs a;
     a.q = (const half_t*)q;

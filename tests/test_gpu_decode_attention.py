@@ -319,3 +319,29 @@ def test_decode_split_workspace_shared_across_head_counts(capi):
         check(out, ref, "shared workspace, b=%d" % b)
         assert (out.float() - single.float()).abs().max().item() <= 2e-3
         assert torch.count_nonzero(ws[:1024]).item() == 0
+
+
+@pytest.mark.parametrize("device_length", [False, True])
+@pytest.mark.parametrize("b,h,d", [(1, 3, 128), (1, 3, 64), (2, 50, 128), (5, 25, 64)])
+def test_decode_shares_at_the_edges_of_passes(capi, b, h, d, device_length):
+    # A workgroup asks for 128 rows (d = 128) or 256 (d = 64) at once; rows are shared from three such passes on (with at
+    # most two workgroups per head, from four on), and where only the device knows the length, by the rows that are there.
+    # The workspace serves every length in turn: its counters have to be zero again after each.
+    step = 128 if d == 128 else 256
+    edges = [1, step, step + 1, 2 * step - 1, 2 * step, 2 * step + 1, 3 * step, 3 * step + 1, 4 * step + 1]
+    edges += [15 * step + 7, 16 * step, 17 * step + 1] if b == 1 else []
+    lmax = edges[-1] + 3
+    q, k, v = make(b, h, lmax, d, seed=b + h + d)
+    kt, vt = torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda()
+    qt = torch.from_numpy(q).cuda()
+    for l in edges + edges[::-1]:
+        kc, vc = kt.clone(), vt.clone()
+        kc[:, :, l:] = float("nan")  # rows behind the end must not matter
+        vc[:, :, l:] = float("nan")
+        kc[:, :, l - 1] = float("nan")  # appended below
+        length = torch.tensor([l - 1], device="cuda") if device_length else l - 1
+        new = (kt[:, :, l - 1].contiguous(), vt[:, :, l - 1].contiguous())
+        out = capi.decode_attention(qt, kc, vc, length, d ** -0.5, k_new=new[0], v_new=new[1])
+        ref = att.decode_attention_ref(q, k[:, :, :l], v[:, :, :l], d ** -0.5)
+        check(out, ref, "l = %d" % l)
+        assert torch.equal(kc[:, :, l - 1], new[0]) and torch.equal(vc[:, :, l - 1], new[1])
