@@ -40,6 +40,7 @@ __host__ __device__ constexpr int pass_rows(int D) { return DA_WAVES * (64 / (D 
 // shared only where that saves two passes.  us, by two passes' worth of rows as it was / so: 1 x 32 heads x 256 rows x 128
 // 6.7 / 5.8, x 501 8.2 / 6.9; 4 x 32 x 301 x 128 8.7 / 6.8; 8 x 12 x 501 x 64 7.5 / 6.2; 1 x 32 x 401 x 64 6.5 / 5.5.
 __host__ __device__ inline int shares_of(int rows, int most, int D) {
+    if (most <= 1) return 1;  // (no division in front of the first request where nothing is shared)
     const int passes = (rows + pass_rows(D) - 1) / pass_rows(D);
     const int shares = passes < most ? passes : most;
     return shares > 1 && passes - (passes + shares - 1) / shares >= 2 ? shares : 1;
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     const int slots = gridDim.y, share = blockIdx.y;
     const int nsplit = shares_of(L, slots, D);
     if (share >= nsplit) return;
-    const int rows_per = (L + nsplit - 1) / nsplit;
+    const int rows_per = nsplit == 1 ? L : (L + nsplit - 1) / nsplit;
     const int r0 = imin(share * rows_per, L);
     const int r1 = imin(r0 + rows_per, L);
 
