@@ -50,6 +50,11 @@ __host__ __device__ inline int shares_of(int rows, int most, int D) {
 // 301 x 128 6.5 / 8.4 us) and hardly faster beyond (x 2001 19.6 / 19.3).
 constexpr int DA_WGS = 256;
 
+// Rows of a head are shared only with fewer than 256 (batch, head) pairs, so 256 counters are
+// always enough: the counter region has one fixed size and the partial states one fixed offset,
+// whatever B * H a workspace is used with next.
+constexpr size_t DECODE_ATTN_COUNTER_BYTES = 256 * sizeof(unsigned);
+
 struct DecodeAttnArgs {
     const half_t* q;
     const half_t* kn;
@@ -64,11 +69,12 @@ struct DecodeAttnArgs {
     long m_bs;        // ... of the additive mask over batch
     int H, Lmax, cache_len;
     const long long* cache_len_dev;
+    int slots;  // grid y
     float scale;
     // Shares of a head's cache rows, one workgroup each (grid y), for launches with too few heads to fill the chip: the
-    // partial softmax states meet in `part`, one counter per head in `counters` (zero between calls), the last arriver merges.
-    float* part;
-    unsigned* counters;
+    // partial softmax states meet in the workspace behind its counters, one per head (zero between calls), and the last arriver
+    // merges them.
+    void* ws;
 };
 
 __device__ __forceinline__ float xor_sum(float v, int m) { return v + __shfl_xor(v, m, 64); }
@@ -101,7 +107,7 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     const int L = n0 + (append ? 1 : 0);  // rows attended; the appended row is row n0
     // This workgroup's share of the rows: [r0, r1).  The launch is sized for the whole cache where only the device knows the
     // length: the workgroups that the rows are too few for leave (64 rows of a cache of 1024, 1 x 32 heads x 128: 9.8 -> 3.4 us).
-    const int slots = gridDim.y, share = blockIdx.y;
+    const int slots = a.slots, share = blockIdx.y;
     const int nsplit = shares_of(L, slots, D);
     if (share >= nsplit) return;
     const int rows_per = nsplit == 1 ? L : (L + nsplit - 1) / nsplit;
@@ -246,7 +252,7 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     }
     // Partial states of a head: [share][D] outputs, then [share] (m, l), exchanged at the device-coherent level (relaxed
     // agent-scope accesses, ordered by the wait below and the counter; no device-wide fence).
-    float* const outs = a.part + (long)blockIdx.x * slots * (D + 2);
+    float* const outs = (float*)((char*)a.ws + DECODE_ATTN_COUNTER_BYTES) + (long)blockIdx.x * slots * (D + 2);
     unsigned long long* const states = (unsigned long long*)(outs + slots * D);
     if (tid < D) __hip_atomic_store(outs + share * D + tid, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tid == 0)
@@ -255,7 +261,7 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-        const unsigned old = __hip_atomic_fetch_add(&a.counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned old = __hip_atomic_fetch_add((unsigned*)a.ws + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         last_flag = (old == (unsigned)(nsplit - 1)) ? 1u : 0u;
     }
     __syncthreads();
@@ -294,7 +300,7 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
         }
         a.o[(long)blockIdx.x * D + tid] = (half_t)(og / lg);
     }
-    if (tid == 0) __hip_atomic_store(&a.counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store((unsigned*)a.ws + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <int D>
@@ -307,11 +313,6 @@ hipError_t launch_d(const DecodeAttnArgs& a, int B, int nsplit, hipStream_t st) 
 }
 
 }  // namespace
-
-// Rows of a head are shared only with fewer than 256 (batch, head) pairs, so 256 counters are
-// always enough: the counter region has one fixed size and the partial states one fixed offset,
-// whatever B * H a workspace is used with next.
-constexpr size_t DECODE_ATTN_COUNTER_BYTES = 256 * sizeof(unsigned);
 
 size_t decode_attention_workspace_bytes(int B, int H, int D) {
     return DECODE_ATTN_COUNTER_BYTES + (size_t)B * H * DECODE_ATTN_MAX_SPLIT * (D + 2) * sizeof(float);
@@ -351,8 +352,8 @@ hipError_t launch_decode_attention(const void* q, const void* k_new, const void*
     a.cache_len = cache_len;
     a.cache_len_dev = cache_len_dev;
     a.scale = sm_scale;
-    a.counters = (unsigned*)workspace;
-    a.part = workspace ? (float*)((char*)workspace + DECODE_ATTN_COUNTER_BYTES) : nullptr;
+    a.slots = nsplit;
+    a.ws = workspace;
     return D == 64 ? launch_d<64>(a, B, nsplit, st) : launch_d<128>(a, B, nsplit, st);
 }
 

@@ -51,12 +51,12 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const half_t* __restric
 template <int MT>
 __global__ __launch_bounds__(64 * LMH_WAVES) void f16_gemv_kernel(const half_t* __restrict__ W, const half_t* __restrict__ X,
                                                                  half_t* __restrict__ Y, float* __restrict__ part_val,
-                                                                 int* __restrict__ part_idx, int M, int N, int K, int iters) {
+                                                                 int* __restrict__ part_idx, int M, int N, int K, int iters,
+                                                                 int G) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lmh_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = lane & 3, b = lane >> 2;
     const int sel = wave >> 2, part = wave & 3;
-    const int G = gridDim.x;
     const int steps = K >> 9;  // 128-wide k-steps of a quarter of K
     const int xbytes = (K >> 7) * (4 * MT) * 256;
     const int cbytes = (4 * MT) * iters * 8 * 4;
@@ -251,7 +251,7 @@ hipError_t launch_f16_gemv(const void* x, const void* w, void* y, float* part_va
             allowed[0][dev] = true;
         }
         hipLaunchKernelGGL((f16_gemv_kernel<1>), dim3(G), dim3(64 * LMH_WAVES), lds, st, (const half_t*)w, (const half_t*)x,
-                           (half_t*)y, part_val, part_idx, M, N, K, iters);
+                           (half_t*)y, part_val, part_idx, M, N, K, iters, G);
     } else {
         if (lds > 64 * 1024 && !allowed[1][dev]) {
             const hipError_t e = hipFuncSetAttribute((const void*)f16_gemv_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -259,7 +259,7 @@ hipError_t launch_f16_gemv(const void* x, const void* w, void* y, float* part_va
             allowed[1][dev] = true;
         }
         hipLaunchKernelGGL((f16_gemv_kernel<2>), dim3(G), dim3(64 * LMH_WAVES), lds, st, (const half_t*)w, (const half_t*)x,
-                           (half_t*)y, part_val, part_idx, M, N, K, iters);
+                           (half_t*)y, part_val, part_idx, M, N, K, iters, G);
     }
     return hipGetLastError();
 }
