@@ -8,17 +8,20 @@
 namespace sq {
 
 // Layout L1.  One thread = one packed word = 8 outputs = one 16-byte store, so a
-// wave reads 256 contiguous bytes and writes 1 KiB contiguous bytes.
+// wave reads 256 contiguous bytes and writes 1 KiB contiguous bytes.  A thread has one to a few words, so what stands in front
+// of its loads counts: a word's row takes a division, which in 64 bits is some hundred instructions with a branch that the word's
+// own load waited behind (4128x2688 at group size 32, 6.8 -> 6.5 us).  I: 32 bits up to 2^31 words, 64 beyond (launch_indexed).
+template <typename I>
 __global__ __launch_bounds__(256) void dequant_l1_kernel(const uint32_t* __restrict__ w,
                                                          const half2_t* __restrict__ zs,
                                                          half8_t* __restrict__ out, int K8, int gshift8,
-                                                         int groups, long total_words) {
+                                                         int groups, I total_words, int blocks) {
     const NibbleMasks nm = nibble_masks();
-    const long stride = (long)gridDim.x * blockDim.x;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total_words; i += stride) {
-        const int n = (int)(i / K8);
-        const int k8 = (int)(i - (long)n * K8);
+    const I stride = (I)blocks * 256;
+    for (I i = (I)blockIdx.x * 256 + threadIdx.x; i < total_words; i += stride) {
         const uint32_t word = __builtin_nontemporal_load(w + i);
+        const I n = i / (I)K8;
+        const int k8 = (int)(i - n * (I)K8);
         const half2_t p = zs[(long)n * groups + (k8 >> gshift8)];
         const half2_t z64 = {p.x, p.x};
         const half2_t s = {p.y, p.y};
@@ -43,14 +46,17 @@ __device__ __forceinline__ uint32_t l2_nibble(const uint32_t* __restrict__ w, in
 
 // Layout L2.  One thread = 8 consecutive k of one row; a one-time conversion, so
 // the gather through the closed form is not tuned.
+template <typename I>
 __global__ __launch_bounds__(256) void dequant_l2_kernel(const uint32_t* __restrict__ w,
                                                          const half2_t* __restrict__ zs,
-                                                         half8_t* __restrict__ out, int N, int K, int g) {
-    const long total = (long)N * (K / 8);
-    const long stride = (long)gridDim.x * blockDim.x;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        const int n = (int)(i / (K / 8));
-        const int k0 = (int)(i - (long)n * (K / 8)) * 8;
+                                                         half8_t* __restrict__ out, int N, int K, int g,
+                                                         int blocks) {
+    const I K8 = (I)(K / 8);
+    const I total = (I)N * K8;
+    const I stride = (I)blocks * 256;
+    for (I i = (I)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) {
+        const int n = (int)(i / K8);
+        const int k0 = (int)(i - (I)n * K8) * 8;
         const half2_t p = zs[(long)(k0 / g) * N + n];
         half8_t r;
 #pragma unroll
@@ -68,22 +74,30 @@ static int log2i(int v) {
     return s;
 }
 
-hipError_t launch_dequant_l1(const void* w, const void* zs, void* out, int N, int K, int g, hipStream_t st) {
-    const long total = (long)N * (K / 8);
+// The width of the index that `total` words need; a trip past the end must not wrap, hence 31 bits.
+template <typename F>
+static hipError_t launch_indexed(long total, F&& launch) {
     long blocks = (total + 255) / 256;
     if (blocks > 256 * 32) blocks = 256 * 32;
-    hipLaunchKernelGGL(dequant_l1_kernel, dim3((unsigned)blocks), dim3(256), 0, st, (const uint32_t*)w,
-                       (const half2_t*)zs, (half8_t*)out, K / 8, log2i(g) - 3, K / g, total);
+    if (total < (1l << 31))
+        launch((int)blocks, (uint32_t)total);
+    else
+        launch((int)blocks, total);
     return hipGetLastError();
 }
 
+hipError_t launch_dequant_l1(const void* w, const void* zs, void* out, int N, int K, int g, hipStream_t st) {
+    return launch_indexed((long)N * (K / 8), [&](int blocks, auto total) {
+        hipLaunchKernelGGL((dequant_l1_kernel<decltype(total)>), dim3(blocks), dim3(256), 0, st, (const uint32_t*)w,
+                           (const half2_t*)zs, (half8_t*)out, K / 8, log2i(g) - 3, K / g, total, blocks);
+    });
+}
+
 hipError_t launch_dequant_l2(const void* w, const void* zs, void* out, int N, int K, int g, hipStream_t st) {
-    const long total = (long)N * (K / 8);
-    long blocks = (total + 255) / 256;
-    if (blocks > 256 * 32) blocks = 256 * 32;
-    hipLaunchKernelGGL(dequant_l2_kernel, dim3((unsigned)blocks), dim3(256), 0, st, (const uint32_t*)w,
-                       (const half2_t*)zs, (half8_t*)out, N, K, g);
-    return hipGetLastError();
+    return launch_indexed((long)N * (K / 8), [&](int blocks, auto total) {
+        hipLaunchKernelGGL((dequant_l2_kernel<decltype(total)>), dim3(blocks), dim3(256), 0, st, (const uint32_t*)w,
+                           (const half2_t*)zs, (half8_t*)out, N, K, g, blocks);
+    });
 }
 
 }  // namespace sq

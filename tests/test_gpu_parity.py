@@ -72,6 +72,15 @@ def test_dequant_l1_bit_exact(capi, n, k, g):
     assert np.array_equal(bits(out), d["w_hat"].view(np.int16))
 
 
+# rows of an odd number of words, from one word group to several trips per thread (2^21 threads at most)
+@pytest.mark.parametrize("n,k,g", [(8, 96, 32), (24, 1056, 32), (72, 2880, 64), (4104, 4128, 32)])
+def test_dequant_l1_odd_rows(capi, n, k, g):
+    d = linear(n, k, g, seed=4)
+    out = capi.dequant(d["w_dev"], d["zs_dev"], n, k, g)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(out), d["w_hat"].view(np.int16))
+
+
 def test_dequant_handmade_word(capi):
     # nibbles 0,2,4,6,1,3,5,7 -> q = 0..7 in natural order; z = 3, s = 0.5
     w = np.array([[0x20, 0x64, 0x31, 0x75] * 4] * 8, dtype=np.uint8)
