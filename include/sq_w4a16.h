@@ -396,7 +396,9 @@ int sq_lut_attention_strided(const void* q, const void* k, const void* v, void* 
  *   out        fp16 [B, H, D] contiguous (= [B, 1, H*D], the layout the output projection reads)
  *   cache_len  rows already valid; cache_len_dev, if not NULL, points to that number on the
  *              device (int64) and overrides cache_len -- read by the kernel, so a captured HIP
- *              graph follows a growing cache; the kernel clamps it to the cache size.
+ *              graph follows a growing cache; the kernel clamps it to the cache size.  Written by work
+ *              that is ordered before or behind the call: one that changes while the launch runs leaves
+ *              that call's out and appended row undefined (the workspace stays good for the next).
  *   workspace  NULL, or sq_decode_attention_workspace_bytes(B, H, D) bytes, 16-byte aligned, its
  *              first 1024 bytes (256 counters, a fixed region whatever B*H is) zero before the first call
  *              (every call leaves them zero), so one workspace serves calls with different B*H.  The kernel

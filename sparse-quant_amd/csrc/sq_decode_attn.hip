@@ -73,7 +73,8 @@ struct DecodeAttnArgs {
     float scale;
     // Shares of a head's cache rows, one workgroup each (grid y), for launches with too few heads to fill the chip: the
     // partial softmax states meet in the workspace behind its counters, one per head (zero between calls), and the last arriver
-    // merges them.
+    // merges them.  The whole grid arrives at a counter that wraps, however many shares a workgroup works out: where a length
+    // on the device changes under a running launch, workgroups disagree on them, and counters would stay behind for later calls.
     void* ws;
 };
 
@@ -106,10 +107,15 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     n0 = n0 < 0 ? 0 : (n0 > n0max ? n0max : n0);
     const int L = n0 + (append ? 1 : 0);  // rows attended; the appended row is row n0
     // This workgroup's share of the rows: [r0, r1).  The launch is sized for the whole cache where only the device knows the
-    // length: the workgroups that the rows are too few for leave (64 rows of a cache of 1024, 1 x 32 heads x 128: 9.8 -> 3.4 us).
+    // length: where one workgroup takes all rows the others arrive and leave, unused shares of several are empty (64 rows of a
+    // cache of 1024, 1 x 32 heads x 128: 9.8 -> 4.0 us, 3.6 without the arrivals).
     const int slots = a.slots, share = blockIdx.y;
     const int nsplit = shares_of(L, slots, D);
-    if (share >= nsplit) return;
+    auto arrive = [&]() { return atomicInc((unsigned*)a.ws + blockIdx.x, (unsigned)(slots - 1)); };  // agent scope, relaxed
+    if (nsplit == 1 && slots > 1) {
+        if (tid == 0) arrive();
+        if (share > 0) return;
+    }
     const int rows_per = nsplit == 1 ? L : (L + nsplit - 1) / nsplit;
     const int r0 = imin(share * rows_per, L);
     const int r1 = imin(r0 + rows_per, L);
@@ -260,15 +266,13 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
                            __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) {
-        const unsigned old = __hip_atomic_fetch_add((unsigned*)a.ws + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last_flag = (old == (unsigned)(nsplit - 1)) ? 1u : 0u;
-    }
+    if (tid == 0) last_flag = arrive() == (unsigned)(slots - 1) ? 1u : 0u;
     __syncthreads();
     if (!last_flag) return;
     // Everything is asked for at once: four outputs of a share per thread, and in every wave lane s the state of share s
     // (unused ones count as empty).  Each thread walking over the shares for its output took a round trip per share, twice:
-    // 1 x 32 heads x 128 (us) x 2001 rows 13.9 -> 10.4, x 4001 18.2 -> 14.7; 1 x 12 x 4001 x 64 16.9 -> 8.5.
+    // 1 x 32 heads x 128 (us) x 2001 rows 13.9 -> 10.3, x 4001 18.2 -> 15.0; 1 x 12 x 4001 x 64 16.9 -> 8.4; with a counter that
+    // wraps instead of one that the last arriver clears 10.0, 14.8 and 8.2.
     // The sums run over the shares in their order: bit-reproducible.
     constexpr int QD = D / 4;
     const int sp = tid / QD, d4 = tid % QD * 4;
@@ -300,7 +304,6 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
         }
         a.o[(long)blockIdx.x * D + tid] = (half_t)(og / lg);
     }
-    if (tid == 0) __hip_atomic_store((unsigned*)a.ws + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <int D>

@@ -345,3 +345,23 @@ def test_decode_shares_at_the_edges_of_passes(capi, b, h, d, device_length):
         ref = att.decode_attention_ref(q, k[:, :, :l], v[:, :, :l], d ** -0.5)
         check(out, ref, "l = %d" % l)
         assert torch.equal(kc[:, :, l - 1], new[0]) and torch.equal(vc[:, :, l - 1], new[1])
+
+
+@pytest.mark.parametrize("l", [1, 64, 256, 300, 513, 1000, 1024])
+def test_decode_every_workgroup_arrives_whatever_the_length_is(capi, l):
+    """A length on the device may change under a running launch (that call's output is then undefined), so that its workgroups
+    disagree on the number of shares.  The counters must be zero afterwards all the same: each of the grid's workgroups arrives
+    once, not each of the shares that the length calls for, and a counter wraps behind the last.  Started beyond the wrap, a
+    counter shows how many came: 8 of 1024 rows of 1 x 32 heads x 128, the first of which sets it to zero."""
+    b, h, d, lmax = 1, 32, 128, 1024
+    q, k, v = (torch.from_numpy(a).cuda() for a in make(b, h, lmax, d, seed=l))
+    ws = torch.zeros(capi.lib().sq_decode_attention_workspace_bytes(b, h, d), dtype=torch.uint8, device="cuda")
+    counters = ws[:1024].view(torch.int32)
+    counters[:h] = 100
+    capi.decode_attention(q, k, v, torch.tensor([l], device="cuda"), 0.1, ws=ws)
+    assert counters[:h].tolist() == [7] * h and torch.count_nonzero(counters[h:]).item() == 0
+    counters.zero_()
+    out = capi.decode_attention(q, k, v, torch.tensor([l], device="cuda"), 0.1, ws=ws)
+    ref = att.decode_attention_ref(q.cpu().numpy(), k[:, :, :l].cpu().numpy(), v[:, :, :l].cpu().numpy(), 0.1)
+    check(out, ref, "l = %d" % l)
+    assert torch.count_nonzero(ws[:1024]).item() == 0
