@@ -1005,13 +1005,18 @@ static const RingTile kRingTiles[] = {
     {256, 256, 64, 9.097f, 0.833f, 0.661f, 0.f, 0.f, 0.f, 1.343f},  // never split, see plan_ring
 };
 // The same with the scale on the sums (up to 64 tokens), where other constants hold: shapes 1..5, of which the fourth is
-// not built for it.  Adjusted for the choice on 96 weights x token counts (768 .. 22016 rows, K 768 .. 16384, 17 .. 64 tokens) with
-// the zeros/scales of several stages at once: 0.3 % above the best in the geometric mean (0.5 with the constants before), at worst 6 %.
+// not built for it; the second's at 17..32 tokens alone.  The zeros/scales of several stages at once made its stages 5..8 % faster,
+// and only there is it the better choice more often for it: over random weights (256 .. 32768 rows, K 768 .. 16384) whose plan
+// changes with its constant, 0.754 -> 0.706, time 0.973 and 0.984 in the geometric mean of two samples of 45 (at best 0.89, at
+// worst 1.05); at 1..4 tokens 1.045, at 5..16 1.025, at 33..64 0.99 and 1.01.  Against the best of all shapes and splits of 1500
+// weights and token counts (1..64, one weight or gate and up): 0.45 % in the geometric mean, 5 % of them more than 3.9 %.
 static const RingTile kRingSumsTiles[] = {
-    kRingTiles[0], {32, 128, 256, 1.498f, 0.706f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f},
-    {64, 128, 256, 2.740f, 0.778f, 0.244f, 0.211f, 0.576f, 0.409f, 0.f},
+    kRingTiles[0], {32, 128, 256, 1.498f, 0.706f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f}, {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f, 0.f},
     kRingTiles[3], {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f, 0.f},
 };
+static const RingTile& ring_tile(int s, int M, bool sums) {
+    return sums && s < 5 && (s != 1 || (M > 16 && M <= 32)) ? kRingSumsTiles[s] : kRingTiles[s];
+}
 constexpr int RING_SHAPES = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
 #define X_(id, MI, NI, WM, WN, WK, ST)                                                                              \
     static_assert(id >= 1 && id <= RING_SHAPES, "a row of kRingTiles per shape");
@@ -1037,7 +1042,7 @@ static RingPlan plan_ring(int M, int N, int K, size_t ws_bytes, bool sums) {
     float best_us = 3.4e38f;
     const int rows32 = (M + 31) / 32 * 32;
     for (int s = 0; s < RING_SHAPES; s++) {
-        const RingTile& t = sums && s < 5 ? kRingSumsTiles[s] : kRingTiles[s];
+        const RingTile& t = ring_tile(s, M, sums);
         const int mt = (M + t.bm - 1) / t.bm;
         // a third of the matrix work would be padding; up to 64 rows the others are the ones with the scale on the sums
         if (t.bm > 64 && (M <= 64 || mt * t.bm * 2 > rows32 * 3)) continue;

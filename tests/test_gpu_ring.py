@@ -181,6 +181,30 @@ def test_ring_multiplicand(capi, shape, m, n, k, g):
         assert ran >= 1
 
 
+@pytest.mark.parametrize("pair,m,n,k,taken,other", [
+    (False, 8, 7616, 8704, (1, 2), (2, 4)), (False, 16, 8192, 8448, (1, 2), (2, 4)), (True, 3, 3776, 8448, (1, 2), (2, 4)),
+    (False, 32, 10944, 10880, (2, 2), (1, 1)), (False, 52, 20288, 8320, (5, 3), (3, 1)), (True, 47, 10624, 10112, (5, 3), (3, 1))])
+def test_ring_plans_the_faster_shape_at_few_tokens(capi, pair, m, n, k, taken, other):
+    """Shape and K split of the automatic choice with the scale on the sums, by its bits: of those timed, the other one takes 7 %
+    (up to 16 tokens) to 13 % longer."""
+    g = 128
+    x, dev, _, _ = gated_operands(m, n, k, g, seed=n)
+    ws = torch.zeros(65536 + 300 * 128 * 256 * 4, dtype=torch.uint8, device=DEV)
+    L, p = capi.lib(), lambda t: t.data_ptr()
+
+    def run(algo):
+        if not pair:
+            return capi.gemm_ws(x, dev[0], dev[1], n, k, g, algo=algo, ws=ws)
+        y = torch.empty((m, n), dtype=torch.float16, device=DEV)
+        assert L.sq_w4a16_gemm_silu_dot_one(p(x), *(p(t) for t in dev), p(y), m, n, k, g, capi.SQ_LAYOUT_L1, algo, p(ws), ws.numel(),
+                                            capi._stream(None)) == 0
+        return y
+
+    forced = [run(capi.SQ_ALGO_RING | ((shape | SUMS | (parts << 8)) << 8)) for shape, parts in (taken, other)]
+    assert not torch.equal(*forced)  # (the sums' order is another)
+    assert torch.equal(run(capi.SQ_ALGO_AUTO), forced[0])
+
+
 def gated_operands(m, n, k, g, seed):
     """x, then weight and zeros/scales of gate and of up, with their float64 products: of W_hat, and of (q - z) s unrounded."""
     from sqamd import capi as c
