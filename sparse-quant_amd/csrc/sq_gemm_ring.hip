@@ -83,7 +83,7 @@ constexpr int ring_trip(int l, int cap, int unit) {
     return u;
 }
 
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS>
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SETS>
 struct RingShape {
     static constexpr int NW = WM * WN * WK, NT = 64 * NW;
     static constexpr int BM = 32 * MI * WM, BN = 32 * NI * WN, KS = 64 * WK;
@@ -91,7 +91,6 @@ struct RingShape {
     static constexpr int P = (KS >> GS) ? (KS >> GS) : 1;  // zeros/scales pairs per column and stage
     // Zeros/scales: a stage's own with its other operands, or (SETS) those of ZN stages, ZD of a row, in two buffers behind
     // the stages: see issue_set.
-    static constexpr bool SETS = SUMS && P <= 2;
     static constexpr int ZD = SETS ? 8 : P, ZN = ZD / P;
     static constexpr int ZB = BN * ZD * 4;
     static constexpr int SB = XB + WB + (SETS ? 0 : ZB);
@@ -200,19 +199,19 @@ __device__ __forceinline__ void load_to_lds_x1_masked(const void* base, uint32_t
 // outputs' in the same workgroup, so that the product is formed in the store and the tiles of both fill the chip's rounds
 // together (us, two launches / one: 11008x4096 at 32 tokens 25.1 / 19.5, at 333 and group size 64 101 / 80.0; 13696x5120 at
 // 100 62.7 / 43.4; 11008x4096 at 2048 396 / 329).  Nothing is rounded between the products.
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool PAIR>
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool SETS, bool PAIR>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4))) void gemm_ring_kernel(
     const uint8_t* __restrict__ W, const half2_t* __restrict__ ZS, const half_t* __restrict__ X, half_t* __restrict__ Y,
     int M, int N, int K, int mtiles, int tiles, int nfull, int ksplit, Epilogue epi, float* part, unsigned* counters,
     const uint8_t* __restrict__ W2, const half2_t* __restrict__ ZS2, half_t* __restrict__ U) {
-    using S = RingShape<MI, NI, WM, WN, WK, GS, ST, SUMS>;
+    using S = RingShape<MI, NI, WM, WN, WK, GS, ST, SETS>;
     constexpr int BM = S::BM, BN = S::BN, KS = S::KS, SB = S::SB, XI = S::XI, WI = S::WI, ZI = S::ZI, ZL = S::ZL, PER = S::PER, P = S::P;
-    constexpr bool SETS = S::SETS;
     constexpr int ZD = S::ZD, ZN = S::ZN;
     constexpr int X_OFF = 0, W_OFF = S::XB, Z_OFF = SETS ? ST * SB : S::XB + S::WB;
     constexpr int H = 4;  // 16-wide k slices per stage and wave
     constexpr bool ALTERNATE = SUMS || MI == 1;  // two groups of waves in turn (see the head of this file)
     static_assert(!ALTERNATE || S::NW == 8, "waves 0..3 and 4..7");
+    static_assert(!SETS || (SUMS && S::P <= 2), "eight pairs of a row at once are four or eight stages'");
     static_assert(!SUMS || (MI * NI <= 4 && GS == 7 && S::NW == 8), "a stage of a wave lies in one group, and the registers suffice");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S::LDS];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
@@ -288,11 +287,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         zlane[j] = (uint32_t)((long)imin(n0 + d / ZD % BO, N - 1) * groups * 4) + (SETS ? 0 : d % P * 4);
     }
     // A stage's own zeros/scales are 4 or 8 bytes of a row, each in a line of its own: with 32 rows per tile a third of the lines
-    // that a stage asks for, and the loads come back in order.  So 32 bytes of a row at once, in front of the first of the ZN
-    // stages that they serve (us: 64 tokens 12288x4096 in tiles of 64 x 128 23.2 -> 21.9, 64 x 256 split in two 26.5 -> 25.4; 32
-    // tokens 4096x11008 in tiles of 32 x 128 split in two 24.4 -> 22.7, gate and up of 11008x4096 19.4 -> 17.8).  Two buffers: set s
-    // goes out when all have read stage ZN s - ST, which is no earlier than the last one of set s - 2.  Not for the waves in step:
-    // the branch in their loop costs what it saves (100 tokens 15360x5120 in tiles of 96 x 128 32.3 -> 33.8, 200 12288x4096 in 96 x 256
+    // that a stage asks for, and the loads come back in order.  So, where that is ahead (ring_sets), 32 bytes of a row at once, in
+    // front of the first of the ZN stages that they serve (us: 64 tokens 12288x4096 in tiles of 64 x 128 23.2 -> 21.9, 64 x 256 split
+    // in two 26.5 -> 25.4; 32 tokens 4096x11008 in tiles of 32 x 128 split in two 24.4 -> 22.7, gate and up of 11008x4096 19.4 -> 17.8).
+    // Two buffers: set s goes out when all have read stage ZN s - ST, which is no earlier than the last one of set s - 2.  Not for
+    // the waves in step: the branch in their loop costs what it saves (100 tokens 15360x5120 in tiles of 96 x 128 32.3 -> 33.8, 200 12288x4096 in 96 x 256
     // 34.9 -> 37.3, 333 at group size 64 41.4 -> 42.3).
     auto issue_set = [&](int set) {
         const int g = ((it0 * KS) >> GS) + set * ZD;
@@ -962,16 +961,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     SQ_RING_LOW_SHAPES(X_) X_(4, 3, 1, 1, 4, 2, 4) X_(6, 3, 2, 1, 4, 2, 3) X_(7, 4, 1, 1, 4, 2, 3)        \
         X_(8, 4, 2, 1, 4, 2, 3) X_(9, 8, 2, 1, 4, 1, 3)
 
-template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool PAIR>
+template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool SETS, bool PAIR>
 static hipError_t launch_shape(const void* x, const void* w, const void* zs, const void* w2, const void* zs2, void* y, void* u, int M,
                                int N, int K, int nfull, int ksplit, Epilogue epi, void* ws, hipStream_t st) {
-    using S = RingShape<MI, NI, WM, WN, WK, GS, ST, SUMS>;
+    using S = RingShape<MI, NI, WM, WN, WK, GS, ST, SETS>;
     const int mt = (M + S::BM - 1) / S::BM;
     constexpr int BO = PAIR ? S::BN / 2 : S::BN;
     const int tiles = mt * ((N + BO - 1) / BO);
     if (ksplit == 1) nfull = tiles;
     const int grid = ksplit == 1 ? (tiles + 7) / 8 * 8 : nfull + ((tiles - nfull) * ksplit + 7) / 8 * 8;
-    hipLaunchKernelGGL((gemm_ring_kernel<MI, NI, WM, WN, WK, GS, ST, SUMS, PAIR>), dim3(grid), dim3(S::NT), 0, st, (const uint8_t*)w,
+    hipLaunchKernelGGL((gemm_ring_kernel<MI, NI, WM, WN, WK, GS, ST, SUMS, SETS, PAIR>), dim3(grid), dim3(S::NT), 0, st, (const uint8_t*)w,
                        (const half2_t*)zs, (const half_t*)x, (half_t*)y, M, N, K, mt, tiles, nfull, ksplit, epi,
                        ws ? (float*)((char*)ws + RING_COUNTER_BYTES) : nullptr, (unsigned*)ws, (const uint8_t*)w2,
                        (const half2_t*)zs2, (half_t*)u);
@@ -1005,11 +1004,12 @@ static const RingTile kRingTiles[] = {
     {256, 256, 64, 9.097f, 0.833f, 0.661f, 0.f, 0.f, 0.f, 1.343f},  // never split, see plan_ring
 };
 // The same with the scale on the sums (up to 64 tokens), where other constants hold: shapes 1..5, of which the fourth is
-// not built for it; the second's at 17..32 tokens alone.  The zeros/scales of several stages at once made its stages 5..8 % faster,
-// and only there is it the better choice more often for it: over random weights (256 .. 32768 rows, K 768 .. 16384) whose plan
-// changes with its constant, 0.754 -> 0.706, time 0.973 and 0.984 in the geometric mean of two samples of 45 (at best 0.89, at
-// worst 1.05); at 1..4 tokens 1.045, at 5..16 1.025, at 33..64 0.99 and 1.01.  Against the best of all shapes and splits of 1500
-// weights and token counts (1..64, one weight or gate and up): 0.45 % in the geometric mean, 5 % of them more than 3.9 %.
+// not built for it; the second's at 17..32 tokens alone.  There its stages are faster with the zeros/scales of several at once
+// (ring_sets), and where 0.706 for 0.754 changes the plan of random weights (256 .. 32768 rows, K 768 .. 16384) it takes 0.979 of
+// the time in the geometric mean (12 of 1300, at worst 1.06); at fewer tokens most plans have them by the stage (with 0.706 there
+// and sets 1.045 at 1..4 tokens, 1.025 at 5..16), at 33..64 the two constants are level (0.99 and 1.01 of 30 each).  Against the
+// best of all shapes and splits of those 1300 (1..64 tokens, one weight or gate and up): 0.5 % in the geometric mean, 5 % of them
+// more than 4.1 %.
 static const RingTile kRingSumsTiles[] = {
     kRingTiles[0], {32, 128, 256, 1.498f, 0.706f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f}, {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f, 0.f},
     kRingTiles[3], {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f, 0.f},
@@ -1089,6 +1089,28 @@ size_t gemm_ring_workspace_bytes(int M, int N, int K) {
     return b > sums ? b : sums;
 }
 
+// With the scale on the sums and tiles of 128 or 256 columns: zeros/scales of several stages at once (SETS of the kernel), or a
+// stage's with its other operands.  `k`: columns of K of a workgroup.  A set is a burst in front of its first stage, which a K of
+// one or two sets shows, and so does a loop that waits for latency; it saves lines, which counts where the rows of a tile ask
+// for many, and more of them where a row has an odd number of pairs, so that a stage's two are no aligned 8 bytes.  Time with
+// sets / without, 32 x 128 tiles, 16..256 workgroups, geometric means (an even number of groups; an odd one has 1 more):
+//   k        512  1024  1536  2048  2560  3072  4096  5120  6144  8192 12288     an odd number of groups
+//   2 rows  1.04  1.06  1.06  1.07  1.07  1.07  1.08  1.01  1.03  1.03  1.03     1.06 1.07 1.03 1.05 1.06 1.03 1.00 1.00 0.97 0.97 0.94
+//   8       1.05  1.07  1.07  1.06  1.06  1.06  1.05  0.99  1.00  1.01  1.01     1.05 1.06 1.03 1.03 1.03 1.01 0.98 0.97 0.96 0.94 0.91
+//   16      1.05  1.06  1.06  1.06  1.04  1.03  1.02  0.95  0.98  0.98  0.96     1.06 1.06 1.03 1.00 1.00 0.98 0.96 0.95 0.94 0.92 0.88
+//   24      1.04  1.07  1.05  1.04  1.02  1.01  0.99  0.93  0.94  0.95  0.92     1.05 1.06 1.02 1.00 0.98 0.97 0.94 0.91 0.91 0.90 0.86
+//   32      1.04  1.05  1.04  1.03  0.98  0.97  0.96  0.89  0.92  0.92  0.88     1.04 1.04 1.00 0.98 0.96 0.95 0.91 0.91 0.90 0.88 0.84
+// 64 x 128 tiles by the share of rows that are there are within 0.03 of that, 64 x 256 tiles lose less and gain up to twice as
+// much (64 rows of an odd number of groups 0.97 0.96 0.97 0.97 0.95 0.92 0.87 0.81 0.81 0.78 0.77).  Over 1050 random weights,
+// token counts and K splits, one weight and gate and up: by this rule 0.965, 0.978 and 0.905 of the time without for the three
+// tiles, always with sets 0.972, 0.979 and 0.905, the better one each time 0.961, 0.973 and 0.903.
+static bool ring_sets(const RingTile& t, int M, int K, int parts) {
+    const int k = K / parts;
+    const long rows = (long)(M + t.bm - 1) / t.bm * t.bm;
+    if (K / 128 % 2) return k > (4L * M <= rows ? 4096 : 2048);
+    return 2L * M > rows && k > (4L * M <= 3 * rows ? 4096 : 2048);
+}
+
 // tune = 0 for the cost model's choice, else shape id | 0x10: only the tiles of the last, part-filled round of 256
 // workgroups split K | K split << 8; RING_SUMS: the scale on the sums (also with the model's choice; group size 128, tiles
 // of 32 and 64 rows).  hipErrorInvalidValue: not applicable (or the workspace is missing or too small).
@@ -1115,14 +1137,16 @@ static hipError_t launch_ring(const void* x, const void* w, const void* zs, cons
                 return hipErrorInvalidValue;
         }
     }
-#define SQ_RING_LAUNCH(MI, NI, WM, WN, WK, GS, ST, SUMS) \
-    launch_shape<MI, NI, WM, WN, WK, GS, ST, SUMS, PAIR>(x, w, zs, w2, zs2, y, u, M, N, K, p.nfull, p.ksplit, epi, ws, st)
+#define SQ_RING_LAUNCH(MI, NI, WM, WN, WK, GS, ST, SUMS, SETS) \
+    launch_shape<MI, NI, WM, WN, WK, GS, ST, SUMS, SETS, PAIR>(x, w, zs, w2, zs2, y, u, M, N, K, p.nfull, p.ksplit, epi, ws, st)
     if (tune & RING_SUMS) {
         if (g != 128) return hipErrorInvalidValue;
+        const bool sets = ring_sets(kRingTiles[p.shape - 1], M, K, p.nfull ? 1 : p.ksplit);
         switch (p.shape) {
-#define X_(id, MI, NI, WM, WN, WK, ST) \
-    case id:                           \
-        return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 7, ST, true);
+#define X_(id, MI, NI, WM, WN, WK, ST)                                           \
+    case id:                                                                     \
+        return sets ? SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 7, ST, true, (WK <= 4)) \
+                    : SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 7, ST, true, false);
             SQ_RING_LOW_SHAPES(X_)
 #undef X_
         }
@@ -1131,9 +1155,9 @@ static hipError_t launch_ring(const void* x, const void* w, const void* zs, cons
     switch (p.shape) {
 #define X_(id, MI, NI, WM, WN, WK, ST)                                              \
     case id:                                                                        \
-        if (g == 128) return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 7, ST, false);      \
-        if (g == 64) return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 6, ST, false);       \
-        return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 5, ST, false);
+        if (g == 128) return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 7, ST, false, false);      \
+        if (g == 64) return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 6, ST, false, false);       \
+        return SQ_RING_LAUNCH(MI, NI, WM, WN, WK, 5, ST, false, false);
         SQ_RING_SHAPES(X_)
 #undef X_
     }

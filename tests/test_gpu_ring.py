@@ -359,6 +359,33 @@ def test_ring_sums_every_count_of_stages(capi, shape, stage, short):
             assert np.all(np.abs(got - ref) <= bound), (stages, parts, np.max(np.abs(got - ref) / bound))
 
 
+@pytest.mark.parametrize("shape,rows", [(2, 32), (3, 64), (5, 64)])
+@pytest.mark.parametrize("quarters,k", [(1, 3200), (1, 2176), (2, 4352), (2, 5120), (3, 2560), (3, 2304)])
+def test_ring_sums_zeros_and_scales_by_the_set_and_by_the_stage(capi, shape, rows, quarters, k):
+    """One token more than a quarter (an odd number of groups), half and three quarters of a tile's rows brings zeros and scales
+    by the set: the bits of the other tokens stay, unsplit and with K split, for one weight and for gate and up."""
+    n, g, m = 136, 128, rows * quarters // 4
+    L, p = capi.lib(), lambda t: t.data_ptr()
+    ws = torch.zeros(65536 + (8 << 20), dtype=torch.uint8, device=DEV)
+    for parts in (1, 2):  # an odd number of groups in two parts begins inside a group's stage of two
+        kk = k * parts + (g if parts == 2 and k // g % 2 else 0)
+        x, dev, _, real = gated_operands(m + 1, n, kk, g, seed=kk + m)
+        word = capi.SQ_ALGO_RING | ((shape | SUMS | (parts << 8)) << 8)
+        y = [capi.gemm_ws(x[:i], dev[0], dev[1], n, kk, g, algo=word, ws=ws) for i in (m, m + 1)]
+        assert torch.equal(y[0], y[1][:m])
+        # one rounding to fp16 and the fp32 sums, norm-wise far below it
+        assert (y[1].double() - real[0]).norm() <= (2.0 ** -11 + 2.0 ** -17) * real[0].norm()
+        u = []
+        for i in (m, m + 1):
+            u.append(torch.empty((i, n), dtype=torch.float16, device=DEV))
+            assert L.sq_w4a16_gemm_silu_dot_one(p(x), *(p(t) for t in dev), p(u[-1]), i, n, kk, g, capi.SQ_LAYOUT_L1, word, p(ws),
+                                                ws.numel(), capi._stream(None)) == 0
+        assert torch.equal(u[0], u[1][:m])
+        ref = torch.nn.functional.silu(real[0]) * real[1]
+        assert (u[1].double() - ref).norm() <= (2.0 ** -10 + 2.0 ** -15) * ref.norm()
+        assert capi.workspace_is_clean(ws)
+
+
 def test_ring_has_the_scale_on_the_sums_where_it_says(capi):
     d = orc.synth_linear(64, 128, 32, seed=1)
     x, w, zs = to_dev(orc.synth_x(8, 128)), to_dev(d["w_l1"]), to_dev(d["zs_l1"])
