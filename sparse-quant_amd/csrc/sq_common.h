@@ -149,7 +149,7 @@ struct LnPre {
 // step of four layers at 8 sequences from a graph 305.5 instead of 308.  (The ring kernel keeps 136 bytes, none of them
 // implicit: with 104, 2048 tokens through a layer of 4096 x 16384 took 753 us instead of 751, a prompt of 8 x 512 3037
 // instead of 3022.)
-// The lm_head, decode attention (152 bytes instead of 416) and the layout conversions take their grid as an argument as well: that
+// The lm_head and decode attention (152 bytes instead of 416) take their grid as an argument as well: that
 // decode step 306.6 -> 304.3 us, 1.3 of it the divisions in front of an unshared head's rows.
 
 // What happens to an fp32 accumulator on its way to Y[m, n]: + bias[n], activation,
