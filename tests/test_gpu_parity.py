@@ -72,13 +72,47 @@ def test_dequant_l1_bit_exact(capi, n, k, g):
     assert np.array_equal(bits(out), d["w_hat"].view(np.int16))
 
 
-# rows of an odd number of words, from one word group to several trips per thread (2^21 threads at most)
-@pytest.mark.parametrize("n,k,g", [(8, 96, 32), (24, 1056, 32), (72, 2880, 64), (4104, 4128, 32)])
+# numbers of words that are no power of two; the last two begin a second and a third trip per thread (2^21 threads at most)
+@pytest.mark.parametrize("n,k,g", [(8, 96, 32), (24, 1056, 32), (72, 2880, 64), (4104, 4128, 32), (8200, 4128, 32)])
 def test_dequant_l1_odd_rows(capi, n, k, g):
     d = linear(n, k, g, seed=4)
     out = capi.dequant(d["w_dev"], d["zs_dev"], n, k, g)
     torch.cuda.synchronize()
     assert np.array_equal(bits(out), d["w_hat"].view(np.int16))
+
+
+@pytest.mark.parametrize("layout", ["l1", "l2"])
+def test_dequant_beyond_32_bit_indexes(capi, layout):
+    """2^31 packed words take the kernels' 64-bit indexes, and parts of the same weight the 32-bit ones (a thread's second to
+    128th trip among them; against the oracle above and below).  L1 is cut between rows, L2 between groups of K."""
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 47 GiB of device memory")
+    n = k = 1 << 17
+    g, parts = 128, 8
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    w = torch.randint(0, 256, (n * k // 2,), dtype=torch.uint8, device=DEV, generator=gen)
+    zs = torch.empty((n * k // g, 2), dtype=torch.float16, device=DEV)
+    zs[:, 0] = torch.randint(64, 80, (n * k // g,), device=DEV, generator=gen)
+    zs[:, 1] = torch.rand(n * k // g, device=DEV, generator=gen) * 0.02
+    of = capi.SQ_LAYOUT_L1 if layout == "l1" else capi.SQ_LAYOUT_L2
+    whole = capi.dequant(w, zs, n, k, g, layout=of)
+    for i in range(parts):
+        wi, zi = w.chunk(parts)[i], zs.chunk(parts)[i]
+        if layout == "l1":
+            part, same = capi.dequant(wi, zi, n // parts, k, g, layout=of), whole.chunk(parts)[i]
+        else:
+            part, same = capi.dequant(wi, zi, n, k // parts, g, layout=of), whole.chunk(parts, dim=1)[i]
+        assert torch.equal(part, same)
+    del whole, part, same, w, zs, wi, zi
+    torch.cuda.empty_cache()
+
+
+def test_dequant_l2_several_trips(capi):
+    n, k, g = 4128, 4224, 128  # 2179584 words: a thread's second trip begins
+    d = orc.synth_linear(n, k, g, seed=6)
+    zs = np.stack([d["z"].astype(np.float16).T + np.float16(64), d["s"].T], axis=-1)
+    out = capi.dequant(to_dev(orc.pack_l2(d["q"])), to_dev(np.ascontiguousarray(zs)), n, k, g, layout=capi.SQ_LAYOUT_L2)
+    assert np.array_equal(bits(out), orc.dequant_l1(d["w_l1"], d["zs_l1"], g).view(np.int16))
 
 
 def test_dequant_handmade_word(capi):

@@ -335,15 +335,17 @@ def test_ring_parity_with_the_scale_on_the_sums(capi, shape, m, n, k, g):
         assert capi.workspace_is_clean(ws)
 
 
-@pytest.mark.parametrize("shape,stage", [(1, 512), (2, 256), (3, 256), (5, 128)])
-@pytest.mark.parametrize("short", [0, 128])
-def test_ring_sums_every_count_of_stages(capi, shape, stage, short):
-    """Zeros and scales come for four or eight stages at once: a last set that is whole, one stage long and ends early, a part
-    of K that begins inside what would be another part's set, and row ends of the last weight row."""
-    m, n, g = 19, 136, 128
+@pytest.mark.parametrize("shape,stage,short", [(1, 512, 0), (1, 512, 128), (2, 256, 0), (2, 256, 128), (3, 256, 0), (3, 256, 128),
+                                               (5, 128, 0)])
+@pytest.mark.parametrize("m", [19, 50])
+def test_ring_sums_every_count_of_stages(capi, shape, stage, short, m):
+    """Zeros and scales by the stage, and (50 tokens, K of a part over 2048) for four or eight stages at once: a last set that is
+    whole, one stage long and ends early, a part of K that begins inside what would be another part's set, and row ends of the
+    last weight row."""
+    n, g = 136, 128
     ws = torch.zeros(65536 + (8 << 20), dtype=torch.uint8, device=DEV)
     for stages in (1, 2, 3, 4, 5, 7, 8, 9, 12, 13, 16, 17, 18, 25) if stage < 512 else (1, 2, 3, 5):
-        k = stage * stages - (short if stage > 128 else 0)
+        k = stage * stages - short
         d = orc.synth_linear(n, k, g, seed=k)
         w64, x = real_weight(d, g), orc.synth_x(m, k, seed=shape)
         x64 = x.astype(np.float64)
