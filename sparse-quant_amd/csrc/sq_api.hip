@@ -239,19 +239,21 @@ int ring_tune(int M, int g) { return g == 128 && M <= 64 ? sq::RING_SUMS : 0; }
 // 0.8 of the two in the geometric mean, at worst 1.05.
 // Group size 64, 5 tokens up, where the two would be the streaming or the ring kernel's (W_hat there as here): 7680x2560 17.6 /
 // 9.9, 2816x1024 6.3 / 5.7, 13824x4608 29.2 / 22.8, 12288x4096 20.4 / 19.8; but 24576x2048 at 5 20.7 / 21.1, 8512x3968 17.0 / 18.1.
-// Group size 128 (the scale on the sums here as there):
-//   the streaming kernel's K ranges leave its chunk slots part empty: 13696x5120 at 8 tokens 30.7 / 25.3, 5632x2048 8.7 / 7.6,
-//   2816x1024 6.3 / 5.8, 28672x5120 52.6 / 47.6; but at 3 19072x4992 without a workspace 32.0 / 36.8, 26112x5504 42.7 / 48.2
-//   they fill them: one launch where its 32 x 128 tiles leave neither half the chip nor most of a round idle: 8192x4096 16.4 /
-//   13.1, 14336x4096 20.4 / 20.0, 16384x4096 22.1 / 20.8; but 8256x4096 14.2 / 17.5 (129 tiles), 11008x4096 17.6 / 19.3 (172),
-//   2048x4096 8.7 / 8.8 (32), and at 3 without a workspace 8384x10112 32.4 / 37.4
-//   1 and 2 tokens (the GEMV): 8192x5120 17.8 / 15.7, 15360x5120 29.0 / 24.5; but 7680x3072 10.5 / 10.8, and at 1 9856x5120 18.2 /
-//   20.2 (154 tiles), 12992x5248 21.5 / 22.9 (203)
-// With few tokens a last stage of K that is half empty (K % 256 != 0) is time: 11584x5760 at 3 22.3 / 24.7, 11200x3712 at 5 and
+// Group size 128 (the scale on the sums here as there; timed again after the lines were drawn, with zeros/scales as ring_sets has
+// them and the streaming kernel's short arguments: 163 random weights where it is taken 0.82 in the geometric mean, at worst 1.10):
+//   the streaming kernel's K ranges leave its chunk slots part empty: 13696x5120 at 8 tokens 29.7 / 23.5, 5632x2048 9.5 / 8.2,
+//   2816x1024 6.2 / 6.1, 28672x5120 46.7 / 45.3; but at 3 19072x4992 without a workspace 33.6 / 38.7, 26112x5504 43.6 / 46.5
+//   they fill them: one launch where its 32 x 128 tiles leave neither half the chip nor most of a round idle: 8192x4096 at 8 14.6 /
+//   11.9, 14336x4096 18.3 / 18.6, at 16 19.0 / 19.1, 16384x4096 at 8 19.5 / 19.2, at 16 20.5 / 19.9; but at 8 8256x4096 14.6 / 17.4
+//   (129 tiles), 11008x4096 16.1 / 17.8 (172), 2048x4096 9.3 / 8.9 (32; at 16 10.9 / 9.0, where the line is behind), and at 3
+//   without a workspace 8384x10112 32.8 / 34.6
+//   1 and 2 tokens (the GEMV): at 2 8192x5120 18.7 / 13.6, 15360x5120 30.6 / 22.7; but at 1 7680x3072 10.3 / 10.0, 9856x5120 18.5 /
+//   20.6 (154 tiles), 12992x5248 22.1 / 21.9 (203)
+// With few tokens a last stage of K that is half empty (K % 256 != 0) is time: 11584x5760 at 3 22.7 / 23.1, 11200x3712 at 5 and
 // group size 64 17.5 / 18.4.
 // Up to 8 tokens and 64 tiles the latency of two decode launches stands against one ring launch's and the exchange of its K
-// ranges, or a K that is not split: 2048x2048 at 3 6.9 / 8.0, at 5 and group size 64 7.1 / 7.7; 1408x2304 at 3 7.2 / 8.0;
-// 4096x3328 at 5 and group size 64 9.9 / 10.9, without a workspace 512x3840 8.7 / 10.8; 3520x2944 at 5 8.9 / 9.5;
+// ranges, or a K that is not split: 2048x2048 at 3 6.4 / 7.7, at 5 and group size 64 7.1 / 7.7; 1408x2304 at 3 7.1 / 7.8;
+// 4096x3328 at 5 and group size 64 9.9 / 10.9, without a workspace 512x3840 8.7 / 10.8; 3520x2944 at 5 9.3 / 9.2;
 // 3328x3712 at 16 and group size 64 without a workspace 11.3 / 12.2.
 bool pair_at_few_tokens(int M, int N, int K, int g, int each, bool ws_ok) {  // each: the kernel of the two launches
     const long tiles = (2L * N + 127) / 128;

@@ -141,16 +141,16 @@ struct LnPre {
     float eps;
 };
 
-// Arguments of a small linear's launch: at most 112 bytes, the implicit ones included, which gridDim and blockDim bring in.
-// Writing them costs the host 2.75 us a launch up to there and 3.5 beyond (4.4 at 280 bytes and implicit ones).  So the
+// Arguments of a launch of skinny2_kernel, skinny3_kernel, gemm_kernel, gemm_lds_kernel and the GEMVs: at most 112 bytes, none of
+// them implicit, which gridDim and blockDim would bring in.  (Grouped launches keep 260 to 272 bytes, skinny_kernel 336 with its
+// implicit ones.)  Writing them costs the host 2.75 us a launch up to there and 3.5 beyond (4.4 at 280 bytes and implicit ones).  So the
 // workspace is one pointer, the counters at its start, and the kernels work their grid out: 376, 360 and 352 bytes -> 112, 96
-// and 96.  Called from Python, 4 linears of a layer of 1280 x 5120 at 12 tokens take 31.9 us a pass instead of 33.2, of
-// 4096 x 16384 at 8 tokens 36.0 instead of 36.6, a gated MLP block of 1024 x 2816 at 8 tokens 23.7 instead of 24.8; a decode
-// step of four layers at 8 sequences from a graph 305.5 instead of 308.  (The ring kernel keeps 136 bytes, none of them
-// implicit: with 104, 2048 tokens through a layer of 4096 x 16384 took 753 us instead of 751, a prompt of 8 x 512 3037
-// instead of 3022.)
-// The lm_head and decode attention (152 bytes instead of 416) take their grid as an argument as well: that
-// decode step 306.6 -> 304.3 us, 1.3 of it the divisions in front of an unshared head's rows.
+// and 96.  Called from Python, 4 linears of a layer of 1280 x 5120 at 12 tokens take 36.7 us a pass instead of 37.6, of
+// 4096 x 16384 at 8 tokens 36.3 instead of 37.0, a gated MLP block of 1024 x 2816 at 8 tokens 26.9 instead of 28.0.  (The ring
+// kernel keeps 136 bytes, none of them implicit: with 104, 2048 tokens through a layer of 4096 x 16384 took 753 us instead of
+// 751, a prompt of 8 x 512 3037 instead of 3022.)
+// The lm_head and decode attention (152 bytes instead of 416) take their grid as an argument as well.  A decode step of four layers
+// at 8 sequences from a graph is 1.5 us shorter or 1 longer for all of it together, by the run: 305.0 -> 303.5, 305.4 -> 306.5.
 
 // What happens to an fp32 accumulator on its way to Y[m, n]: + bias[n], activation,
 // * mul[m, n], + residual[m, n] (each optional), one rounding to fp16 at the end.

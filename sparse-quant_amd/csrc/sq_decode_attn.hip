@@ -38,7 +38,7 @@ __host__ __device__ constexpr int pass_rows(int D) { return DA_WAVES * (64 / (D 
 // Shares of a head's rows, at most `most`: one pass each where there are enough.  A pass costs 1 to 1.3 us after the first and
 // the meeting of the shares 2.2 us (stores, counter and loads through the level that the eight L2s share), so the rows are
 // shared only where that saves two passes.  us, by two passes' worth of rows as it was / so: 1 x 32 heads x 256 rows x 128
-// 6.7 / 5.8, x 501 8.2 / 6.9; 4 x 32 x 301 x 128 8.7 / 6.8; 8 x 12 x 501 x 64 7.5 / 6.2; 1 x 32 x 401 x 64 6.5 / 5.5.
+// 6.5 / 5.6, x 501 8.0 / 6.4; 4 x 32 x 301 x 128 8.4 / 6.5; 8 x 12 x 501 x 64 7.3 / 6.1; 1 x 32 x 401 x 64 6.5 / 5.4.
 __host__ __device__ inline int shares_of(int rows, int most, int D) {
     if (most <= 1) return 1;  // (no division in front of the first request where nothing is shared)
     const int passes = (rows + pass_rows(D) - 1) / pass_rows(D);
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     const int L = n0 + (append ? 1 : 0);  // rows attended; the appended row is row n0
     // This workgroup's share of the rows: [r0, r1).  The launch is sized for the whole cache where only the device knows the
     // length: where one workgroup takes all rows the others arrive and leave, unused shares of several are empty (64 rows of a
-    // cache of 1024, 1 x 32 heads x 128: 9.8 -> 4.0 us, 3.6 without the arrivals).
+    // cache of 1024, 1 x 32 heads x 128: 9.8 -> 4.1 us, 3.6 without the arrivals).
     const int slots = a.slots, share = blockIdx.y;
     const int nsplit = shares_of(L, slots, D);
     auto arrive = [&]() { return atomicInc((unsigned*)a.ws + blockIdx.x, (unsigned)(slots - 1)); };  // agent scope, relaxed
@@ -271,8 +271,8 @@ __global__ __launch_bounds__(64 * DA_WAVES) void decode_attn_kernel(DecodeAttnAr
     if (!last_flag) return;
     // Everything is asked for at once: four outputs of a share per thread, and in every wave lane s the state of share s
     // (unused ones count as empty).  Each thread walking over the shares for its output took a round trip per share, twice:
-    // 1 x 32 heads x 128 (us) x 2001 rows 13.9 -> 10.3, x 4001 18.2 -> 15.0; 1 x 12 x 4001 x 64 16.9 -> 8.4; with a counter that
-    // wraps instead of one that the last arriver clears 10.0, 14.8 and 8.2.
+    // 1 x 32 heads x 128 (us) x 2001 rows 13.9 -> 10.1, x 4001 18.4 -> 14.9; 1 x 12 x 4001 x 64 17.0 -> 8.3 (10.3, 15.0 and 8.4
+    // with a counter that the last arriver clears instead of one that wraps).
     // The sums run over the shares in their order: bit-reproducible.
     constexpr int QD = D / 4;
     const int sp = tid / QD, d4 = tid % QD * 4;

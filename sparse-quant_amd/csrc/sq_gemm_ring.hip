@@ -65,9 +65,10 @@ namespace {
 __device__ __forceinline__ int swz8(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 // LDS layout of a stage: activations as WK tiles [BM rows][128 bytes], weights [BN rows][32 WK bytes], zeros/scales
-// [BN columns][pairs].  The 16-byte chunks of a row are permuted (by the lane that requests them: a direct load puts
-// lane l at 16 l) so that the 128-bit operand reads, lane = row, of eight and of sixteen consecutive rows fall on
-// different banks: swz8 for rows of eight chunks, wswz for weight rows of 2 WK.
+// [BN columns][P pairs]; with SETS the stages hold none and behind them stand two buffers [BN columns][8 pairs].  The
+// 16-byte chunks of a row are permuted (by the lane that requests them: a direct load puts lane l at 16 l) so that the
+// 128-bit operand reads, lane = row, of eight and of sixteen consecutive rows fall on different banks: swz8 for rows of
+// eight chunks, wswz for weight rows of 2 WK.
 template <int WK>
 __device__ __forceinline__ int wswz(int row) {
     if constexpr (WK == 8) return row & 15;
@@ -190,14 +191,14 @@ __device__ __forceinline__ void load_to_lds_x1_masked(const void* base, uint32_t
 // SUMS: the matrix instructions see the integers q - z and the scale meets the sums of a stage (64 k of one group) in
 // fp32, as in the decode kernels at group size 128; without it they see W_hat.  Sixteen vector instructions per 64 k and
 // column tile go and sixteen per row tile come: the same count with one row tile, more with two.  Measured (us, W_hat / sums):
-// 32 tokens 12288x4096 11.96 / 12.03, 5120x13696 16.3 / 16.4; 48 tokens 12288x4096 16.4 / 16.1, 5120x13696 20.6 / 21.1;
-// 64 tokens 4096x11008 16.6 / 16.6, 15360x5120 20.4 / 21.0.  Its loop keeps the two alternating groups of waves (0..3 fetch
+// 32 tokens 12288x4096 12.5 / 12.5, 5120x13696 17.1 / 17.2; 48 tokens 12288x4096 16.9 / 16.7, 5120x13696 22.4 / 22.5;
+// 64 tokens 4096x11008 17.6 / 17.3, 12288x4096 17.9 / 17.3, 15360x5120 23.7 / 22.6.  Its loop keeps the two alternating groups of waves (0..3 fetch
 // phase p + 1 while 4..7 compute phase p): in step it would need a second set of sums, which tiles of 64 rows (222..226 registers
 // of 256) have no room for, and tiles of 32 rows are slower in step as they are.
 //
 // PAIR: silu(X W^T) * (X W2^T), both weights [N, K], in one launch: half of a tile's columns are W's and half W2's, the same
 // outputs' in the same workgroup, so that the product is formed in the store and the tiles of both fill the chip's rounds
-// together (us, two launches / one: 11008x4096 at 32 tokens 25.1 / 19.5, at 333 and group size 64 101 / 80.0; 13696x5120 at
+// together (us, two launches / one: 11008x4096 at 32 tokens 24.9 / 18.4, at 333 and group size 64 101 / 80.0; 13696x5120 at
 // 100 62.7 / 43.4; 11008x4096 at 2048 396 / 329).  Nothing is rounded between the products.
 template <int MI, int NI, int WM, int WN, int WK, int GS, int ST, bool SUMS, bool SETS, bool PAIR>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4))) void gemm_ring_kernel(
@@ -288,11 +289,13 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     }
     // A stage's own zeros/scales are 4 or 8 bytes of a row, each in a line of its own: with 32 rows per tile a third of the lines
     // that a stage asks for, and the loads come back in order.  So, where that is ahead (ring_sets), 32 bytes of a row at once, in
-    // front of the first of the ZN stages that they serve (us: 64 tokens 12288x4096 in tiles of 64 x 128 23.2 -> 21.9, 64 x 256 split
-    // in two 26.5 -> 25.4; 32 tokens 4096x11008 in tiles of 32 x 128 split in two 24.4 -> 22.7, gate and up of 11008x4096 19.4 -> 17.8).
+    // front of the first of the ZN stages that they serve (gate and up of 11008x4096 at 32 tokens: 1.52 M accesses of the L1s
+    // instead of 2.14, 0.82 M requests to the L2s instead of 1.05, the same reads from memory; us: 64 tokens 12288x4096 in tiles
+    // of 64 x 128 23.2 -> 21.9, 64 x 256 split in two 26.5 -> 25.4; 32 tokens 4096x11008 in tiles of 32 x 128 split in two 24.4 ->
+    // 22.7, gate and up of 11008x4096 19.4 -> 17.8).
     // Two buffers: set s goes out when all have read stage ZN s - ST, which is no earlier than the last one of set s - 2.  Not for
-    // the waves in step: the branch in their loop costs what it saves (100 tokens 15360x5120 in tiles of 96 x 128 32.3 -> 33.8, 200 12288x4096 in 96 x 256
-    // 34.9 -> 37.3, 333 at group size 64 41.4 -> 42.3).
+    // the waves in step: the branch in their loop costs what it saves (100 tokens 15360x5120 in tiles of 96 x 128 32.3 -> 33.8, 200
+    // 12288x4096 in 96 x 256 34.9 -> 37.3, 333 at group size 64 41.4 -> 42.3).
     auto issue_set = [&](int set) {
         const int g = ((it0 * KS) >> GS) + set * ZD;
 #pragma unroll
@@ -1011,7 +1014,8 @@ static const RingTile kRingTiles[] = {
 // best of all shapes and splits of those 1300 (1..64 tokens, one weight or gate and up): 0.5 % in the geometric mean, 5 % of them
 // more than 4.1 %.
 static const RingTile kRingSumsTiles[] = {
-    kRingTiles[0], {32, 128, 256, 1.498f, 0.706f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f}, {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f, 0.f},
+    kRingTiles[0], {32, 128, 256, 1.498f, 0.706f, 0.096f, 0.448f, 0.304f, 0.649f, 0.f},
+    {64, 128, 256, 2.615f, 0.896f, 0.244f, 0.211f, 0.515f, 0.409f, 0.f},
     kRingTiles[3], {64, 256, 128, 2.020f, 0.843f, 0.222f, 0.814f, 0.857f, 0.394f, 0.f},
 };
 static const RingTile& ring_tile(int s, int M, bool sums) {
